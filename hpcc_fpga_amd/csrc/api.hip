@@ -4,8 +4,8 @@
 // (LINPACK/src/host/execution_types/execution_pcie.hpp:53-728).  Where the
 // reference launches one single-work-item kernel per block and round-trips
 // every panel through the host, here one step of the blocked right-looking
-// factorisation is four stream-ordered launches on device-resident data:
-//   lu (diagonal block) -> prep (inverses of 32x32 diagonal sub-systems)
+// factorisation is three stream-ordered launches on device-resident data:
+//   lu (diagonal block, with the inverses of its 32x32 diagonal sub-systems)
 //   -> trsm (whole top and left strips) -> gemm (whole trailing matrix).
 #include <hip/hip_runtime.h>
 
@@ -125,8 +125,6 @@ hpl_status alloc_factor_ws(hpl_ctx* c, uint32_t B) {
     if (st) return st;
     st = ensure(c, c->dInv, c->capInv, w.inv);
     if (st) return st;
-    st = ensure(c, c->dInner, c->capInner, w.inner);
-    if (st) return st;
     st = ensure(c, c->dTinv, c->capTinv, c->strip_inverse ? w.tinv : 0);
     if (st) return st;
     st = ensure(c, c->dLpT, c->capLpT, w.lp);
@@ -230,26 +228,33 @@ hpl_status launch_update2(hpl_ctx* c, hipStream_t st, int64_t k0, UpdRegion a, U
     return HPL_SUCCESS;
 }
 
-// Factorise the B x B diagonal block at (off, off) in place.  Blocks above the
-// leaf size are split 2 x 2: LU(D11), solve D12/D21, D22 -= D21 D12, LU(D22).
-hpl_status factor_diag(hpl_ctx* c, hipStream_t st, int64_t off, uint32_t B, float* scratch) {
+// Factorise the B x B diagonal block at (off, off) in place and prepare what
+// the strip solves read: the block transposed in DT (leading dimension ldt)
+// and the inverses of its 32 x 32 sub-blocks in inv (types inv_ts apart).
+// Blocks above the leaf size are split 2 x 2: LU(D11), solve D12/D21, D22 -=
+// D21 D12, LU(D22).  The solve's transposed copy of D21, the update's operand,
+// is the part of DT above D22's, so DT and inv fill up in place.
+hpl_status factor_diag(hpl_ctx* c, hipStream_t st, int64_t off, uint32_t B, float* DT, int64_t ldt,
+                       float* inv, int64_t inv_ts) {
+    const int64_t lda = (int64_t)c->lda;
     if (B <= (uint32_t)kMaxLeafLU) {
-        HIPCHK(c, launch_lu_diag(c->dA, c->lda, off, B, c->dStatus, st));
+        // Beside an FP32 bulk update of many tiles (two workgroups of 16 waves
+        // on every CU) the 8-wave workgroup waits longer for a place than its
+        // shorter run gains: n = 32768 207.0 ms with 8 waves throughout, 201.0
+        // with 4, 200.9 with 4 while more than 6144 of the order are left; n =
+        // 2048: 1.71 ms with 8, 1.81 with 4.  The 16-bit and 8-bit updates
+        // leave room for either (n = 65536 BF16: 252.4 ms with 8, 253.5 with 4).
+        const bool narrow = c->prec == HPL_PREC_FP32 && (int64_t)c->n - off > 6144;
+        HIPCHK(c, launch_lu_diag(c->dA, lda, off, B, c->dStatus, DT, ldt, inv, inv_ts, narrow, st));
         return HPL_SUCCESS;
     }
     const uint32_t h = B / 2;
-    float* Lt = scratch;
-    float* DT = Lt + (size_t)h * h;
-    float* inv = DT + (size_t)h * h;
-    float* next = inv + 3 * (h / 32) * 1024;
-    hpl_status r = factor_diag(c, st, off, h, next);
+    hpl_status r = factor_diag(c, st, off, h, DT, ldt, inv, inv_ts);
     if (r) return r;
-    HIPCHK(c, launch_prep(c->dA, c->lda, off, h, DT, inv, st));
-    HIPCHK(c, launch_trsm(c->dA, c->lda, off, h, h, DT, inv, Lt, h, st));
-    const int64_t lda = (int64_t)c->lda;
-    HIPCHK(c, launch_gemm_update_f32(c->dA + (off + h) * lda + off + h, lda, Lt, h,
+    HIPCHK(c, launch_trsm(c->dA, lda, off, h, h, DT, ldt, inv, inv_ts, DT + h, ldt, st));
+    HIPCHK(c, launch_gemm_update_f32(c->dA + (off + h) * lda + off + h, lda, DT + h, ldt,
                                      c->dA + off * lda + off + h, lda, h, h, h, st));
-    return factor_diag(c, st, off + h, h, next);
+    return factor_diag(c, st, off + h, h, DT + h * ldt + h, ldt, inv + (h / 32) * 1024, inv_ts);
 }
 
 // Step k's buffer of diagonal-block inverses for the strip solves of the
@@ -267,11 +272,10 @@ float* step_tinv(hpl_ctx* c, int64_t k, uint32_t B) {
 hpl_status panel_diag(hpl_ctx* c, hipStream_t st, int64_t k, uint32_t B) {
     const int64_t lda = (int64_t)c->lda;
     const int64_t off = k * B;
-    hpl_status r = factor_diag(c, st, off, B, c->dInner);
-    if (r) return r;
     float* inv = c->dInv + k * (int64_t)(3 * (B / 32) * 1024);
     float* DT = c->dDT + (k & 1) * (int64_t)B * B;
-    HIPCHK(c, launch_prep(c->dA, lda, off, B, DT, inv, st));
+    hpl_status r = factor_diag(c, st, off, B, DT, B, inv, (B / 32) * 1024);
+    if (r) return r;
     // BF16: the inverses for the strip solve are the substitution's own, so
     // they go to their slot of dBInv when the factorisation fills it
     if (float* t = step_tinv(c, k, B))
@@ -310,8 +314,8 @@ hpl_status panel_strips(hpl_ctx* c, hipStream_t st, int64_t k, uint32_t B) {
         if (const float* t = step_tinv(c, k, B))
             HIPCHK(c, launch_trsm_inv(c->dA, lda, off, m, B, t, st, c->prec, lpT, lpL, B));
         else
-            HIPCHK(c, launch_trsm(c->dA, lda, off, m, B, DT, inv, Lt, n, st, c->prec, lpT, lpL,
-                                  B, scT, scL));
+            HIPCHK(c, launch_trsm(c->dA, lda, off, m, B, DT, B, inv, (B / 32) * 1024, Lt, n, st,
+                                  c->prec, lpT, lpL, B, scT, scL));
     }
     return HPL_SUCCESS;
 }
@@ -589,15 +593,6 @@ WsPlan plan_factor_ws(uint64_t n, uint32_t B, int prec, int depth, bool linear) 
     w.lt = prec == HPL_PREC_FP32 ? slots * B * n * sizeof(float) : 0;
     w.dt = 2 * (size_t)B * B * sizeof(float);
     w.inv = N * (size_t)(3 * (B / 32) * 1024) * sizeof(float);
-    w.inner = 0;
-    if (B > (uint32_t)kMaxLeafLU) {
-        // recursion scratch per level h = B/2, B/4, .., 128: Lt and DT (h x h
-        // each) and the 3 h/32 inverses of 32 x 32
-        size_t need = 0;
-        for (uint32_t h = B / 2; h >= (uint32_t)kMaxLeafLU; h /= 2)
-            need += 2 * (size_t)h * h + 3 * (h / 32) * 1024;
-        w.inner = need * sizeof(float);
-    }
     w.lp = prec == HPL_PREC_FP32 ? 0 : slots * n * B * lp_elem_bytes(prec);
     w.sc = prec == HPL_PREC_FP8 ? slots * (n / 32) * sizeof(float) : 0;
     w.status = 64;
@@ -833,7 +828,7 @@ void hpl_destroy(hpl_ctx* c) {
     if (!c->external)
         for (void* p : {(void*)c->dA, (void*)c->dA0, (void*)c->db, (void*)c->dx, (void*)c->db64,
                         (void*)c->dxt, (void*)c->dLt, (void*)c->dDT, (void*)c->dInv,
-                        (void*)c->dInner, (void*)c->dTinv, (void*)c->dStatus, (void*)c->dWork, (void*)c->dOut4,
+                        (void*)c->dTinv, (void*)c->dStatus, (void*)c->dWork, (void*)c->dOut4,
                         c->dLpT, c->dLpL, (void*)c->dScT, (void*)c->dScL, (void*)c->dX64,
                         (void*)c->dIrR, (void*)c->dIrXs, (void*)c->dIrOut, (void*)c->dRhsB,
                         (void*)c->dRhsX, (void*)c->dGmV, (void*)c->dGmW, (void*)c->dGmC,

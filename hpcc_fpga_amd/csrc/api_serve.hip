@@ -71,7 +71,6 @@ class HipExecutor : public hplserve::Executor {
             const hplx::IrPlan ir = hplx::plan_ir(np, cfg_.max_nrhs);
             k.lt = std::max(k.lt, w.lt);
             k.dt = std::max(k.dt, w.dt);
-            k.inner = std::max(k.inner, w.inner);
             k.lp = std::max(k.lp, w.lp);
             k.sc = std::max(k.sc, w.sc);
             k.work = std::max(k.work, ir.work);
@@ -80,7 +79,7 @@ class HipExecutor : public hplserve::Executor {
             k.out = std::max(k.out, ir.out);
             k.vec = std::max(k.vec, (size_t)np * cfg_.max_nrhs * sizeof(double));
         }
-        return al(k.lt) + al(k.dt) + al(k.inner) + 2 * al(k.lp) + 2 * al(k.sc) + al(k.work) +
+        return al(k.lt) + al(k.dt) + 2 * al(k.lp) + 2 * al(k.sc) + al(k.work) +
                al(k.r) + al(k.xs) + al(k.out) + 2 * al(k.vec) + al(kStatusBytes);
     }
 
@@ -99,8 +98,6 @@ class HipExecutor : public hplserve::Executor {
         c->capLt = k.lt;
         c->dDT = reinterpret_cast<float*>(take(k.dt));
         c->capDT = k.dt;
-        c->dInner = reinterpret_cast<float*>(take(k.inner));
-        c->capInner = k.inner;
         c->dLpT = take(k.lp);
         c->capLpT = k.lp;
         c->dLpL = take(k.lp);
@@ -230,7 +227,7 @@ class HipExecutor : public hplserve::Executor {
     std::vector<Slot> slots_;
     char* factor_base_ = nullptr;
     struct SlotCaps {
-        size_t lt = 0, dt = 0, inner = 0, lp = 0, sc = 0, work = 0, r = 0, xs = 0, out = 0,
+        size_t lt = 0, dt = 0, lp = 0, sc = 0, work = 0, r = 0, xs = 0, out = 0,
                vec = 0;
     } caps_;
     static constexpr size_t kStatusBytes = 64;

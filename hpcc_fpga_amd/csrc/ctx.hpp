@@ -97,8 +97,6 @@ struct hpl_ctx {
     size_t capGeslWs = 0;
     bool binv_ready = false;    // dBInv holds the inverses of the current factor
     bool binv_in_gefa = false;  // the running factorisation fills dBInv
-    float* dInner = nullptr;    // recursion scratch for blocks > 128
-    size_t capInner = 0;
     // BF16 factorisation: the current steps' diagonal-block inverses for
     // the strip solves (two buffers, step parity), and whether to use them
     // (HPL_STRIP_SOLVE=recurrence: the 32 x 32 block recurrence instead)
@@ -197,7 +195,7 @@ hpl_status init_pipeline_streams(hpl_ctx* c);
 // Device bytes of the factorisation workspaces of an n x n system at block B
 // with the given trailing-update precision and update depth.
 struct WsPlan {
-    size_t lt, dt, inner, lp, sc, status;
+    size_t lt, dt, lp, sc, status;
     size_t inv;   // per-block 32 x 32 inverses (kept with the factor)
     size_t binv;  // full diagonal-block inverses for the substitution (kept with the factor)
     size_t tinv;  // 16-bit factorisations: two steps' inverses for the strip solves

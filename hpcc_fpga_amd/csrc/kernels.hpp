@@ -4,8 +4,14 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-// diagonal-block LU (lu.hip); status[0] is raised to 1 on a zero/non-finite pivot
-hipError_t launch_lu_diag(float* A, int64_t lda, int64_t off, int B, int* status, hipStream_t s);
+// diagonal-block LU of a block of 32, 64 or 128 (lu.hip); status[0] is raised
+// to 1 on a zero/non-finite pivot.  DT (leading dimension ldt) receives the
+// factorised block transposed, and inv the inverses of its 32 x 32 diagonal
+// sub-blocks as launch_prep writes them, those of one type inv_ts floats apart
+// (a larger block's parts pass their places in its DT and inv).  narrow: 256
+// threads instead of 512, for a device that other launches fill.
+hipError_t launch_lu_diag(float* A, int64_t lda, int64_t off, int B, int* status, float* DT,
+                          int64_t ldt, float* inv, int64_t inv_ts, bool narrow, hipStream_t s);
 
 // panel solves (trsm.hip)
 hipError_t launch_prep(const float* A, int64_t lda, int64_t off, int B, float* DT, float* inv,
@@ -15,10 +21,11 @@ hipError_t launch_prep_all(const float* A, int64_t lda, int B, int nblocks, floa
 // lp_prec 0: FP32 only; 1/2: also write BF16/FP16 k-contiguous copies of the
 // top strip (lpT[c][k]) and left strip (lpL[r][k]), leading dimension ldlp;
 // 3: FP8 E4M3 copies with the scale of vectors 32 g .. 32 g + 31 at scT[g] /
-// scL[g] (vectors counted from the strip start).
+// scL[g] (vectors counted from the strip start).  lddt: leading dimension of
+// DT; inv_ts: distance of the inverses' types.
 hipError_t launch_trsm(float* A, int64_t lda, int64_t off, int64_t m, int B, const float* DT,
-                       const float* inv, float* Lt, int64_t ldt, hipStream_t s, int lp_prec = 0,
-                       void* lpT = nullptr, void* lpL = nullptr, int64_t ldlp = 0,
+                       int64_t lddt, const float* inv, int64_t inv_ts, float* Lt, int64_t ldt,
+                       hipStream_t s, int lp_prec = 0, void* lpT = nullptr, void* lpL = nullptr, int64_t ldlp = 0,
                        float* scT = nullptr, float* scL = nullptr);
 
 // Strip solves of the BF16 factorisation through the diagonal block's full

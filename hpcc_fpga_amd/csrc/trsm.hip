@@ -146,8 +146,8 @@ __global__ __launch_bounds__(64) void prep_kernel(const float* __restrict__ A, i
 // and lpL[r][k] (left strip, row r), k-contiguous with leading dimension ldlp.
 template <int B, typename LP>
 __global__ __launch_bounds__(64) void trsm_kernel(float* __restrict__ A, int64_t lda, int64_t off,
-                                                  int64_t m, const float* __restrict__ DT,
-                                                  const float* __restrict__ inv,
+                                                  int64_t m, const float* __restrict__ DT, int64_t lddt,
+                                                  const float* __restrict__ inv, int64_t inv_ts,
                                                   float* __restrict__ Lt, int64_t ldt,
                                                   int ngroups_top, LP* __restrict__ lpT,
                                                   LP* __restrict__ lpL, int64_t ldlp,
@@ -166,8 +166,8 @@ __global__ __launch_bounds__(64) void trsm_kernel(float* __restrict__ A, int64_t
     const float* D = A + off * lda + off;
     // coefficient matrix read as X[p][i]: top -> D^T, left -> D
     const float* Xc = top ? DT : D;
-    const int64_t ldx = top ? (int64_t)B : lda;
-    const float* G = inv + (top ? 0 : NQ * 1024);
+    const int64_t ldx = top ? lddt : lda;
+    const float* G = inv + (top ? 0 : inv_ts);
     float* stripT = A + off * lda + off + B;          // top strip: rows off.., cols off+B..
     float* stripL = A + (off + B) * lda + off;        // left strip: rows off+B.., cols off..
 
@@ -317,8 +317,8 @@ __global__ __launch_bounds__(64) void trsm_kernel(float* __restrict__ A, int64_t
 template <int B, typename LP>
 __global__ __launch_bounds__(64) void trsm_reg_kernel(float* __restrict__ A, int64_t lda,
                                                       int64_t off, int64_t m,
-                                                      const float* __restrict__ DT,
-                                                      const float* __restrict__ inv,
+                                                      const float* __restrict__ DT, int64_t lddt,
+                                                      const float* __restrict__ inv, int64_t inv_ts,
                                                       float* __restrict__ Lt, int64_t ldt,
                                                       int ngroups_top, LP* __restrict__ lpT,
                                                       LP* __restrict__ lpL, int64_t ldlp,
@@ -334,8 +334,8 @@ __global__ __launch_bounds__(64) void trsm_reg_kernel(float* __restrict__ A, int
     const int64_t v0 = (int64_t)(top ? blockIdx.x : blockIdx.x - ngroups_top) * 32;
     const float* D = A + off * lda + off;
     const float* Xc = top ? DT : D;  // coefficients read as X[p][i]
-    const int64_t ldx = top ? (int64_t)B : lda;
-    const float* G = inv + (top ? 0 : NQ * 1024);
+    const int64_t ldx = top ? lddt : lda;
+    const float* G = inv + (top ? 0 : inv_ts);
     float* stripT = A + off * lda + off + B;
     float* stripL = A + (off + B) * lda + off;
 
@@ -711,15 +711,15 @@ hipError_t launch_prep_all(const float* A, int64_t lda, int B, int nblocks, floa
 
 template <typename LP>
 static hipError_t launch_trsm_t(float* A, int64_t lda, int64_t off, int64_t m, int B,
-                                const float* DT, const float* inv, float* Lt, int64_t ldt,
-                                LP* lpT, LP* lpL, int64_t ldlp, hipStream_t s,
+                                const float* DT, int64_t lddt, const float* inv, int64_t inv_ts,
+                                float* Lt, int64_t ldt, LP* lpT, LP* lpL, int64_t ldlp, hipStream_t s,
                                 float* scT = nullptr, float* scL = nullptr) {
     const int groups = (int)(m / 32);
     dim3 grid(2 * groups);
 #define HPL_TRSM_CASE(BB, KERNEL)                                                             \
     case BB:                                                                                  \
-        KERNEL<BB, LP><<<grid, 64, 0, s>>>(A, lda, off, m, DT, inv, Lt, ldt, groups, lpT, lpL,  \
-                                           ldlp, scT, scL);                                   \
+        KERNEL<BB, LP><<<grid, 64, 0, s>>>(A, lda, off, m, DT, lddt, inv, inv_ts, Lt, ldt, groups, \
+                                           lpT, lpL, ldlp, scT, scL);                         \
         break;
     switch (B) {
         HPL_TRSM_CASE(32, trsm_reg_kernel)
@@ -740,8 +740,9 @@ hipError_t launch_trsm_top(float* A, int64_t lda, int64_t off, int64_t m, int B,
     const int groups = (int)(m / 32);
 #define HPL_TRSM_TOP(BB)                                                                      \
     case BB:                                                                                  \
-        trsm_reg_kernel<BB, float><<<groups, 64, 0, s>>>(A, lda, off, m, DT, inv, nullptr, 0, \
-                                                         groups, nullptr, nullptr, 0, nullptr, \
+        trsm_reg_kernel<BB, float><<<groups, 64, 0, s>>>(A, lda, off, m, DT, BB, inv,         \
+                                                         (BB / 32) * 1024, nullptr, 0, groups, \
+                                                         nullptr, nullptr, 0, nullptr,        \
                                                          nullptr);                            \
         break;
     switch (B) {
@@ -756,24 +757,24 @@ hipError_t launch_trsm_top(float* A, int64_t lda, int64_t off, int64_t m, int B,
 }
 
 hipError_t launch_trsm(float* A, int64_t lda, int64_t off, int64_t m, int B, const float* DT,
-                       const float* inv, float* Lt, int64_t ldt, hipStream_t s, int lp_prec,
+                       int64_t lddt, const float* inv, int64_t inv_ts, float* Lt, int64_t ldt, hipStream_t s, int lp_prec,
                        void* lpT, void* lpL, int64_t ldlp, float* scT, float* scL) {
     if (m <= 0) return hipSuccess;
     if (m % 32) return hipErrorInvalidValue;
     switch (lp_prec) {
         case 0:
-            return launch_trsm_t<float>(A, lda, off, m, B, DT, inv, Lt, ldt, nullptr, nullptr, 0, s);
+            return launch_trsm_t<float>(A, lda, off, m, B, DT, lddt, inv, inv_ts, Lt, ldt, nullptr, nullptr, 0, s);
         case 1:
-            return launch_trsm_t<__bf16>(A, lda, off, m, B, DT, inv, Lt, ldt,
+            return launch_trsm_t<__bf16>(A, lda, off, m, B, DT, lddt, inv, inv_ts, Lt, ldt,
                                          static_cast<__bf16*>(lpT), static_cast<__bf16*>(lpL),
                                          ldlp, s);
         case 2:
-            return launch_trsm_t<_Float16>(A, lda, off, m, B, DT, inv, Lt, ldt,
+            return launch_trsm_t<_Float16>(A, lda, off, m, B, DT, lddt, inv, inv_ts, Lt, ldt,
                                            static_cast<_Float16*>(lpT),
                                            static_cast<_Float16*>(lpL), ldlp, s);
         case 3:
             if (!scT || !scL || ldlp % 16) return hipErrorInvalidValue;
-            return launch_trsm_t<fp8e4m3>(A, lda, off, m, B, DT, inv, Lt, ldt,
+            return launch_trsm_t<fp8e4m3>(A, lda, off, m, B, DT, lddt, inv, inv_ts, Lt, ldt,
                                           static_cast<fp8e4m3*>(lpT), static_cast<fp8e4m3*>(lpL),
                                           ldlp, s, scT, scL);
         default:
