@@ -424,6 +424,26 @@ hipError_t binv_range(hpl_ctx* c, hipStream_t st, int64_t k0, int64_t k1, uint32
                                 c->dInv + k0 * is, is, c->dBInv + k0 * 2 * (int64_t)B * B, st);
 }
 
+// The last blocks, k0 and on, one launch after the other on s0: the pending
+// steps p0 .. k0 - 1 on the whole trailing matrix, then per block its panel
+// and the whole trailing update by that one step.
+hpl_status gefa_serial(hpl_ctx* c, uint32_t B, int64_t k0, int64_t p0) {
+    const int64_t n = (int64_t)c->n, N = n / B;
+    int64_t from = p0;
+    for (int64_t k = k0; k < N; ++k) {
+        const int64_t kb = k * B;
+        hpl_status r = HPL_SUCCESS;
+        if (k > from)
+            r = launch_update(c, c->s0, from, kb, kb, (int)(n - kb), (int)(n - kb),
+                              (int)((k - from) * B), B);
+        if (!r) r = panel(c, c->s0, k, B);
+        if (r) return r;
+        from = k;
+    }
+    if (c->binv_in_gefa && !step_tinv(c, p0, B)) HIPCHK(c, binv_range(c, c->s0, p0, N, B));
+    return HPL_SUCCESS;
+}
+
 hpl_status gefa_pipelined(hpl_ctx* c, uint32_t B) {
     hpl_status r = hplx::init_pipeline_streams(c);
     if (r) return r;
@@ -434,6 +454,8 @@ hpl_status gefa_pipelined(hpl_ctx* c, uint32_t B) {
                            c->prec == HPL_PREC_BF16 || c->prec == HPL_PREC_FP16);
     const int64_t G = (int64_t)bnd.size() - 1;
     for (int64_t g = 0; g < G; ++g) {
+        if (n - bnd[g] * (int64_t)B <= c->serial_m)
+            return gefa_serial(c, B, bnd[g], g ? bnd[g - 1] : bnd[g]);
         const int64_t s = bnd[g + 1] * (int64_t)B;
         const bool wide = (c->prec == HPL_PREC_BF16 || c->prec == HPL_PREC_FP16) &&
                           (n - s) % 256 == 0;
@@ -803,6 +825,7 @@ hpl_status hpl_create(int device, hpl_ctx** out) {
         hipSuccess)
         c->num_cu = 0;
     if (const char* e = getenv("HPL_TAIL_M")) c->tail_m = std::max(0LL, atoll(e));
+    if (const char* e = getenv("HPL_SERIAL_M")) c->serial_m = std::max(0LL, atoll(e));
     if (const char* e = getenv("HPL_HEAD_M")) c->head_m = std::max(0LL, atoll(e));
     if (const char* e = getenv("HPL_HEAD_DEPTH")) c->head_depth = std::max(0, std::min(32, atoi(e)));
     if (const char* e = getenv("HPL_TAIL_DEPTH")) c->tail_depth = std::max(0, std::min(32, atoi(e)));

@@ -49,6 +49,16 @@ struct hpl_ctx {
     // 65536 BF16 320 ms against 324.5.
     int64_t tail_m = -1;
     int tail_depth = 0;
+    // End of the pipelined schedule: once the order still to factorise is at
+    // most serial_m (HPL_SERIAL_M), one launch after the other on one stream.
+    // A step's whole trailing update is then a few microseconds, less than the
+    // fork and join of the streams that would hide it (a wait on another
+    // stream's event costs 6-25 us, a launch on the same stream about 1): n =
+    // 2048 block 128 1.49 ms without, 1.34 from order 1024, 1.23 from 2048,
+    // 1.24 from 4096; n = 7488 block 64 8.94, 8.62, 7.63, 7.48 (7.90 from
+    // 6144); FP8 GMRES n = 6144 6.55, 6.44, 6.19, 5.42 (5.71); n = 32768 FP32
+    // and n = 65536 BF16 the same within 0.3%.
+    int64_t serial_m = 4096;
     // Head of the pipelined schedule for the BF16/FP16 update: while the order
     // still to factorise exceeds head_m (-1: 5n/8; 0: no head), groups hold
     // head_depth steps (0: 5/4 of the depth).  There the chain of a group
