@@ -726,6 +726,9 @@ hpl_status ir_solve(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_
     const GeslWs* ws = nrhs == 1 ? gesl_workspace(c, &wsbuf) : nullptr;
     const int B = (int)c->B;
     const int64_t inv_stride = 3 * (B / 32) * 1024;
+    // the substitution of several columns: between two residuals, whose
+    // partial sums (at least n (nrhs + 1) doubles) it overwrites
+    float* scratch = reinterpret_cast<float*>(c->dWork);
     double sc_in[16], sc_out[16], h[64];
     int iters[16];
     for (int j = 0; j < nrhs; ++j) {
@@ -736,7 +739,7 @@ hpl_status ir_solve(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_
     const int* perm = c->pivoted ? c->dPerm : nullptr;
     HIPCHK(c, launch_d2f_multi(dB, n, c->dIrXs, n, n, nrhs, sc_in, c->s0, perm));
     HIPCHK(c, launch_gesl_multi(c->dA, (int64_t)c->lda, n, B, c->dInv, inv_stride, c->dIrXs, n,
-                                nrhs, c->s0, c->binv_ready ? c->dBInv : nullptr, ws));
+                                nrhs, c->s0, c->binv_ready ? c->dBInv : nullptr, ws, scratch));
     HIPCHK(c, launch_axpy_multi(dX, n, c->dIrXs, n, n, nrhs, sc_out, 1, c->s0));
     for (int it = 0;; ++it) {
         HIPCHK(c, launch_residual_multi(c->dA0, (int64_t)c->lda, n, dX, n, dB, n, nrhs, c->dWork,
@@ -770,7 +773,8 @@ hpl_status ir_solve(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_
         // columns get scale 0 and stay unchanged)
         HIPCHK(c, launch_d2f_multi(c->dIrR, n, c->dIrXs, n, n, nrhs, sc_in, c->s0, perm));
         HIPCHK(c, launch_gesl_multi(c->dA, (int64_t)c->lda, n, B, c->dInv, inv_stride, c->dIrXs,
-                                    n, nrhs, c->s0, c->binv_ready ? c->dBInv : nullptr, ws));
+                                    n, nrhs, c->s0, c->binv_ready ? c->dBInv : nullptr, ws,
+                                    scratch));
         HIPCHK(c, launch_axpy_multi(dX, n, c->dIrXs, n, n, nrhs, sc_out, 0, c->s0));
     }
     st = gesl_check(c, ws);

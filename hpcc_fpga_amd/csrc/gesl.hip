@@ -17,7 +17,8 @@
 // of solved rows is a dot product spread over the workgroup, and the 32 x 32
 // triangular system is applied as its inverse (computed by the panel prep);
 // with the full inverses of the diagonal blocks (launch_block_inverse, B <=
-// 256) the diagonal solve is instead one coalesced GEMV.
+// 256) the diagonal solve is instead one coalesced GEMV (one right-hand side)
+// or a matrix product (several, below).
 //
 // Right-hand sides: column r of X at X + r * ldx.  NR is the compile-time
 // capacity (1, 4, 16), nr <= NR the count in use.
@@ -173,27 +174,6 @@ __device__ void diag_solve(const float* __restrict__ A, int64_t lda, int64_t Qof
     }
 }
 
-// Diagonal block at Qoff with its full inverse: X[Qoff..Qoff+B) := W^T z,
-// z the current entries, W[p][i] the stored inverse (SIGN -1: negated).
-template <int NR, int SIGN>
-__device__ void diag_apply(const float* __restrict__ W, int64_t Qoff, int B, float* __restrict__ X,
-                           int64_t ldx, int nr, float* zbuf, float* red) {
-    constexpr int MAXB = gesl_cfg<NR>::MAXB;
-    const int t = threadIdx.x;
-    if (NR == 1) nr = 1;
-    for (int idx = t; idx < nr * B; idx += NT) {
-        const int r = idx / B, e = idx % B;
-        zbuf[r * MAXB + e] = X[r * ldx + Qoff + e];
-        X[r * ldx + Qoff + e] = 0.0f;
-    }
-    __syncthreads();
-    for (int e0 = 0; e0 < B; e0 += kDiagPass) {
-        const int ncols = min(kDiagPass, B - e0) / 4;
-        block_gemv<NR, SIGN>(W, B, 0, Qoff + e0, ncols, B, zbuf, MAXB, nr, red, Qoff + B, X, ldx,
-                             Qoff);
-    }
-}
-
 template <int NR>
 struct gesl_smem {
     float ybuf[NR * gesl_cfg<NR>::MAXB];  // diagonal system being solved
@@ -209,7 +189,6 @@ __global__ __launch_bounds__(NT) void gesl_fwd_kernel(const float* __restrict__ 
                                                       int64_t n, int B, int q,
                                                       const float* __restrict__ inv,
                                                       int64_t inv_stride,
-                                                      const float* __restrict__ binv,
                                                       float* __restrict__ X, int64_t ldx, int nr) {
     constexpr int MAXB = gesl_cfg<NR>::MAXB, CH = gesl_cfg<NR>::CH;
     __shared__ gesl_smem<NR> sm;
@@ -234,12 +213,8 @@ __global__ __launch_bounds__(NT) void gesl_fwd_kernel(const float* __restrict__ 
             }
             __syncthreads();
         }
-        if (binv)
-            diag_apply<NR, 1>(binv + (int64_t)(q + 1) * 2 * B * B, Q, B, X, ldx, nr, sm.ybuf,
-                              sm.red);
-        else
-            diag_solve<NR, true>(A, lda, Q, B, inv + (int64_t)(q + 1) * inv_stride + NQ * 1024, X,
-                                 ldx, nr, sm.ybuf, sm.part, sm.zbuf);
+        diag_solve<NR, true>(A, lda, Q, B, inv + (int64_t)(q + 1) * inv_stride + NQ * 1024, X, ldx,
+                             nr, sm.ybuf, sm.part, sm.zbuf);
         return;
     }
     // entries [(q+2)B, n) in chunks of CH
@@ -253,7 +228,6 @@ __global__ __launch_bounds__(NT) void gesl_bwd_kernel(const float* __restrict__ 
                                                       int B, int q, int N,
                                                       const float* __restrict__ inv,
                                                       int64_t inv_stride,
-                                                      const float* __restrict__ binv,
                                                       float* __restrict__ X, int64_t ldx, int nr) {
     constexpr int MAXB = gesl_cfg<NR>::MAXB, CH = gesl_cfg<NR>::CH;
     __shared__ gesl_smem<NR> sm;
@@ -277,12 +251,8 @@ __global__ __launch_bounds__(NT) void gesl_bwd_kernel(const float* __restrict__ 
             }
             __syncthreads();
         }
-        if (binv)
-            diag_apply<NR, -1>(binv + (int64_t)(q - 1) * 2 * B * B + (int64_t)B * B, Q, B, X, ldx,
-                               nr, sm.ybuf, sm.red);
-        else
-            diag_solve<NR, false>(A, lda, Q, B, inv + (int64_t)(q - 1) * inv_stride + 2 * NQ * 1024,
-                                  X, ldx, nr, sm.ybuf, sm.part, sm.zbuf);
+        diag_solve<NR, false>(A, lda, Q, B, inv + (int64_t)(q - 1) * inv_stride + 2 * NQ * 1024, X,
+                              ldx, nr, sm.ybuf, sm.part, sm.zbuf);
         return;
     }
     // entries [0, (q-1)B)
@@ -293,21 +263,19 @@ __global__ __launch_bounds__(NT) void gesl_bwd_kernel(const float* __restrict__ 
 
 template <int NR>
 hipError_t gesl_sweeps(const float* A, int64_t lda, int64_t n, int B, const float* inv,
-                       int64_t inv_stride, const float* binv, float* X, int64_t ldx, int nr,
-                       hipStream_t s) {
+                       int64_t inv_stride, float* X, int64_t ldx, int nr, hipStream_t s) {
     constexpr int CH = gesl_cfg<NR>::CH;
     if (B > gesl_cfg<NR>::MAXB) return hipErrorInvalidValue;
     const int N = (int)(n / B);
     for (int q = -1; q <= N - 2; ++q) {
         const int64_t rest = n - (int64_t)(q + 2) * B;
         const int grid = 1 + (q >= 0 ? (int)((rest + CH - 1) / CH) : 0);
-        gesl_fwd_kernel<NR><<<grid, NT, 0, s>>>(A, lda, n, B, q, inv, inv_stride, binv, X, ldx, nr);
+        gesl_fwd_kernel<NR><<<grid, NT, 0, s>>>(A, lda, n, B, q, inv, inv_stride, X, ldx, nr);
     }
     for (int q = N; q >= 1; --q) {
         const int64_t rest = (int64_t)(q - 1) * B;
         const int grid = 1 + (q < N ? (int)((rest + CH - 1) / CH) : 0);
-        gesl_bwd_kernel<NR><<<grid, NT, 0, s>>>(A, lda, B, q, N, inv, inv_stride, binv, X, ldx,
-                                                nr);
+        gesl_bwd_kernel<NR><<<grid, NT, 0, s>>>(A, lda, B, q, N, inv, inv_stride, X, ldx, nr);
     }
     return hipGetLastError();
 }
@@ -402,6 +370,107 @@ hipError_t gesl_sweeps_split(const float* A, int64_t lda, int64_t n, int B, cons
         gesl_apply1_kernel<-1><<<(int)((e1 + CH - 1) / CH), NT, 0, s>>>(A, lda, B, e1, 0, e1, X);
         gesl_diag1_kernel<-1><<<1, NTD, 0, s>>>(binv + (int64_t)(q - 1) * 2 * BB + BB, B,
                                                 (int64_t)(q - 1) * B, X);
+    }
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Several right-hand sides with full diagonal-block inverses: every step is a
+// product of a B-row strip (of the factor, or of a block's inverse) with the
+// B x nr block of solved vectors, on v_mfma_f32_16x16x4_f32 with 16 entries
+// as its rows and the right-hand sides as its columns.  A workgroup takes 32
+// entries and splits the B rows over its waves, so every load of a wave is in
+// flight before its first product; the waves' sums are added in wave order.
+// Two launches per block step: the update of all further entries by block q,
+// then block q + 1's product with its inverse (on B / 32 workgroups).  The
+// solved vectors go to a second array (a block's product reads the whole
+// block), the forward sweep from X to Y and the backward sweep from Y to X.
+// Bound: the chain of 4 n / B launches, about 4 us each.  n = 4096, B = 256,
+// 16 right-hand sides: one workgroup per block step doing the dependent
+// products on vector instructions took 156 us a step, 10 ms for the two
+// solves of a refinement; solve_rhs64 as a whole 12.17 -> 1.57 ms.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// out[r][e] := (ASSIGN ? 0 : out[r][e]) + SIGN sum_{p < B} W[p * ldw + e] v[r][p]
+// for the 32 entries e of workgroup blockIdx.x, r < nr <= 16
+template <int SIGN, bool ASSIGN>
+__global__ __launch_bounds__(NT) void gesl_mrhs_kernel(const float* __restrict__ W, int64_t ldw,
+                                                       int B, const float* __restrict__ v,
+                                                       float* __restrict__ out, int64_t ldx,
+                                                       int nr) {
+    __shared__ float red[4][16][33];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int c = lane & 15, kk = lane >> 4;
+    const int waves = min(4, B / 16), rows = B / waves;  // 16, 32 or 64 rows per wave
+    const int64_t e0 = (int64_t)blockIdx.x * 32;
+    if (wave < waves) {
+        // lane group kk takes rows 16 j + 4 kk + s of the wave's, s = 0..3
+        const int k0 = wave * rows + 4 * kk;
+        const float* w = W + (int64_t)k0 * ldw + e0 + c;
+        const float* y = v + (int64_t)c * ldx + k0;
+        f32x4 yv[4];
+        float a0[4][4], a1[4][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (16 * j < rows) {
+                yv[j] = c < nr ? *reinterpret_cast<const f32x4*>(y + 16 * j) : f32x4{0, 0, 0, 0};
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    a0[j][s] = w[(int64_t)(16 * j + s) * ldw];
+                    a1[j][s] = w[(int64_t)(16 * j + s) * ldw + 16];
+                }
+            }
+        }
+        f32x4 d0 = {0, 0, 0, 0}, d1 = {0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (16 * j < rows) {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    d0 = mfma16(a0[j][s], yv[j][s], d0);
+                    d1 = mfma16(a1[j][s], yv[j][s], d1);
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            red[wave][c][4 * kk + i] = d0[i];
+            red[wave][c][16 + 4 * kk + i] = d1[i];
+        }
+    }
+    __syncthreads();
+    for (int r = t >> 5; r < nr; r += NT / 32) {
+        const int e = t & 31;
+        float sum = red[0][r][e];
+        for (int g = 1; g < waves; ++g) sum += red[g][r][e];
+        float* o = out + (int64_t)r * ldx + e0 + e;
+        *o = ASSIGN ? SIGN * sum : *o + SIGN * sum;
+    }
+}
+
+hipError_t gesl_sweeps_mrhs(const float* A, int64_t lda, int64_t n, int B, const float* binv,
+                            float* X, float* Y, int64_t ldx, int nr, hipStream_t s) {
+    const int N = (int)(n / B);
+    const int64_t BB = (int64_t)B * B;
+    const unsigned gb = (unsigned)(B / 32);
+    gesl_mrhs_kernel<1, true><<<gb, NT, 0, s>>>(binv, B, B, X, Y, ldx, nr);
+    for (int q = 0; q + 1 < N; ++q) {
+        const int64_t q0 = (int64_t)q * B, e0 = q0 + B;
+        gesl_mrhs_kernel<1, false><<<(unsigned)((n - e0) / 32), NT, 0, s>>>(
+            A + q0 * lda + e0, lda, B, Y + q0, X + e0, ldx, nr);
+        gesl_mrhs_kernel<1, true><<<gb, NT, 0, s>>>(binv + (int64_t)(q + 1) * 2 * BB, B, B, X + e0,
+                                                    Y + e0, ldx, nr);
+    }
+    for (int q = N - 1; q >= 0; --q) {
+        const int64_t q0 = (int64_t)q * B;
+        gesl_mrhs_kernel<-1, true><<<gb, NT, 0, s>>>(binv + (int64_t)q * 2 * BB + BB, B, B, Y + q0,
+                                                     X + q0, ldx, nr);
+        if (q)
+            gesl_mrhs_kernel<-1, false><<<(unsigned)(q0 / 32), NT, 0, s>>>(A + q0 * lda, lda, B,
+                                                                           X + q0, Y, ldx, nr);
     }
     return hipGetLastError();
 }
@@ -668,8 +737,8 @@ hipError_t gesl_persist(const float* A, int64_t lda, int64_t n, int B, const flo
 
 hipError_t launch_gesl_multi(const float* A, int64_t lda, int64_t n, int B, const float* inv,
                              int64_t inv_stride, float* X, int64_t ldx, int nrhs, hipStream_t s,
-                             const float* binv, const GeslWs* ws) {
-    if (B > 512 || B < 32 || B % 32 || n % B || nrhs < 1 || (nrhs > 1 && (ldx < n || ldx % 4)))
+                             const float* binv, const GeslWs* ws, float* scratch) {
+    if (B > 512 || B < 32 || B % 32 || n % B || nrhs < 1 || (nrhs > 1 && (ldx < n || ldx % 4 || (binv && !scratch))))
         return hipErrorInvalidValue;
     for (int r0 = 0; r0 < nrhs; r0 += 16) {
         const int nr = std::min(16, nrhs - r0);
@@ -681,11 +750,13 @@ hipError_t launch_gesl_multi(const float* A, int64_t lda, int64_t n, int B, cons
         else if (nr == 1 && binv && B <= 256)
             e = gesl_sweeps_split(A, lda, n, B, binv, Xr, s);
         else if (nr == 1)
-            e = gesl_sweeps<1>(A, lda, n, B, inv, inv_stride, binv, Xr, ldx, 1, s);
+            e = gesl_sweeps<1>(A, lda, n, B, inv, inv_stride, Xr, ldx, 1, s);
+        else if (binv && B <= 256)
+            e = gesl_sweeps_mrhs(A, lda, n, B, binv, Xr, scratch, ldx, nr, s);
         else if (nr <= 4)
-            e = gesl_sweeps<4>(A, lda, n, B, inv, inv_stride, binv, Xr, ldx, nr, s);
+            e = gesl_sweeps<4>(A, lda, n, B, inv, inv_stride, Xr, ldx, nr, s);
         else
-            e = gesl_sweeps<16>(A, lda, n, B, inv, inv_stride, binv, Xr, ldx, nr, s);
+            e = gesl_sweeps<16>(A, lda, n, B, inv, inv_stride, Xr, ldx, nr, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

@@ -118,10 +118,12 @@ hipError_t launch_gesl(const float* A, int64_t lda, int64_t n, int B, const floa
                        int64_t inv_stride, float* x, hipStream_t s, const float* binv = nullptr,
                        const GeslWs* ws = nullptr);
 // nrhs right-hand sides, column r at X + r * ldx (ldx a multiple of 4, >= n);
-// blocks up to 256 for more than 4 right-hand sides
+// blocks up to 256 for more than 4 right-hand sides.  Several right-hand
+// sides with binv need scratch: nrhs columns of the same leading dimension.
 hipError_t launch_gesl_multi(const float* A, int64_t lda, int64_t n, int B, const float* inv,
                              int64_t inv_stride, float* X, int64_t ldx, int nrhs, hipStream_t s,
-                             const float* binv = nullptr, const GeslWs* ws = nullptr);
+                             const float* binv = nullptr, const GeslWs* ws = nullptr,
+                             float* scratch = nullptr);
 
 // partial pivoting (pivot.hip); X is the transposed matrix X[i][j] = M(i, j)
 hipError_t launch_transpose_square(float* A, int64_t ld, int64_t n, hipStream_t s);
