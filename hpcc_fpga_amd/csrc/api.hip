@@ -560,8 +560,7 @@ hpl_status gefa_pipelined(hpl_ctx* c, uint32_t B) {
 
 hpl_status check_status(hpl_ctx* c) {
     int h = 0;
-    HIPCHK(c, hipMemcpyAsync(&h, c->dStatus, sizeof(int), hipMemcpyDeviceToHost, c->s0));
-    HIPCHK(c, hipStreamSynchronize(c->s0));
+    HIPCHK(c, c->stage.to_host(c->s0, &h, c->dStatus, sizeof(int)));
     if (h & 2)
         return fail(c, HPL_ERR_HIP,
                     "pivot panel: a grid barrier timed out (workgroups not co-resident)");
@@ -665,8 +664,7 @@ const GeslWs* gesl_workspace(hpl_ctx* c, GeslWs* ws) {
 hpl_status gesl_check(hpl_ctx* c, const GeslWs* ws) {
     if (!ws) return HPL_SUCCESS;
     int h = 0;
-    HIPCHK(c, hipMemcpyAsync(&h, ws->status, sizeof(int), hipMemcpyDeviceToHost, c->s0));
-    HIPCHK(c, hipStreamSynchronize(c->s0));
+    HIPCHK(c, c->stage.to_host(c->s0, &h, ws->status, sizeof(int)));
     if (h & 2)
         return fail(c, HPL_ERR_HIP,
                     "substitution: a bounded wait gave up (workgroups not co-resident)");
@@ -744,9 +742,7 @@ hpl_status ir_solve(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_
     for (int it = 0;; ++it) {
         HIPCHK(c, launch_residual_multi(c->dA0, (int64_t)c->lda, n, dX, n, dB, n, nrhs, c->dWork,
                                         c->dIrR, n, c->dIrOut, c->s0));
-        HIPCHK(c, hipMemcpyAsync(h, c->dIrOut, 4 * nrhs * sizeof(double), hipMemcpyDeviceToHost,
-                                 c->s0));
-        HIPCHK(c, hipStreamSynchronize(c->s0));
+        HIPCHK(c, c->stage.to_host(c->s0, h, c->dIrOut, 4 * nrhs * sizeof(double)));
         bool any = false;
         for (int j = 0; j < nrhs; ++j) {
             const double* hj = h + 4 * j;
@@ -904,10 +900,10 @@ hpl_status hpl_upload(hpl_ctx* c, const float* a, uint64_t n, uint64_t lda, cons
     hpl_status st = alloc_system(c, n);
     if (st) return st;
     HIPCHK(c, hipEventRecord(c->e0, c->s0));
-    HIPCHK(c, hipMemcpy2DAsync(c->dA, c->lda * sizeof(float), a, lda * sizeof(float),
-                               n * sizeof(float), n, hipMemcpyHostToDevice, c->s0));
+    HIPCHK(c, c->stage.to_device(c->s0, c->dA, c->lda * sizeof(float), a, lda * sizeof(float),
+                                 n * sizeof(float), n));
     if (b)
-        HIPCHK(c, hipMemcpyAsync(c->db, b, n * sizeof(float), hipMemcpyHostToDevice, c->s0));
+        HIPCHK(c, c->stage.to_device(c->s0, c->db, b, n * sizeof(float)));
     else
         HIPCHK(c, hipMemsetAsync(c->db, 0, n * sizeof(float), c->s0));
     if (c->keep_orig) {
@@ -992,9 +988,8 @@ hpl_status hpl_gefa_dev(hpl_ctx* c, uint32_t block, hpl_prec prec, hpl_timing* t
                         : gefa_schedule(c, block);
     if (st) return st;
     HIPCHK(c, hipEventRecord(c->e1, c->s0));
-    HIPCHK(c, hipStreamSynchronize(c->s0));
+    st = check_status(c);  // waits for the stream
     if (t) t->gefa_s = elapsed_s(c);
-    st = check_status(c);
     if (st) return st;
     c->B = block;
     c->factored = true;
@@ -1021,9 +1016,10 @@ hpl_status hpl_gesl_dev(hpl_ctx* c, hpl_timing* t) {
                           3 * (c->B / 32) * 1024, c->dx, c->s0, c->binv_ready ? c->dBInv : nullptr,
                           ws));
     HIPCHK(c, hipEventRecord(c->e1, c->s0));
-    HIPCHK(c, hipStreamSynchronize(c->s0));
+    st = hplx::gesl_check(c, ws);  // waits for the stream where there is a status
+    if (!ws) HIPCHK(c, hipStreamSynchronize(c->s0));
     if (t) t->gesl_s = elapsed_s(c);
-    return hplx::gesl_check(c, ws);
+    return st;
 }
 
 hpl_status hpl_download(hpl_ctx* c, float* a, uint64_t lda, float* x, hpl_timing* t) {
@@ -1033,9 +1029,9 @@ hpl_status hpl_download(hpl_ctx* c, float* a, uint64_t lda, float* x, hpl_timing
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, hipEventRecord(c->e0, c->s0));
     if (a)
-        HIPCHK(c, hipMemcpy2DAsync(a, lda * sizeof(float), c->dA, c->lda * sizeof(float),
-                                   c->n * sizeof(float), c->n, hipMemcpyDeviceToHost, c->s0));
-    if (x) HIPCHK(c, hipMemcpyAsync(x, c->dx, c->n * sizeof(float), hipMemcpyDeviceToHost, c->s0));
+        HIPCHK(c, c->stage.to_host(c->s0, a, lda * sizeof(float), c->dA, c->lda * sizeof(float),
+                                   c->n * sizeof(float), c->n));
+    if (x) HIPCHK(c, c->stage.to_host(c->s0, x, c->dx, c->n * sizeof(float)));
     HIPCHK(c, hipEventRecord(c->e1, c->s0));
     HIPCHK(c, hipStreamSynchronize(c->s0));
     if (t) t->d2h_s = elapsed_s(c);
@@ -1048,12 +1044,9 @@ hpl_status hpl_download_vectors(hpl_ctx* c, float* b, double* b64, double* xtrue
     if (!c->dA) return fail(c, HPL_ERR_STATE, "no resident system");
     HIPCHK(c, hipSetDevice(c->device));
     const size_t n = c->n;
-    if (b) HIPCHK(c, hipMemcpyAsync(b, c->db, n * sizeof(float), hipMemcpyDeviceToHost, c->s0));
-    if (b64)
-        HIPCHK(c, hipMemcpyAsync(b64, c->db64, n * sizeof(double), hipMemcpyDeviceToHost, c->s0));
-    if (xtrue)
-        HIPCHK(c, hipMemcpyAsync(xtrue, c->dxt, n * sizeof(double), hipMemcpyDeviceToHost, c->s0));
-    HIPCHK(c, hipStreamSynchronize(c->s0));
+    if (b) HIPCHK(c, c->stage.to_host(c->s0, b, c->db, n * sizeof(float)));
+    if (b64) HIPCHK(c, c->stage.to_host(c->s0, b64, c->db64, n * sizeof(double)));
+    if (xtrue) HIPCHK(c, c->stage.to_host(c->s0, xtrue, c->dxt, n * sizeof(double)));
     return HPL_SUCCESS;
 }
 
@@ -1095,7 +1088,7 @@ hpl_status hpl_gesl(hpl_ctx* c, const float* lu, float* b, uint64_t n, uint64_t 
     c->binv_ready = false;
     st = hpl_gesl_dev(c, t);
     if (st) return st;
-    HIPCHK(c, hipMemcpy(b, c->dx, n * sizeof(float), hipMemcpyDeviceToHost));
+    HIPCHK(c, c->stage.to_host(c->s0, b, c->dx, n * sizeof(float)));
     return HPL_SUCCESS;
 }
 
@@ -1113,8 +1106,7 @@ hpl_status hpl_residual(hpl_ctx* c, double out[4]) {
     }
     HIPCHK(c, launch_residual_f32x(c->dA0, (int64_t)c->lda, n, c->dx, c->db, c->dWork, nullptr,
                                    c->dOut4, c->s0));
-    HIPCHK(c, hipMemcpyAsync(out, c->dOut4, 4 * sizeof(double), hipMemcpyDeviceToHost, c->s0));
-    HIPCHK(c, hipStreamSynchronize(c->s0));
+    HIPCHK(c, c->stage.to_host(c->s0, out, c->dOut4, 4 * sizeof(double)));
     return HPL_SUCCESS;
 }
 
@@ -1252,15 +1244,14 @@ hpl_status hpl_solve_gmres(hpl_ctx* c, uint32_t block, hpl_prec prec, int restar
     st = precond_apply(c, c->db64, c->dX64);
     if (st) return st;
     std::vector<double> H((size_t)(m + 1) * m), cs(m), sn(m), g(m + 1), h1(m + 1), h2(m + 1),
-        y(m);
+        y(m), coef(2 * m + 2);
     double hres[4];
     int inner_total = 0, outer = 0;
     double berr = 0.0;
     for (;; ++outer) {
         HIPCHK(c, launch_residual_multi(c->dA0, (int64_t)c->lda, n, c->dX64, n, c->db64, n, 1,
                                         c->dWork, c->dIrR, n, c->dIrOut, c->s0));
-        HIPCHK(c, hipMemcpyAsync(hres, c->dIrOut, sizeof hres, hipMemcpyDeviceToHost, c->s0));
-        HIPCHK(c, hipStreamSynchronize(c->s0));
+        HIPCHK(c, c->stage.to_host(c->s0, hres, c->dIrOut, sizeof hres));
         berr = hres[0] / (hres[1] * hres[2] + hres[3]);
         if (berr <= tol || outer >= max_iter || !(hres[0] > 0.0) || !(hres[0] < HUGE_VAL)) break;
         // GMRES on F^-1 M d = F^-1 r, d0 = 0: V0 = z / beta
@@ -1268,8 +1259,7 @@ hpl_status hpl_solve_gmres(hpl_ctx* c, uint32_t block, hpl_prec prec, int restar
         if (st) return st;
         HIPCHK(c, launch_multi_dot(W, n, 1, W, n, dh, work, c->s0));
         double beta2 = 0.0;
-        HIPCHK(c, hipMemcpyAsync(&beta2, dh, sizeof(double), hipMemcpyDeviceToHost, c->s0));
-        HIPCHK(c, hipStreamSynchronize(c->s0));
+        HIPCHK(c, c->stage.to_host(c->s0, &beta2, dh, sizeof(double)));
         const double beta = std::sqrt(beta2);
         if (!(beta > 0.0) || !(beta < HUGE_VAL)) break;
         HIPCHK(c, launch_scale_copy(V, W, 1.0 / beta, n, c->s0));
@@ -1289,14 +1279,12 @@ hpl_status hpl_solve_gmres(hpl_ctx* c, uint32_t block, hpl_prec prec, int restar
             HIPCHK(c, launch_multi_dot(V, n, i + 1, W, n, dh + m + 1, work, c->s0));
             HIPCHK(c, launch_multi_axpy(W, 1.0, -1.0, V, n, i + 1, dh + m + 1, n, c->s0));
             double nw2 = 0.0;
-            HIPCHK(c, hipMemcpyAsync(h1.data(), dh, (i + 1) * sizeof(double),
-                                     hipMemcpyDeviceToHost, c->s0));
-            HIPCHK(c, hipMemcpyAsync(h2.data(), dh + m + 1, (i + 1) * sizeof(double),
-                                     hipMemcpyDeviceToHost, c->s0));
             HIPCHK(c, launch_multi_dot(W, n, 1, W, n, dh + 2 * m + 1, work, c->s0));
-            HIPCHK(c, hipMemcpyAsync(&nw2, dh + 2 * m + 1, sizeof(double), hipMemcpyDeviceToHost,
-                                     c->s0));
-            HIPCHK(c, hipStreamSynchronize(c->s0));
+            // all coefficients in one copy: pass 1, pass 2, ||W||^2
+            HIPCHK(c, c->stage.to_host(c->s0, coef.data(), dh, (2 * m + 2) * sizeof(double)));
+            std::copy(coef.begin(), coef.begin() + i + 1, h1.begin());
+            std::copy(coef.begin() + m + 1, coef.begin() + m + 2 + i, h2.begin());
+            nw2 = coef[2 * m + 1];
             const double hn = std::sqrt(nw2);
             double* col = &H[(size_t)i * (m + 1)];  // column i of H, rows 0..i+1
             for (int q = 0; q <= i; ++q) col[q] = h1[q] + h2[q];
@@ -1326,7 +1314,7 @@ hpl_status hpl_solve_gmres(hpl_ctx* c, uint32_t block, hpl_prec prec, int restar
             for (int p2 = q + 1; p2 < k; ++p2) sum -= H[(size_t)p2 * (m + 1) + q] * y[p2];
             y[q] = sum / H[(size_t)q * (m + 1) + q];
         }
-        HIPCHK(c, hipMemcpyAsync(dh, y.data(), k * sizeof(double), hipMemcpyHostToDevice, c->s0));
+        HIPCHK(c, c->stage.to_device(c->s0, dh, y.data(), k * sizeof(double)));
         HIPCHK(c, launch_multi_axpy(c->dX64, 1.0, 1.0, V, n, k, dh, n, c->s0));
         inner_total += k;
     }
@@ -1369,27 +1357,28 @@ hpl_status hpl_solve_rhs64(hpl_ctx* c, int nrhs, const double* b, uint64_t ldb, 
     if (st) return st;
     st = ensure(c, c->dRhsX, c->capRhsX, bytes);
     if (st) return st;
-    HIPCHK(c, hipMemcpy2DAsync(c->dRhsB, n * sizeof(double), b, ldb * sizeof(double),
-                               n * sizeof(double), (size_t)nrhs, hipMemcpyHostToDevice, c->s0));
+    HIPCHK(c, c->stage.to_device(c->s0, c->dRhsB, n * sizeof(double), b, ldb * sizeof(double),
+                                 n * sizeof(double), (size_t)nrhs));
     st = hplx::ir_solve(c, nrhs, c->dRhsB, c->dRhsX, max_iter, tol, res);
     if (st && st != HPL_ERR_NOT_CONVERGED) return st;
-    HIPCHK(c, hipMemcpy2DAsync(x, ldx * sizeof(double), c->dRhsX, n * sizeof(double),
-                               n * sizeof(double), (size_t)nrhs, hipMemcpyDeviceToHost, c->s0));
-    HIPCHK(c, hipStreamSynchronize(c->s0));
+    HIPCHK(c, c->stage.to_host(c->s0, x, ldx * sizeof(double), c->dRhsX, n * sizeof(double),
+                               n * sizeof(double), (size_t)nrhs));
     return st;
 }
 
 hpl_status hpl_download_solution64(hpl_ctx* c, double* x) {
     if (!c || !x) return HPL_ERR_INVALID_ARG;
     if (!c->dX64) return fail(c, HPL_ERR_STATE, "no refined solution");
-    HIPCHK(c, hipMemcpy(x, c->dX64, c->n * sizeof(double), hipMemcpyDeviceToHost));
+    HIPCHK(c, hipSetDevice(c->device));
+    HIPCHK(c, c->stage.to_host(c->s0, x, c->dX64, c->n * sizeof(double)));
     return HPL_SUCCESS;
 }
 
 hpl_status hpl_upload_rhs64(hpl_ctx* c, const double* b) {
     if (!c || !b) return HPL_ERR_INVALID_ARG;
     if (!c->dA) return fail(c, HPL_ERR_STATE, "no resident system");
-    HIPCHK(c, hipMemcpy(c->db64, b, c->n * sizeof(double), hipMemcpyHostToDevice));
+    HIPCHK(c, hipSetDevice(c->device));
+    HIPCHK(c, c->stage.to_device(c->s0, c->db64, b, c->n * sizeof(double)));
     HIPCHK(c, launch_d2f_scaled(c->db64, c->db, (int64_t)c->n, 1.0, c->s0));
     HIPCHK(c, hipStreamSynchronize(c->s0));
     return HPL_SUCCESS;

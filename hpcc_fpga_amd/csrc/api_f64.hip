@@ -201,10 +201,10 @@ hpl_status hpl_upload_f64(hpl_ctx* c, const double* a, uint64_t n, uint64_t lda,
     hpl_status st = alloc_f64(c, n);
     if (st) return st;
     FCHK(c, hipEventRecord(c->e0, c->s0));
-    FCHK(c, hipMemcpy2DAsync(c->dA64, c->lda64 * sizeof(double), a, lda * sizeof(double),
-                             n * sizeof(double), n, hipMemcpyHostToDevice, c->s0));
+    FCHK(c, c->stage.to_device(c->s0, c->dA64, c->lda64 * sizeof(double), a, lda * sizeof(double),
+                               n * sizeof(double), n));
     if (b)
-        FCHK(c, hipMemcpyAsync(c->dB64s, b, n * sizeof(double), hipMemcpyHostToDevice, c->s0));
+        FCHK(c, c->stage.to_device(c->s0, c->dB64s, b, n * sizeof(double)));
     else
         FCHK(c, launch_fill_f64(c->dB64s, (int64_t)n, 0.0, c->s0));
     FCHK(c, hipMemcpyAsync(c->dA064, c->dA64, n * c->lda64 * sizeof(double),
@@ -260,10 +260,9 @@ hpl_status hpl_gefa_dev_f64(hpl_ctx* c, hpl_timing* t) {
     st = c->f64_linear ? schedule64_pipelined(c) : schedule64(c);
     if (st) return st;
     FCHK(c, hipEventRecord(c->e1, c->s0));
-    FCHK(c, hipStreamSynchronize(c->s0));
-    if (t) t->gefa_s = seconds(c->e0, c->e1);
     int h = 0;
-    FCHK(c, hipMemcpy(&h, c->dStatus, sizeof(int), hipMemcpyDeviceToHost));
+    FCHK(c, c->stage.to_host(c->s0, &h, c->dStatus, sizeof(int)));  // waits for the stream
+    if (t) t->gefa_s = seconds(c->e0, c->e1);
     if (h) return fail(c, HPL_ERR_ZERO_PIVOT, "zero or non-finite pivot met during FP64 GEFA");
     c->factored64 = true;
     return HPL_SUCCESS;
@@ -290,10 +289,9 @@ hpl_status hpl_download_f64(hpl_ctx* c, double* a, uint64_t lda, double* x, hpl_
     FCHK(c, hipSetDevice(c->device));
     FCHK(c, hipEventRecord(c->e0, c->s0));
     if (a)
-        FCHK(c, hipMemcpy2DAsync(a, lda * sizeof(double), c->dA64, c->lda64 * sizeof(double),
-                                 c->n64 * sizeof(double), c->n64, hipMemcpyDeviceToHost, c->s0));
-    if (x)
-        FCHK(c, hipMemcpyAsync(x, c->dX64s, c->n64 * sizeof(double), hipMemcpyDeviceToHost, c->s0));
+        FCHK(c, c->stage.to_host(c->s0, a, lda * sizeof(double), c->dA64,
+                                 c->lda64 * sizeof(double), c->n64 * sizeof(double), c->n64));
+    if (x) FCHK(c, c->stage.to_host(c->s0, x, c->dX64s, c->n64 * sizeof(double)));
     FCHK(c, hipEventRecord(c->e1, c->s0));
     FCHK(c, hipStreamSynchronize(c->s0));
     if (t) t->d2h_s = seconds(c->e0, c->e1);
@@ -306,8 +304,7 @@ hpl_status hpl_residual_f64(hpl_ctx* c, double out[4]) {
     FCHK(c, hipSetDevice(c->device));
     FCHK(c, launch_residual_f64(c->dA064, (int64_t)c->lda64, (int64_t)c->n64, c->dX64s, c->dB64s,
                                 c->dWork64, c->dOut64, c->s0));
-    FCHK(c, hipMemcpyAsync(out, c->dOut64, 4 * sizeof(double), hipMemcpyDeviceToHost, c->s0));
-    FCHK(c, hipStreamSynchronize(c->s0));
+    FCHK(c, c->stage.to_host(c->s0, out, c->dOut64, 4 * sizeof(double)));
     return HPL_SUCCESS;
 }
 
@@ -328,7 +325,7 @@ hpl_status hpl_gesl_f64(hpl_ctx* c, const double* lu, double* b, uint64_t n, uin
     c->factored64 = true;
     st = hpl_gesl_dev_f64(c, t);
     if (st) return st;
-    FCHK(c, hipMemcpy(b, c->dX64s, n * sizeof(double), hipMemcpyDeviceToHost));
+    FCHK(c, c->stage.to_host(c->s0, b, c->dX64s, n * sizeof(double)));
     return HPL_SUCCESS;
 }
 

@@ -180,8 +180,8 @@ hpl_status pivot_factor_to_host(hpl_ctx* c, float* a, uint64_t lda) {
     const uint64_t n = c->n;
     std::vector<int32_t> ipvt(n);
     std::vector<float> u(n);
-    PCHK(c, hipMemcpy(ipvt.data(), c->dPiv, n * sizeof(int32_t), hipMemcpyDeviceToHost));
-    PCHK(c, hipMemcpy(u.data(), c->dDiagU, n * sizeof(float), hipMemcpyDeviceToHost));
+    PCHK(c, c->stage.to_host(c->s0, ipvt.data(), c->dPiv, n * sizeof(int32_t)));
+    PCHK(c, c->stage.to_host(c->s0, u.data(), c->dDiagU, n * sizeof(float)));
     // stored row k is M's column k: u_kk on the diagonal, and the exchanges
     // of the later steps j > k (positions j and ipvt[j] > j) undone in
     // reverse order
@@ -210,7 +210,7 @@ hpl_status hpl_get_pivots(hpl_ctx* c, int32_t* ipvt) {
     if (!c || !ipvt) return HPL_ERR_INVALID_ARG;
     if (!c->factored || !c->pivoted) return fail(c, HPL_ERR_STATE, "no pivoted factor resident");
     PCHK(c, hipSetDevice(c->device));
-    PCHK(c, hipMemcpy(ipvt, c->dPiv, c->n * sizeof(int32_t), hipMemcpyDeviceToHost));
+    PCHK(c, c->stage.to_host(c->s0, ipvt, c->dPiv, c->n * sizeof(int32_t)));
     return HPL_SUCCESS;
 }
 
@@ -270,9 +270,9 @@ hpl_status hpl_gesl_pvt(hpl_ctx* c, const float* lu, float* b, const int32_t* ip
     PvLayout L{};
     st = bind_pivot_block(c, B, &L);
     if (st) return st;
-    PCHK(c, hipMemcpy(c->dPiv, ipvt, n * sizeof(int32_t), hipMemcpyHostToDevice));
-    PCHK(c, hipMemcpy(c->dPerm, perm.data(), n * sizeof(int32_t), hipMemcpyHostToDevice));
-    PCHK(c, hipMemcpy(c->dDiagU, u.data(), n * sizeof(float), hipMemcpyHostToDevice));
+    PCHK(c, c->stage.to_device(c->s0, c->dPiv, ipvt, n * sizeof(int32_t)));
+    PCHK(c, c->stage.to_device(c->s0, c->dPerm, perm.data(), n * sizeof(int32_t)));
+    PCHK(c, c->stage.to_device(c->s0, c->dDiagU, u.data(), n * sizeof(float)));
     PCHK(c, launch_prep_all(c->dA, (int64_t)c->lda, (int)B, (int)(n / B), c->dInv,
                             3 * (B / 32) * 1024, c->s0));
     c->B = B;
@@ -281,7 +281,7 @@ hpl_status hpl_gesl_pvt(hpl_ctx* c, const float* lu, float* b, const int32_t* ip
     c->binv_ready = false;
     st = hpl_gesl_dev(c, t);
     if (st) return st;
-    PCHK(c, hipMemcpy(b, c->dx, n * sizeof(float), hipMemcpyDeviceToHost));
+    PCHK(c, c->stage.to_host(c->s0, b, c->dx, n * sizeof(float)));
     return HPL_SUCCESS;
 }
 

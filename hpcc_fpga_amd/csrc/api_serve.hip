@@ -131,6 +131,8 @@ class HipExecutor : public hplserve::Executor {
             slots_.push_back(S);
             if (hplx::init_streams(S.c) != HPL_SUCCESS)
                 return set_err(HPL_ERR_HIP, "stream creation failed for a serving slot");
+            if (S.c->stage.make() != hipSuccess)
+                return set_err(HPL_ERR_OUT_OF_MEMORY, "pinned host memory for a serving slot");
         }
         return HPL_SUCCESS;
     }
@@ -169,8 +171,8 @@ class HipExecutor : public hplserve::Executor {
         if (job.fresh) {
             hipError_t e;
             if (rq.a)
-                e = hipMemcpy2DAsync(c->dA0, lda * sizeof(float), rq.a, rq.lda * sizeof(float),
-                                     n * sizeof(float), n, hipMemcpyHostToDevice, s0);
+                e = c->stage.to_device(s0, c->dA0, lda * sizeof(float), rq.a,
+                                       rq.lda * sizeof(float), n * sizeof(float), n);
             else
                 e = launch_generate(c->dA0, (int64_t)lda, (int64_t)n, 0, rq.seed, 1.0, nullptr,
                                     nullptr, nullptr, s0);
@@ -194,16 +196,15 @@ class HipExecutor : public hplserve::Executor {
         hipError_t e = hipSuccess;
         if (np > n) e = launch_fill_f64(S.b64, (int64_t)(np * nr), 0.0, s0);
         if (e == hipSuccess)
-            e = hipMemcpy2DAsync(S.b64, np * sizeof(double), rq.b, rq.ldb * sizeof(double),
-                                 n * sizeof(double), (size_t)nr, hipMemcpyHostToDevice, s0);
+            e = c->stage.to_device(s0, S.b64, np * sizeof(double), rq.b, rq.ldb * sizeof(double),
+                                   n * sizeof(double), (size_t)nr);
         if (e != hipSuccess) return fail(job, c, HPL_ERR_HIP, hipGetErrorString(e));
         hpl_ir_result res[16];
         hpl_status st =
             hplx::ir_solve(c, nr, S.b64, S.x64, cfg_.max_iter, cfg_.tol_per_n * (double)n, res);
         if (st != HPL_SUCCESS && st != HPL_ERR_NOT_CONVERGED) return fail(job, c, st, c->err.c_str());
-        e = hipMemcpy2DAsync(rq.x, rq.ldx * sizeof(double), S.x64, np * sizeof(double),
-                             n * sizeof(double), (size_t)nr, hipMemcpyDeviceToHost, s0);
-        if (e == hipSuccess) e = hipStreamSynchronize(s0);
+        e = c->stage.to_host(s0, rq.x, rq.ldx * sizeof(double), S.x64, np * sizeof(double),
+                             n * sizeof(double), (size_t)nr);
         if (e != hipSuccess) return fail(job, c, HPL_ERR_HIP, hipGetErrorString(e));
         job.resp.iterations = 0;
         job.resp.backward_error = 0.0;

@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/hpl_hip.h"
+#include "transfer.hpp"
 
 struct hpl_ctx {
     int device = 0;
@@ -25,6 +26,7 @@ struct hpl_ctx {
     hipStream_t s2 = nullptr;   // row and column blocks' last update in the pipelined schedule
     hipStream_t s3 = nullptr;   // its look-ahead updates of the next block
     hipEvent_t e0 = nullptr, e1 = nullptr;
+    hplx::HostStage stage;      // pinned buffers of the copies from and to the host
     hipEvent_t evA = nullptr, evP = nullptr;  // next-panel region updated / panel ready
     hipEvent_t evS = nullptr, evD = nullptr;  // strips solved / row and column blocks updated
     hipEvent_t evL = nullptr;                 // next block's look-ahead update done

@@ -1,0 +1,49 @@
+// Copies between host buffers of any kind and device memory through pinned
+// staging memory (internal to libhpl_hip.so).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <stddef.h>
+
+namespace hplx {
+
+// A few pinned buffers with an event each, owned by one context, slot or batch
+// and used by one thread at a time.  Made on first use, given back by free().
+//
+// The runtime moves a pitched copy from ordinary host memory row by row, each
+// row pinned and queued by itself (about 10 us a row where the buffer has not
+// been seen before: 27 ms for the three transfers of a 1024 x 1024 solve, 1.3
+// ms through these buffers), and its copies were seen to overtake or be
+// overtaken by kernels of the same stream under a profiler.  Here rows are
+// packed at the device's pitch by the host while the previous piece is on its
+// way, so the device sees plain copies from pinned memory.
+class HostStage {
+   public:
+    ~HostStage() { free(); }
+    // `rows` rows of `width` bytes, `pitch` apart on each side.  to_device: the
+    // device rows' bytes between width and pitch become zero where the pitch
+    // fits a buffer (the last row's excepted; else they stay); the host buffer
+    // may be reused on return, the copies run on `s`.  to_host: returns when the rows are in place, after everything
+    // enqueued on `s` before.
+    hipError_t to_device(hipStream_t s, void* dev, size_t dev_pitch, const void* host,
+                         size_t host_pitch, size_t width, size_t rows);
+    hipError_t to_host(hipStream_t s, void* host, size_t host_pitch, const void* dev,
+                       size_t dev_pitch, size_t width, size_t rows);
+    // contiguous bytes
+    hipError_t to_device(hipStream_t s, void* dev, const void* host, size_t bytes);
+    hipError_t to_host(hipStream_t s, void* host, const void* dev, size_t bytes);
+    hipError_t make();
+    void free();
+
+   private:
+    static constexpr int kBufs = 4;
+    // 1 MiB: packed in 30 us, on its way for 20 us; shorter pieces pay the
+    // launch of a copy, longer ones the wait for the first and last piece
+    static constexpr size_t kBytes = 1u << 20;
+    char* mem_ = nullptr;
+    hipEvent_t ev_[kBufs] = {};
+    int next_ = 0;
+};
+
+}  // namespace hplx
