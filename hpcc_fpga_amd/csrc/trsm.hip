@@ -458,77 +458,171 @@ __global__ __launch_bounds__(64) void trsm_reg_kernel(float* __restrict__ A, int
 //   top  recurrence on e_c :  y = -(U^T)^-1 e_c -> OutU[i][c] = -(U^-1)(c, i)
 // stored per block at out + k * 2 * B * B (OutL, then OutU), both row-major
 // B x B, so the substitution applies them as coalesced GEMVs.  Launch: grid
-// (B/32 vector groups, 2 types, blocks), one wave each; coefficients are read
-// straight from the factor (the transposed copy DT of the panel is gone).
+// (B/16 vector groups, 2 types, blocks), four waves each; coefficients are
+// read straight from the factor.
+//
+// Bound: the chain of B/32 blocks, per block one update by the block before
+// and the product with its 32 x 32 inverse.  Wave w owns the 32-row blocks w
+// and w + 4 of the group's 16 vectors; as soon as block p is solved every
+// wave updates its blocks beyond p by it, the next one first.  With 16
+// vectors a product of 32 x 32 coefficients is 16 v_mfma_f32_16x16x4_f32 of
+// 32 cycles, half the chain of 32 vectors on 32x32x2; blocks before the unit
+// vectors' own are zero and skipped.  (B = 256: 38 us with one wave solving
+// all blocks of 32 vectors in turn, 13 us here; hpl_gesl_noalloc at n = 1024
+// 72.3 -> 47.6 us, BF16 refinement at n = 65536 279.7 -> 278.2 ms.)
+//
+// Operand layout: step (t, r) of a product takes k = 16 t + 4 (lane / 16) + r,
+// the row that register r of accumulator tile t holds in that lane, so a
+// solved block is the next product's B operand as it stands (its own inverse)
+// or as two 16-byte LDS reads (the other waves).
+//
+// pk, if not null: the inverses' BF16 operand copies of the strip solves
+// (below), written from the same registers.
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
 template <int B>
-__global__ __launch_bounds__(64) void block_inverse_kernel(const float* __restrict__ A,
-                                                           int64_t lda,
-                                                           const float* __restrict__ inv,
-                                                           int64_t inv_stride,
-                                                           float* __restrict__ out) {
-    constexpr int NQ = B / 32;
-    const int lane = threadIdx.x;
-    const int lr = lane & 31;
-    const int v0 = blockIdx.x * 32;
+__global__ __launch_bounds__(256) void block_inverse_kernel(const float* __restrict__ A,
+                                                            int64_t lda,
+                                                            const float* __restrict__ inv,
+                                                            int64_t inv_stride,
+                                                            float* __restrict__ out,
+                                                            bf16x8_t* __restrict__ pk) {
+    constexpr int NQ = B / 32, NB = NQ * (NQ + 1) / 2;
+    constexpr int NO = (NQ + 3) / 4;  // blocks per wave
+    __shared__ __attribute__((aligned(16))) float Y[2][16][36];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c = lane & 15, kk = lane >> 4;
+    const int v0 = blockIdx.x * 16, vb = v0 / 32;
     const bool top = blockIdx.y == 0;
     const int64_t k = blockIdx.z;
     const float* D = A + k * B * lda + k * B;
-    // coefficient X[p][i]: top C[i][p] = D[i][p], left C[i][p] = D[p][i]
-    const int64_t sp = top ? 1 : lda, si = top ? lda : 1;
     const float* G = inv + k * inv_stride + (top ? 0 : NQ * 1024);
     float* o = out + k * 2 * (int64_t)B * B + (top ? (int64_t)B * B : 0);
-
-    // Every load is issued one block ahead of its use (the 32 x 32 inverse of
-    // the next block and the first coefficient block of the next column
-    // block while this one multiplies), and the stores' layout is selected by
-    // address, not by a branch, so the unrolled loop stays one stretch of code
-    // the compiler can schedule.
-    f32x16 Y[NQ];
-    float g[2][16], c[2][16];
-    int cb = 0;  // buffer of c holding the next product's coefficients
-#pragma unroll
-    for (int r = 0; r < 16; ++r) g[0][r] = G[acc_row(r, lane) * 32 + lr];
-    if (NQ > 1) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) c[0][r] = D[(int64_t)acc_row(r, lane) * sp + (int64_t)(32 + lr) * si];
-    }
     const int64_t ostep_i = top ? B : 1, ostep_v = top ? 1 : B;  // o offset per element / vector
+
+    // zeros above the unit vectors' block
+    for (int e = threadIdx.x; e < vb * 32 * 16; e += 256) {
+        const int i = top ? e / 16 : e % (vb * 32), v = top ? e % 16 : e / (vb * 32);
+        o[i * ostep_i + (v0 + v) * ostep_v] = 0.0f;
+    }
+
+    // coefficients of block (q, p) for step (t2, r) and row tile t: X[p][i],
+    // top D[i][p], left D[p][i]
+    auto load_c = [&](float (&x)[2][2][4], int q, int p) {
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        if (q + 1 < NQ) {
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
-                g[(q + 1) & 1][r] = G[(q + 1) * 1024 + acc_row(r, lane) * 32 + lr];
-        }
-        f32x16 acc;
+            for (int t2 = 0; t2 < 2; ++t2) {
+                const int64_t i = q * 32 + 16 * t + c, kp = p * 32 + 16 * t2 + 4 * kk;
+                if (top) {
+                    const f32x4 v = *reinterpret_cast<const f32x4*>(D + i * lda + kp);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[r] = (q * 32 + acc_row(r, lane) == v0 + lr) ? 1.0f : 0.0f;
+                    for (int r = 0; r < 4; ++r) x[t][t2][r] = v[r];
+                } else {
 #pragma unroll
-        for (int pb = 0; pb < q; ++pb) {
-            // the coefficients of the next product: block pb + 1 of this
-            // column block, or block 0 of the next one
-            const int nq = pb + 1 < q ? q : q + 1, np = pb + 1 < q ? pb + 1 : 0;
-            if (nq < NQ) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    c[cb ^ 1][r] = D[(int64_t)(np * 32 + acc_row(r, lane)) * sp +
-                                     (int64_t)(nq * 32 + lr) * si];
+                    for (int r = 0; r < 4; ++r) x[t][t2][r] = D[(kp + r) * lda + i];
+                }
             }
+    };
+    float g[NO][2][2][4], cn[NO][2][2][4];
+    f32x4 acc[NO][2];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc = mfma32(c[cb][r], Y[pb][r], acc);
-            cb ^= 1;
+    for (int m = 0; m < NO; ++m) {
+        const int q = wave + 4 * m;
+        const bool mine = q < NQ && q >= vb;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                acc[m][t][r] = q * 32 + 16 * t + 4 * kk + r == v0 + c ? 1.0f : 0.0f;
+                g[m][t][0][r] = g[m][t][1][r] = cn[m][t][0][r] = cn[m][t][1][r] = 0.0f;
+            }
+        if (mine) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        g[m][t][t2][r] = G[q * 1024 + (16 * t2 + 4 * kk + r) * 32 + 16 * t + c];
+            if (q > vb) load_c(cn[m], q, vb);
         }
-        f32x16 y = {0};
+    }
+    for (int p = vb; p < NQ; ++p) {
+        if ((p & 3) == wave) {
+            // y_p = G_p z_p
+            f32x4 y[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
 #pragma unroll
-        for (int r = 0; r < 16; ++r) y = mfma32(g[q & 1][r], acc[r], y);
-        Y[q] = y;
-        // element i = q*32 + acc_row(r) of vector v0 + lr
+            for (int m = 0; m < NO; ++m)
+                if (p == wave + 4 * m) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r)
-            o[(int64_t)(q * 32 + acc_row(r, lane)) * ostep_i + (int64_t)(v0 + lr) * ostep_v] = y[r];
+                    for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+#pragma unroll
+                            for (int t = 0; t < 2; ++t)
+                                y[t] = mfma16(g[m][t][t2][r], acc[m][t2][r], y[t]);
+                }
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                *reinterpret_cast<f32x4*>(&Y[p & 1][c][16 * t + 4 * kk]) = y[t];
+                // element i = p*32 + 16 t + 4 kk + r of vector v0 + c
+                const int64_t i = p * 32 + 16 * t + 4 * kk;
+                if (top) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[(i + r) * B + v0 + c] = y[t][r];
+                } else {
+                    *reinterpret_cast<f32x4*>(o + (v0 + c) * (int64_t)B + i) = y[t];
+                }
+                if (pk) {
+                    // operand copy: row i % 32, k = v0 + c of block (p, vb)
+                    __bf16* d = reinterpret_cast<__bf16*>(
+                        pk + ((top ? 0 : NB) + p * (p + 1) / 2 + vb) * (int64_t)256);
+                    const int kc = (v0 & 31) + c, kb = kc >> 4, h = (kc >> 3) & 1, e = kc & 7;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int l = 16 * t + 4 * kk + r + 32 * h;
+                        const __bf16 hi = static_cast<__bf16>(y[t][r]);
+                        d[((kb * 2 + 0) * 64 + l) * 8 + e] = hi;
+                        d[((kb * 2 + 1) * 64 + l) * 8 + e] =
+                            static_cast<__bf16>(y[t][r] - static_cast<float>(hi));
+                    }
+                }
+            }
+        }
+        if (p + 1 == NQ) break;
+        __syncthreads();
+        f32x4 yv[2];
+#pragma unroll
+        for (int t2 = 0; t2 < 2; ++t2)
+            yv[t2] = *reinterpret_cast<const f32x4*>(&Y[p & 1][c][16 * t2 + 4 * kk]);
+#pragma unroll
+        for (int m = 0; m < NO; ++m) {
+            const int q = wave + 4 * m;
+            if (q > p && q < NQ) {
+                float x[2][2][4];
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) x[t][t2][r] = cn[m][t][t2][r];
+                if (q > p + 1) load_c(cn[m], q, p + 1);  // for the next block
+#pragma unroll
+                for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+#pragma unroll
+                        for (int t = 0; t < 2; ++t)
+                            acc[m][t] = mfma16(x[t][t2][r], yv[t2][r], acc[m][t]);
+            }
+        }
     }
 }
-
 
 // ----------------------------------------------------------------------------
 // Strip solves of the BF16 factorisation as products with the diagonal
@@ -546,42 +640,12 @@ __global__ __launch_bounds__(64) void block_inverse_kernel(const float* __restri
 // i, v[16 kb + 8 h + e], e = 0..7.  tinv_pack_kernel writes G in that layout
 // once per step: block (q, p), p <= q, at index q (q + 1) / 2 + p, 2048
 // halves each -- [kb][hi, lo][lane][8].
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-
 __device__ __forceinline__ void split_bf16(const float (&x)[8], bf16x8_t& hi, bf16x8_t& lo) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         const __bf16 h = static_cast<__bf16>(x[e]);
         hi[e] = h;
         lo[e] = static_cast<__bf16>(x[e] - static_cast<float>(h));
-    }
-}
-
-template <int B>
-__global__ __launch_bounds__(64) void tinv_pack_kernel(const float* __restrict__ binv,
-                                                       bf16x8_t* __restrict__ pk) {
-    constexpr int NQ = B / 32, NB = NQ * (NQ + 1) / 2;
-    const int bi = blockIdx.x;
-    int q = 0;
-    while ((q + 1) * (q + 2) / 2 <= bi) ++q;
-    const int p = bi - q * (q + 1) / 2;
-    const bool top = blockIdx.y == 0;
-    const int lane = threadIdx.x, i = lane & 31, h = lane >> 5;
-    const float* OutL = binv;
-    const float* OutU = binv + B * B;
-    bf16x8_t* dst = pk + (int64_t)((top ? 0 : NB) + bi) * 256;
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-        float x[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int k = p * 32 + 16 * kb + 8 * h + e, r = q * 32 + i;
-            x[e] = top ? OutU[r * B + k] : OutL[k * B + r];
-        }
-        bf16x8_t hi, lo;
-        split_bf16(x, hi, lo);
-        dst[(kb * 2 + 0) * 64 + lane] = hi;
-        dst[(kb * 2 + 1) * 64 + lane] = lo;
     }
 }
 
@@ -675,19 +739,32 @@ __global__ __launch_bounds__(64) void trsm_inv_kernel(float* __restrict__ A, int
 
 }  // namespace
 
-hipError_t launch_block_inverse(const float* A, int64_t lda, int64_t n, int B, const float* inv,
-                                int64_t inv_stride, float* out, hipStream_t s) {
-    if (n % B) return hipErrorInvalidValue;
-    const int NQ = B / 32;
-    dim3 grid(NQ, 2, (unsigned)(n / B));
+static hipError_t block_inverse(dim3 grid, const float* A, int64_t lda, int B, const float* inv,
+                                int64_t inv_stride, float* out, bf16x8_t* pk, hipStream_t s) {
+    // 16-byte row vectors
+    if ((lda & 3) || (reinterpret_cast<uintptr_t>(A) & 15) ||
+        (reinterpret_cast<uintptr_t>(out) & 15))
+        return hipErrorInvalidValue;
     switch (B) {
-        case 32: block_inverse_kernel<32><<<grid, 64, 0, s>>>(A, lda, inv, inv_stride, out); break;
-        case 64: block_inverse_kernel<64><<<grid, 64, 0, s>>>(A, lda, inv, inv_stride, out); break;
-        case 128: block_inverse_kernel<128><<<grid, 64, 0, s>>>(A, lda, inv, inv_stride, out); break;
-        case 256: block_inverse_kernel<256><<<grid, 64, 0, s>>>(A, lda, inv, inv_stride, out); break;
+#define HPL_BINV(BB)                                                                   \
+    case BB:                                                                           \
+        block_inverse_kernel<BB><<<grid, 256, 0, s>>>(A, lda, inv, inv_stride, out, pk); \
+        break;
+        HPL_BINV(32)
+        HPL_BINV(64)
+        HPL_BINV(128)
+        HPL_BINV(256)
+#undef HPL_BINV
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
+}
+
+hipError_t launch_block_inverse(const float* A, int64_t lda, int64_t n, int B, const float* inv,
+                                int64_t inv_stride, float* out, hipStream_t s) {
+    if (n % B) return hipErrorInvalidValue;
+    dim3 grid(B / 16, 2, (unsigned)(n / B));
+    return block_inverse(grid, A, lda, B, inv, inv_stride, out, nullptr, s);
 }
 
 hipError_t launch_prep(const float* A, int64_t lda, int64_t off, int B, float* DT, float* inv,
@@ -792,25 +869,9 @@ hipError_t launch_tinv_prepare(const float* A, int64_t lda, int64_t off, int B, 
                                float* tinv, float* out, hipStream_t s) {
     if (B % 32 || B > 256 || B < 32 || (reinterpret_cast<uintptr_t>(tinv) & 15))
         return hipErrorInvalidValue;
-    const int NQ = B / 32;
-    const float* D = A + off * lda + off;
     bf16x8_t* pk = reinterpret_cast<bf16x8_t*>(tinv + 2 * (int64_t)B * B);
-    float* o = out ? out : tinv;
-    dim3 g1(NQ, 2, 1), g2(NQ * (NQ + 1) / 2, 2);
-    switch (B) {
-#define HPL_TINV(BB)                                                                     \
-    case BB:                                                                             \
-        block_inverse_kernel<BB><<<g1, 64, 0, s>>>(D, lda, inv, 0, o);                   \
-        tinv_pack_kernel<BB><<<g2, 64, 0, s>>>(o, pk);                                   \
-        break;
-        HPL_TINV(32)
-        HPL_TINV(64)
-        HPL_TINV(128)
-        HPL_TINV(256)
-#undef HPL_TINV
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    return block_inverse(dim3(B / 16, 2, 1), A + off * lda + off, lda, B, inv, 0,
+                         out ? out : tinv, pk, s);
 }
 
 hipError_t launch_trsm_inv(float* A, int64_t lda, int64_t off, int64_t m, int B,
