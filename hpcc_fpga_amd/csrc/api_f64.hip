@@ -79,14 +79,20 @@ int64_t lt_slot64(const hpl_ctx* c, int64_t k) {
     return ((k / D) % 2) * D + (k % D);
 }
 
-// C += L T over rows [r0, r0+M) and columns [c0, c0+N), steps k0 .. k0+K/64-1
-hpl_status update64(hpl_ctx* c, hipStream_t st, int64_t k0, int64_t r0, int64_t c0, int64_t M,
-                    int64_t N, int K) {
-    if (M <= 0 || N <= 0) return HPL_SUCCESS;
+// Rows [r0, r0+M) and columns [c0, c0+N) of the trailing matrix.
+struct Part {
+    int64_t r0, c0, M, N;
+};
+
+// C += L T over one region or two, steps k0 .. k0+K/64-1
+hpl_status update64(hpl_ctx* c, hipStream_t st, int64_t k0, Part a, int K,
+                    Part b = Part{0, 0, 0, 0}) {
     const int64_t n = (int64_t)c->n64, lda = (int64_t)c->lda64, B = f64_block();
-    const double* Lt = c->dLt64 + lt_slot64(c, k0) * B * n + r0;
-    const double* T = c->dA64 + k0 * B * lda + c0;
-    FCHK(c, launch_update_f64(c->dA64 + r0 * lda + c0, lda, Lt, n, T, lda, (int)M, (int)N, K, st));
+    const double* Lt = c->dLt64 + lt_slot64(c, k0) * B * n;
+    const double* T = c->dA64 + k0 * B * lda;
+    FCHK(c, launch_update_f64(c->dA64 + a.r0 * lda + a.c0, lda, Lt + a.r0, n, T + a.c0, lda,
+                              (int)a.M, (int)a.N, c->dA64 + b.r0 * lda + b.c0, Lt + b.r0, T + b.c0,
+                              (int)b.M, (int)b.N, K, st));
     return HPL_SUCCESS;
 }
 
@@ -116,13 +122,13 @@ hpl_status schedule64(hpl_ctx* c) {
         const int K = (int)((j + 1) * B);
         const int64_t k0 = k - j;
         if (m <= B) {
-            r = update64(c, c->s0, k0, k1, k1, m, m, K);
+            r = update64(c, c->s0, k0, Part{k1, k1, m, m}, K);
             if (!r) r = panel64(c, c->s0, k + 1);
             if (r) return r;
             continue;
         }
-        r = update64(c, c->s0, k0, k1, k1, B, m, K);  // row block of the next panel
-        if (!r) r = update64(c, c->s0, k0, k1 + B, k1, m - B, B, K);  // column block
+        // row and column block of the next panel
+        r = update64(c, c->s0, k0, Part{k1, k1, B, m}, K, Part{k1 + B, k1, m - B, B});
         if (r) return r;
         FCHK(c, hipEventRecord(c->evA, c->s0));
         FCHK(c, hipStreamWaitEvent(c->s1, c->evA, 0));
@@ -130,10 +136,28 @@ hpl_status schedule64(hpl_ctx* c) {
         if (r) return r;
         FCHK(c, hipEventRecord(c->evP, c->s1));
         if (j == f64_depth(c) - 1) {
-            r = update64(c, c->s0, k0, k1 + B, k1 + B, m - B, m - B, K);
+            r = update64(c, c->s0, k0, Part{k1 + B, k1 + B, m - B, m - B}, K);
             if (r) return r;
         }
         FCHK(c, hipStreamWaitEvent(c->s0, c->evP, 0));
+    }
+    return HPL_SUCCESS;
+}
+
+// The last blocks, k0 and on, launch after launch on s0, as the FP32 path's end:
+// the pending steps p0 .. k0 - 1 first, then per block its panel and the
+// whole trailing update.
+hpl_status serial64(hpl_ctx* c, int64_t k0, int64_t p0) {
+    const int64_t n = (int64_t)c->n64, B = f64_block();
+    int64_t from = p0;
+    for (int64_t k = k0; k < n / B; ++k) {
+        const int64_t kb = k * B;
+        hpl_status r = HPL_SUCCESS;
+        if (k > from)
+            r = update64(c, c->s0, from, Part{kb, kb, n - kb, n - kb}, (int)((k - from) * B));
+        if (!r) r = panel64(c, c->s0, k);
+        if (r) return r;
+        from = k;
     }
     return HPL_SUCCESS;
 }
@@ -148,8 +172,12 @@ hpl_status schedule64_pipelined(hpl_ctx* c) {
     // tail groups of at most 3 steps
     const std::vector<int64_t> bnd = hplx::group_bounds(c, N, B, f64_depth(c), 3);
     const int64_t G = (int64_t)bnd.size() - 1;
+    // n = 4096: 6.41 ms without the serial end, 6.23 from 2048, 6.75 from 4096;
+    // n = 1024 1.35, 1.20
+    const int64_t serial_m = std::min<int64_t>(c->serial_m, 2048);
     hpl_status r;
     for (int64_t g = 0; g < G; ++g) {
+        if (n - bnd[g] * B <= serial_m) return serial64(c, bnd[g], g ? bnd[g - 1] : bnd[g]);
         const int64_t s = bnd[g + 1] * B;
         if (g >= 1 && s < n) {
             const int64_t steps = bnd[g] - bnd[g - 1];
@@ -159,7 +187,7 @@ hpl_status schedule64_pipelined(hpl_ctx* c) {
             for (int64_t i = 0; i < S; ++i) {
                 const int64_t a = s + tiles * i / S * 128;
                 const int64_t b = i + 1 == S ? n : s + tiles * (i + 1) / S * 128;
-                r = update64(c, c->s1, bnd[g - 1], s, a, w, b - a, (int)(steps * B));
+                r = update64(c, c->s1, bnd[g - 1], Part{s, a, w, b - a}, (int)(steps * B));
                 if (r) return r;
             }
         }
@@ -169,8 +197,8 @@ hpl_status schedule64_pipelined(hpl_ctx* c) {
             const int64_t kb = k * B, m = n - kb;
             if (k > k0) {
                 const int K = (int)((k - k0) * B);
-                r = update64(c, c->s0, k0, kb, kb, B, m, K);  // row block k
-                if (!r) r = update64(c, c->s0, k0, kb + B, kb, m - B, B, K);  // column block k
+                // row and column block k
+                r = update64(c, c->s0, k0, Part{kb, kb, B, m}, K, Part{kb + B, kb, m - B, B});
                 if (r) return r;
             }
             r = panel64(c, c->s0, k);

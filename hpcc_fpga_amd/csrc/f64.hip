@@ -233,6 +233,81 @@ __global__ __launch_bounds__(UNT, 4) void update_f64_kernel(double* __restrict__
             }
 }
 
+// The update of small regions, as the FP32 one (gemm.hip): a wave owns a 16 x
+// 32 block of C and reads its operands straight into the MFMA registers, 16 k
+// values at a time, three chunks ahead; four waves (32 x 64 of C) share them
+// through the CU's L1.  The row and column blocks on a step's critical path
+// are 64 wide: the tiled kernel, one 128 x 128 tile per CU and half of it
+// empty, takes 68 us for K = 640, all of it one CU's matrix rate.
+// Bound: one memory round trip, then the wave's chain of K / 2 MFMAs (64
+// cycles each).  C first, then k in order: the bits of the tiled kernel.
+struct Region64 {
+    double* C;
+    const double* At;
+    const double* Bt;
+    int M, N;
+};
+constexpr int SCH = 4;   // 16 k values: 4 MFMA steps per chunk
+constexpr int SBUF = 4;
+
+__global__ __launch_bounds__(256) void update_small_f64_kernel(Region64 g, int64_t ldc, int64_t lda,
+                                                               int64_t ldb, int K, Region64 g2) {
+    int tiles_n = (g.N + 63) / 64, bid = blockIdx.x;
+    const int nblk = ((g.M + 31) / 32) * tiles_n;
+    if (bid >= nblk) {  // second region
+        bid -= nblk;
+        g = g2;
+        tiles_n = (g.N + 63) / 64;
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c = lane & 15, kk = lane >> 4;
+    const int m0 = (bid / tiles_n) * 32 + (wave & 1) * 16;
+    const int n0 = (bid % tiles_n) * 64 + (wave >> 1) * 32;
+    if (m0 >= g.M || n0 >= g.N) return;  // regions are whole 16 x 32 blocks
+    const double* a = g.At + (int64_t)kk * lda + m0 + c;
+    const double* b = g.Bt + (int64_t)kk * ldb + n0 + c;
+    double va[SBUF][SCH], vb[SBUF][SCH][2];
+    auto load = [&](int ch, int buf) {
+#pragma unroll
+        for (int i = 0; i < SCH; ++i) {
+            const int64_t k = 4 * (ch * SCH + i);
+            va[buf][i] = a[k * lda];
+            vb[buf][i][0] = b[k * ldb];
+            vb[buf][i][1] = b[k * ldb + 16];
+        }
+    };
+    // accumulator register q: row kk + 4 q
+    double* p = g.C + (int64_t)(m0 + kk) * ldc + n0 + c;
+    f64x4 acc[2];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        acc[0][q] = p[(int64_t)(4 * q) * ldc];
+        acc[1][q] = p[(int64_t)(4 * q) * ldc + 16];
+    }
+    const int nch = K / (4 * SCH);
+#pragma unroll
+    for (int u = 0; u < SBUF - 1; ++u)
+        if (u < nch) load(u, u);
+    for (int ch0 = 0; ch0 < nch; ch0 += SBUF) {
+#pragma unroll
+        for (int u = 0; u < SBUF; ++u) {
+            const int ch = ch0 + u;
+            if (ch >= nch) break;
+            if (ch + SBUF - 1 < nch) load(ch + SBUF - 1, (u + SBUF - 1) % SBUF);
+#pragma unroll
+            for (int i = 0; i < SCH; ++i) {
+                acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(va[u][i], vb[u][i][0], acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(va[u][i], vb[u][i][1], acc[1], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        p[(int64_t)(4 * q) * ldc] = acc[0][q];
+        p[(int64_t)(4 * q) * ldc + 16] = acc[1][q];
+    }
+}
+
 // ---------------------------------------------------------------- substitution
 // forward, block q (64 entries from k0): x_i += x_k * a[k][i] (k < i, inside
 // the block), the block staged in LDS, one wave; then x_i += sum_{k in block}
@@ -381,11 +456,32 @@ hipError_t launch_strips_f64(double* A, int64_t lda, int64_t off, int64_t m, dou
 }
 
 hipError_t launch_update_f64(double* C, int64_t ldc, const double* Lt, int64_t ldl,
-                             const double* T, int64_t ldt, int M, int N, int K, hipStream_t s) {
-    if (M <= 0 || N <= 0) return hipSuccess;
-    if (K % UBK || (M & 1) || (N & 1)) return hipErrorInvalidValue;
-    const int tiles = ((M + UBM - 1) / UBM) * ((N + UBN - 1) / UBN);
-    update_f64_kernel<<<tiles, UNT, 0, s>>>(C, ldc, Lt, ldl, T, ldt, M, N, K);
+                             const double* T, int64_t ldt, int M, int N, double* C2,
+                             const double* Lt2, const double* T2, int M2, int N2, int K,
+                             hipStream_t s) {
+    if (M <= 0 || N <= 0) M = N = 0;
+    if (M2 <= 0 || N2 <= 0) M2 = N2 = 0;
+    if (!M && !M2) return hipSuccess;
+    if (K % UBK || (M & 1) || (N & 1) || (M2 & 1) || (N2 & 1)) return hipErrorInvalidValue;
+    const auto tiles = [](int m, int n, int tm, int tn) {
+        return ((m + tm - 1) / tm) * ((n + tn - 1) / tn);
+    };
+    const int t1 = tiles(M, N, UBM, UBN), t2 = tiles(M2, N2, UBM, UBN);
+    // One or two 64-wide blocks (half a tile each) up to two tiles per CU, other
+    // regions while half the CUs would have no tile: with every region up to
+    // 128 tiles on the small path GEFA at n = 8192 takes 17.2 ms, up to 256
+    // 17.8, up to 512 18.7 (none: 33.5); n = 16384 89.5, 73.5, 74.0 (99.3) and
+    // n = 32768 464.6, 459.1, 449.7 (474.2), where the row and column blocks
+    // make up the larger counts.
+    const bool narrow = std::min(M, N) <= FB && std::min(M2, N2) <= FB;
+    if (t1 + t2 <= (narrow ? 512 : 128) && M % 16 == 0 && N % 32 == 0 && M2 % 16 == 0 && N2 % 32 == 0) {
+        update_small_f64_kernel<<<(unsigned)(tiles(M, N, 32, 64) + tiles(M2, N2, 32, 64)), 256, 0,
+                                  s>>>(Region64{C, Lt, T, M, N}, ldc, ldl, ldt, K,
+                                       Region64{C2, Lt2, T2, M2, N2});
+        return hipGetLastError();
+    }
+    if (t1) update_f64_kernel<<<t1, UNT, 0, s>>>(C, ldc, Lt, ldl, T, ldt, M, N, K);
+    if (t2) update_f64_kernel<<<t2, UNT, 0, s>>>(C2, ldc, Lt2, ldl, T2, ldt, M2, N2, K);
     return hipGetLastError();
 }
 

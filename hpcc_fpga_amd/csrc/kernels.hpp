@@ -175,10 +175,12 @@ hipError_t launch_lu_f64(double* A, int64_t lda, int64_t off, int* status, hipSt
 // off+64.., columns off..off+63); the left strip also into Lt[k][v] (ldl)
 hipError_t launch_strips_f64(double* A, int64_t lda, int64_t off, int64_t m, double* Lt,
                              int64_t ldl, hipStream_t s);
-// C[r][c] += sum_k Lt[k][r] T[k][c] (K a multiple of 16, M and N even)
+// C[r][c] += sum_k Lt[k][r] T[k][c] (K a multiple of 16, M and N even), over
+// one region or two of the same leading dimensions (M2 or N2 0: one)
 hipError_t launch_update_f64(double* C, int64_t ldc, const double* Lt, int64_t ldl,
-                             const double* T, int64_t ldt, int M, int N, int K, hipStream_t s);
-// x := M^-1 x with the factor (gesl_ref_nopvt's order; n a multiple of 64)
+                             const double* T, int64_t ldt, int M, int N, double* C2,
+                             const double* Lt2, const double* T2, int M2, int N2, int K,
+                             hipStream_t s);
 hipError_t launch_gesl_f64(const double* A, int64_t lda, int64_t n, double* x, hipStream_t s);
 int64_t residual_f64_work(int64_t n);
 hipError_t launch_residual_f64(const double* A, int64_t lda, int64_t n, const double* x,

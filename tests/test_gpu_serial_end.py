@@ -49,3 +49,24 @@ def test_serial_end(monkeypatch, n, B, prec, depth):
         # the generator's solution is 1; FP32 substitution, low-precision factors
         # to their update's rounding (2^-4 for E4M3 on entries of size 1 / n)
         assert np.max(np.abs(x - 1.0)) <= np.max(np.abs(xg - 1.0)) + 1e-5, serial
+
+
+@pytest.mark.parametrize("n,depth", [(64, 8), (192, 2), (1600, 6), (2688, 8)])
+def test_serial_end_fp64(monkeypatch, n, depth):
+    """The FP64 schedules (blocks of 64): grouped, pipelined to the end, and
+    with the serial end from several orders on."""
+    d = {"HPL_F64_DEPTH": str(depth)}
+    out = []
+    for env in ({"HPL_SCHEDULE": "grouped"}, {"HPL_SERIAL_M": "0"}, {"HPL_SERIAL_M": "640"},
+                {"HPL_SERIAL_M": "640", "HPL_TAIL_M": "1000", "HPL_TAIL_DEPTH": "2"}, {}):
+        for k in [k for k in os.environ if k.startswith("HPL_")]:
+            monkeypatch.delenv(k)
+        for k, v in {**env, **d}.items():
+            monkeypatch.setenv(k, v)
+        print(f"{env} n={n} FP64", flush=True)
+        with Context(0) as c:
+            c.generate_f64(n, 0, 3)
+            c.gefa_dev_f64()
+            out.append(c.download_f64(matrix=True, solution=False)[0])
+    for a in out[1:]:
+        assert np.array_equal(out[0].view(np.uint64), a.view(np.uint64))
