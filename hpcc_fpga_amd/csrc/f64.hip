@@ -2,13 +2,13 @@
 // build, LINPACK/src/host/linpack_data.cpp:166-229 with HOST_DATA_TYPE
 // double).  Same algorithm and storage as the FP32 path (row-major a,
 // M = a^T, dgefa encoding without pivoting); the kernels:
-//   * lu_f64_kernel: the 64 x 64 diagonal block in the registers of one wave
+//   * lu_f64_kernel: the 64 x 64 diagonal block in the registers of four waves
 //     (lane c holds stored column c), pivots and multipliers broadcast with
 //     v_readlane; the operation order of gefa_ref_nopvt with contraction off,
 //     so the block is bit-identical to it;
-//   * strip_f64_kernel: the top strip (one thread per column of the strip,
+//   * strip_f64_kernel: the top strip (two lanes per column of the strip,
 //     the closed form of test_kernel_communication.cpp:776-789) and the left
-//     strip (one thread per row, :624-632) with the 64 values of the vector in
+//     strip (two lanes per row, :624-632) with the 64 values of the vector in
 //     registers, coefficients from LDS; the left strip is also written
 //     transposed (k-major) for the update;
 //   * update_f64_kernel: C += Lt^T T on v_mfma_f64_16x16x4f64, 128 x 128
@@ -22,6 +22,7 @@
 #include "kernels.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
@@ -37,83 +38,184 @@ __device__ __forceinline__ double bcast64(double v, int lane) {
 }
 
 // ---------------------------------------------------------------- diagonal LU
-// Stored row r of the block is M's column r; lane c holds d[r] = D[r][c].
+// Stored row r of the block is M's column r; lane c of every wave belongs to
+// column c, wave w holds the rows r with r % 4 = w.
 //   for gk: D[gk][gk] = -1/D[gk][gk]; D[gk][c] *= D[gk][gk] (c > gk);
 //           D[r][c] += D[gk][c] * D[r][gk] (r > gk, c > gk)
-__global__ __launch_bounds__(64) void lu_f64_kernel(double* __restrict__ A, int64_t lda,
-                                                    int64_t off, int* __restrict__ status) {
+// Bound: the chain of 64 pivot steps -- a division, the scaled row through LDS
+// to the other waves, one row's update.  The wave of the next pivot updates
+// that row first, divides and publishes it, and catches up on its other rows
+// behind the barrier, while the other waves are on theirs.  22 us; one wave
+// holding all 64 rows took 36.
+constexpr int LW = 4, LR = FB / LW;  // waves, rows per wave
+
+__global__ __launch_bounds__(64 * LW) void lu_f64_kernel(double* __restrict__ A, int64_t lda,
+                                                         int64_t off, int* __restrict__ status) {
 #pragma clang fp contract(off)
-    const int c = threadIdx.x;
+    __shared__ double row[2][FB];
+    const int c = threadIdx.x & 63, wave = threadIdx.x >> 6;
     double* base = A + off * lda + off;
-    double d[FB];
+    double d[LR];
 #pragma unroll
-    for (int r = 0; r < FB; ++r) d[r] = base[(int64_t)r * lda + c];
+    for (int i = 0; i < LR; ++i) d[i] = base[(int64_t)(LW * i + wave) * lda + c];
     bool bad = false;
-#pragma unroll
-    for (int gk = 0; gk < FB; ++gk) {
-        const double piv = bcast64(d[gk], gk);
+    // row gk = LW i + (its wave), already updated by the steps before
+    auto pivot = [&](double& x, int gk) {
+        const double piv = bcast64(x, gk);
         const double inv = -1.0 / piv;
         bad |= (piv == 0.0) || !__builtin_isfinite(inv);
-        d[gk] = (c > gk) ? d[gk] * inv : ((c == gk) ? inv : d[gk]);
+        x = (c > gk) ? x * inv : ((c == gk) ? inv : x);
+        row[gk & 1][c] = x;
+    };
+    if (wave == 0) pivot(d[0], 0);
 #pragma unroll
-        for (int r = gk + 1; r < FB; ++r) {
-            const double s = bcast64(d[r], gk);
-            if (c > gk) d[r] = d[r] + d[gk] * s;
+    for (int gk = 0; gk < FB; ++gk) {
+        const int i0 = gk / LW, i1 = (gk + 1) / LW;
+        __syncthreads();  // row gk is there; everyone is past row gk - 1
+        if (gk + 1 == FB) break;
+        const double u = row[gk & 1][c];
+        if (wave == (gk + 1) % LW) {
+            const double s = bcast64(d[i1], gk);
+            if (c > gk) d[i1] = d[i1] + u * s;
+            pivot(d[i1], gk + 1);
+        } else if (wave > gk % LW) {
+            // the wave's row LW i0 + wave > gk
+            const double s = bcast64(d[i0], gk);
+            if (c > gk) d[i0] = d[i0] + u * s;
+        }
+#pragma unroll
+        for (int i = i0 + 1; i < LR; ++i) {
+            if (i == i1 && wave == (gk + 1) % LW) continue;
+            const double s = bcast64(d[i], gk);
+            if (c > gk) d[i] = d[i] + u * s;
         }
     }
 #pragma unroll
-    for (int r = 0; r < FB; ++r) base[(int64_t)r * lda + c] = d[r];
+    for (int i = 0; i < LR; ++i) base[(int64_t)(LW * i + wave) * lda + c] = d[i];
     if (bad && c == 0 && status) atomicMax(status, 1);
 }
 
 // ---------------------------------------------------------------- strips
-// Workgroup of 256 threads; blocks [0, gtop) take top-strip columns, the rest
-// left-strip rows, 256 vectors each.  D (the factored diagonal block) in LDS.
+// 32 vectors per wave, each held by two lanes: half h of the wave has the
+// elements e = 4 q + 2 h + b in x[2 q + b] (pairs, so that a row's elements
+// move as 16-byte vectors).  Blocks [0, gtop) take top-strip columns, the rest
+// left-strip rows, 128 vectors each.  The factored diagonal block lies in LDS
+// in the order the lanes use it: S[k][h][2 q + b] = the coefficient of step k
+// and element 4 q + 2 h + b, 16-byte broadcasts read one step ahead.
+// Bound: the 64-step recurrence's instructions: 18 us, 46 with one vector per
+// thread and 2016 scalar LDS reads each.  With both, GEFA at n = 8192 went
+// from 17.2 to 13.5 ms (1024: 1.19 -> 0.72, 32768: 450 -> 437).
+template <int H>
+__device__ __forceinline__ double from_half64(double v) {
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    const uint32_t l = (uint32_t)u, g = (uint32_t)(u >> 32);
+    const auto a = __builtin_amdgcn_permlane32_swap(l, l, false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(g, g, false, false);
+    return __longlong_as_double((long long)(((uint64_t)b[H] << 32) | a[H]));
+}
+
+template <int J, int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (J < N) {
+        f(std::integral_constant<int, J>{});
+        static_for<J + 1, N>(f);
+    }
+}
+
+template <bool TOP>
+__device__ __forceinline__ void strip_solve64(double (&x)[FB / 2], const double* S, int h) {
+#pragma clang fp contract(off)
+    const double* Sh = S + h * (FB / 2);
+    double2 nx[2][FB / 4];
+#pragma unroll
+    for (int q = 0; q < FB / 4; ++q) nx[0][q] = *reinterpret_cast<const double2*>(Sh + 2 * q);
+    // the scale of step k: element k's own coefficient
+    auto dg_at = [&](int k) { return S[k * FB + ((k >> 1) & 1) * (FB / 2) + 2 * (k >> 2) + (k & 1)]; };
+    double dg = TOP ? dg_at(0) : 0.0;
+    static_for<0, FB>([&](auto kc) {
+        constexpr int k = kc.value, q0 = k >> 2, kr = k & 3, hk = kr >> 1, ik = 2 * q0 + (k & 1);
+        if constexpr (k + 1 < FB) {
+#pragma unroll
+            for (int q = (k + 1) >> 2; q < FB / 4; ++q)
+                nx[(k + 1) & 1][q] = *reinterpret_cast<const double2*>(Sh + (k + 1) * FB + 2 * q);
+        }
+        double s = x[ik];
+        if constexpr (TOP) s = s * dg;
+        const double v = from_half64<hk>(s);
+        if constexpr (TOP) {
+            x[ik] = h == hk ? s : x[ik];
+            if constexpr (k + 1 < FB) dg = dg_at(k + 1);
+        }
+        // the elements of k's own group of four that come after k
+        if constexpr (kr < 2) {
+            const double w = x[2 * q0] + v * nx[k & 1][q0].x;
+            x[2 * q0] = h == 1 ? w : x[2 * q0];
+        }
+        if constexpr (kr < 3) {
+            const double w = x[2 * q0 + 1] + v * nx[k & 1][q0].y;
+            x[2 * q0 + 1] = kr == 0 || h == 1 ? w : x[2 * q0 + 1];
+        }
+#pragma unroll
+        for (int q = q0 + 1; q < FB / 4; ++q) {
+            const double2 f = nx[k & 1][q];
+            x[2 * q] = x[2 * q] + v * f.x;
+            x[2 * q + 1] = x[2 * q + 1] + v * f.y;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    });
+}
+
 __global__ __launch_bounds__(256) void strip_f64_kernel(double* __restrict__ A, int64_t lda,
                                                         int64_t off, int64_t m, int gtop,
                                                         double* __restrict__ Lt, int64_t ldl) {
-#pragma clang fp contract(off)
-    __shared__ double Ds[FB][FB + 1];
+    __shared__ __attribute__((aligned(16))) double S[FB * FB];
     const int t = threadIdx.x;
     const double* D = A + off * lda + off;
-    for (int e = t; e < FB * FB; e += 256) Ds[e / FB][e % FB] = D[(int64_t)(e / FB) * lda + e % FB];
-    __syncthreads();
     const bool top = (int)blockIdx.x < gtop;
-    const int64_t v = (int64_t)(top ? blockIdx.x : blockIdx.x - gtop) * 256 + t;
-    if (v >= m) return;
-    double x[FB];
+    for (int e = t; e < FB * FB; e += 256) {
+        const int i = e / FB, j = e % FB;
+        // top: step j, element i; left: step i, element j
+        const int k = top ? j : i, el = top ? i : j;
+        S[k * FB + ((el >> 1) & 1) * (FB / 2) + 2 * (el >> 2) + (el & 1)] = D[(int64_t)i * lda + j];
+    }
+    __syncthreads();
+    const int lane = t & 63, h = lane >> 5;
+    const int64_t v = (int64_t)(top ? blockIdx.x : blockIdx.x - gtop) * 128 + (t >> 6) * 32 + (lane & 31);
+    if (v >= m) return;  // m is a multiple of 64: whole waves
+    double x[FB / 2];
     if (top) {
-        // x = column off+FB+v of stored rows off..off+FB-1:
+        // column off+FB+v of stored rows off..off+FB-1:
         //   for k: x_k *= D[k][k]; x_j += x_k * D[j][k] (j > k)
-        double* col = A + off * lda + off + FB + v;
+        double* col = A + (off + 2 * h) * lda + off + FB + v;
 #pragma unroll
-        for (int k = 0; k < FB; ++k) x[k] = col[(int64_t)k * lda];
-#pragma unroll
-        for (int k = 0; k < FB; ++k) {
-            x[k] = x[k] * Ds[k][k];
-#pragma unroll
-            for (int j = k + 1; j < FB; ++j) x[j] = x[j] + x[k] * Ds[j][k];
+        for (int q = 0; q < FB / 4; ++q) {
+            x[2 * q] = col[(int64_t)(4 * q) * lda];
+            x[2 * q + 1] = col[(int64_t)(4 * q + 1) * lda];
         }
+        strip_solve64<true>(x, S, h);
 #pragma unroll
-        for (int k = 0; k < FB; ++k) col[(int64_t)k * lda] = x[k];
+        for (int q = 0; q < FB / 4; ++q) {
+            col[(int64_t)(4 * q) * lda] = x[2 * q];
+            col[(int64_t)(4 * q + 1) * lda] = x[2 * q + 1];
+        }
     } else {
-        // x = stored row off+FB+v, columns off..off+FB-1:
+        // stored row off+FB+v, columns off..off+FB-1:
         //   for k: x_i += x_k * D[k][i] (i > k)
-        double* row = A + (off + FB + v) * lda + off;
+        double* row = A + (off + FB + v) * lda + off + 2 * h;
 #pragma unroll
-        for (int k = 0; k < FB; k += 2) {
-            const double2 p = *reinterpret_cast<const double2*>(row + k);
-            x[k] = p.x;
-            x[k + 1] = p.y;
+        for (int q = 0; q < FB / 4; ++q) {
+            const double2 p = *reinterpret_cast<const double2*>(row + 4 * q);
+            x[2 * q] = p.x;
+            x[2 * q + 1] = p.y;
         }
+        strip_solve64<false>(x, S, h);
+        double* lt = Lt + (int64_t)(2 * h) * ldl + v;
 #pragma unroll
-        for (int k = 0; k < FB; ++k)
-#pragma unroll
-            for (int i = k + 1; i < FB; ++i) x[i] = x[i] + x[k] * Ds[k][i];
-#pragma unroll
-        for (int k = 0; k < FB; k += 2) *reinterpret_cast<double2*>(row + k) = double2{x[k], x[k + 1]};
-#pragma unroll
-        for (int k = 0; k < FB; ++k) Lt[(int64_t)k * ldl + v] = x[k];
+        for (int q = 0; q < FB / 4; ++q) {
+            *reinterpret_cast<double2*>(row + 4 * q) = double2{x[2 * q], x[2 * q + 1]};
+            lt[(int64_t)(4 * q) * ldl] = x[2 * q];
+            lt[(int64_t)(4 * q + 1) * ldl] = x[2 * q + 1];
+        }
     }
 }
 
@@ -443,14 +545,15 @@ __global__ void f32_to_f64_kernel(const float* __restrict__ s, int64_t lds, doub
 int f64_block() { return FB; }
 
 hipError_t launch_lu_f64(double* A, int64_t lda, int64_t off, int* status, hipStream_t s) {
-    lu_f64_kernel<<<1, 64, 0, s>>>(A, lda, off, status);
+    lu_f64_kernel<<<1, 64 * LW, 0, s>>>(A, lda, off, status);
     return hipGetLastError();
 }
 
 hipError_t launch_strips_f64(double* A, int64_t lda, int64_t off, int64_t m, double* Lt,
                              int64_t ldl, hipStream_t s) {
     if (m <= 0) return hipSuccess;
-    const int g = (int)((m + 255) / 256);
+    if (m % 32) return hipErrorInvalidValue;
+    const int g = (int)((m + 127) / 128);
     strip_f64_kernel<<<2 * g, 256, 0, s>>>(A, lda, off, m, g, Lt, ldl);
     return hipGetLastError();
 }
