@@ -60,7 +60,9 @@ hpl_status alloc_f64(hpl_ctx* c, uint64_t n) {
         if (!st) st = grow(c, c->dOut64, cap, 4 * sizeof(double));
         if (!st) c->capV64 = n * sizeof(double);
     }
-    if (!st) st = grow(c, c->dWork64, c->capWork64, residual_f64_work((int64_t)n) * sizeof(double));
+    // the residual's partial sums or the substitution's state
+    const int64_t work = std::max(residual_f64_work((int64_t)n), gesl_f64_work((int64_t)n));
+    if (!st) st = grow(c, c->dWork64, c->capWork64, work * sizeof(double));
     if (!st) st = hplx::ensure_mem(c, reinterpret_cast<void**>(&c->dStatus), &c->capStatus, 64);
     if (st) return st;
     c->n64 = n;
@@ -303,10 +305,15 @@ hpl_status hpl_gesl_dev_f64(hpl_ctx* c, hpl_timing* t) {
     FCHK(c, hipEventRecord(c->e0, c->s0));
     FCHK(c, hipMemcpyAsync(c->dX64s, c->dB64s, c->n64 * sizeof(double), hipMemcpyDeviceToDevice,
                            c->s0));
-    FCHK(c, launch_gesl_f64(c->dA64, (int64_t)c->lda64, (int64_t)c->n64, c->dX64s, c->s0));
+    const int64_t n = (int64_t)c->n64;
+    FCHK(c, launch_gesl_f64(c->dA64, (int64_t)c->lda64, n, c->dX64s, c->dWork64, c->s0));
     FCHK(c, hipEventRecord(c->e1, c->s0));
-    FCHK(c, hipStreamSynchronize(c->s0));
+    int h = 0;
+    FCHK(c, c->stage.to_host(c->s0, &h, gesl_f64_status(c->dWork64, n), sizeof h));
     if (t) t->gesl_s = seconds(c->e0, c->e1);
+    if (h)
+        return fail(c, HPL_ERR_HIP,
+                    "FP64 substitution: a bounded wait gave up (workgroups not co-resident)");
     return HPL_SUCCESS;
 }
 

@@ -14,9 +14,10 @@
 //   * update_f64_kernel: C += Lt^T T on v_mfma_f64_16x16x4f64, 128 x 128
 //     workgroup tiles of four 64 x 64 wave tiles, k-slabs of 16 through
 //     double-buffered LDS, XCD-aware tile order as the FP32 update;
-//   * gesl: per 64-block a one-wave diagonal solve (block staged in LDS) and a
-//     column-parallel update of the rest of x (the factor streamed once per
-//     sweep);
+//   * gesl: one launch of a wave per 64 entries that pass solved blocks on by
+//     flags; beyond what the device holds at once, per 64-block a one-wave
+//     diagonal solve (block staged in LDS) and a column-parallel update of the
+//     rest of x (the factor streamed once per sweep);
 //   * residual r = b - M x with per-chunk partial sums added in fixed order.
 #include "common.hpp"
 #include "kernels.hpp"
@@ -485,6 +486,111 @@ __global__ __launch_bounds__(256) void gesl_gemv_f64(const double* __restrict__ 
     x[i] = acc;
 }
 
+// Single-launch substitution: one wave per 64 entries, which stay in its
+// registers (lane l, entry l).  Forward, it takes block q's contribution as
+// soon as q is solved, q ascending, then solves its own block; backward the
+// same descending.  The arithmetic and its order are those of the kernels
+// above.  A solved block is published by agent-scope stores, then, once they
+// have completed, its flag (1 forward, 2 backward; cleared by a small kernel
+// before); waits are bounded and a wave that gives up raises status bit 2 and
+// leaves.  The tile of a contribution (and the wave's own diagonal block, the
+// same access) is loaded into the registers that the tile before it leaves,
+// so only the flag and the arithmetic follow a wait.
+// Bound: the chain of 2 n / 64 block solves, each a flag's trip, 64 steps of
+// contribution and 64 of the solve.  0.99 ms at n = 8192, 2.92 launch after
+// launch, 4 n / 64 of them (n = 1024 0.31 -> 0.12, 32768 12.5 -> 4.7).
+constexpr long kGesl64SpinLimit = 1L << 22;
+
+__global__ void gesl_reset_f64(unsigned* __restrict__ flags, int count, int* __restrict__ status) {
+    for (int i = threadIdx.x; i < count; i += blockDim.x) flags[i] = 0u;
+    if (threadIdx.x == 0) *status = 0;
+}
+
+__global__ __launch_bounds__(64) void gesl_persist_f64(const double* __restrict__ A, int64_t lda,
+                                                       int N, double* __restrict__ x,
+                                                       double* __restrict__ pf,
+                                                       double* __restrict__ pb,
+                                                       unsigned* __restrict__ flags,
+                                                       int* __restrict__ status, long spin_limit) {
+#pragma clang fp contract(off)
+    const int l = threadIdx.x, s = blockIdx.x;
+    const double* col = A + (int64_t)s * FB + l;  // this lane's column of the factor
+    auto put = [&](double* p, double v) {
+        __hip_atomic_store(reinterpret_cast<unsigned long long*>(p + (int64_t)s * FB + l),
+                           (unsigned long long)__double_as_longlong(v), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    };
+    auto get = [&](const double* p, int q) {
+        return __longlong_as_double((long long)__hip_atomic_load(
+            reinterpret_cast<const unsigned long long*>(p + (int64_t)q * FB + l), __ATOMIC_RELAXED,
+            __HIP_MEMORY_SCOPE_AGENT));
+    };
+    auto publish = [&](unsigned v) {
+        __builtin_amdgcn_s_waitcnt(0);  // the wave's stores have completed
+        if (l == 0)
+            __hip_atomic_store(flags + s, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    // true: gave up
+    auto wait = [&](int q, unsigned v) {
+        long spins = 0;
+        while (__hip_atomic_load(flags + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < v) {
+            if (++spins > spin_limit ||
+                (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 2)) {
+                if (l == 0) atomicOr(status, 2);
+                return true;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        return false;
+    };
+    double a[FB];
+    auto load = [&](int q) {
+#pragma unroll
+        for (int u = 0; u < FB; ++u) a[u] = col[((int64_t)q * FB + u) * lda];
+    };
+    double xi = x[(int64_t)s * FB + l];
+    // ---- forward: L y = b
+    load(0);
+    for (int q = 0; q < s; ++q) {
+        if (wait(q, 1u)) return;
+        const double xs = get(pf, q);
+        const double* next = col + (int64_t)(q + 1) * FB * lda;
+#pragma unroll
+        for (int u = 0; u < FB; ++u) {
+            xi = xi + bcast64(xs, u) * a[u];
+            a[u] = next[u * lda];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < FB - 1; ++k) {
+        const double xk = bcast64(xi, k);
+        if (l > k) xi = xi + xk * a[k];
+    }
+    put(pf, xi);
+    publish(1u);
+    // ---- backward: U x = y
+    load(N - 1);
+    for (int q = N - 1; q > s; --q) {
+        if (wait(q, 2u)) return;
+        const double xs = -get(pb, q);
+        const double* next = col + (int64_t)(q - 1) * FB * lda;
+#pragma unroll
+        for (int u = FB - 1; u >= 0; --u) {
+            xi = xi + bcast64(xs, u) * a[u];
+            a[u] = next[u * lda];
+        }
+    }
+#pragma unroll
+    for (int k = FB - 1; k >= 0; --k) {
+        const double sk = bcast64(xi, k) * bcast64(a[k], k);
+        if (l == k) xi = -sk;
+        if (l < k) xi = xi + sk * a[k];
+    }
+    put(pb, xi);
+    publish(2u);
+    x[(int64_t)s * FB + l] = xi;
+}
+
 // ---------------------------------------------------------------- residual
 // partial[c][i] = sum_{j in chunk c} M(i, j) x_j, M(i, j) = A[j][i]
 constexpr int RCH64 = 256;
@@ -588,8 +694,38 @@ hipError_t launch_update_f64(double* C, int64_t ldc, const double* Lt, int64_t l
     return hipGetLastError();
 }
 
-hipError_t launch_gesl_f64(const double* A, int64_t lda, int64_t n, double* x, hipStream_t s) {
+int64_t gesl_f64_work(int64_t n) {
+    // both sweeps' published blocks, a flag per block, the status
+    return 2 * n + n / FB / 2 + 8;
+}
+
+const int* gesl_f64_status(const double* work, int64_t n) {
+    return reinterpret_cast<const int*>(work + 2 * n);
+}
+
+hipError_t launch_gesl_f64(const double* A, int64_t lda, int64_t n, double* x, double* work,
+                           hipStream_t s) {
     if (n % FB) return hipErrorInvalidValue;
+    int* status = reinterpret_cast<int*>(work + 2 * n);
+    unsigned* flags = reinterpret_cast<unsigned*>(work + 2 * n + 8);
+    const int64_t N = n / FB;
+    // Every wave has to be resident at once: at most half of what the device
+    // holds, so that other work on it leaves room (n up to 65536); beyond, or
+    // where the device does not say, launch after launch.
+    int per_cu = 0, dev = 0, cus = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &per_cu, reinterpret_cast<const void*>(gesl_persist_f64), 64, 0) != hipSuccess ||
+        hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+        (void)hipGetLastError();
+        per_cu = cus = 0;
+    }
+    gesl_reset_f64<<<1, 256, 0, s>>>(flags, (int)N, status);
+    if (N <= (int64_t)per_cu * cus / 2) {
+        gesl_persist_f64<<<(unsigned)N, 64, 0, s>>>(A, lda, (int)N, x, work, work + n, flags, status,
+                                                    kGesl64SpinLimit);
+        return hipGetLastError();
+    }
     for (int64_t k0 = 0; k0 < n; k0 += FB) {
         gesl_diag_fwd_f64<<<1, 64, 0, s>>>(A, lda, k0, x);
         const int64_t i0 = k0 + FB;

@@ -181,7 +181,12 @@ hipError_t launch_update_f64(double* C, int64_t ldc, const double* Lt, int64_t l
                              const double* T, int64_t ldt, int M, int N, double* C2,
                              const double* Lt2, const double* T2, int M2, int N2, int K,
                              hipStream_t s);
-hipError_t launch_gesl_f64(const double* A, int64_t lda, int64_t n, double* x, hipStream_t s);
+// work: gesl_f64_work(n) doubles; *gesl_f64_status(work, n) is non-zero
+// afterwards where a bounded wait of the single launch gave up
+int64_t gesl_f64_work(int64_t n);
+const int* gesl_f64_status(const double* work, int64_t n);
+hipError_t launch_gesl_f64(const double* A, int64_t lda, int64_t n, double* x, double* work,
+                           hipStream_t s);
 int64_t residual_f64_work(int64_t n);
 hipError_t launch_residual_f64(const double* A, int64_t lda, int64_t n, const double* x,
                                const double* b, double* work, double* out4, hipStream_t s);
