@@ -102,13 +102,12 @@ hpl_status gefa_pivot(hpl_ctx* c, uint32_t B) {
         PCHK(c, panel_pivot_prepare((int)B, &c->pv_max_groups));
         c->pv_B = B;
     }
-    const int R = panel_pivot_rows((int)B);
-    const int64_t groups = (n + R - 1) / R;
+    const int64_t groups = panel_pivot_groups(n, (int)B);
     if (groups > c->pv_max_groups)
         return fail(c, HPL_ERR_UNSUPPORTED,
-                    "pivot panel of %lld rows needs %lld co-resident workgroups of %d rows, the "
-                    "device holds %d (use a smaller block)",
-                    (long long)n, (long long)groups, R, c->pv_max_groups);
+                    "pivot panel of %lld rows needs %lld co-resident workgroups, the device holds "
+                    "%d (use a smaller block)",
+                    (long long)n, (long long)groups, c->pv_max_groups);
     PvLayout L{};
     hpl_status st = bind_pivot_block(c, B, &L);
     if (st) return st;

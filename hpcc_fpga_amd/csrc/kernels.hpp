@@ -127,15 +127,13 @@ hipError_t launch_gesl_multi(const float* A, int64_t lda, int64_t n, int B, cons
 
 // partial pivoting (pivot.hip); X is the transposed matrix X[i][j] = M(i, j)
 hipError_t launch_transpose_square(float* A, int64_t ld, int64_t n, hipStream_t s);
-// rows per workgroup of the panel kernel at block B; workgroups of a panel
-// of m rows
-int panel_pivot_rows(int B);
-int panel_pivot_groups(int64_t m, int B);
+// most workgroups of any panel of up to n rows at block B
+int panel_pivot_groups(int64_t n, int B);
 // set the panel kernel up and return how many of its workgroups are co-resident
 hipError_t panel_pivot_prepare(int B, int* max_groups);
 // factorise panel k0 (m = n - k0 rows of X, B columns) with partial pivoting;
 // pub, krow, kslot: the exchange words of the panel's workgroups (G =
-// panel_pivot_groups(m, B) <= max_groups; kslot has gslots > G slots per
+// panel_pivot_groups(n, B) <= max_groups; kslot has gslots > G slots per
 // parity), carved from panel_exchange_words(n, B) words that
 // launch_zero_words clears before each factorisation; writes the panel (-1/u
 // on the diagonal), Lt[c][pos] for pos >= k0 + B, diagU/ipvt at k0.., and the

@@ -42,6 +42,19 @@
 // one panel is bit-identical to gefa_ref after the exchanges of the earlier
 // columns are undone (a data movement done on download).
 //
+// Bound: the chain of one column, about 7000 cycles (m = 6144, B = 128, cycle
+// counter): 3100 until every key is seen (store, load and the slowest
+// workgroup), 1170 the update of the other columns, the rest the workgroup's
+// own instructions, so their count is what matters: one thread takes a row
+// through its multiplier, its update of column c+1 and its key without a
+// barrier between (four barriers a column), maxima go over DPP, positions are
+// 32 bits wide, the key slot is published by a wave of its own, and the update
+// keeps eight rows per wave in flight with multipliers from v_readlane.  With
+// eight barriers, 64-bit positions and 256 rows per workgroup a column took
+// 13000 (3450 the exchange, 1670 the search, 4700 the update) and the panel
+// 730 us; now 400.  GEFA: n = 4096 B = 128 25.3 -> 14.3 ms, n = 9216 57.9 ->
+// 36.6, n = 32768 B = 256 388 -> 346.
+//
 // Every wait spins with a bound: a workgroup that waits longer than about a
 // second raises the status, marks its key slots with the abort tag (which
 // every waiter takes as a release) and exits, so every wave exits (the host
@@ -108,6 +121,36 @@ __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v)
     }
     return v;
 }
+// A key's order among keys of rising positions in rising lanes: its magnitude
+// plus one; none (key 0) lowest, the diagonal's NaN (all ones) highest.
+__device__ __forceinline__ unsigned key_rank(unsigned long long key) {
+    return key == 0 ? 0u : key == ~0ULL ? ~0u : (unsigned)(key >> 32) + 1u;
+}
+// The first lane of the wave with the largest rank (0: no lane has a key).  On
+// DPP moves, in registers (shuffles go through LDS, six in a row for a key).
+__device__ __forceinline__ int first_best(unsigned rank) {
+    unsigned m = rank;
+#define HPL_DPP_MAX(ctrl)                                                                 \
+    m = max(m, (unsigned)__builtin_amdgcn_update_dpp(0, (int)m, ctrl, 0xf, 0xf, false))
+    HPL_DPP_MAX(0x111);  // row_shr:1
+    HPL_DPP_MAX(0x112);
+    HPL_DPP_MAX(0x114);
+    HPL_DPP_MAX(0x118);
+    HPL_DPP_MAX(0x142);  // row_bcast:15
+    HPL_DPP_MAX(0x143);  // row_bcast:31
+#undef HPL_DPP_MAX
+    m = (unsigned)__builtin_amdgcn_readlane((int)m, 63);
+    return __ffsll((unsigned long long)__ballot(rank == m)) - 1;
+}
+__device__ __forceinline__ float bcast_lane(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ unsigned lane_u32(unsigned v, int l) {
+    return (unsigned)__builtin_amdgcn_readlane((int)v, l);
+}
+__device__ __forceinline__ unsigned long long lane_u64(unsigned long long v, int l) {
+    return ((unsigned long long)lane_u32((unsigned)(v >> 32), l) << 32) | lane_u32((unsigned)v, l);
+}
 
 // 64-bit exchange words: (tag << 32) | payload
 __device__ __forceinline__ void put_tagged(unsigned long long* p, unsigned payload, unsigned tag) {
@@ -130,27 +173,30 @@ __device__ __forceinline__ unsigned word_payload(unsigned long long w) { return 
 // row k's (written by its owner only).
 template <int B>
 __global__ __launch_bounds__(PNT) void panel_pivot_kernel(
-    float* __restrict__ X, int64_t ldx, int64_t n, int64_t k0, int R,
+    float* __restrict__ X, int64_t ldx, int64_t n, int64_t k0, int R_sh,
     unsigned long long* __restrict__ pub, unsigned long long* __restrict__ krow,
     unsigned long long* __restrict__ kslot, int gslots, float* __restrict__ Lt, int64_t ldl,
     float* __restrict__ diagU, int* __restrict__ ipvt, int* __restrict__ src,
     int* __restrict__ status, long spin_limit, unsigned phantom) {
 #pragma clang fp contract(off)
     constexpr int LDT = B + 1;
-    constexpr int TPC = PNT / B;  // threads per column in the update
     constexpr int NF = (B + PNT) / PNT;  // row words per thread (B + 1 of them)
     extern __shared__ __attribute__((aligned(16))) float sm[];
     float* tile = sm;
-    float* urow = sm + (size_t)R * LDT;
+    float* urow = sm + ((size_t)LDT << R_sh);
     float* lcol = urow + LDT;
     __shared__ unsigned long long skey[PNT / 64], wkey[PNT / 64];
     __shared__ float wval[PNT / 64][2];
     __shared__ float kval[2];
     __shared__ int abort_flag;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int R = 1 << R_sh;
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int G = gridDim.x, g = blockIdx.x;
-    const int64_t p0 = k0 + (int64_t)g * R;  // position of local row 0
-    const int rows = (int)min<int64_t>((int64_t)R, n - p0);
+    // positions fit 32 bits (the host checks n)
+    const int kb = (int)k0, nn = (int)n;
+    const int p0 = kb + (g << R_sh);  // position of local row 0
+    const int rows = min(R, nn - p0);
     const size_t kstride = (size_t)gslots * kSlotWords;
     if (t == 0) abort_flag = 0;
 
@@ -165,7 +211,7 @@ __global__ __launch_bounds__(PNT) void panel_pivot_kernel(
             for (int u = 0; u < 16; ++u) {
                 const int e = e0 + u * PNT;
                 if (e < nv)
-                    v[u] = *reinterpret_cast<const float4*>(X + (p0 + e / Q) * ldx + k0 +
+                    v[u] = *reinterpret_cast<const float4*>(X + (int64_t)(p0 + e / Q) * ldx + k0 +
                                                             (e % Q) * 4);
             }
 #pragma unroll
@@ -181,21 +227,20 @@ __global__ __launch_bounds__(PNT) void panel_pivot_kernel(
             }
         }
     }
-    for (int r = t; r < rows; r += PNT) tile[r * LDT + B] = __int_as_float((int)(p0 + r));
+    for (int r = t; r < rows; r += PNT) tile[r * LDT + B] = __int_as_float(p0 + r);
     __syncthreads();
 
-    // the workgroup's best candidate of column c (rows at positions >= k)
-    auto search = [&](int c) {
-        const int64_t k = k0 + c;
-        unsigned long long b = 0;
-        for (int r = (int)max<int64_t>(0, k - p0) + t; r < rows; r += PNT)
-            b = max(b, pivot_key(tile[r * LDT + c], p0 + r, k));
-        b = wave_max_u64(b);
-        if (lane == 0) skey[wave] = b;
+    // The workgroup's best candidate among its threads' keys: thread t holds row
+    // t's (R <= PNT), rising positions in rising lanes.  One barrier, which
+    // also orders what the threads wrote before.
+    auto best_of = [&](unsigned long long b) {
+        if (wave * 64 < R) {
+            b = lane_u64(b, first_best(key_rank(b)));
+            if (lane == 0) skey[wave] = b;
+        }
         __syncthreads();
         b = skey[0];
-#pragma unroll
-        for (int w = 1; w < PNT / 64; ++w) b = max(b, skey[w]);
+        for (int w = 1; w * 64 < R; ++w) b = max(b, skey[w]);
         return b;
     };
     // Publish column c's candidate `best`: the whole row, row k when this
@@ -205,37 +250,38 @@ __global__ __launch_bounds__(PNT) void panel_pivot_kernel(
     // beyond c (the same float product and sum), and the workgroup updates
     // those columns after publishing, while the others arrive.
     auto publish = [&](int c, unsigned long long best, bool upd) {
-        const int64_t k = k0 + c;
-        const unsigned tag = (unsigned)(k + 1);
+        const int kp = kb + c;
+        const unsigned tag = (unsigned)(kp + 1);
         const int buf = c & 1;
-        const int64_t rk = k - p0;
+        const int rk = kp - p0;
         const bool own_k = rk >= 0 && rk < rows;
+        const bool some = best != 0;
+        const int rl = some ? (int)key_position(best, kp) - p0 : 0;
         auto cur = [&](int r, int j) {
             float v = tile[r * LDT + j];
             if (upd && j > c && j < B) v = v + lcol[r] * urow[j];
             return v;
         };
-        const int rl = best != 0 ? (int)(key_position(best, k) - p0) : 0;
-        if (best != 0) {
-            unsigned long long* slot = pub + ((int64_t)buf * G + g) * LDT;
-            for (int j = t; j <= B; j += PNT) put_tagged(slot + j, __float_as_uint(cur(rl, j)), tag);
+        // the key slot, which every workgroup polls, by the last wave while
+        // the first ones publish the rows: lanes 0..5 a word each
+        if (wave == PNT / 64 - 1) {
+            if (lane < 6 && (lane < 2 || (lane < 4 ? some : own_k))) {
+                unsigned v = lane == 0 ? (unsigned)best : (unsigned)(best >> 32);
+                if (lane >= 2) {
+                    const int j = c + (lane & 1);
+                    v = j < B ? __float_as_uint(cur(lane < 4 ? rl : rk, j)) : 0u;
+                }
+                put_tagged(kslot + (size_t)buf * kstride + (size_t)g * kSlotWords + lane, v, tag);
+            }
+            return;
+        }
+        if (some) {
+            unsigned long long* slot = pub + (size_t)(buf * G + g) * LDT;
+            for (int j = t; j <= B; j += PNT - 64) put_tagged(slot + j, __float_as_uint(cur(rl, j)), tag);
         }
         if (own_k)
-            for (int j = t; j <= B; j += PNT)
-                put_tagged(krow + buf * LDT + j, __float_as_uint(cur((int)rk, j)), tag);
-        if (t == 0) {
-            unsigned long long* w = kslot + (size_t)buf * kstride + (size_t)g * kSlotWords;
-            if (best != 0) {
-                put_tagged(w + 2, __float_as_uint(cur(rl, c)), tag);
-                put_tagged(w + 3, c + 1 < B ? __float_as_uint(cur(rl, c + 1)) : 0u, tag);
-            }
-            if (own_k) {
-                put_tagged(w + 4, __float_as_uint(cur((int)rk, c)), tag);
-                put_tagged(w + 5, c + 1 < B ? __float_as_uint(cur((int)rk, c + 1)) : 0u, tag);
-            }
-            put_tagged(w + 0, (unsigned)best, tag);
-            put_tagged(w + 1, (unsigned)(best >> 32), tag);
-        }
+            for (int j = t; j <= B; j += PNT - 64)
+                put_tagged(krow + buf * LDT + j, __float_as_uint(cur(rk, j)), tag);
     };
     // give up: raise the status, mark this workgroup's key slots (both
     // parities) with the abort tag so that every waiter is released
@@ -256,10 +302,10 @@ __global__ __launch_bounds__(PNT) void panel_pivot_kernel(
     // gave up or another workgroup did.  wkey / wval are next written after
     // several barriers, so they need no barrier after the reads here.
     auto exchange = [&](int c, bool* ok, float* u0, float* u1) {
-        const unsigned tag = (unsigned)(k0 + c + 1);
+        const unsigned tag = (unsigned)(kb + c + 1);
         const unsigned long long* ks = kslot + (size_t)(c & 1) * kstride;
         const int GW = G + (int)phantom;
-        const int gk = c / R;  // the group holding position k
+        const int gk = c >> R_sh;  // the group holding position k
         unsigned long long mx = 0;
         float m0 = 0.0f, m1 = 0.0f;
         bool fail = false;
@@ -301,16 +347,19 @@ __global__ __launch_bounds__(PNT) void panel_pivot_kernel(
         }
         if (fail) abort_flag = 1;
         // the maximum key with its values, over the wave, then the workgroup
-        for (int o = 32; o > 0; o >>= 1) {
-            const unsigned lo = __shfl_xor((unsigned)mx, o);
-            const unsigned hi = __shfl_xor((unsigned)(mx >> 32), o);
-            const float o0 = __shfl_xor(m0, o), o1 = __shfl_xor(m1, o);
-            const unsigned long long om = ((unsigned long long)hi << 32) | lo;
-            if (om > mx) {
-                mx = om;
-                m0 = o0;
-                m1 = o1;
+        if (GW <= PNT) {  // one slot per thread: rising positions in rising lanes
+            if (wave * 64 < GW) {
+                const int bl = first_best(key_rank(mx));
+                mx = lane_u64(mx, bl);
+                m0 = __uint_as_float(lane_u32(__float_as_uint(m0), bl));
+                m1 = __uint_as_float(lane_u32(__float_as_uint(m1), bl));
             }
+        } else {
+            const unsigned long long best = wave_max_u64(mx);
+            const int bl = __ffsll((unsigned long long)__ballot(mx == best)) - 1;
+            mx = best;
+            m0 = __uint_as_float(lane_u32(__float_as_uint(m0), bl));
+            m1 = __uint_as_float(lane_u32(__float_as_uint(m1), bl));
         }
         if (lane == 0) {
             wkey[wave] = mx;
@@ -321,8 +370,7 @@ __global__ __launch_bounds__(PNT) void panel_pivot_kernel(
         *ok = abort_flag == 0;
         int bw = 0;
         mx = wkey[0];
-#pragma unroll
-        for (int w = 1; w < PNT / 64; ++w)
+        for (int w = 1; w < PNT / 64 && w * 64 < GW; ++w)
             if (wkey[w] > mx) {
                 mx = wkey[w];
                 bw = w;
@@ -332,7 +380,8 @@ __global__ __launch_bounds__(PNT) void panel_pivot_kernel(
         return mx;
     };
 
-    publish(0, search(0), false);
+    publish(0, best_of(t < rows && p0 + t >= kb ? pivot_key(tile[t * LDT], p0 + t, kb) : 0ull),
+            false);
     for (int c = 0; c < B; ++c) {
         bool ok = true;
         float piv = 0.0f, u1 = 0.0f;
@@ -341,23 +390,22 @@ __global__ __launch_bounds__(PNT) void panel_pivot_kernel(
             give_up();
             return;
         }
-        const int64_t k = k0 + c;
-        const unsigned tag = (unsigned)(k + 1);
+        const int kp = kb + c;
+        const unsigned tag = (unsigned)(kp + 1);
         const int buf = c & 1;
-        const int64_t rk = k - p0;  // local row of position k (may be outside)
-        int64_t p = key_position(win, k);
-        if (p < k || p >= n) {  // cannot happen with a complete exchange; never index with it
+        const int rk = kp - p0;  // local row of position kp (may be outside)
+        int p = (int)key_position(win, kp);
+        if (p < kp || p >= nn) {  // cannot happen with a complete exchange; never index with it
             if (t == 0) atomicOr(status, 4);
-            p = k;
+            p = kp;
         }
-        const int gw = (int)((p - k0) / R);
-        const int64_t rp = p - p0;
-        const bool swap = p != k;
+        const int rp = p - p0;
+        const bool swap = p != kp;
         const bool own_k = swap && rk >= 0 && rk < rows;
         const bool own_p = swap && rp >= 0 && rp < rows;
-        // the whole winning row (and row k where position p is ours) start
+        // the whole winning row (and row kp where position p is ours) start
         // now and are checked after the search of column c+1
-        const unsigned long long* wrow = pub + ((int64_t)buf * G + gw) * LDT;
+        const unsigned long long* wrow = pub + (size_t)(buf * G + ((p - kb) >> R_sh)) * LDT;
         const unsigned long long* krw = krow + buf * LDT;
         unsigned long long fw[NF], fk[NF];
 #pragma unroll
@@ -366,44 +414,32 @@ __global__ __launch_bounds__(PNT) void panel_pivot_kernel(
             fw[i] = j <= B ? get_tagged(wrow + j) : 0ull;
             fk[i] = (own_p && j <= B) ? get_tagged(krw + j) : 0ull;
         }
-        if (t == 0) {
-            if (g == 0) {
-                ipvt[k] = (int)p;
-                diagU[k] = piv;
-                if (!(piv != 0.0f) || !__builtin_isfinite(piv)) atomicOr(status, 1);
-            }
-            // the exchanged rows' values at columns c and c+1 (the rest of
-            // the rows follows from the fetches)
-            if (own_k) {
-                tile[rk * LDT + c] = piv;
-                if (c + 1 < B) tile[rk * LDT + c + 1] = u1;
-            }
-            if (own_p) {
-                tile[rp * LDT + c] = kval[0];
-                if (c + 1 < B) tile[rp * LDT + c + 1] = kval[1];
+        if (t == 0 && g == 0) {
+            ipvt[kp] = p;
+            diagU[kp] = piv;
+            if (!(piv != 0.0f) || !__builtin_isfinite(piv)) atomicOr(status, 1);
+        }
+        // ---- one thread per row below position kp, no barrier between: its
+        // multiplier (gefa_ref: double reciprocal and product, rounded once),
+        // its update of column c+1 and its key there.  Row kp's values, where
+        // they move here, come with the exchange.
+        const int rs1 = max(0, rk + 1);
+        unsigned long long key = 0;
+        if (t >= rs1 && t < rows) {
+            const bool moved = own_p && t == rp;
+            const double inv = -1.0 / (double)piv;
+            const float l = (float)((double)(moved ? kval[0] : tile[t * LDT + c]) * inv);
+            tile[t * LDT + c] = l;
+            lcol[t] = l;
+            if (c + 1 < B) {
+                const float v = (moved ? kval[1] : tile[t * LDT + c + 1]) + l * u1;
+                tile[t * LDT + c + 1] = v;
+                key = pivot_key(v, p0 + t, kp + 1);
             }
         }
-        __syncthreads();
-        // ---- multipliers of the rows below position k (gefa_ref: double
-        // reciprocal and product, rounded once)
-        const int rs1 = (int)max<int64_t>(0, k + 1 - p0);
-        const double inv = -1.0 / (double)piv;
-        for (int r = rs1 + t; r < rows; r += PNT) {
-            const float l = (float)((double)tile[r * LDT + c] * inv);
-            tile[r * LDT + c] = l;
-            lcol[r] = l;
-        }
-        __syncthreads();
-        unsigned long long next = 0;
-        if (c + 1 < B) {
-            // column c+1 first, one row per thread: the next search reads it
-            for (int r = rs1 + t; r < rows; r += PNT)
-                tile[r * LDT + c + 1] = tile[r * LDT + c + 1] + lcol[r] * u1;
-            __syncthreads();
-            next = search(c + 1);
-        }
-        // ---- the fetched rows: the pivot row into urow and position k, row k
-        // into position p (its columns c and c+1 are already in place)
+        const unsigned long long next = best_of(key);
+        // ---- the fetched rows: the pivot row into urow and position kp, row
+        // kp into position p (its columns c and c+1 are already in place)
         bool fail = false;
 #pragma unroll
         for (int i = 0; i < NF; ++i) {
@@ -437,24 +473,38 @@ __global__ __launch_bounds__(PNT) void panel_pivot_kernel(
         if (c + 1 == B) break;
         publish(c + 1, next, true);
         __syncthreads();  // the published rows were read before they change
-        // the other columns, one column per TPC threads, 16 rows in flight
-        const int j = t % B;
-        if (j > c + 1) {
-            const float uj = urow[j];
-            int r = rs1 + t / B;
-            for (; r + 15 * TPC < rows; r += 16 * TPC) {
-                float v[16], lv[16];
+        // ---- the other columns: a lane per column, 64 rows at a time from the
+        // last one up, eight of them per wave and all in flight; a row's
+        // multiplier comes from the lane that read it.  (The next exchange's
+        // barrier orders this with what reads these columns.)
+        for (int rt = rows; rt > rs1; rt -= 64) {
+            const int r0 = rt - 64 + wave;  // rows r0 + 8 i
+            const int rl = r0 + 8 * (lane & 7);
+            const float lv = rl >= rs1 ? lcol[rl] : 0.0f;
+            for (int jb = c + 2; jb < B; jb += 64) {
+                const int j = jb + lane;
+                if (j >= B) continue;
+                const float uj = urow[j];
+                float* q = tile + r0 * LDT + j;
+                if (r0 >= rs1) {
+                    float v[8];
 #pragma unroll
-                for (int u = 0; u < 16; ++u) {
-                    v[u] = tile[(r + u * TPC) * LDT + j];
-                    lv[u] = lcol[r + u * TPC];
+                    for (int i = 0; i < 8; ++i) v[i] = q[8 * i * LDT];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) v[i] = v[i] + bcast_lane(lv, i) * uj;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) q[8 * i * LDT] = v[i];
+                } else {
+                    // part of the rows lie above: only those from rs1 on
+                    float v[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) v[i] = r0 + 8 * i >= rs1 ? q[8 * i * LDT] : 0.0f;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        if (r0 + 8 * i >= rs1) q[8 * i * LDT] = v[i] + bcast_lane(lv, i) * uj;
                 }
-#pragma unroll
-                for (int u = 0; u < 16; ++u) tile[(r + u * TPC) * LDT + j] = v[u] + lv[u] * uj;
             }
-            for (; r < rows; r += TPC) tile[r * LDT + j] = tile[r * LDT + j] + lcol[r] * uj;
         }
-        __syncthreads();
     }
     // ---- write back: the panel (-1/u_kk on the diagonal, the encoding of
     // the unpivoted path), the transposed multipliers below the block for the
@@ -462,12 +512,12 @@ __global__ __launch_bounds__(PNT) void panel_pivot_kernel(
     for (int e = t; e < rows * B; e += PNT) {
         const int r = e / B, c = e % B;
         float v = tile[r * LDT + c];
-        if (p0 + r == k0 + c) v = (float)(-1.0 / (double)v);
-        X[(p0 + r) * ldx + k0 + c] = v;
+        if (p0 + r == kb + c) v = (float)(-1.0 / (double)v);
+        X[(int64_t)(p0 + r) * ldx + k0 + c] = v;
     }
     for (int c = 0; c < B; ++c)
         for (int r = t; r < rows; r += PNT)
-            if (p0 + r >= k0 + B) Lt[(int64_t)c * ldl + p0 + r] = tile[r * LDT + c];
+            if (p0 + r >= kb + B) Lt[(int64_t)c * ldl + p0 + r] = tile[r * LDT + c];
     for (int r = t; r < rows; r += PNT) src[p0 + r] = __float_as_int(tile[r * LDT + B]);
 }
 
@@ -617,11 +667,22 @@ hipError_t launch_transpose_square(float* A, int64_t ld, int64_t n, hipStream_t 
     return hipGetLastError();
 }
 
-int panel_pivot_rows(int B) { return B >= 256 ? 128 : 256; }
+namespace {
+// log2 of the rows per workgroup of a panel of m rows.  A workgroup's share of
+// each column's update sits on the column's chain, so the panel spreads over
+// up to half the CUs with 64 rows each before the workgroups grow (the other
+// half runs the trailing update beside it); at most what the LDS holds.  A
+// 128-column panel alone, us, with 64 / 128 / 256 rows: m = 2048 377 / 440 /
+// 572, 6144 396 / 443 / 556, 12288 426 / 461 / 556, 16384 461 / 462 / 561; with
+// 32 rows 6144 takes 457 (twice the slots to poll).
+int panel_rows_sh(int64_t m, int B) {
+    const int most = B >= 256 ? 7 : 8;
+    return std::min(most, m <= 64 * 128 ? 6 : m <= 128 * 128 ? 7 : 8);
+}
+}  // namespace
 
 namespace {
-size_t panel_pivot_lds(int B) {
-    const int R = panel_pivot_rows(B);
+size_t panel_pivot_lds(int R, int B) {
     return ((size_t)R * (B + 1) + (B + 1) + R) * sizeof(float);
 }
 // Dynamic LDS requested at least, so that a CU holds at most one panel
@@ -630,13 +691,19 @@ size_t panel_pivot_lds(int B) {
 constexpr size_t kSpreadLds = 96 * 1024;
 }  // namespace
 
-int panel_pivot_groups(int64_t m, int B) {
-    const int R = panel_pivot_rows(B);
-    return (int)((m + R - 1) / R);
+int panel_pivot_groups(int64_t n, int B) {
+    // the largest count of any panel of up to n rows: shorter panels can have
+    // more, smaller workgroups
+    int64_t g = 0;
+    for (int64_t m : {n, std::min<int64_t>(n, 64 * 128), std::min<int64_t>(n, 128 * 128)}) {
+        const int sh = panel_rows_sh(m, B);
+        g = std::max<int64_t>(g, (m + (1 << sh) - 1) >> sh);
+    }
+    return (int)g;
 }
 
 hipError_t panel_pivot_prepare(int B, int* max_groups) {
-    const size_t lds = panel_pivot_lds(B);
+    const size_t lds = panel_pivot_lds(B >= 256 ? 128 : 256, B);  // the largest workgroup's
     const void* k = nullptr;
     switch (B) {
         case 32: k = reinterpret_cast<const void*>(panel_pivot_kernel<32>); break;
@@ -665,25 +732,25 @@ hipError_t launch_panel_pivot(float* X, int64_t ldx, int64_t n, int64_t k0, int 
                               unsigned long long* kslot, int gslots, float* Lt, int64_t ldl,
                               float* diagU, int* ipvt, int* src, int* status, int max_groups,
                               int num_cu, hipStream_t s, long spin_limit) {
-    const int R = panel_pivot_rows(B);
     // spin_limit < 0: give up after -spin_limit polls, waiting for one more
     // workgroup than the grid holds, so that every exchange gives up (the
     // error path, exercised from the host with every kernel exiting)
     const unsigned phantom = spin_limit < 0 ? 1u : 0u;
     spin_limit = spin_limit == 0 ? kSpinLimit : (spin_limit < 0 ? -spin_limit : spin_limit);
     const int64_t m = n - k0;
-    const int G = panel_pivot_groups(m, B);
+    const int sh = panel_rows_sh(m, B);
+    const int G = (int)((m + (1 << sh) - 1) >> sh);
     if (G < 1 || G > max_groups || G + (int)phantom > gslots ||
         G + (int)phantom > kMaxPanelGroups)
         return hipErrorInvalidConfiguration;
     // 16-byte row vectors; tags are positions + 1 and must stay below the abort tag
     if ((ldx & 3) || (k0 & 3) || (reinterpret_cast<uintptr_t>(X) & 15) || n >= (1LL << 31))
         return hipErrorInvalidValue;
-    size_t lds = panel_pivot_lds(B);
+    size_t lds = panel_pivot_lds(1 << sh, B);
     if (G <= num_cu) lds = std::max(lds, kSpreadLds);
 #define HPL_PANEL(BB)                                                                        \
     case BB:                                                                                 \
-        panel_pivot_kernel<BB><<<G, PNT, lds, s>>>(X, ldx, n, k0, R, pub, krow, kslot, gslots, \
+        panel_pivot_kernel<BB><<<G, PNT, lds, s>>>(X, ldx, n, k0, sh, pub, krow, kslot, gslots, \
                                                    Lt, ldl, diagU, ipvt, src, status,          \
                                                    spin_limit, phantom);                       \
         break;
