@@ -634,13 +634,12 @@ hpl_status ensure_block_inverses(hpl_ctx* c) {
     if (c->binv_ready) return HPL_SUCCESS;
     const uint32_t B = c->B;
     if (B > 256) return HPL_SUCCESS;  // sequential diagonal solves
-    // a pivoted factor keeps the 32 x 32 diagonal solves: the diagonal blocks
-    // of U of a matrix that is not diagonally dominant can be poorly
-    // conditioned, and applying a whole B x B inverse loses up to a digit
-    // there (B = 256, uniform matrices: 1.8e-3 against 4e-4 with 32 x 32)
-    if (c->pivoted) return HPL_SUCCESS;
     const hplx::WsPlan w = plan_factor_ws(c->n, B, c->prec, 1);
     hpl_status st = ensure(c, c->dBInv, c->capBInv, w.binv);
+    if (st && c->pivoted) {
+        c->err.clear();  // no room: the per-step launches solve
+        return HPL_SUCCESS;
+    }
     if (st) return st;
     HIPCHK(c, launch_block_inverse(c->dA, (int64_t)c->lda, (int64_t)c->n, (int)B, c->dInv,
                                    3 * (B / 32) * 1024, c->dBInv, c->s0));
@@ -991,7 +990,7 @@ hpl_status hpl_gefa_dev(hpl_ctx* c, uint32_t block, hpl_prec prec, hpl_timing* t
     st = check_status(c);  // waits for the stream
     if (t) t->gefa_s = elapsed_s(c);
     if (st) return st;
-    c->B = block;
+    c->B = c->pivoting ? 32 : block;  // a pivoted factor is substituted in blocks of 32
     c->factored = true;
     c->pivoted = c->pivoting;
     c->binv_ready = c->binv_in_gefa;

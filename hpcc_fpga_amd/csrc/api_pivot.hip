@@ -95,6 +95,21 @@ void parallel_rows(uint64_t n, F f) {
 
 namespace hplx {
 
+// A pivoted factor is substituted in blocks of 32: the diagonal blocks of U of
+// a matrix that is not diagonally dominant can be poorly conditioned, and
+// applying a whole B x B inverse loses up to a digit there (B = 256, uniform
+// matrices: 1.8e-3 against 4e-4 with 32 x 32).  So c->B is 32 for it and the
+// substitutions that apply whole inverses take the 32 x 32 ones: one launch for
+// a right-hand side (n = 6144: 1.4 ms as 96 launches, now 0.69; n = 32768
+// B = 256 10.3 -> 4.6; n = 64 0.019 -> 0.016), the MFMA sweeps for several (16
+// refined at n = 4096: 13.7 -> 5.0 ms).  Residual of an unrefined solution,
+// means over 8 to 16 matrices: n = 1024 8.1e-7 -> 7.9e-7, 2048 1.13e-6 ->
+// 1.17e-6, 4096 1.67e-6 -> 1.57e-6, 6144 2.05e-6 -> 2.03e-6.
+hpl_status prep_solve_blocks(hpl_ctx* c) {
+    PCHK(c, launch_prep_all(c->dA, (int64_t)c->lda, 32, (int)(c->n / 32), c->dInv, 3 * 1024, c->s0));
+    return HPL_SUCCESS;
+}
+
 hpl_status gefa_pivot(hpl_ctx* c, uint32_t B) {
     const int64_t n = (int64_t)c->n, lda = (int64_t)c->lda;
     if (B < 32 || B > 256) return fail(c, HPL_ERR_UNSUPPORTED, "pivoting needs a block in [32, 256]");
@@ -171,7 +186,7 @@ hpl_status gefa_pivot(hpl_ctx* c, uint32_t B) {
     if (rest_pending) PCHK(c, hipStreamWaitEvent(s, c->evP, 0));
     PCHK(c, launch_transpose_square(c->dA, lda, n, s));
     // the substitution's 32 x 32 inverses, from the final factor
-    PCHK(c, launch_prep_all(c->dA, lda, (int)B, (int)N, c->dInv, inv_stride, s));
+    if (hpl_status ps = prep_solve_blocks(c)) return ps;
     return HPL_SUCCESS;
 }
 
@@ -272,9 +287,9 @@ hpl_status hpl_gesl_pvt(hpl_ctx* c, const float* lu, float* b, const int32_t* ip
     PCHK(c, c->stage.to_device(c->s0, c->dPiv, ipvt, n * sizeof(int32_t)));
     PCHK(c, c->stage.to_device(c->s0, c->dPerm, perm.data(), n * sizeof(int32_t)));
     PCHK(c, c->stage.to_device(c->s0, c->dDiagU, u.data(), n * sizeof(float)));
-    PCHK(c, launch_prep_all(c->dA, (int64_t)c->lda, (int)B, (int)(n / B), c->dInv,
-                            3 * (B / 32) * 1024, c->s0));
-    c->B = B;
+    st = hplx::prep_solve_blocks(c);
+    if (st) return st;
+    c->B = 32;
     c->factored = true;
     c->pivoted = true;
     c->binv_ready = false;

@@ -258,6 +258,8 @@ hpl_status alloc_factor_workspace(hpl_ctx* c, uint32_t B);
 // Partial-pivoting factorisation of the resident matrix (FP32, B <= 256) on
 // stream s0, leaving the factor, dPiv, dPerm, dDiagU and the GESL inverses.
 hpl_status gefa_pivot(hpl_ctx* c, uint32_t B);
+// the 32 x 32 inverses that a pivoted factor's substitution applies, into dInv
+hpl_status prep_solve_blocks(hpl_ctx* c);
 // Rewrite a downloaded pivoted factor (host, row-major, lda) into gefa_ref's
 // layout: u_kk on the diagonal, each column's multipliers in the row order of
 // its own step.

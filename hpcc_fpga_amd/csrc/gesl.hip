@@ -530,7 +530,12 @@ __global__ __launch_bounds__(NT) void gesl_persist_kernel(const float* __restric
     constexpr int RPT = B / RG;         // rows of a tile per thread
     static_assert(RPT >= 1 && RPT * RG == B, "tile split");
     static_assert(B <= NT && T <= kMaxT, "one share column per thread");
-    __shared__ float zown[kMaxOwn * S];  // running sums of the owned slices
+    // running sums of the owned slices; a sum over blocks of 32 has up to n/32
+    // serial terms, so it carries its rounding errors along (zlo), which keeps
+    // the residual below that of the sums over whole blocks it stands in for
+    constexpr bool kCarry = B == 32;
+    __shared__ float zown[kMaxOwn * S];
+    __shared__ float zlo[kCarry ? kMaxOwn * S : 1];
     __shared__ float vbuf[B];            // the awaited block vector
     __shared__ float red[RG * S];
     __shared__ int abort_flag;
@@ -541,7 +546,10 @@ __global__ __launch_bounds__(NT) void gesl_persist_kernel(const float* __restric
     unsigned* flag = ws.flags;
 
     for (int k = 0; k < own; ++k)
-        for (int c = t; c < S; c += NT) zown[k * S + c] = x[(int64_t)(g + k * G) * S + c];
+        for (int c = t; c < S; c += NT) {
+            zown[k * S + c] = x[(int64_t)(g + k * G) * S + c];
+            if (kCarry) zlo[k * S + c] = 0.0f;
+        }
 
     f32x4 tile[RPT];
     // rows p = rg + RG i (stride ld) of base, the 4 columns of group cg
@@ -550,8 +558,9 @@ __global__ __launch_bounds__(NT) void gesl_persist_kernel(const float* __restric
         for (int i = 0; i < RPT; ++i)
             tile[i] = *reinterpret_cast<const f32x4*>(base + (int64_t)(rg + RG * i) * ld + 4 * cg);
     };
-    // out[c] += sign * sum_p tile[p][c] vbuf[p]
-    auto gemv = [&](float* out, float sign) {
+    // zown[k S + c] += sign * sum_p tile[p][c] vbuf[p]
+    auto gemv = [&](int k, float sign) {
+        float* out = zown + k * S;
         f32x4 a = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int i = 0; i < RPT; ++i) {
@@ -567,7 +576,13 @@ __global__ __launch_bounds__(NT) void gesl_persist_kernel(const float* __restric
             float sum = 0.0f;
 #pragma unroll 8
             for (int r = 0; r < RG; ++r) sum += red[r * S + t];
-            out[t] = out[t] + sign * sum;
+            if (kCarry) {
+                const float z = out[t], y = fmaf(sign, sum, zlo[k * S + t]), w = z + y;
+                zlo[k * S + t] = fabsf(z) >= fabsf(y) ? y - (w - z) : z - (w - y);
+                out[t] = w;
+            } else {
+                out[t] = out[t] + sign * sum;
+            }
         }
         __syncthreads();
     };
@@ -634,7 +649,7 @@ __global__ __launch_bounds__(NT) void gesl_persist_kernel(const float* __restric
         load_tile(A + (int64_t)q * B * lda + (int64_t)s * S, lda);
         if (wait(flag + (int64_t)q * T, fwd ? 1u : 2u)) return true;
         fetch_sum(q, fwd ? ws.pf : ws.pb, 0, B, vbuf);
-        gemv(zown + k * S, fwd ? 1.0f : -1.0f);
+        gemv(k, fwd ? 1.0f : -1.0f);
         return false;
     };
     __syncthreads();
@@ -659,6 +674,7 @@ __global__ __launch_bounds__(NT) void gesl_persist_kernel(const float* __restric
         if (blk == N - 1) share_load(N - 1, s, false);
         if (wait(flag + (int64_t)blk * T, 1u)) return;
         fetch_sum(blk, ws.pf, (s - blk * T) * S, S, zown + k * S);
+        if (kCarry && t < S) zlo[k * S + t] = 0.0f;
         if (blk == N - 1) share(k, s, false);
     }
     for (int q = N - 1; q >= 1; --q)

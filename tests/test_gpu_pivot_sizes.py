@@ -56,3 +56,25 @@ def test_short_last_workgroup(ctx, n, B):
     # rounding of another summation order
     assert np.array_equal(f[:B].view(np.uint32), f_ref[:B].view(np.uint32))
     assert np.max(np.abs(f - f_ref)) <= 1e-3 * np.max(np.abs(f_ref))
+
+
+@pytest.mark.parametrize("n,B", [(32, 32), (96, 32), (320, 64), (512, 256)])
+@pytest.mark.parametrize("nrhs", [1, 3, 16])
+def test_substitution_in_blocks_of_32(ctx, n, B, nrhs):
+    print(f"pivoted n={n} B={B} nrhs={nrhs}", flush=True)
+    ctx.keep_original(True)
+    ctx.set_pivoting(True)
+    try:
+        ctx.generate(n, 2, n)
+        a, _ = ctx.download(matrix=True, solution=False)
+        ctx.gefa_dev(B)
+        b = np.random.default_rng(n).random((n, nrhs)) - 0.5
+        x, res = ctx.solve_rhs64(b)
+    finally:
+        ctx.set_pivoting(False)
+        ctx.keep_original(False)
+    M = a.astype(np.float64).T
+    r = np.abs(b - M @ x).max(axis=0)
+    scale = np.abs(M).sum(axis=1).max() * np.abs(x).max(axis=0) + np.abs(b).max(axis=0)
+    assert all(q["converged"] for q in res)
+    assert np.all(r <= 1e-14 * n * scale)
