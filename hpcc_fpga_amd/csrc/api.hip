@@ -239,11 +239,9 @@ hpl_status factor_diag(hpl_ctx* c, hipStream_t st, int64_t off, uint32_t B, floa
     const int64_t lda = (int64_t)c->lda;
     if (B <= (uint32_t)kMaxLeafLU) {
         // Beside an FP32 bulk update of many tiles (two workgroups of 16 waves
-        // on every CU) the 8-wave workgroup waits longer for a place than its
-        // shorter run gains: n = 32768 207.0 ms with 8 waves throughout, 201.0
-        // with 4, 200.9 with 4 while more than 6144 of the order are left; n =
-        // 2048: 1.71 ms with 8, 1.81 with 4.  The 16-bit and 8-bit updates
-        // leave room for either (n = 65536 BF16: 252.4 ms with 8, 253.5 with 4).
+        // on every CU) a 16-wave workgroup waits longer for a place than its
+        // shorter run gains (figures at the launch); while no more than 6144 of
+        // the order are left it does not (n = 7168: 5.4 ms either way).
         const bool narrow = c->prec == HPL_PREC_FP32 && (int64_t)c->n - off > 6144;
         HIPCHK(c, launch_lu_diag(c->dA, lda, off, B, c->dStatus, DT, ldt, inv, inv_ts, narrow, st));
         return HPL_SUCCESS;

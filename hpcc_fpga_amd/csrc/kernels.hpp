@@ -8,8 +8,8 @@
 // to 1 on a zero/non-finite pivot.  DT (leading dimension ldt) receives the
 // factorised block transposed, and inv the inverses of its 32 x 32 diagonal
 // sub-blocks as launch_prep writes them, those of one type inv_ts floats apart
-// (a larger block's parts pass their places in its DT and inv).  narrow: 256
-// threads instead of 512, for a device that other launches fill.
+// (a larger block's parts pass their places in its DT and inv).  narrow: 8
+// waves instead of 16 at B = 128, for a device that other launches fill.
 hipError_t launch_lu_diag(float* A, int64_t lda, int64_t off, int B, int* status, float* DT,
                           int64_t ldt, float* inv, int64_t inv_ts, bool narrow, hipStream_t s);
 

@@ -9,36 +9,39 @@
 // Every element receives the same multiplies and adds in the same order as in
 // the reference loop (no FMA contraction), so the result is bit-identical.
 //
-// One workgroup; the block lives in LDS and is processed in panels of 32
-// pivot rows, three stages per panel:
-//   A. wave 0 factorises the panel's 32 x 32 diagonal sub-block.  The other
-//      waves apply the previous panel's rank-32 update to the blocks that
-//      this panel's stage C does not need, and at the last panel store what
-//      is finished.
-//   B. every column right of the sub-block (top strip) and every row below it
-//      (left strip) is solved against the sub-block, 32 vectors per wave, and
-//      one further wave of each kind solves for the 32 unit vectors: those
-//      are the sub-block's inverses.
-//   C. the next diagonal sub-block alone receives this panel's update.
-// So the chain from pivot to pivot holds A, one strip solve and one 32 x 32
-// update per panel, not the whole trailing update.
+// One workgroup; the block lives in LDS and is processed in panels of 16
+// pivot rows, two stages per panel:
+//   1. wave 0 applies the previous panel's rank-16 update to the panel's 16 x 16
+//      diagonal sub-block and factorises it in registers.  The other waves apply
+//      that update to the rest, carry on the solves of the unit vectors that
+//      give the inverses, and in the last half of the panels store what is
+//      finished.
+//   2. every column right of the sub-block (top strip) and every row below it
+//      (left strip) is solved against the sub-block, 16 vectors per wave.
+// So the chain from pivot to pivot holds one 16 x 16 update, one factorisation
+// and one 16-step solve per panel, not the whole trailing update.
 //
-// Bound: instruction latency of stage A's single wave (a pivot step is about
-// 45 instructions, 320 cycles) and of the 32-step strip solves (180 cycles a
-// step).  In A and B a lane holds 16 values of one vector -- rows (or
-// columns) of one parity, the two halves of the wave holding the two
-// parities -- so a step's updates take half the instructions of one lane per
-// vector.  A's multipliers are broadcast within each half by ds_swizzle right
-// after the row's update, one step ahead of their use; the next pivot's row
-// goes first and its reciprocal's chain is issued between the other rows.
-// B = 128 alone on the device: 39.6 us with the inverses and DT, against
-// 62.2 us for the former one-stage-at-a-time kernel and a further launch of 8
-// us for those (B = 64: 21.3 against 26.1 + 8; B = 32: 11.0 against 9.2 + 7);
-// GEFA + GESL at n = 2048, B = 128: 2.36 -> 1.91 ms.
-// At most 128 VGPRs and 91 KiB of LDS: the workgroup fits into what one of
-// the two workgroups of the FP32 trailing update on a CU leaves, whichever of
-// the two ends first (with 109 KiB, a second buffer of the left strip, only
-// after the second one: 4% on n = 32768).
+// Bound: the instructions of one wave, of which one issues every 6 to 8 cycles
+// whether the next depends on it or not: a pivot step of stage 1 is 25 of them
+// (168 cycles), a step of stage 2 15 (100).  Hence 16-wide panels (a step of a
+// 32-wide one took 45 and 320 cycles): the columns of a sub-block lie in the 16
+// lanes of a DPP row, so that a multiplier is broadcast within the multiply
+// (row_newbcast) and needs neither LDS nor an instruction of its own; the
+// strips have an element of their vectors per lane for the same reason.  Masks
+// are immediates of the exec register, one change for all rows of a step.  The
+// scaled rows stay in registers of their own beside the multipliers and are
+// put together once per panel.
+// A tile of the trailing update is 4000 to 5000 cycles of one wave, also when it
+// is alone on its SIMD, so B = 128 takes 16 waves: with 8, 35.4 us.  Panels 1
+// and 2 are still bound by that update (8300 and 6400 cycles of stage 1, 3700
+// the others).
+// Alone on the device, with the inverses and DT: B = 128 31.9 us (32-wide
+// panels 39.6; one stage at a time 62.2 and a further launch of 8 for the
+// inverses), B = 64 14.4 (21.3; 26.1 + 8), B = 32 8.9 (11.0; 9.2 + 7).  GEFA at
+// B = 128: n = 1024 0.454 -> 0.379 ms, 2048 1.008 -> 0.860, 4096 2.43 -> 2.12;
+// B = 64 n = 7488 6.75 -> 6.0.
+// With 8 waves at most 128 VGPRs and 77 KiB of LDS: the workgroup fits into
+// what one of the two workgroups of the FP32 trailing update on a CU leaves.
 // Blocks up to 128 are handled here; larger diagonal blocks are factorised by
 // the host schedule as a 2 x 2 recursion on top of this kernel.
 #include "common.hpp"
@@ -52,43 +55,81 @@ __device__ __forceinline__ float bcast(float v, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
-// b where the mask has the lane, else a
-__device__ __forceinline__ float pick(unsigned long long mask, float a, float b) {
-    float r;
-    asm("v_cndmask_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "s"(mask));
-    return r;
-}
-
-constexpr unsigned long long kLowHalf = 0xffffffffull, kHighHalf = kLowHalf << 32;
-
-// d[i] += m[i], i < n <= 4, in the lanes of the mask: one change of the exec
-// mask instead of a select per value (every lane of the wave is active here)
-__device__ __forceinline__ void add_in(unsigned long long mask, int n, float* d, const float* m) {
-    if (n == 4)
-        asm("s_mov_b64 exec, %8\n\tv_add_f32 %0, %0, %4\n\tv_add_f32 %1, %1, %5\n\t"
-            "v_add_f32 %2, %2, %6\n\tv_add_f32 %3, %3, %7\n\ts_mov_b64 exec, -1"
-            : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3])
-            : "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "s"(mask));
-    else if (n == 3)
-        asm("s_mov_b64 exec, %6\n\tv_add_f32 %0, %0, %3\n\tv_add_f32 %1, %1, %4\n\t"
-            "v_add_f32 %2, %2, %5\n\ts_mov_b64 exec, -1"
-            : "+v"(d[0]), "+v"(d[1]), "+v"(d[2])
-            : "v"(m[0]), "v"(m[1]), "v"(m[2]), "s"(mask));
-    else if (n == 2)
-        asm("s_mov_b64 exec, %4\n\tv_add_f32 %0, %0, %2\n\tv_add_f32 %1, %1, %3\n\t"
+// d[i] += m[i], i < N, in the lanes that the mask M has in each half of the wave:
+// one change of the exec mask instead of a select per value (every lane of the
+// wave is active here)
+template <unsigned M, int N>
+__device__ __forceinline__ void add_in(float* d, const float* m) {
+    static_assert(N >= 1 && N <= 8, "up to eight values");
+    if constexpr (N == 1)
+        asm("s_mov_b32 exec_lo, %2\n\ts_mov_b32 exec_hi, %2\n\t"
+            "v_add_f32 %0, %0, %1\n\t"
+            "s_mov_b64 exec, -1"
+            : "+v"(d[0])
+            : "v"(m[0]), "i"(M));
+    else if constexpr (N == 2)
+        asm("s_mov_b32 exec_lo, %4\n\ts_mov_b32 exec_hi, %4\n\t"
+            "v_add_f32 %0, %0, %2\n\tv_add_f32 %1, %1, %3\n\t"
             "s_mov_b64 exec, -1"
             : "+v"(d[0]), "+v"(d[1])
-            : "v"(m[0]), "v"(m[1]), "s"(mask));
-    else
-        asm("s_mov_b64 exec, %2\n\tv_add_f32 %0, %0, %1\n\ts_mov_b64 exec, -1"
-            : "+v"(d[0])
-            : "v"(m[0]), "s"(mask));
+            : "v"(m[0]), "v"(m[1]), "i"(M));
+    else if constexpr (N == 3)
+        asm("s_mov_b32 exec_lo, %6\n\ts_mov_b32 exec_hi, %6\n\t"
+            "v_add_f32 %0, %0, %3\n\tv_add_f32 %1, %1, %4\n\t"
+            "v_add_f32 %2, %2, %5\n\t"
+            "s_mov_b64 exec, -1"
+            : "+v"(d[0]), "+v"(d[1]), "+v"(d[2])
+            : "v"(m[0]), "v"(m[1]), "v"(m[2]), "i"(M));
+    else if constexpr (N == 4)
+        asm("s_mov_b32 exec_lo, %8\n\ts_mov_b32 exec_hi, %8\n\t"
+            "v_add_f32 %0, %0, %4\n\tv_add_f32 %1, %1, %5\n\t"
+            "v_add_f32 %2, %2, %6\n\tv_add_f32 %3, %3, %7\n\t"
+            "s_mov_b64 exec, -1"
+            : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3])
+            : "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "i"(M));
+    else if constexpr (N == 5)
+        asm("s_mov_b32 exec_lo, %10\n\ts_mov_b32 exec_hi, %10\n\t"
+            "v_add_f32 %0, %0, %5\n\tv_add_f32 %1, %1, %6\n\t"
+            "v_add_f32 %2, %2, %7\n\tv_add_f32 %3, %3, %8\n\t"
+            "v_add_f32 %4, %4, %9\n\t"
+            "s_mov_b64 exec, -1"
+            : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]), "+v"(d[4])
+            : "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "v"(m[4]), "i"(M));
+    else if constexpr (N == 6)
+        asm("s_mov_b32 exec_lo, %12\n\ts_mov_b32 exec_hi, %12\n\t"
+            "v_add_f32 %0, %0, %6\n\tv_add_f32 %1, %1, %7\n\t"
+            "v_add_f32 %2, %2, %8\n\tv_add_f32 %3, %3, %9\n\t"
+            "v_add_f32 %4, %4, %10\n\tv_add_f32 %5, %5, %11\n\t"
+            "s_mov_b64 exec, -1"
+            : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]), "+v"(d[4]), "+v"(d[5])
+            : "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "v"(m[4]), "v"(m[5]), "i"(M));
+    else if constexpr (N == 7)
+        asm("s_mov_b32 exec_lo, %14\n\ts_mov_b32 exec_hi, %14\n\t"
+            "v_add_f32 %0, %0, %7\n\tv_add_f32 %1, %1, %8\n\t"
+            "v_add_f32 %2, %2, %9\n\tv_add_f32 %3, %3, %10\n\t"
+            "v_add_f32 %4, %4, %11\n\tv_add_f32 %5, %5, %12\n\t"
+            "v_add_f32 %6, %6, %13\n\t"
+            "s_mov_b64 exec, -1"
+            : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]), "+v"(d[4]), "+v"(d[5]), "+v"(d[6])
+            : "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "v"(m[4]), "v"(m[5]), "v"(m[6]), "i"(M));
+    else if constexpr (N == 8)
+        asm("s_mov_b32 exec_lo, %16\n\ts_mov_b32 exec_hi, %16\n\t"
+            "v_add_f32 %0, %0, %8\n\tv_add_f32 %1, %1, %9\n\t"
+            "v_add_f32 %2, %2, %10\n\tv_add_f32 %3, %3, %11\n\t"
+            "v_add_f32 %4, %4, %12\n\tv_add_f32 %5, %5, %13\n\t"
+            "v_add_f32 %6, %6, %14\n\tv_add_f32 %7, %7, %15\n\t"
+            "s_mov_b64 exec, -1"
+            : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]), "+v"(d[4]), "+v"(d[5]), "+v"(d[6]),
+              "+v"(d[7])
+            : "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "v"(m[4]), "v"(m[5]), "v"(m[6]),
+              "v"(m[7]), "i"(M));
 }
 
-// lane J of each half of the wave to all lanes of that half
+// lane J of each row of 16 lanes to all lanes of that row
 template <int J>
-__device__ __forceinline__ float half_bcast(float v) {
-    return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), J << 5));
+__device__ __forceinline__ float row_bcast(float v) {
+    return __int_as_float(
+        __builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + J, 0xf, 0xf, true));
 }
 
 // the lower (H = 0) or upper (H = 1) half of v in both halves of the wave
@@ -98,15 +139,15 @@ __device__ __forceinline__ float from_half(float v) {
     return __uint_as_float(r[H]);
 }
 
-template <int J, typename F>
-__device__ __forceinline__ void static_for32(F&& f) {
-    if constexpr (J < 32) {
+template <int J, int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (J < N) {
         f(std::integral_constant<int, J>{});
-        static_for32<J + 1>(f);
+        static_for<J + 1, N>(f);
     }
 }
 
-// -1/p from the hardware reciprocal and two Newton steps in FMA: correctly
+// -1/p from the hardware reciprocal and a Newton step in FMA: correctly
 // rounded (checked against the division for every mantissa) while neither p
 // nor 1/p comes near the ends of the exponent range; the kernel checks that
 // on the results and factorises the panel again by divisions where it fails.
@@ -114,60 +155,42 @@ __device__ __forceinline__ bool rcp_in_range(float inv) {
     return ((__float_as_uint(inv) >> 23) & 0xffu) - 28u < 198u;
 }
 
-// Forward substitution of one vector per half-lane pair against the
-// factorised sub-block: lane (c, h) holds x[i] = element 2 i + h of vector c.
+// lanes r > j of every row of 16 lanes, for one half of the wave
+constexpr unsigned above(int j) { return (0xffffu << (j + 1) & 0xffffu) * 0x10001u; }
+
+// Forward substitution of 4 NR vectors against a factorised 16 x 16 sub-block,
+// an element per lane: lane (r, q) holds element r of vector 4 q' + k, k < NR.
 //   SCALED: x_j *= dg_j, then x_r += x_j S[j][r], r > j (top strip)
 //   else:   x_r += x_j S[j][r], r > j                   (left strip)
-// with S[j][r] at S[32 j + 16 (r % 2) + r / 2]: a step's coefficients are
-// 16-byte LDS broadcasts, read two steps ahead.
-template <bool SCALED>
-__device__ __forceinline__ void solve32(float (&x)[16], const float* S, float dgl, int h) {
+// S[j] is S[j][r] in lane r, dg lane r's dg_r.  A lane's element is scaled
+// for its use at step j and, final by then, once more at the end.
+template <bool SCALED, int NR>
+__device__ __forceinline__ void solve16(float (&x)[NR], const float (&S)[16], float dg) {
 #pragma clang fp contract(off)
-    float dg[SCALED ? 32 : 1];
-    if constexpr (SCALED) {
+    static_for<0, 15>([&](auto jc) {
+        constexpr int j = jc.value;
+        float u[NR];
 #pragma unroll
-        for (int j = 0; j < 32; ++j) dg[j] = bcast(dgl, j);
-    }
-    const float* Sh = S + h * 16;
-    float4 nx[2][4];
+        for (int k = 0; k < NR; ++k) u[k] = SCALED ? x[k] * dg : x[k];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        nx[0][g] = *reinterpret_cast<const float4*>(Sh + 4 * g);
-        nx[1][g] = *reinterpret_cast<const float4*>(Sh + 32 + 4 * g);
-    }
-    static_for32<0>([&](auto jc) {
-        constexpr int j = jc.value, i0 = j >> 1, hj = j & 1;
-        float s4[16];
-#pragma unroll
-        for (int g = (i0 + hj) / 4; g < 4; ++g) {
-            float4& q = nx[hj][g];
-            // whole 16-byte reads, also where a step needs part of one
-            asm volatile("" : "+v"(q.x), "+v"(q.y), "+v"(q.z), "+v"(q.w));
-            s4[4 * g] = q.x;
-            s4[4 * g + 1] = q.y;
-            s4[4 * g + 2] = q.z;
-            s4[4 * g + 3] = q.w;
-        }
-        if constexpr (j < 30) {
-#pragma unroll
-            for (int g = (j + 3) / 8; g < 4; ++g)
-                nx[hj][g] = *reinterpret_cast<const float4*>(Sh + (j + 2) * 32 + 4 * g);
-        }
-        float s = x[i0];
-        if constexpr (SCALED) s = s * dg[j];
-        const float v = from_half<hj>(s);
-        if constexpr (SCALED) x[i0] = pick(hj ? kHighHalf : kLowHalf, x[i0], s);
-        if constexpr (hj == 0) {
-            const float u = v * s4[i0];
-            const float w = x[i0] + u;
-            x[i0] = pick(kHighHalf, x[i0], w);
-        }
-#pragma unroll
-        for (int i = i0 + 1; i < 16; ++i) s4[i] = v * s4[i];
-#pragma unroll
-        for (int i = i0 + 1; i < 16; ++i) x[i] = x[i] + s4[i];
-        __builtin_amdgcn_sched_barrier(0);
+        for (int k = 0; k < NR; ++k) u[k] = row_bcast<j>(u[k]) * S[j];
+        add_in<above(j), NR>(x, u);
     });
+    if (SCALED)
+#pragma unroll
+        for (int k = 0; k < NR; ++k) x[k] = x[k] * dg;
+}
+
+// a lane's 16 consecutive floats
+__device__ __forceinline__ void read16(float (&S)[16], const float* p) {
+#pragma unroll
+    for (int g = 0; g < 16; g += 4) {
+        const float4 v = *reinterpret_cast<const float4*>(p + g);
+        S[g] = v.x;
+        S[g + 1] = v.y;
+        S[g + 2] = v.z;
+        S[g + 3] = v.w;
+    }
 }
 
 template <int B, int NT>
@@ -176,19 +199,19 @@ __global__ __launch_bounds__(NT) void lu_diag_kernel(float* __restrict__ A, int6
                                                      float* __restrict__ DT, int64_t ldt,
                                                      float* __restrict__ inv, int64_t inv_ts) {
 #pragma clang fp contract(off)
-    constexpr int LD = B + 4, NP = B / 32, NW = NT / 64;
+    constexpr int LD = B + 4, NP = B / 16, NW = NT / 64, LS = 20;
     __shared__ __attribute__((aligned(16))) float Ds[B * LD];
-    // the panel's left strip transposed (k-major)
-    __shared__ __attribute__((aligned(16))) float LT[B > 32 ? 32 * LD : 4];
-    // the factorised sub-block by columns and by rows, each column's (row's)
-    // even elements before its odd ones
-    __shared__ __attribute__((aligned(16))) float Sc[1024], Sr[1024];
+    // the panel's left strip transposed (k-major); row 4 i + 2 e + h of each
+    // block of 16 at 8 h + 4 e + i, the order in which a lane of the diagonal
+    // update needs four of them
+    __shared__ __attribute__((aligned(16))) float LT[16 * LD];
+    __shared__ __attribute__((aligned(16))) float Sr[2 * 16 * LS];  // the sub-block transposed, by the panel's parity
     const int t = threadIdx.x;
-    const int wave = t >> 6;
-    int lane = t & 63, c = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     float* base = A + off * lda + off;
     constexpr int V = B * B / 4 / NT;
     static_assert(V >= 1 && V * NT * 4 == B * B, "block must split evenly over the threads");
+    static_assert(NW >= 4, "waves 0, NW - 2 and NW - 1 have parts of their own");
     {
         float4 v[V];
 #pragma unroll
@@ -204,283 +227,280 @@ __global__ __launch_bounds__(NT) void lu_diag_kernel(float* __restrict__ A, int6
     }
     __syncthreads();
 
-    // rank-32 update of the 4 x 4 register tile of each lane in the 32 x 32
-    // block (bi, bj) by panel q
-    auto tile32 = [&](int q, int bi, int bj) {
-        const int rr = bi * 32 + (lane >> 3) * 4, cc = bj * 32 + (lane & 7) * 4;
-        float acc[4][4];
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            const float4 v = *reinterpret_cast<const float4*>(&Ds[(rr + a) * LD + cc]);
-            acc[a][0] = v.x;
-            acc[a][1] = v.y;
-            acc[a][2] = v.z;
-            acc[a][3] = v.w;
-        }
-        const float* lt = &LT[rr];
-        const float* tp = &Ds[q * 32 * LD + cc];
-#pragma unroll 4
-        for (int k = 0; k < 32; ++k) {
-            const float4 l = *reinterpret_cast<const float4*>(lt + k * LD);
-            const float4 u = *reinterpret_cast<const float4*>(tp + k * LD);
-            const float lv[4] = {l.x, l.y, l.z, l.w}, uv[4] = {u.x, u.y, u.z, u.w};
-            float pr[4][4];
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-#pragma unroll
-                for (int b = 0; b < 4; ++b) pr[a][b] = uv[b] * lv[a];
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-#pragma unroll
-                for (int b = 0; b < 4; ++b) acc[a][b] = acc[a][b] + pr[a][b];
-        }
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-            *reinterpret_cast<float4*>(&Ds[(rr + a) * LD + cc]) =
-                float4{acc[a][0], acc[a][1], acc[a][2], acc[a][3]};
-    };
-    // the same for the 16 x 16 quarter qt of block (b, b), 2 x 2 per lane
-    auto tile16 = [&](int q, int b, int qt) {
-        const int rr = b * 32 + (qt >> 1) * 16 + (lane >> 3) * 2;
-        const int cc = b * 32 + (qt & 1) * 16 + (lane & 7) * 2;
-        float acc[2][2];
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            acc[a][0] = Ds[(rr + a) * LD + cc];
-            acc[a][1] = Ds[(rr + a) * LD + cc + 1];
-        }
-        const float* lt = &LT[rr];
-        const float* tp = &Ds[q * 32 * LD + cc];
-        // the next four operand pairs are read while four are multiplied
-        float2 l[4], u[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            l[k] = *reinterpret_cast<const float2*>(lt + k * LD);
-            u[k] = *reinterpret_cast<const float2*>(tp + k * LD);
-        }
-#pragma unroll 1
-        for (int kb = 4; kb <= 32; kb += 4) {
-            float2 ln[4], un[4];
-            const int kn = kb < 32 ? kb : 28;  // the last turn reads again what it has
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                ln[k] = *reinterpret_cast<const float2*>(lt + (kn + k) * LD);
-                un[k] = *reinterpret_cast<const float2*>(tp + (kn + k) * LD);
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const float p0 = u[k].x * l[k].x, p1 = u[k].y * l[k].x;
-                const float p2 = u[k].x * l[k].y, p3 = u[k].y * l[k].y;
-                acc[0][0] = acc[0][0] + p0;
-                acc[0][1] = acc[0][1] + p1;
-                acc[1][0] = acc[1][0] + p2;
-                acc[1][1] = acc[1][1] + p3;
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                l[k] = ln[k];
-                u[k] = un[k];
-            }
-        }
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            Ds[(rr + a) * LD + cc] = acc[a][0];
-            Ds[(rr + a) * LD + cc + 1] = acc[a][1];
+    // the rows and columns of panels lo..hi-1 (their parts outside earlier
+    // panels') to the matrix and transposed to DT, by wave w of nw: a block of
+    // 16 x 16 at a time, whose place is the same for the whole wave
+    auto store = [&](int w, int nw, int lo, int hi) {
+        const int lane = t & 63, y = lane >> 2, x = 4 * (lane & 3);
+        float* ap = base + (int64_t)y * lda + x;
+        float* dp = DT + (int64_t)y * ldt + x;
+        for (int g = w; g < NP * NP; g += nw) {
+            const int r0 = g / NP * 16, c0 = g % NP * 16, b = min(r0, c0) >> 4;
+            if (b < lo || b >= hi) continue;
+            const float4 v = *reinterpret_cast<const float4*>(&Ds[(r0 + y) * LD + c0 + x]);
+            const float* q = &Ds[(c0 + x) * LD + r0 + y];
+            const float4 d = {q[0], q[LD], q[2 * LD], q[3 * LD]};
+            *reinterpret_cast<float4*>(ap + (int64_t)r0 * lda + c0) = v;
+            *reinterpret_cast<float4*>(dp + (int64_t)r0 * ldt + c0) = d;
         }
     };
-    // the elements of the last 32 x 32 block, or all others, to the matrix and
-    // transposed to DT: 8 rows x 8 float4 columns per wave, so that a wave's
-    // stores fill 128-byte lines and its LDS reads by column meet few conflicts
-    auto store = [&](int s, int ns, bool last) {
-        constexpr int G = B / 8, GC = B / 32;
-        for (int g = s >> 6; g < G * GC; g += ns >> 6) {
-            const int r = (g / GC) * 8 + (s & 7), cc = (g % GC) * 32 + ((s >> 3) & 7) * 4;
-            if (last != (r >= B - 32 && cc >= B - 32)) continue;
-            const int r2 = (g / GC) * 8 + ((s >> 3) & 7), c2 = (g % GC) * 32 + (s & 7) * 4;
-            *reinterpret_cast<float4*>(base + (int64_t)r2 * lda + c2) =
-                *reinterpret_cast<const float4*>(&Ds[r2 * LD + c2]);
-            *reinterpret_cast<float4*>(DT + (int64_t)r * ldt + cc) =
-                float4{Ds[cc * LD + r], Ds[(cc + 1) * LD + r], Ds[(cc + 2) * LD + r],
-                       Ds[(cc + 3) * LD + r]};
+    // Panel p's part of the unit vectors' solves, for the top or the left strip's
+    // recurrence: elements 0..15 of vectors 4 q + k of a 32 x 32 block in its
+    // first half, elements 16..31 of those (from yu) and of vectors 16 + 4 q + k
+    // (hi) in its second.
+    float xu[4], yu[4];
+    auto units = [&](int p, int lane, bool top, bool hi) {
+        const int P0 = p * 16, r = lane & 15, q = lane >> 4;
+        const bool odd = p & 1;
+        float x[4], S[16];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            x[k] = odd != hi ? (odd ? yu[k] : 0.0f) : (4 * q + k == r ? 1.0f : 0.0f);
+        if (top) {
+            read16(S, &Ds[(P0 + r) * LD + P0]);
+            solve16<true, 4>(x, S, Ds[(P0 + r) * LD + P0 + r]);
+        } else {
+            read16(S, &Sr[(p & 1) * 16 * LS + r * LS]);
+            solve16<false, 4>(x, S, 0.0f);
         }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) xu[k] = x[k];
+        // top: the inverse (S^-1 - C)^-1 of the top recurrence, stored
+        // transposed, and its negated transpose, which is the inverse of the
+        // sub-block's U
+        const int row = (odd ? 16 : 0) + r, col = (hi ? 16 : 0) + 4 * q;
+        float* o = inv + (top ? 0 : inv_ts) + (p >> 1) * 1024 + row + col * 32;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[k * 32] = x[k];
+        if (top)
+            *reinterpret_cast<float4*>(inv + 2 * inv_ts + (p >> 1) * 1024 + row * 32 + col) =
+                float4{-x[0], -x[1], -x[2], -x[3]};
     };
     bool bad = false;
 #pragma unroll 1
-    for (int p = 0; p < NP; ++p) {
-        const int P0 = p * 32;
+    for (int p = 0; p <= NP; ++p) {
+        const int P0 = p * 16;
         // opaque per panel: or every LDS address of the loop is formed before
-        // it and held (100 registers)
-        lane = t & 63;
+        // it and held
+        int lane = t & 63;
         asm volatile("" : "+v"(lane));
-        c = lane & 31;
-        h = lane >> 5;
-        // ---- A: lane (c, h) holds rows 2 i + h of column P0 + c
-        if (wave == 0) {
-            float d[16];
+        const int r = lane & 15, q = lane >> 4;
+        // ---- 1
+        if (wave == 0 && p < NP) {
+            const int c = r, e = q & 1, h = q >> 1;
+            // lane (c, e, h): column P0 + c, rows 4 i + 2 e + h of the sub-block
+            float z[4];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) d[i] = Ds[(P0 + 2 * i + h) * LD + P0 + c];
-            // lanes (both halves) whose column is above j, shifted along: kept
-            // out of the compiler's sight, or it hoists and spills 32 masks
-            unsigned long long gt = 0xfffffffefffffffeull;
-            asm volatile("" : "+s"(gt));
-            float m[16];
+            for (int i = 0; i < 4; ++i) z[i] = Ds[(P0 + 4 * i + 2 * e + h) * LD + P0 + c];
+            if (p > 0) {
+                const float* up = &Ds[(P0 - 16) * LD + P0 + c];
+                const float* lp = &LT[P0 + 8 * h + 4 * e];
+                float uv[16];
+                float4 lv[16];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) m[i] = half_bcast<0>(d[i]);
-            // row j scaled by -1/pivot, the pivot itself replaced by -1/pivot
+                for (int k = 0; k < 16; ++k) {
+                    uv[k] = up[k * LD];
+                    lv[k] = *reinterpret_cast<const float4*>(lp + k * LD);
+                }
+#pragma unroll
+                for (int k = 0; k < 16; ++k) {
+                    const float m0 = uv[k] * lv[k].x, m1 = uv[k] * lv[k].y;
+                    const float m2 = uv[k] * lv[k].z, m3 = uv[k] * lv[k].w;
+                    z[0] = z[0] + m0;
+                    z[1] = z[1] + m1;
+                    z[2] = z[2] + m2;
+                    z[3] = z[3] + m3;
+                }
+            }
+            // both e hold all rows 2 i + h
+            float d[8], d0[8];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const auto w = __builtin_amdgcn_permlane16_swap(
+                    __float_as_uint(z[i]), __float_as_uint(z[i]), false, false);
+                d[2 * i] = __uint_as_float(w[0]);
+                d[2 * i + 1] = __uint_as_float(w[1]);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) d0[i] = d[i];
+            // V[j]: row j scaled by -1/pivot, in both halves; d keeps the columns
+            // <= j of it, the multipliers and the pivot
+            float V[16];
             const float piv0 = bcast(d[0], 0);
             float r0 = __builtin_amdgcn_rcpf(piv0);
             r0 = fmaf(fmaf(-piv0, r0, 1.0f), r0, r0);
-            r0 = fmaf(fmaf(-piv0, r0, 1.0f), r0, r0);
-            float sc = pick(1ull, d[0], 1.0f) * -r0;
-            static_for32<0>([&](auto jc) {
-                constexpr int j = jc.value, i0 = j >> 1, hj = j & 1;
-                constexpr int j1 = (j + 1) & 31, i1 = j1 >> 1, h1 = j1 & 1;
-                const unsigned long long ge = gt | (1ull << j) | (1ull << (j + 32));
-                // row j scaled, in both halves
-                const float v = from_half<hj>(sc);
-                if constexpr (j < 31) {
-                    // the next pivot's row first; its reciprocal's chain goes
-                    // between the other rows' updates
-                    float u = v * m[i1], w = d[i1] + u;
-                    d[i0] = pick(ge & (hj ? kHighHalf : kLowHalf), d[i0], sc);
-                    d[i1] = pick(hj == 0 ? gt & kHighHalf : gt, d[i1], w);
-                    const float piv = bcast(d[i1], h1 * 32 + j1);
-                    if constexpr (h1 == 0) m[i1] = half_bcast<j1>(d[i1]);
-                    float r = __builtin_amdgcn_rcpf(piv), e = 0.0f, x1 = 0.0f;
-                    auto link = [&](int n) {
-                        if (n == 0) x1 = pick(1ull << (j1 + 32 * h1), d[i1], 1.0f);
-                        if (n == 1) e = fmaf(-piv, r, 1.0f);
-                        if (n == 2) r = fmaf(e, r, r);
-                        if (n == 3) e = fmaf(-piv, r, 1.0f);
-                        if (n == 4) r = fmaf(e, r, r);
-                        if (n == 5) sc = x1 * -r;
-                        __builtin_amdgcn_sched_barrier(0);
-                    };
-                    __builtin_amdgcn_sched_barrier(0);
-                    // four rows at a time, operation by operation: a result
-                    // is not ready for the next instruction
-                    constexpr int NG = (15 - i1 + 3) / 4;
+            V[0] = from_half<0>(d[0]) * -r0;
+            static_for<0, 15>([&](auto jc) {
+                constexpr int j = jc.value, i1 = (j + 1) >> 1, h1 = (j + 1) & 1;
+                float m[8];
 #pragma unroll
-                    for (int g = 0; g < NG; ++g) {
-                        const int ia = i1 + 1 + 4 * g, ib = ia + 4 < 16 ? ia + 4 : 16;
-                        asm volatile("" : "+v"(m[ib - 1]));  // one wait for the group's values
-#pragma unroll
-                        for (int i = ia; i < ib; ++i) m[i] = v * m[i];
-                        link(2 * g);
-                        add_in(gt, ib - ia, d + ia, m + ia);
-                        link(2 * g + 1);
-#pragma unroll
-                        for (int i = ia; i < ib; ++i) m[i] = half_bcast<j1>(d[i]);
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-#pragma unroll
-                    for (int n = 2 * NG; n < 6; ++n) link(n);
-                } else {
-                    d[i0] = pick(ge & (hj ? kHighHalf : kLowHalf), d[i0], sc);
-                }
-                gt = (gt & 0x7fffffff7fffffffull) << 1;
+                for (int i = i1; i < 8; ++i) m[i] = V[j] * row_bcast<j>(d[i]);
+                add_in<above(j), 8 - i1>(d + i1, m + i1);
+                const float piv = bcast(d[i1], h1 * 32 + j + 1);
+                const float y = from_half<h1>(d[i1]);
+                float rc = __builtin_amdgcn_rcpf(piv);
+                rc = fmaf(fmaf(-piv, rc, 1.0f), rc, rc);
+                V[j + 1] = y * -rc;
             });
-            bool fine = true;
+            // -1/pivot of the lane's own column, where it has that row
+            float dinv = 1.0f;
 #pragma unroll
-            for (int i = 0; i < 16; ++i)
-                if (2 * i + h == c) fine = rcp_in_range(d[i]);
+            for (int i = 0; i < 8; ++i)
+                if (2 * i + h == c) dinv = d[i];
+            {
+                const float r1 = __builtin_amdgcn_rcpf(dinv);
+                dinv = -fmaf(fmaf(-dinv, r1, 1.0f), r1, r1);
+            }
+            const bool fine = rcp_in_range(dinv);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float up = h ? V[2 * i + 1] : V[2 * i];
+                d[i] = 2 * i + h == c ? dinv : 2 * i + h < c ? up : d[i];
+            }
             if (__ballot(!fine)) {
                 // a pivot near the ends of the exponent range (or zero): the
-                // same steps with divisions, on the panel as it still lies in LDS
-                for (int j = 0; j < 32; ++j) {
+                // same steps with divisions, in LDS
+#pragma unroll
+                for (int i = 0; i < 8; ++i) Ds[(P0 + 2 * i + h) * LD + P0 + c] = d0[i];
+                wave_lds_sync();
+                for (int j = 0; j < 16; ++j) {
                     float* row = &Ds[(P0 + j) * LD + P0];
                     const float rinv = -1.0f / row[j];
                     const float s = c == j ? rinv : row[c] * rinv;
                     wave_lds_sync();
-                    if (lane < 32 && c >= j) row[c] = s;
-                    for (int r = j + 1; r < 32; ++r) {
-                        float* q = &Ds[(P0 + r) * LD + P0];
-                        const float u = s * q[j];
-                        const float w = q[c] + u;
-                        if (lane < 32 && c > j) q[c] = w;
+                    if (lane < 16 && c >= j) row[c] = s;
+                    for (int rr = j + 1; rr < 16; ++rr) {
+                        float* o = &Ds[(P0 + rr) * LD + P0];
+                        const float u = s * o[j];
+                        const float w = o[c] + u;
+                        if (lane < 16 && c > j) o[c] = w;
                     }
                     wave_lds_sync();
                 }
 #pragma unroll
-                for (int i = 0; i < 16; ++i) d[i] = Ds[(P0 + 2 * i + h) * LD + P0 + c];
+                for (int i = 0; i < 8; ++i) d[i] = Ds[(P0 + 2 * i + h) * LD + P0 + c];
             }
+            float* o = e ? &Sr[(p & 1) * 16 * LS + c * LS + h] : &Ds[(P0 + h) * LD + P0 + c];
+            const int os = e ? 2 : 2 * LD;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int r = 2 * i + h;
-                Ds[(P0 + r) * LD + P0 + c] = d[i];
-                Sr[r * 32 + (c & 1) * 16 + (c >> 1)] = d[i];
-                if (r == c) bad |= !__builtin_isfinite(d[i]);
+            for (int i = 0; i < 8; ++i) {
+                o[i * os] = d[i];
+                if (2 * i + h == c) bad |= !__builtin_isfinite(d[i]);
             }
+        } else if (wave > 0) {
+            // panel p - 1's update of the w x w blocks of 16 without the first,
+            // which is wave 0's: a row of 16 lanes per block, 4 x 4 per lane
+            const int w = NP - p, nb = p > 0 ? w * w : 0;
+            const int rcpw = 65536 / max(w, 1) + 1;
+            for (int b0 = 4 * wave - 3; b0 < nb; b0 += 4 * (NW - 1)) {
+                const bool in = b0 + q < nb;
+                const int id = in ? b0 + q : b0;
+                const int bi = (id * rcpw) >> 16, bj = id - bi * w;
+                const int a = r >> 2, cc = P0 + 16 * bj + 4 * (r & 3);
+                const int r0 = P0 + 16 * bi + 2 * (a & 1) + (a >> 1);  // rows r0 + 4 i
+                const float* lp = &LT[P0 + 16 * bi + 4 * a];
+                const float* up = &Ds[(P0 - 16) * LD + cc];
+                float acc[4][4];
 #pragma unroll
-            for (int i = 0; i < 16; i += 4)
-                *reinterpret_cast<float4*>(&Sc[c * 32 + h * 16 + i]) =
-                    float4{d[i], d[i + 1], d[i + 2], d[i + 3]};
-        } else if (NP == 4 && (p == 1 || p == 2)) {
-            // panel p - 1's update of blocks p..3 x p..3 without (p, p), which is done
-            const int w = 4 - p;
-            for (int x = wave; x < w * w; x += NW - 1) tile32(p - 1, p + x / w, p + x % w);
+                for (int i = 0; i < 4; ++i) {
+                    const float4 v = *reinterpret_cast<const float4*>(&Ds[(r0 + 4 * i) * LD + cc]);
+                    acc[i][0] = v.x;
+                    acc[i][1] = v.y;
+                    acc[i][2] = v.z;
+                    acc[i][3] = v.w;
+                }
+#pragma unroll 4
+                for (int k = 0; k < 16; ++k) {
+                    const float4 l = *reinterpret_cast<const float4*>(lp + k * LD);
+                    const float4 u = *reinterpret_cast<const float4*>(up + k * LD);
+                    const float lv[4] = {l.x, l.y, l.z, l.w}, uv[4] = {u.x, u.y, u.z, u.w};
+                    float pr[4][4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int b = 0; b < 4; ++b) pr[i][b] = uv[b] * lv[i];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int b = 0; b < 4; ++b) acc[i][b] = acc[i][b] + pr[i][b];
+                }
+                if (in)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        *reinterpret_cast<float4*>(&Ds[(r0 + 4 * i) * LD + cc]) =
+                            float4{acc[i][0], acc[i][1], acc[i][2], acc[i][3]};
+            }
+            if (p > 0) {
+                // waves NW - 1 and NW - 2 the low vectors, two others the high ones
+                // (with four waves one takes both)
+                if (wave < NW - 2)
+                    for (int u = 0; u < 2; ++u) {
+                        if (wave == (NW > 4 ? NW - 3 - u : 1)) units(p - 1, lane, u == 0, true);
+                    }
+                else
+                    units(p - 1, lane, wave == NW - 1, false);
+            }
+            if ((p & 1) && wave >= NW - 2) {
+                // elements 16..31 of the first 16 unit vectors
+                const float* sp = wave == NW - 1
+                                      ? &LT[P0 + (r & 1) * 8 + ((r >> 1) & 1) * 4 + (r >> 2)]
+                                      : &Ds[(P0 - 16) * LD + P0 + r];
+                float S[16];
+#pragma unroll
+                for (int j = 0; j < 16; ++j) S[j] = sp[j * LD];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) yu[k] = 0.0f;
+                static_for<0, 16>([&](auto jc) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const float u = row_bcast<jc.value>(xu[k]) * S[jc.value];
+                        yu[k] = yu[k] + u;
+                    }
+                });
+            }
+            // what is final, where the updates leave time for it
+            if (p >= NP / 2) {
+                const int lo = min(2 * (p - NP / 2), NP - 1);
+                // (of 16 waves, those that have neither a tile nor unit vectors)
+                constexpr int W0 = NW > 8 ? 5 : 1, W1 = NW > 8 ? 12 : NW;
+                if (wave >= W0 && wave < W1)
+                    store(wave - W0, W1 - W0, lo, p == NP ? NP : min(lo + 2, p));
+            }
         }
-        if (NP > 1 && p == NP - 1 && wave > 0) store(t - 64, NT - 64, false);
+        if (p == NP) break;
         __syncthreads();
-        // ---- B: wave g the top group g, wave ng the unit vectors, then the same
-        // of the left strip
-        const int R0 = P0 + 32;
-        const int ng = NP - 1 - p;
+        // ---- 2
+        const int R0 = P0 + 16, ng = NP - 1 - p;
+        const float dg = Ds[(P0 + r) * LD + P0 + r];
+        const float* scol = &Ds[(P0 + r) * LD + P0];
+        const float* srow = &Sr[(p & 1) * 16 * LS + r * LS];
 #pragma unroll 1
-        for (int g = wave; g < 2 * (ng + 1); g += NW) {
-            float x[16];
-            if (g <= ng) {
-                const bool unit = g == ng;
-                const int cc = unit ? P0 + c : R0 + g * 32 + c;
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const float v = Ds[(P0 + 2 * i + h) * LD + cc];
-                    x[i] = unit ? (2 * i + h == c ? 1.0f : 0.0f) : v;
-                }
-                solve32<true>(x, Sc, Sc[c * 32 + (c & 1) * 16 + (c >> 1)], h);
-                if (unit) {
-                    // the inverse (S^-1 - C)^-1 of the top recurrence, stored
-                    // transposed, and its negated transpose, which is the
-                    // inverse of the sub-block's U
-                    float* o = inv + p * 1024;
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        o[c * 32 + 2 * i + h] = x[i];
-                        o[2 * inv_ts + (2 * i + h) * 32 + c] = -x[i];
-                    }
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) Ds[(P0 + 2 * i + h) * LD + cc] = x[i];
-                }
+        for (int g = wave; g < 2 * ng; g += NW) {
+            float x[4], S[16];
+            if (g < ng) {
+                float4* xp = reinterpret_cast<float4*>(&Ds[(P0 + r) * LD + R0 + 16 * g + 4 * q]);
+                const float4 v = *xp;
+                x[0] = v.x;
+                x[1] = v.y;
+                x[2] = v.z;
+                x[3] = v.w;
+                read16(S, scol);
+                solve16<true, 4>(x, S, dg);
+                *xp = float4{x[0], x[1], x[2], x[3]};
             } else {
-                const bool unit = g == 2 * ng + 1;
-                const int rr = unit ? P0 + c : R0 + (g - ng - 1) * 32 + c;
+                // register k: row 4 k + q of the group
+                const int rr = R0 + 16 * (g - ng);
+                float* xp = &Ds[(rr + q) * LD + P0 + r];
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const float v = Ds[rr * LD + P0 + 2 * i + h];
-                    x[i] = unit ? (2 * i + h == c ? 1.0f : 0.0f) : v;
-                }
-                solve32<false>(x, Sr, 0.0f, h);
-                if (unit) {
-                    float* o = inv + inv_ts + p * 1024 + c * 32 + h;
+                for (int k = 0; k < 4; ++k) x[k] = xp[4 * k * LD];
+                read16(S, srow);
+                solve16<false, 4>(x, S, 0.0f);
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) o[2 * i] = x[i];
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        Ds[rr * LD + P0 + 2 * i + h] = x[i];
-                        LT[(2 * i + h) * LD + rr] = x[i];
-                    }
-                }
+                for (int k = 0; k < 4; ++k) xp[4 * k * LD] = x[k];
+                *reinterpret_cast<float4*>(&LT[r * LD + rr + (q & 1) * 8 + (q >> 1) * 4]) =
+                    float4{x[0], x[1], x[2], x[3]};
             }
         }
-        if (p + 1 == NP) {
-            if (wave >= 2) store(t - 128, NT - 128, true);
-            break;
-        }
-        __syncthreads();
-        // ---- C: (1, 1), (2, 2), (3, 3)
-        if (wave < 4) tile16(p, p + 1, wave);
         __syncthreads();
     }
     if (bad && status) atomicMax(status, 1);
@@ -499,12 +519,15 @@ hipError_t launch_lu_diag(float* A, int64_t lda, int64_t off, int B, int* status
     switch (B) {
         case 32: HPL_LU(32, 256); break;
         case 64:
-            if (narrow) HPL_LU(64, 256);
-            else HPL_LU(64, 512);
+            HPL_LU(64, 512);
             break;
         case 128:
-            if (narrow) HPL_LU(128, 256);
-            else HPL_LU(128, 512);
+            // 16 waves need a CU to themselves, which a large FP32 update beside
+            // them does not leave: GEFA n = 32768 199.9 ms with 8 waves, 203.9
+            // with 16, n = 16384 30.8 and 32.0; without one n = 2048 0.910 and
+            // 0.860
+            if (narrow) HPL_LU(128, 512);
+            else HPL_LU(128, 1024);
             break;
         default: return hipErrorInvalidValue;
     }

@@ -61,3 +61,16 @@ def test_recursive_block(ctx, B):
     ctx.gefa(f, B)
     ref = O.gefa_nopvt(a)
     assert np.max(np.abs(f - ref)) <= 2e-5 * np.max(np.abs(ref))
+
+
+def test_block_beside_a_large_update(ctx):
+    """The narrower workgroup of large orders: the first diagonal block, which no
+    update precedes, bit for bit."""
+    n, B = 6656, 128
+    print(f"lu block B={B} of n={n}", flush=True)
+    ctx.generate(n, 0, 5)
+    a, _ = ctx.download(matrix=True, solution=False)
+    ctx.gefa_dev(B)
+    f, _ = ctx.download(matrix=True, solution=False)
+    ref = O.gefa_nopvt(np.ascontiguousarray(a[:B, :B]))
+    assert np.array_equal(np.ascontiguousarray(f[:B, :B]).view(np.uint32), ref.view(np.uint32))
