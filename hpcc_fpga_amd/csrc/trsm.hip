@@ -451,6 +451,189 @@ __global__ __launch_bounds__(64) void trsm_reg_kernel(float* __restrict__ A, int
 }
 
 // ----------------------------------------------------------------------------
+// The same solve for strips that leave most of the device idle: one workgroup
+// per 32 vectors, 16 vectors to each half of it, the 32-row blocks of those
+// dealt out to W waves.  As soon as block p is solved every wave updates its
+// blocks beyond p by it, the next one first.
+//
+// Bound: the chain of B/32 blocks.  With 16 vectors a product of 32 x 32
+// coefficients is 16 v_mfma_f32_16x16x4_f32 of 32 cycles, half of the chain of 32
+// vectors on 32x32x2, and a block's chain holds one update and the product
+// with its inverse, not an update by every block before it.
+//
+// Operand layout: step (t, r) of a product takes k = 16 t + 4 (lane / 16) + r,
+// the row that register r of accumulator tile t holds in that lane, so a
+// solved block is the next product's B operand as it stands (its own inverse)
+// or as two 16-byte LDS reads (the other waves).
+//
+// GEFA: n = 1024 B = 128 0.378 -> 0.324 ms, 2048 0.853 -> 0.738, 4096 B = 256
+// 2.51 -> 1.94, B = 64 2.15 -> 2.00; FP8 n = 6144 B = 128 3.3 -> 2.95, B = 256
+// 3.69 -> 2.86.
+__device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+template <int B>
+constexpr int kSplitWaves = B / 32 < 4 ? B / 32 : 4;  // per half
+
+template <int B, typename LP>
+__global__ __launch_bounds__(128 * kSplitWaves<B>) void trsm_split_kernel(
+    float* __restrict__ A, int64_t lda, int64_t off, const float* DT, int64_t lddt,
+    const float* __restrict__ inv, int64_t inv_ts, float* Lt, int64_t ldt, int ngroups_top,
+    LP* __restrict__ lpT, LP* __restrict__ lpL, int64_t ldlp, float* __restrict__ scT,
+    float* __restrict__ scL) {
+    constexpr int NQ = B / 32, W = kSplitWaves<B>, NO = NQ / W;  // blocks per wave
+    constexpr bool kFp8 = std::is_same<LP, fp8e4m3>::value;
+    constexpr bool kLp = !std::is_same<LP, float>::value && !kFp8;
+    __shared__ __attribute__((aligned(16))) float Ys[2][2][16][36];
+    __shared__ float am_sh[2 * W];
+    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) % W;
+    const int half = (threadIdx.x >> 6) / W;
+    const int c = lane & 15, kk = lane >> 4;
+    const bool top = (int)blockIdx.x < ngroups_top;
+    const int64_t g32 = top ? blockIdx.x : blockIdx.x - ngroups_top;
+    const int64_t v = g32 * 32 + 16 * half + c;  // this lane's vector
+    const float* G = inv + (top ? 0 : inv_ts);
+    float* stripT = A + off * lda + off + B + v;
+    float* stripL = A + (off + B + v) * lda + off;
+    auto Y = Ys[half];
+
+    // coefficients X[p][i] of block (q, p) for step (t2, r) and row tile t: top
+    // D^T, left D
+    const float* X = top ? DT : A + off * lda + off;
+    const int64_t ldx = top ? lddt : lda;
+    auto load_c = [&](float (&x)[2][2][4], int q, int p) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    x[t][t2][r] = X[(p * 32 + 16 * t2 + 4 * kk + r) * ldx + q * 32 + 16 * t + c];
+    };
+    float g[NO][2][2][4], cn[NO][2][2][4];
+    f32x4 acc[NO][2];
+#pragma unroll
+    for (int m = 0; m < NO; ++m) {
+        const int q = wave + W * m;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int64_t k = q * 32 + 16 * t + 4 * kk;
+            if (top) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[m][t][r] = stripT[(k + r) * lda];
+            } else {
+                acc[m][t] = *reinterpret_cast<const f32x4*>(stripL + k);
+            }
+#pragma unroll
+            for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    g[m][t][t2][r] = G[q * 1024 + (16 * t2 + 4 * kk + r) * 32 + 16 * t + c];
+        }
+        if (q > 0) load_c(cn[m], q, 0);
+    }
+    for (int p = 0; p < NQ; ++p) {
+        if (p % W == wave) {
+            // y_p = G_p z_p
+            f32x4 y[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+            for (int m = 0; m < NO; ++m)
+                if (p == wave + W * m) {
+#pragma unroll
+                    for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+#pragma unroll
+                            for (int t = 0; t < 2; ++t)
+                                y[t] = mfma16(g[m][t][t2][r], acc[m][t2][r], y[t]);
+                    acc[m][0] = y[0];
+                    acc[m][1] = y[1];
+                }
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                *reinterpret_cast<f32x4*>(&Y[p & 1][c][16 * t + 4 * kk]) = y[t];
+        }
+        if (p + 1 == NQ) break;
+        __syncthreads();
+        f32x4 yv[2];
+#pragma unroll
+        for (int t2 = 0; t2 < 2; ++t2)
+            yv[t2] = *reinterpret_cast<const f32x4*>(&Y[p & 1][c][16 * t2 + 4 * kk]);
+#pragma unroll
+        for (int m = 0; m < NO; ++m) {
+            const int q = wave + W * m;
+            if (q > p) {
+                float x[2][2][4];
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) x[t][t2][r] = cn[m][t][t2][r];
+                if (q > p + 1) load_c(cn[m], q, p + 1);  // for the next block
+#pragma unroll
+                for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+#pragma unroll
+                        for (int t = 0; t < 2; ++t)
+                            acc[m][t] = mfma16(x[t][t2][r], yv[t2][r], acc[m][t]);
+            }
+        }
+    }
+    // ---- write back: acc[m][t][r] is element 32 q + 16 t + 4 kk + r
+    float sinv = 1.0f;
+    if constexpr (kFp8) {
+        // one power-of-two scale for the workgroup's 32 vectors x B
+        float am = 0.0f;
+#pragma unroll
+        for (int m = 0; m < NO; ++m)
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) am = fmaxf(am, fabsf(acc[m][t][r]));
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) am = fmaxf(am, __shfl_xor(am, o));
+        if (lane == 0) am_sh[threadIdx.x >> 6] = am;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < 2 * W; ++w) am = fmaxf(am, am_sh[w]);
+        const int e = fp8_scale_exp(am);
+        sinv = exp2i(-e);
+        if (threadIdx.x == 0) (top ? scT : scL)[g32] = exp2i(e);
+    }
+#pragma unroll
+    for (int m = 0; m < NO; ++m)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int64_t k = (wave + W * m) * 32 + 16 * t + 4 * kk;
+            const f32x4 y = acc[m][t];
+            if (top) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) stripT[(k + r) * lda] = y[r];
+            } else {
+                *reinterpret_cast<f32x4*>(stripL + k) = y;
+                if (Lt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) Lt[(k + r) * ldt + v] = y[r];
+            }
+            if constexpr (kLp) {
+                struct alignas(8) P4 { LP e[4]; } p4;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) p4.e[r] = static_cast<LP>(y[r]);
+                *reinterpret_cast<P4*>((top ? lpT : lpL) + v * ldlp + k) = p4;
+            }
+            if constexpr (kFp8) {
+                uint8_t* dst = reinterpret_cast<uint8_t*>(top ? lpT : lpL) + v * ldlp + k;
+                *reinterpret_cast<uint32_t*>(dst) =
+                    fp8_e4m3_code(y[0] * sinv) | (fp8_e4m3_code(y[1] * sinv) << 8) |
+                    (fp8_e4m3_code(y[2] * sinv) << 16) | (fp8_e4m3_code(y[3] * sinv) << 24);
+            }
+        }
+}
+
+// ----------------------------------------------------------------------------
 // Full inverses of the diagonal blocks for the substitution.  The strip
 // recurrences above, run on unit vectors, give for diagonal block k (with
 // L unit lower and U upper as the substitution uses them, M terms):
@@ -479,10 +662,6 @@ __global__ __launch_bounds__(64) void trsm_reg_kernel(float* __restrict__ A, int
 // pk, if not null: the inverses' BF16 operand copies of the strip solves
 // (below), written from the same registers.
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
 
 template <int B>
 __global__ __launch_bounds__(256) void block_inverse_kernel(const float* __restrict__ A,
@@ -786,6 +965,18 @@ hipError_t launch_prep_all(const float* A, int64_t lda, int B, int nblocks, floa
     return hipGetLastError();
 }
 
+// Strips of up to this many vectors a side take trsm_split_kernel: 16 waves of
+// registers per 64 vectors where trsm_reg_kernel has two, which beside a large
+// update costs more than the shorter chain gives (GEFA n = 32768, B = 256, all
+// steps by it 201.1 ms, none 198.6, up to 12288 196.7; n = 16384 29.2, none 30.5).
+constexpr int64_t kSplitStrips = 12288;
+
+// ... where the left strip's 16-byte vectors are aligned
+static bool split_ok(const float* A, int64_t lda, int64_t off, int64_t m, int64_t ldlp) {
+    return m <= kSplitStrips && !(lda & 3) && !(off & 3) && !(ldlp & 3) &&
+           !(reinterpret_cast<uintptr_t>(A) & 15);
+}
+
 template <typename LP>
 static hipError_t launch_trsm_t(float* A, int64_t lda, int64_t off, int64_t m, int B,
                                 const float* DT, int64_t lddt, const float* inv, int64_t inv_ts,
@@ -793,6 +984,20 @@ static hipError_t launch_trsm_t(float* A, int64_t lda, int64_t off, int64_t m, i
                                 float* scT = nullptr, float* scL = nullptr) {
     const int groups = (int)(m / 32);
     dim3 grid(2 * groups);
+    if (split_ok(A, lda, off, m, ldlp)) {
+#define HPL_TRSM_SPLIT(BB)                                                                    \
+    case BB:                                                                                  \
+        trsm_split_kernel<BB, LP><<<grid, 128 * kSplitWaves<BB>, 0, s>>>(                     \
+            A, lda, off, DT, lddt, inv, inv_ts, Lt, ldt, groups, lpT, lpL, ldlp, scT, scL);   \
+        return hipGetLastError();
+        switch (B) {
+            HPL_TRSM_SPLIT(64)
+            HPL_TRSM_SPLIT(128)
+            HPL_TRSM_SPLIT(256)
+            default: break;
+        }
+#undef HPL_TRSM_SPLIT
+    }
 #define HPL_TRSM_CASE(BB, KERNEL)                                                             \
     case BB:                                                                                  \
         KERNEL<BB, LP><<<grid, 64, 0, s>>>(A, lda, off, m, DT, lddt, inv, inv_ts, Lt, ldt, groups, \
@@ -815,6 +1020,8 @@ hipError_t launch_trsm_top(float* A, int64_t lda, int64_t off, int64_t m, int B,
     if (m <= 0) return hipSuccess;
     if (m % 32) return hipErrorInvalidValue;
     const int groups = (int)(m / 32);
+    // (not trsm_split_kernel: beside the other stream's update its workgroups
+    // wait longer than they gain, n = 6144 25.8 ms against 25.5)
 #define HPL_TRSM_TOP(BB)                                                                      \
     case BB:                                                                                  \
         trsm_reg_kernel<BB, float><<<groups, 64, 0, s>>>(A, lda, off, m, DT, BB, inv,         \
