@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -72,3 +74,21 @@ __device__ __forceinline__ int fp8_scale_exp(float amax) {
 }
 
 __device__ __forceinline__ float exp2i(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
+
+// lane J of each row of 16 lanes to all lanes of that row
+template <int J>
+__device__ __forceinline__ float row_bcast(float v) {
+    return __int_as_float(
+        __builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + J, 0xf, 0xf, true));
+}
+
+template <int J, int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (J < N) {
+        f(std::integral_constant<int, J>{});
+        static_for<J + 1, N>(f);
+    }
+}
+
+// lanes r > j of every row of 16 lanes, for one half of the wave
+constexpr unsigned above(int j) { return (0xffffu << (j + 1) & 0xffffu) * 0x10001u; }

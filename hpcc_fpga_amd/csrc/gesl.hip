@@ -729,8 +729,9 @@ int64_t persist_groups(int64_t n, int B) {
 hipError_t gesl_persist(const float* A, int64_t lda, int64_t n, int B, const float* binv,
                         float* x, const GeslWs& ws, int64_t G, hipStream_t s) {
     const int64_t NS = n / std::min(64, B);
-    gesl_persist_reset_kernel<<<(unsigned)std::min<int64_t>((NS + 255) / 256, 64), 256, 0,
-                                s>>>(ws.flags, NS, ws.status);
+    if (!ws.cleared)
+        gesl_persist_reset_kernel<<<(unsigned)std::min<int64_t>((NS + 255) / 256, 64), 256, 0,
+                                    s>>>(ws.flags, NS, ws.status);
     const unsigned grid = (unsigned)G;
     switch (B) {
         case 32:

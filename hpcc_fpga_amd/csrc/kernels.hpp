@@ -13,11 +13,13 @@
 hipError_t launch_lu_diag(float* A, int64_t lda, int64_t off, int B, int* status, float* DT,
                           int64_t ldt, float* inv, int64_t inv_ts, bool narrow, hipStream_t s);
 
-// panel solves (trsm.hip)
+struct GeslWs;
+
+// panel solves (trsm.hip); launch_prep_all also clears ws's flags and status
 hipError_t launch_prep(const float* A, int64_t lda, int64_t off, int B, float* DT, float* inv,
                        hipStream_t s);
 hipError_t launch_prep_all(const float* A, int64_t lda, int B, int nblocks, float* inv,
-                           int64_t inv_stride, hipStream_t s);
+                           int64_t inv_stride, hipStream_t s, const GeslWs* ws = nullptr);
 // lp_prec 0: FP32 only; 1/2: also write BF16/FP16 k-contiguous copies of the
 // top strip (lpT[c][k]) and left strip (lpL[r][k]), leading dimension ldlp;
 // 3: FP8 E4M3 copies with the scale of vectors 32 g .. 32 g + 31 at scT[g] /
@@ -98,12 +100,14 @@ hipError_t launch_block_inverse(const float* A, int64_t lda, int64_t n, int B, c
 // Workspace of the single-launch substitution of one right-hand side: the
 // forward and backward slice sums zf, zb and the forward solution y (n floats
 // each), two flags per slice and a status word (bit 2: a bounded wait gave
-// up).  Every launch clears the flags and the status itself.
+// up).  Every launch clears the flags and the status itself,
+// unless the caller has (cleared: by launch_prep_all just before).
 struct GeslWs {
     float* pf;  // forward partial solutions, B per slice
     float* pb;  // backward partial solutions, B per slice
     unsigned* flags;
     int* status;
+    bool cleared = false;
 };
 size_t gesl_ws_bytes(int64_t n);
 GeslWs gesl_ws_carve(void* base, int64_t n);  // base: gesl_ws_bytes(n), 16-byte aligned

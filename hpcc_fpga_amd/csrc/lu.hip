@@ -47,8 +47,6 @@
 #include "common.hpp"
 #include "kernels.hpp"
 
-#include <type_traits>
-
 namespace {
 
 __device__ __forceinline__ float bcast(float v, int lane) {
@@ -125,26 +123,11 @@ __device__ __forceinline__ void add_in(float* d, const float* m) {
               "v"(m[7]), "i"(M));
 }
 
-// lane J of each row of 16 lanes to all lanes of that row
-template <int J>
-__device__ __forceinline__ float row_bcast(float v) {
-    return __int_as_float(
-        __builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + J, 0xf, 0xf, true));
-}
-
 // the lower (H = 0) or upper (H = 1) half of v in both halves of the wave
 template <int H>
 __device__ __forceinline__ float from_half(float v) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(r[H]);
-}
-
-template <int J, int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (J < N) {
-        f(std::integral_constant<int, J>{});
-        static_for<J + 1, N>(f);
-    }
 }
 
 // -1/p from the hardware reciprocal and a Newton step in FMA: correctly
@@ -154,9 +137,6 @@ __device__ __forceinline__ void static_for(F&& f) {
 __device__ __forceinline__ bool rcp_in_range(float inv) {
     return ((__float_as_uint(inv) >> 23) & 0xffu) - 28u < 198u;
 }
-
-// lanes r > j of every row of 16 lanes, for one half of the wave
-constexpr unsigned above(int j) { return (0xffffu << (j + 1) & 0xffffu) * 0x10001u; }
 
 // Forward substitution of 4 NR vectors against a factorised 16 x 16 sub-block,
 // an element per lane: lane (r, q) holds element r of vector 4 q' + k, k < NR.

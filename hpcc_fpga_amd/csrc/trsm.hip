@@ -37,103 +37,136 @@ namespace {
 //   inv + 0*NQ*1024 : G^T for top   (S^-1 - C)^-1 with C = D lower, s = diag D
 //   inv + 1*NQ*1024 : G^T for left  (I - C)^-1 with C[i][p] = D[p][i]
 //   inv + 2*NQ*1024 : H^T for the back substitution of GESL, H = U_qq^-1 with
-//                     U[i][p] = D[p][i] (p > i), 1/u_ii = -D[i][i]
+//                     U[i][p] = D[p][i] (p > i), 1/u_ii = -D[i][i]: the
+//                     negated transpose of the first
+// Launch: two waves per inverse of the first two types, then one workgroup per
+// 32 x 32 block of the copy (with DT); grid.y the diagonal blocks.
+//
+// Bound: the recurrence of the unit vectors, x_r += x_j S[j][r] for r > j, 32
+// steps of one wave.  An element per lane of a DPP row: lane (r, g) of wave w
+// holds elements r and 16 + r of vectors 16 w + 4 g + k, a step is a broadcast
+// and a masked FMA per register, and the first half's part of the second is
+// taken over the solved elements at once; wave 1's vectors have no first half.
+// (A column of the inverse per lane, all three types: 8.2 us at n = 1024, 5.2
+// here; hpl_gesl_noalloc there 47.3 -> 42.6 us with the cleared flags.)
+//
+// flags, status: the substitution's, cleared here for a launch that follows.
 // ----------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void prep_kernel(const float* __restrict__ A, int64_t lda,
-                                                  int64_t off, int B, float* __restrict__ DT,
-                                                  float* __restrict__ inv, int64_t inv_stride) {
-    __shared__ float S[32][33];
+// d[k] += m[k] s in the lanes that the mask M has in each half of the wave
+template <unsigned M>
+__device__ __forceinline__ void fma_in(float (&d)[4], const float (&m)[4], float s) {
+    asm("s_mov_b32 exec_lo, %9\n\ts_mov_b32 exec_hi, %9\n\t"
+        "v_fmac_f32 %0, %4, %8\n\tv_fmac_f32 %1, %5, %8\n\t"
+        "v_fmac_f32 %2, %6, %8\n\tv_fmac_f32 %3, %7, %8\n\ts_mov_b64 exec, -1"
+        : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3])
+        : "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "v"(s), "i"(M));
+}
+
+// x_j *= dg_j, then x_r += x_j S[j][r] for r > j, 16 elements
+__device__ __forceinline__ void unit_solve(float (&x)[4], const float (&S)[16], float dg) {
+    static_for<0, 15>([&](auto jc) {
+        constexpr int j = jc.value;
+        float m[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) m[k] = row_bcast<j>(x[k] * dg);
+        fma_in<above(j)>(x, m, S[j]);
+    });
+#pragma unroll
+    for (int k = 0; k < 4; ++k) x[k] *= dg;
+}
+
+__global__ __launch_bounds__(128) void prep_kernel(const float* __restrict__ A, int64_t lda,
+                                                   int64_t off, int B, float* __restrict__ DT,
+                                                   float* __restrict__ inv, int64_t inv_stride,
+                                                   unsigned* __restrict__ flags, int64_t nflags,
+                                                   int* __restrict__ status) {
+    __shared__ __attribute__((aligned(16))) float S[32][36];
     const int NQ = B / 32;
     const int t = threadIdx.x;
     int blk = blockIdx.x;
     const float* D = A + off * lda + off;
     inv += (int64_t)blockIdx.y * inv_stride;
     if (gridDim.y > 1) D += (int64_t)blockIdx.y * (B * lda + B);  // all-blocks mode
-    // a 32 x 32 sub-block into S: four float4 per thread, all issued before
-    // the first is used (rows are 16-byte aligned: off is a multiple of 32,
-    // lda of 4)
+    if (flags) {
+        const int64_t wg = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+        for (int64_t i = wg * 128 + t; i < nflags; i += (int64_t)gridDim.x * gridDim.y * 128)
+            flags[i] = 0u;
+        if (wg == 0 && t == 0) *status = 0;
+    }
+    // a 32 x 32 sub-block into S (rows are 16-byte aligned: off is a multiple
+    // of 32, lda of 4)
     auto load_sub = [&](int r0, int c0) {
-        float4 v[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int e = t + 64 * k, i = e / 8, j = (e % 8) * 4;
-            v[k] = *reinterpret_cast<const float4*>(D + (int64_t)(r0 + i) * lda + c0 + j);
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int e = t + 64 * k, i = e / 8, j = (e % 8) * 4;
-            S[i][j] = v[k].x;
-            S[i][j + 1] = v[k].y;
-            S[i][j + 2] = v[k].z;
-            S[i][j + 3] = v[k].w;
+        for (int k = 0; k < 2; ++k) {
+            const int e = t + 128 * k, i = e / 8, j = (e % 8) * 4;
+            *reinterpret_cast<float4*>(&S[i][j]) =
+                *reinterpret_cast<const float4*>(D + (int64_t)(r0 + i) * lda + c0 + j);
         }
     };
-    if (blk >= 3 * NQ) {
-        if (DT == nullptr) return;
-        blk -= 3 * NQ;
+    if (blk >= 2 * NQ) {
+        blk -= 2 * NQ;
         const int tr = blk / NQ, tc = blk % NQ;
         load_sub(tr * 32, tc * 32);
         __syncthreads();
-        for (int e = t; e < 1024; e += 64) {
+        for (int e = t; e < 1024; e += 128) {
             const int j = e / 32, i = e % 32;
             DT[(int64_t)(tc * 32 + j) * B + tr * 32 + i] = S[i][j];
         }
         return;
     }
-    const int type = blk / NQ, q = blk % NQ;
+    const bool top = blk < NQ;
+    const int q = top ? blk : blk - NQ;
     load_sub(q * 32, q * 32);
     __syncthreads();
-    // Lane j (mod 32) computes column j of the inverse in registers, x[i] =
-    // X[i][j], with the same fmaf sequence per element as the textbook loops
-    // (a from 0, p = j .. i - 1 increasing; backward for type 2): the terms
-    // outside that range are computed and discarded by a select, so the
-    // accumulator stays +0 until the first real term.  The S reads have
-    // lane-independent addresses (LDS broadcasts) and do not depend on the
-    // chain, so only the fmaf chain is serial.
-    const int j = t & 31;
-    float x[32];
-    if (type == 0) {
+    const int r = t & 15, g = (t >> 4) & 3, w = t >> 6;
+    // coefficients S[j][r]: top D[r][j], left D[j][r]
+    auto coeff = [&](float (&s)[16], int j0, int r0) {
+        if (top) {
 #pragma unroll
-        for (int i = 0; i < 32; ++i) {
-            float a = 0.0f;
-#pragma unroll
-            for (int p = 0; p < i; ++p) {
-                const float f = fmaf(S[i][p], x[p], a);
-                a = p >= j ? f : a;
+            for (int j = 0; j < 16; j += 4) {
+                const float4 v = *reinterpret_cast<const float4*>(&S[r0 + r][j0 + j]);
+                s[j] = v.x;
+                s[j + 1] = v.y;
+                s[j + 2] = v.z;
+                s[j + 3] = v.w;
             }
-            const float sii = S[i][i];
-            x[i] = i > j ? a * sii : (i == j ? sii : 0.0f);
-        }
-    } else if (type == 1) {
+        } else {
 #pragma unroll
-        for (int i = 0; i < 32; ++i) {
-            float a = 0.0f;
-#pragma unroll
-            for (int p = 0; p < i; ++p) {
-                const float f = fmaf(S[p][i], x[p], a);
-                a = p >= j ? f : a;
-            }
-            x[i] = i > j ? a : (i == j ? 1.0f : 0.0f);
+            for (int j = 0; j < 16; ++j) s[j] = S[j0 + j][r0 + r];
         }
+    };
+    float lo[4] = {0, 0, 0, 0}, hi[4], s[16];
+    if (w == 0) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            lo[k] = 4 * g + k == r ? 1.0f : 0.0f;
+            hi[k] = 0.0f;
+        }
+        coeff(s, 0, 0);
+        unit_solve(lo, s, top ? S[r][r] : 1.0f);
+        coeff(s, 0, 16);
+        static_for<0, 16>([&](auto jc) {
+            constexpr int j = jc.value;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) hi[k] = fmaf(row_bcast<j>(lo[k]), s[j], hi[k]);
+        });
     } else {
 #pragma unroll
-        for (int i = 31; i >= 0; --i) {
-            float a = 0.0f;
-#pragma unroll
-            for (int p = i + 1; p < 32; ++p) {
-                const float f = fmaf(S[p][i], x[p], a);
-                a = p <= j ? f : a;
-            }
-            const float sii = S[i][i];
-            x[i] = i < j ? a * sii : (i == j ? -sii : 0.0f);
-        }
+        for (int k = 0; k < 4; ++k) hi[k] = 4 * g + k == r ? 1.0f : 0.0f;
     }
-    // out[j][i] = X[i][j]: lane j writes its 32 values as 16-byte vectors
-    if (t < 32) {
-        float* out = inv + (int64_t)(type * NQ + q) * 1024 + j * 32;
+    coeff(s, 16, 16);
+    unit_solve(hi, s, top ? S[16 + r][16 + r] : 1.0f);
+    // out[c][i] = element i of vector c
+    float* o = inv + (int64_t)(top ? q : NQ + q) * 1024 + (16 * w + 4 * g) * 32 + r;
 #pragma unroll
-        for (int i = 0; i < 32; i += 4)
-            *reinterpret_cast<float4*>(out + i) = float4{x[i], x[i + 1], x[i + 2], x[i + 3]};
+    for (int k = 0; k < 4; ++k) {
+        o[k * 32] = lo[k];
+        o[k * 32 + 16] = hi[k];
+    }
+    if (top) {
+        float* h = inv + (int64_t)(2 * NQ + q) * 1024 + r * 32 + 16 * w + 4 * g;
+        *reinterpret_cast<float4*>(h) = float4{-lo[0], -lo[1], -lo[2], -lo[3]};
+        *reinterpret_cast<float4*>(h + 16 * 32) = float4{-hi[0], -hi[1], -hi[2], -hi[3]};
     }
 }
 
@@ -951,17 +984,20 @@ hipError_t launch_prep(const float* A, int64_t lda, int64_t off, int B, float* D
     if ((lda & 3) || (off & 3) || (reinterpret_cast<uintptr_t>(A) & 15))
         return hipErrorInvalidValue;  // 16-byte row vectors
     const int NQ = B / 32;
-    dim3 grid(3 * NQ + (DT ? NQ * NQ : 0), 1);
-    prep_kernel<<<grid, 64, 0, s>>>(A, lda, off, B, DT, inv, 0);
+    dim3 grid(2 * NQ + (DT ? NQ * NQ : 0), 1);
+    prep_kernel<<<grid, 128, 0, s>>>(A, lda, off, B, DT, inv, 0, nullptr, 0, nullptr);
     return hipGetLastError();
 }
 
 hipError_t launch_prep_all(const float* A, int64_t lda, int B, int nblocks, float* inv,
-                           int64_t inv_stride, hipStream_t s) {
+                           int64_t inv_stride, hipStream_t s, const GeslWs* ws) {
     if ((lda & 3) || (reinterpret_cast<uintptr_t>(A) & 15)) return hipErrorInvalidValue;
     const int NQ = B / 32;
-    dim3 grid(3 * NQ, nblocks);
-    prep_kernel<<<grid, 64, 0, s>>>(A, lda, 0, B, nullptr, inv, inv_stride);
+    dim3 grid(2 * NQ, nblocks);
+    prep_kernel<<<grid, 128, 0, s>>>(A, lda, 0, B, nullptr, inv, inv_stride,
+                                     ws ? ws->flags : nullptr,
+                                     (int64_t)nblocks * B / (B < 64 ? B : 64),
+                                     ws ? ws->status : nullptr);
     return hipGetLastError();
 }
 

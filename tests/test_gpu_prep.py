@@ -1,0 +1,42 @@
+"""GPU: the 32 x 32 inverses of hpl_gesl_noalloc and of an uploaded factor.
+
+They come from a kernel that solves for the unit vectors, an element per lane;
+the substitution that applies them is compared with an FP64 substitution of the
+same factor, over orders of one block to several and every inner block (the
+largest power of two up to 256 that divides n).  Bound: the factor is well
+conditioned (diagonally dominant), so the FP32 result differs by a modest
+multiple of the unit roundoff times the root of the number of terms.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+def _x64(f, b):
+    """Substitution with gefa_ref_nopvt's factor in FP64: stored rows are M's
+    columns; negated multipliers right of the diagonal, -1/u_kk on it."""
+    n = len(b)
+    F = f.astype(np.float64).T  # M's factor
+    L = np.tril(-F, -1) + np.eye(n)
+    U = np.triu(F, 1) + np.diag(-1.0 / np.diag(F))
+    return np.linalg.solve(U, np.linalg.solve(L, b.astype(np.float64)))
+
+
+@pytest.mark.parametrize("n", [32, 64, 96, 128, 160, 256, 512, 768, 1056, 1088])
+def test_noalloc(ctx, n):
+    print(f"noalloc n={n}", flush=True)
+    a, b, _, _ = O.generate_ref(n, seed=n)
+    f = O.gefa_nopvt(a)
+    F = torch.from_numpy(f).cuda()
+    x = torch.from_numpy(b).cuda()
+    for _ in range(2):  # the flags of a launch before are cleared
+        x.copy_(torch.from_numpy(b))
+        assert ctx._L.hpl_gesl_noalloc(F.data_ptr(), n, n, x.data_ptr(), None) == 0
+        torch.cuda.synchronize()
+    ref = _x64(f, b)
+    err = np.max(np.abs(x.cpu().numpy() - ref)) / np.max(np.abs(ref))
+    assert err <= 8 * np.sqrt(n) * 2.0 ** -21
