@@ -580,7 +580,10 @@ namespace hplx {
 std::vector<int64_t> group_bounds(const hpl_ctx* c, int64_t N, int64_t B, int64_t depth,
                                   int64_t tail_cap, bool deep_head) {
     const int64_t n = N * B;
-    const int64_t tail_m = c->tail_m < 0 ? n / 2 : c->tail_m;
+    // a tail of single steps (FP32) pays off only where the chain is the longer
+    const int64_t tail_m = c->tail_m >= 0   ? c->tail_m
+                           : tail_cap == 1 ? std::min<int64_t>(n / 2, 8192)
+                                           : n / 2;
     const int64_t tail_d = c->tail_depth > 0
                                ? c->tail_depth
                                : std::max<int64_t>(1, std::min<int64_t>(depth / 2, tail_cap));

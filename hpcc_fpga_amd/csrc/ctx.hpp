@@ -44,11 +44,13 @@ struct hpl_ctx {
     int chain_cus = 0;
     int num_cu = 0;
     // Tail of the pipelined schedule: once the order still to factorise is at
-    // most tail_m (-1: half the order; 0: no tail), groups hold tail_depth
-    // steps (0: half the depth, at least 1).  The row and column-block updates
+    // most tail_m (-1: half the order, for the FP32 update at most 8192; 0: no
+    // tail), groups hold tail_depth steps (0: half the depth, at least 1).  The row and column-block updates
     // on the critical path then carry fewer steps where the bulk update no
-    // longer hides the panels: n = 32768 FP32 204.6 ms against 207.3, n =
-    // 65536 BF16 320 ms against 324.5.
+    // longer hides the panels: n = 65536 BF16 320 ms against 324.5.  The FP32
+    // update hides them down to about 8192: GEFA n = 24576 86.2 ms with half
+    // the order, 85.7 with 8192, 32768 194.8 and 192.9, 40960 375.0 and 370.0,
+    // 65536 1509 and 1482 (n = 16384: 31.1 with 4096 for 29.4).
     int64_t tail_m = -1;
     int tail_depth = 0;
     // End of the pipelined schedule: once the order still to factorise is at
@@ -233,8 +235,8 @@ uint64_t device_lda(uint64_t n);
 // Group boundaries, in blocks, of the pipelined schedule over N blocks of B:
 // b[0] = 0 < b[1] < ... = N, `depth` blocks per group until the order left
 // is at most the tail threshold, then the tail depth (the context's tail_m and
-// tail_depth, or their defaults: half the order, and half the depth but at
-// most tail_cap).  With deep_head, groups before that hold the head depth
+// tail_depth, or their defaults: half the order -- for tail_cap 1 at most
+// 8192 --, and half the depth but at most tail_cap).  With deep_head, groups before that hold the head depth
 // while the order left exceeds the head threshold (head_m, head_depth).
 std::vector<int64_t> group_bounds(const hpl_ctx* c, int64_t N, int64_t B, int64_t depth,
                                   int64_t tail_cap = 16, bool deep_head = false);
