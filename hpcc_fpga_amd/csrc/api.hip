@@ -125,7 +125,7 @@ hpl_status alloc_factor_ws(hpl_ctx* c, uint32_t B) {
     if (st) return st;
     st = ensure(c, c->dInv, c->capInv, w.inv);
     if (st) return st;
-    st = ensure(c, c->dTinv, c->capTinv, c->strip_inverse ? w.tinv : 0);
+    st = ensure(c, c->dTinv, c->capTinv, c->strip_inverse != 0 ? w.tinv : 0);
     if (st) return st;
     st = ensure(c, c->dLpT, c->capLpT, w.lp);
     if (st) return st;
@@ -255,13 +255,24 @@ hpl_status factor_diag(hpl_ctx* c, hipStream_t st, int64_t off, uint32_t B, floa
     return factor_diag(c, st, off + h, h, DT + h * ldt + h, ldt, inv + (h / 32) * 1024, inv_ts);
 }
 
+// Whether a BF16 factorisation solves its strips by the diagonal blocks'
+// inverses: their product reads the strips once and has no chain, but needs
+// the full inverses on the critical path before it.  Up to order 16384 the
+// recurrence (mostly trsm_split_kernel's) is the faster: GEFA n = 1024 B = 128
+// 0.40 ms by inverses, 0.34 by the recurrence, 4096 B = 256 1.99 and 1.59, 8192
+// 4.54 and 3.93, 16384 13.83 and 13.69, then 24576 25.4 and 25.6, 32768 44.7
+// and 45.2.
+bool strips_by_inverse(const hpl_ctx* c) {
+    return c->strip_inverse < 0 ? c->n > 16384 : c->strip_inverse > 0;
+}
+
 // Step k's buffer of diagonal-block inverses for the strip solves of the
 // BF16 factorisation, or null where the strips take the recurrence.  (The
 // split product is exact to about 2^-17, far below BF16's rounding of the
 // update operands (2^-9) but not far enough below FP16's (2^-12): the FP16
 // factorisation keeps the FP32 recurrence.)
 float* step_tinv(hpl_ctx* c, int64_t k, uint32_t B) {
-    if (!c->dTinv || !c->strip_inverse || B > 256 || c->prec != HPL_PREC_BF16) return nullptr;
+    if (!c->dTinv || !strips_by_inverse(c) || B > 256 || c->prec != HPL_PREC_BF16) return nullptr;
     return c->dTinv + (k & 1) * tinv_floats((int)B);
 }
 
@@ -284,8 +295,8 @@ hpl_status panel_diag(hpl_ctx* c, hipStream_t st, int64_t k, uint32_t B) {
 }
 
 // Panel of step k, part 2: solve the top and left strips (the left one also,
-// transposed, into its Lt slot with absolute row indices) -- one wave per 32
-// vectors, as wide as the trailing matrix.
+// transposed, into its Lt slot with absolute row indices), as wide as the
+// trailing matrix.
 hpl_status panel_strips(hpl_ctx* c, hipStream_t st, int64_t k, uint32_t B) {
     const int64_t n = (int64_t)c->n, lda = (int64_t)c->lda;
     const int64_t off = k * B;
@@ -819,7 +830,8 @@ hpl_status hpl_create(int device, hpl_ctx** out) {
     if (const char* e = getenv("HPL_LOOKAHEAD")) c->lookahead = atoi(e) != 0;
     if (const char* e = getenv("HPL_SCHEDULE")) c->pipelined = strcmp(e, "grouped") != 0;
     if (const char* e = getenv("HPL_BULK_SLICES")) c->bulk_slices = std::max(0, atoi(e));
-    if (const char* e = getenv("HPL_STRIP_SOLVE")) c->strip_inverse = strcmp(e, "recurrence") != 0;
+    if (const char* e = getenv("HPL_STRIP_SOLVE")) 
+        c->strip_inverse = !strcmp(e, "inverse") ? 1 : !strcmp(e, "recurrence") ? 0 : -1;
     if (const char* e = getenv("HPL_CHAIN_CUS")) c->chain_cus = std::max(0, atoi(e));
     if (hipDeviceGetAttribute(&c->num_cu, hipDeviceAttributeMultiprocessorCount, device) !=
         hipSuccess)

@@ -113,10 +113,11 @@ struct hpl_ctx {
     bool binv_in_gefa = false;  // the running factorisation fills dBInv
     // BF16 factorisation: the current steps' diagonal-block inverses for
     // the strip solves (two buffers, step parity), and whether to use them
-    // (HPL_STRIP_SOLVE=recurrence: the 32 x 32 block recurrence instead)
+    // (-1: by the order; HPL_STRIP_SOLVE=inverse: 1, =recurrence, the 32 x 32
+    // block recurrence instead: 0)
     float* dTinv = nullptr;
     size_t capTinv = 0;
-    bool strip_inverse = true;
+    int strip_inverse = -1;
     void* dLpT = nullptr;       // low-precision k-contiguous top-strip copies, slots of n x B (as dLt)
     void* dLpL = nullptr;       // low-precision k-contiguous left-strip copies, same layout
     size_t capLpT = 0, capLpL = 0;
