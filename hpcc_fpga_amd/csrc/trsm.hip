@@ -22,8 +22,9 @@
 // Blocking: rows are taken 32 at a time.  For block q the contribution of the
 // already solved rows is a 32 x 32q by 32q x 32 product on MFMA
 // (v_mfma_f32_32x32x2_f32), and the 32 x 32 diagonal system is applied as its
-// precomputed inverse G_q = (S^-1 - C_qq)^-1, also on MFMA.  One wavefront
-// owns 32 vectors for all B rows, so no workgroup barrier is needed.
+// precomputed inverse G_q = (S^-1 - C_qq)^-1, also on MFMA.  Either one
+// wavefront owns 32 vectors for all B rows, so that no workgroup barrier is
+// needed, or (trsm_split_kernel) several share them.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -849,7 +850,7 @@ __global__ __launch_bounds__(256) void block_inverse_kernel(const float* __restr
 //
 // Operand layout of one 32 x 32 block product (two MFMAs of K = 16): lane
 // (i, h) = (l % 32, l / 32) supplies G[i][16 kb + 8 h + e] and, for vector
-// i, v[16 kb + 8 h + e], e = 0..7.  tinv_pack_kernel writes G in that layout
+// i, v[16 kb + 8 h + e], e = 0..7.  block_inverse_kernel writes G in that layout
 // once per step: block (q, p), p <= q, at index q (q + 1) / 2 + p, 2048
 // halves each -- [kb][hi, lo][lane][8].
 __device__ __forceinline__ void split_bf16(const float (&x)[8], bf16x8_t& hi, bf16x8_t& lo) {
