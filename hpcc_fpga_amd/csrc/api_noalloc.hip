@@ -5,7 +5,7 @@
 // allocate device memory (code under HIP graph capture, serving loops,
 // harnesses that forbid hipMalloc) pass the factor and the right-hand side in
 // their own device memory instead; the inverses and the state of the
-// single-launch solve (slice sums, flags -- which each launch clears itself)
+// single-launch solve (the slices' shares -- which each launch clears itself)
 // then live in one fixed device array, `scratch`, of kScratchBytes per GPU.
 // The kernels are hpl_gesl's, in the same order, so the result is hpl_gesl's
 // bit for bit.

@@ -100,8 +100,8 @@ namespace hplx {
 // applying a whole B x B inverse loses up to a digit there (B = 256, uniform
 // matrices: 1.8e-3 against 4e-4 with 32 x 32).  So c->B is 32 for it and the
 // substitutions that apply whole inverses take the 32 x 32 ones: one launch for
-// a right-hand side (n = 6144: 1.4 ms as 96 launches, now 0.69; n = 32768
-// B = 256 10.3 -> 4.6; n = 64 0.019 -> 0.016), the MFMA sweeps for several (16
+// a right-hand side (n = 6144: 1.4 ms as 96 launches, now 0.49; n = 16384
+// B = 256 5.1 -> 1.6; n = 64 0.019 -> 0.014), the MFMA sweeps for several (16
 // refined at n = 4096: 13.7 -> 5.0 ms).  Residual of an unrefined solution,
 // means over 8 to 16 matrices: n = 1024 8.1e-7 -> 7.9e-7, 2048 1.13e-6 ->
 // 1.17e-6, 4096 1.67e-6 -> 1.57e-6, 6144 2.05e-6 -> 2.03e-6.

@@ -92,3 +92,17 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 // lanes r > j of every row of 16 lanes, for one half of the wave
 constexpr unsigned above(int j) { return (0xffffu << (j + 1) & 0xffffu) * 0x10001u; }
+
+// A share of the single-launch substitution that is not yet written: a NaN
+// pattern that no arithmetic result has.
+constexpr unsigned kGeslEmpty = 0xffffffffu;
+
+// The shares and the status before a launch, by thread i of nt.
+__device__ __forceinline__ void gesl_clear(float* pf, float* pb, int64_t words, int* status,
+                                           int64_t i, int64_t nt) {
+    if (i == 0) *status = 0;
+    for (; i < words; i += nt) {
+        pf[i] = __uint_as_float(kGeslEmpty);
+        pb[i] = __uint_as_float(kGeslEmpty);
+    }
+}

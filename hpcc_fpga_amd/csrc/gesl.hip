@@ -489,33 +489,39 @@ hipError_t gesl_sweeps_mrhs(const float* A, int64_t lda, int64_t n, int B, const
 // z followed by a publication of y.  The backward sweep mirrors it
 // (descending, U and -W_U), each slice starting from its entries of y; the
 // owners of a block finally write their entries of x.
-// Publication: values are written with agent-scope coherent stores, every
-// wave drains its stores, then the slice's flag is set (1 forward, 2
-// backward; a small kernel clears the flags before each launch).  A waiter
-// polls the T flags of the block it needs, bounded: past the limit the call
-// fails with status bit 2 and every workgroup leaves.  The factor tile of a
-// contribution and the inverse rows of a share do not depend on the awaited
-// values, so they are loaded before the wait and only the flag latency and
-// the arithmetic stay on the critical path.
+// Publication: a word that is not yet written holds kGeslEmpty, a NaN pattern that
+// no published value has (the workspace is filled with it before each launch),
+// so a value is its own flag: written with an agent-scope coherent store, it is
+// there for whoever reads it, and neither the store has to complete nor a flag
+// to arrive before it.  The workgroups of the next block, which the chain
+// waits for, read the shares until all are there; the others watch one word of
+// each share first, which keeps the traffic of a thousand waiting waves down.
+// Waits are bounded: past the limit the call fails with status bit 2 and every
+// workgroup leaves.  The factor tile of a contribution and the inverse rows of
+// a share do not depend on the awaited values, so they are loaded before the
+// wait and only the round trip and the arithmetic stay on the critical path.
+// (With drained stores, a flag and then the values, three round trips a block:
+// n = 1024 B = 64 71 us, now 57; 2048 B = 128 81, 64; 7488 B = 64 435, 369; in
+// blocks of 32 n = 6144 680, 491; n = 32768 B = 256 1417, 1262, 65536 4.67 ms,
+// 4.12.)
 // ---------------------------------------------------------------------------
 constexpr int kMaxOwn = 16;            // slices per workgroup (LDS capacity)
 constexpr int kMaxT = 4;               // shares per block (B / S, B <= 256)
 constexpr long kGeslSpinLimit = 1L << 22;
 
 __device__ __forceinline__ void pub_f(float* p, float v) {
-    __hip_atomic_store(reinterpret_cast<unsigned*>(p), __float_as_uint(v), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned u = __float_as_uint(v);
+    __hip_atomic_store(reinterpret_cast<unsigned*>(p), u == kGeslEmpty ? 0x7fc00000u : u,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ float get_f(const float* p) {
-    return __uint_as_float(__hip_atomic_load(reinterpret_cast<const unsigned*>(p),
-                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+__device__ __forceinline__ unsigned get_u(const float* p) {
+    return __hip_atomic_load(reinterpret_cast<const unsigned*>(p), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ void gesl_persist_reset_kernel(unsigned* flags, int64_t nflags, int* status) {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nflags;
-         i += (int64_t)gridDim.x * blockDim.x)
-        flags[i] = 0u;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *status = 0;
+__global__ void gesl_persist_reset_kernel(float* pf, float* pb, int64_t words, int* status) {
+    gesl_clear(pf, pb, words, status, blockIdx.x * (int64_t)blockDim.x + threadIdx.x,
+               (int64_t)gridDim.x * blockDim.x);
 }
 
 template <int B>
@@ -543,7 +549,7 @@ __global__ __launch_bounds__(NT) void gesl_persist_kernel(const float* __restric
     const int NS = (int)(n / S), N = (int)(n / B);
     const int own = (NS - g + G - 1) / G;  // slices g, g + G, ...
     const int cg = t % CG, rg = t / CG;
-    unsigned* flag = ws.flags;
+    if (t == 0) abort_flag = 0;
 
     for (int k = 0; k < own; ++k)
         for (int c = t; c < S; c += NT) {
@@ -586,41 +592,57 @@ __global__ __launch_bounds__(NT) void gesl_persist_kernel(const float* __restric
         }
         __syncthreads();
     };
-    // wait until the T flags from f on are >= target; true: the call failed
-    auto wait = [&](const unsigned* f, unsigned target) {
-        if (t == 0) {
-            int ab = 0;
-            long spins = 0;
-            for (int m = 0; m < T && !ab; ++m)
-                while (__hip_atomic_load(f + m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
-                       target) {
-                    if (++spins > spin_limit ||
-                        (__hip_atomic_load(ws.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &
-                         2)) {
-                        atomicOr(ws.status, 2);
-                        ab = 1;
-                        break;
+    auto gave_up = [&](long spins) {
+        return spins > spin_limit ||
+               ((spins & 31) == 0 && (__hip_atomic_load(ws.status, __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_AGENT) &
+                                      2));
+    };
+    // block q's vector, entries lo .. lo + len - 1, once its T shares are there:
+    // their sum, in slice order; urgent: on the chain.  true: the call failed
+    auto fetch_sum = [&](int q, const float* shares, int lo, int len, float* dst, bool urgent) {
+        const float* src = shares + (int64_t)q * T * B + lo;
+        bool bad = false;
+        if (!urgent) {
+            if (t == 0)
+                for (int j = 0; j < T && !bad; ++j)
+                    for (long spins = 1; get_u(src + j * B) == kGeslEmpty; ++spins) {
+                        if (gave_up(spins)) {
+                            bad = true;
+                            break;
+                        }
+                        __builtin_amdgcn_s_sleep(1);
                     }
-                    __builtin_amdgcn_s_sleep(1);
+            __syncthreads();
+        }
+        for (int p = t; p < len && !bad; p += NT) {
+            unsigned w[T];
+            for (long spins = 1;; ++spins) {
+                bool there = true;
+#pragma unroll
+                for (int j = 0; j < T; ++j) w[j] = get_u(src + j * B + p);
+#pragma unroll
+                for (int j = 0; j < T; ++j) there = there && w[j] != kGeslEmpty;
+                if (there) break;
+                if (gave_up(spins)) {
+                    bad = true;
+                    break;
                 }
-            abort_flag = ab;
+            }
+            float v = 0.0f;
+#pragma unroll
+            for (int j = 0; j < T; ++j) v += __uint_as_float(w[j]);
+            dst[p] = v;
+        }
+        if (bad) {
+            atomicOr(ws.status, 2);
+            abort_flag = 1;
         }
         __syncthreads();
         return abort_flag != 0;
     };
-    // block q's vector: the sum of its T shares, in slice order
-    auto fetch_sum = [&](int q, const float* shares, int lo, int len, float* dst) {
-        const float* src = shares + (int64_t)q * T * B;
-        for (int p = t; p < len; p += NT) {
-            float v = 0.0f;
-#pragma unroll
-            for (int j = 0; j < T; ++j) v += get_f(src + j * B + lo + p);
-            dst[p] = v;
-        }
-        __syncthreads();
-    };
     // slice s (owned slice k, block Q): its share sign * W[slice rows]^T z_s,
-    // published with the slice's flag; the inverse rows are loaded first
+    // published; the inverse rows are loaded first
     // (share_load), before the wait for the slice's last contribution
     float wrow[S];
     auto share_load = [&](int Q, int s, bool fwd) {
@@ -639,16 +661,18 @@ __global__ __launch_bounds__(NT) void gesl_persist_kernel(const float* __restric
             for (int r = 0; r < S; ++r) acc = fmaf(wrow[r], z[r], acc);
             pub_f((fwd ? ws.pf : ws.pb) + (int64_t)s * B + t, fwd ? acc : -acc);
         }
-        __builtin_amdgcn_s_waitcnt(0);  // this wave's stores have completed
-        __syncthreads();
-        if (t == 0)
-            __hip_atomic_store(flag + s, fwd ? 1u : 2u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();  // z_s was read before it changes
     };
-    // block q's contribution to owned slice k (= s)
+    // block q's contribution to owned slice k (= s); its vector is fetched for
+    // the first of the workgroup's slices and stays for the others
+    int have = -1;
     auto contrib = [&](int q, int k, int s, bool fwd) {
         load_tile(A + (int64_t)q * B * lda + (int64_t)s * S, lda);
-        if (wait(flag + (int64_t)q * T, fwd ? 1u : 2u)) return true;
-        fetch_sum(q, fwd ? ws.pf : ws.pb, 0, B, vbuf);
+        const int key = fwd ? q : N + q;
+        if (have != key && fetch_sum(q, fwd ? ws.pf : ws.pb, 0, B, vbuf,
+                                     s / T == (fwd ? q + 1 : q - 1)))
+            return true;
+        have = key;
         gemv(k, fwd ? 1.0f : -1.0f);
         return false;
     };
@@ -672,8 +696,7 @@ __global__ __launch_bounds__(NT) void gesl_persist_kernel(const float* __restric
     for (int k = own - 1; k >= 0; --k) {
         const int s = g + k * G, blk = s / T;
         if (blk == N - 1) share_load(N - 1, s, false);
-        if (wait(flag + (int64_t)blk * T, 1u)) return;
-        fetch_sum(blk, ws.pf, (s - blk * T) * S, S, zown + k * S);
+        if (fetch_sum(blk, ws.pf, (s - blk * T) * S, S, zown + k * S, blk == N - 1)) return;
         if (kCarry && t < S) zlo[k * S + t] = 0.0f;
         if (blk == N - 1) share(k, s, false);
     }
@@ -688,8 +711,7 @@ __global__ __launch_bounds__(NT) void gesl_persist_kernel(const float* __restric
     // x: the owners of a block sum its backward shares
     for (int k = 0; k < own; ++k) {
         const int s = g + k * G, blk = s / T;
-        if (wait(flag + (int64_t)blk * T, 2u)) return;
-        fetch_sum(blk, ws.pb, (s - blk * T) * S, S, zown + k * S);
+        if (fetch_sum(blk, ws.pb, (s - blk * T) * S, S, zown + k * S, blk == 0)) return;
         for (int c = t; c < S; c += NT) x[(int64_t)s * S + c] = zown[k * S + c];
     }
 }
@@ -728,10 +750,11 @@ int64_t persist_groups(int64_t n, int B) {
 
 hipError_t gesl_persist(const float* A, int64_t lda, int64_t n, int B, const float* binv,
                         float* x, const GeslWs& ws, int64_t G, hipStream_t s) {
-    const int64_t NS = n / std::min(64, B);
-    if (!ws.cleared)
-        gesl_persist_reset_kernel<<<(unsigned)std::min<int64_t>((NS + 255) / 256, 64), 256, 0,
-                                    s>>>(ws.flags, NS, ws.status);
+    if (!ws.cleared) {
+        const int64_t words = gesl_ws_words(n, B);
+        gesl_persist_reset_kernel<<<(unsigned)std::min<int64_t>((words + 511) / 512, 512), 256, 0,
+                                    s>>>(ws.pf, ws.pb, words, ws.status);
+    }
     const unsigned grid = (unsigned)G;
     switch (B) {
         case 32:
@@ -789,7 +812,7 @@ int64_t gesl_persist_groups(int64_t n, int B) { return persist_groups(n, B); }
 
 size_t gesl_ws_bytes(int64_t n) {
     // forward and backward shares (B per slice of S: at most kMaxT n floats
-    // each), one flag per slice of >= 32 entries, status
+    // each), status
     return (size_t)(2 * kMaxT * n) * sizeof(float) + (size_t)(n / 32 + 64) * sizeof(unsigned);
 }
 
@@ -798,7 +821,6 @@ GeslWs gesl_ws_carve(void* base, int64_t n) {
     float* f = static_cast<float*>(base);
     w.pf = f;
     w.pb = f + kMaxT * n;
-    w.flags = reinterpret_cast<unsigned*>(f + 2 * kMaxT * n);
-    w.status = reinterpret_cast<int*>(w.flags + n / 32);
+    w.status = reinterpret_cast<int*>(f + 2 * kMaxT * n);
     return w;
 }

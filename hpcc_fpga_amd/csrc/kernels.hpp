@@ -15,7 +15,7 @@ hipError_t launch_lu_diag(float* A, int64_t lda, int64_t off, int B, int* status
 
 struct GeslWs;
 
-// panel solves (trsm.hip); launch_prep_all also clears ws's flags and status
+// panel solves (trsm.hip); launch_prep_all also clears ws's shares and status
 hipError_t launch_prep(const float* A, int64_t lda, int64_t off, int B, float* DT, float* inv,
                        hipStream_t s);
 hipError_t launch_prep_all(const float* A, int64_t lda, int B, int nblocks, float* inv,
@@ -98,18 +98,18 @@ hipError_t launch_block_inverse(const float* A, int64_t lda, int64_t n, int B, c
 
 // substitution (gesl.hip)
 // Workspace of the single-launch substitution of one right-hand side: the
-// forward and backward slice sums zf, zb and the forward solution y (n floats
-// each), two flags per slice and a status word (bit 2: a bounded wait gave
-// up).  Every launch clears the flags and the status itself,
-// unless the caller has (cleared: by launch_prep_all just before).
+// forward and backward shares of the slices and a status word (bit 2: a bounded
+// wait gave up).  Every launch clears the shares and the status itself, unless
+// the caller has (cleared: by launch_prep_all just before).
 struct GeslWs {
     float* pf;  // forward partial solutions, B per slice
     float* pb;  // backward partial solutions, B per slice
-    unsigned* flags;
     int* status;
     bool cleared = false;
 };
 size_t gesl_ws_bytes(int64_t n);
+// floats of pf and of pb that a launch uses: B per slice of at most 64 entries
+inline int64_t gesl_ws_words(int64_t n, int B) { return n / (B < 64 ? B : 64) * B; }
 GeslWs gesl_ws_carve(void* base, int64_t n);  // base: gesl_ws_bytes(n), 16-byte aligned
 // workgroups of the single launch for order n at block B; 0: it does not
 // apply (block above 256, or too many slices per workgroup)

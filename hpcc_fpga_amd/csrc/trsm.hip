@@ -49,9 +49,9 @@ namespace {
 // and a masked FMA per register, and the first half's part of the second is
 // taken over the solved elements at once; wave 1's vectors have no first half.
 // (A column of the inverse per lane, all three types: 8.2 us at n = 1024, 5.2
-// here; hpl_gesl_noalloc there 47.3 -> 42.6 us with the cleared flags.)
+// here; hpl_gesl_noalloc there 47.3 -> 42.6 us with the clearing here.)
 //
-// flags, status: the substitution's, cleared here for a launch that follows.
+// pf, pb, status: the substitution's shares, cleared for a launch that follows.
 // ----------------------------------------------------------------------------
 // d[k] += m[k] s in the lanes that the mask M has in each half of the wave
 template <unsigned M>
@@ -79,8 +79,8 @@ __device__ __forceinline__ void unit_solve(float (&x)[4], const float (&S)[16], 
 __global__ __launch_bounds__(128) void prep_kernel(const float* __restrict__ A, int64_t lda,
                                                    int64_t off, int B, float* __restrict__ DT,
                                                    float* __restrict__ inv, int64_t inv_stride,
-                                                   unsigned* __restrict__ flags, int64_t nflags,
-                                                   int* __restrict__ status) {
+                                                   float* pf, float* pb, int64_t words,
+                                                   int* status) {
     __shared__ __attribute__((aligned(16))) float S[32][36];
     const int NQ = B / 32;
     const int t = threadIdx.x;
@@ -88,12 +88,10 @@ __global__ __launch_bounds__(128) void prep_kernel(const float* __restrict__ A, 
     const float* D = A + off * lda + off;
     inv += (int64_t)blockIdx.y * inv_stride;
     if (gridDim.y > 1) D += (int64_t)blockIdx.y * (B * lda + B);  // all-blocks mode
-    if (flags) {
-        const int64_t wg = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
-        for (int64_t i = wg * 128 + t; i < nflags; i += (int64_t)gridDim.x * gridDim.y * 128)
-            flags[i] = 0u;
-        if (wg == 0 && t == 0) *status = 0;
-    }
+    if (pf)
+        gesl_clear(pf, pb, words, status,
+                   ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 128 + t,
+                   (int64_t)gridDim.x * gridDim.y * 128);
     // a 32 x 32 sub-block into S (rows are 16-byte aligned: off is a multiple
     // of 32, lda of 4)
     auto load_sub = [&](int r0, int c0) {
@@ -986,7 +984,8 @@ hipError_t launch_prep(const float* A, int64_t lda, int64_t off, int B, float* D
         return hipErrorInvalidValue;  // 16-byte row vectors
     const int NQ = B / 32;
     dim3 grid(2 * NQ + (DT ? NQ * NQ : 0), 1);
-    prep_kernel<<<grid, 128, 0, s>>>(A, lda, off, B, DT, inv, 0, nullptr, 0, nullptr);
+    prep_kernel<<<grid, 128, 0, s>>>(A, lda, off, B, DT, inv, 0, nullptr, nullptr, 0,
+                                     nullptr);
     return hipGetLastError();
 }
 
@@ -996,8 +995,8 @@ hipError_t launch_prep_all(const float* A, int64_t lda, int B, int nblocks, floa
     const int NQ = B / 32;
     dim3 grid(2 * NQ, nblocks);
     prep_kernel<<<grid, 128, 0, s>>>(A, lda, 0, B, nullptr, inv, inv_stride,
-                                     ws ? ws->flags : nullptr,
-                                     (int64_t)nblocks * B / (B < 64 ? B : 64),
+                                     ws ? ws->pf : nullptr, ws ? ws->pb : nullptr,
+                                     gesl_ws_words((int64_t)nblocks * B, B),
                                      ws ? ws->status : nullptr);
     return hipGetLastError();
 }

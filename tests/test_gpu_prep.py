@@ -40,3 +40,18 @@ def test_noalloc(ctx, n):
     ref = _x64(f, b)
     err = np.max(np.abs(x.cpu().numpy() - ref)) / np.max(np.abs(ref))
     assert err <= 8 * np.sqrt(n) * 2.0 ** -21
+
+
+@pytest.mark.parametrize("n", [32, 128, 1024])
+def test_nan_of_every_pattern_ends(ctx, n):
+    """Published values announce themselves by not being the cleared pattern, a
+    NaN: right-hand sides of that very NaN (and of its payload's neighbours)
+    still come out as NaN, without a wait that gives up."""
+    print(f"gesl of NaN n={n}", flush=True)
+    a, _, _, _ = O.generate_ref(n, seed=n)
+    f = O.gefa_nopvt(a)
+    for bits in (0xFFFFFFFF, 0x7FFFFFFF, 0xFFBFFFFF, 0x7FC00000):
+        x = np.full(n, bits, np.uint32).view(np.float32)
+        st = ctx._L.hpl_gesl(ctx._c, f.ctypes.data, x.ctypes.data, n, n, None)
+        assert st == 0, (hex(bits), st)
+        assert np.all(np.isnan(x)), hex(bits)
