@@ -14,8 +14,8 @@
 //   * update_f64_kernel: C += Lt^T T on v_mfma_f64_16x16x4f64, 128 x 128
 //     workgroup tiles of four 64 x 64 wave tiles, k-slabs of 16 through
 //     double-buffered LDS, XCD-aware tile order as the FP32 update;
-//   * gesl: one launch of a wave per 64 entries that pass solved blocks on by
-//     flags; beyond what the device holds at once, per 64-block a one-wave
+//   * gesl: one launch of a wave per 64 entries that pass solved blocks on, each
+//     value its own flag; beyond what the device holds at once, per 64-block a one-wave
 //     diagonal solve (block staged in LDS) and a column-parallel update of the
 //     rest of x (the factor streamed once per sweep);
 //   * residual r = b - M x with per-chunk partial sums added in fixed order.
@@ -490,58 +490,57 @@ __global__ __launch_bounds__(256) void gesl_gemv_f64(const double* __restrict__ 
 // registers (lane l, entry l).  Forward, it takes block q's contribution as
 // soon as q is solved, q ascending, then solves its own block; backward the
 // same descending.  The arithmetic and its order are those of the kernels
-// above.  A solved block is published by agent-scope stores, then, once they
-// have completed, its flag (1 forward, 2 backward; cleared by a small kernel
-// before); waits are bounded and a wave that gives up raises status bit 2 and
-// leaves.  The tile of a contribution (and the wave's own diagonal block, the
+// above.  A solved block is published by agent-scope stores; an entry not yet
+// there holds kEmpty64, a NaN pattern that no published value has (a small
+// kernel fills it in before), so the values are their own flags.  Waits are
+// bounded and a wave that gives up raises status bit 2 and leaves.  The tile of a contribution (and the wave's own diagonal block, the
 // same access) is loaded into the registers that the tile before it leaves,
-// so only the flag and the arithmetic follow a wait.
-// Bound: the chain of 2 n / 64 block solves, each a flag's trip, 64 steps of
-// contribution and 64 of the solve.  0.99 ms at n = 8192, 2.92 launch after
-// launch, 4 n / 64 of them (n = 1024 0.31 -> 0.12, 32768 12.5 -> 4.7).
+// so only the arithmetic follows a wait.
+// Bound: the chain of 2 n / 64 block solves, each a value's trip, 64 steps of
+// contribution and 64 of the solve.  0.91 ms at n = 8192, 2.92 launch after
+// launch, 4 n / 64 of them (n = 1024 0.31 -> 0.11, 32768 12.5 -> 4.3); with
+// drained stores, flags and then the values 1.00, 0.124 and 4.7.
 constexpr long kGesl64SpinLimit = 1L << 22;
 
-__global__ void gesl_reset_f64(unsigned* __restrict__ flags, int count, int* __restrict__ status) {
-    for (int i = threadIdx.x; i < count; i += blockDim.x) flags[i] = 0u;
-    if (threadIdx.x == 0) *status = 0;
+constexpr unsigned long long kEmpty64 = ~0ull;
+
+__global__ void gesl_reset_f64(double* __restrict__ w, int64_t count, int* __restrict__ status) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < count) w[i] = __longlong_as_double((long long)kEmpty64);
+    if (i == 0) *status = 0;
 }
 
 __global__ __launch_bounds__(64) void gesl_persist_f64(const double* __restrict__ A, int64_t lda,
                                                        int N, double* __restrict__ x,
                                                        double* __restrict__ pf,
                                                        double* __restrict__ pb,
-                                                       unsigned* __restrict__ flags,
                                                        int* __restrict__ status, long spin_limit) {
 #pragma clang fp contract(off)
     const int l = threadIdx.x, s = blockIdx.x;
     const double* col = A + (int64_t)s * FB + l;  // this lane's column of the factor
     auto put = [&](double* p, double v) {
+        const unsigned long long u = (unsigned long long)__double_as_longlong(v);
         __hip_atomic_store(reinterpret_cast<unsigned long long*>(p + (int64_t)s * FB + l),
-                           (unsigned long long)__double_as_longlong(v), __ATOMIC_RELAXED,
+                           u == kEmpty64 ? 0x7ff8000000000000ull : u, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
     };
-    auto get = [&](const double* p, int q) {
-        return __longlong_as_double((long long)__hip_atomic_load(
-            reinterpret_cast<const unsigned long long*>(p + (int64_t)q * FB + l), __ATOMIC_RELAXED,
-            __HIP_MEMORY_SCOPE_AGENT));
-    };
-    auto publish = [&](unsigned v) {
-        __builtin_amdgcn_s_waitcnt(0);  // the wave's stores have completed
-        if (l == 0)
-            __hip_atomic_store(flags + s, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    };
-    // true: gave up
-    auto wait = [&](int q, unsigned v) {
-        long spins = 0;
-        while (__hip_atomic_load(flags + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < v) {
-            if (++spins > spin_limit ||
-                (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 2)) {
+    // this lane's entry of block q once all of them are there; true: gave up
+    auto get = [&](const double* p, int q, double& v) {
+        for (long spins = 1;; ++spins) {
+            const unsigned long long u = __hip_atomic_load(
+                reinterpret_cast<const unsigned long long*>(p + (int64_t)q * FB + l),
+                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            v = __longlong_as_double((long long)u);
+            if (!__any(u == kEmpty64)) return false;
+            if (spins > spin_limit ||
+                ((spins & 31) == 0 &&
+                 (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 2))) {
                 if (l == 0) atomicOr(status, 2);
                 return true;
             }
-            __builtin_amdgcn_s_sleep(1);
+            // on the chain only the next block's wave waits
+            if (q + 1 != s && q - 1 != s) __builtin_amdgcn_s_sleep(1);
         }
-        return false;
     };
     double a[FB];
     auto load = [&](int q) {
@@ -552,8 +551,8 @@ __global__ __launch_bounds__(64) void gesl_persist_f64(const double* __restrict_
     // ---- forward: L y = b
     load(0);
     for (int q = 0; q < s; ++q) {
-        if (wait(q, 1u)) return;
-        const double xs = get(pf, q);
+        double xs;
+        if (get(pf, q, xs)) return;
         const double* next = col + (int64_t)(q + 1) * FB * lda;
 #pragma unroll
         for (int u = 0; u < FB; ++u) {
@@ -567,12 +566,12 @@ __global__ __launch_bounds__(64) void gesl_persist_f64(const double* __restrict_
         if (l > k) xi = xi + xk * a[k];
     }
     put(pf, xi);
-    publish(1u);
     // ---- backward: U x = y
     load(N - 1);
     for (int q = N - 1; q > s; --q) {
-        if (wait(q, 2u)) return;
-        const double xs = -get(pb, q);
+        double xs;
+        if (get(pb, q, xs)) return;
+        xs = -xs;
         const double* next = col + (int64_t)(q - 1) * FB * lda;
 #pragma unroll
         for (int u = FB - 1; u >= 0; --u) {
@@ -587,7 +586,6 @@ __global__ __launch_bounds__(64) void gesl_persist_f64(const double* __restrict_
         if (l < k) xi = xi + sk * a[k];
     }
     put(pb, xi);
-    publish(2u);
     x[(int64_t)s * FB + l] = xi;
 }
 
@@ -695,8 +693,8 @@ hipError_t launch_update_f64(double* C, int64_t ldc, const double* Lt, int64_t l
 }
 
 int64_t gesl_f64_work(int64_t n) {
-    // both sweeps' published blocks, a flag per block, the status
-    return 2 * n + n / FB / 2 + 8;
+    // both sweeps' published blocks, the status
+    return 2 * n + 8;
 }
 
 const int* gesl_f64_status(const double* work, int64_t n) {
@@ -707,7 +705,6 @@ hipError_t launch_gesl_f64(const double* A, int64_t lda, int64_t n, double* x, d
                            hipStream_t s) {
     if (n % FB) return hipErrorInvalidValue;
     int* status = reinterpret_cast<int*>(work + 2 * n);
-    unsigned* flags = reinterpret_cast<unsigned*>(work + 2 * n + 8);
     const int64_t N = n / FB;
     // Every wave has to be resident at once: at most half of what the device
     // holds, so that other work on it leaves room (n up to 65536); beyond, or
@@ -720,9 +717,9 @@ hipError_t launch_gesl_f64(const double* A, int64_t lda, int64_t n, double* x, d
         (void)hipGetLastError();
         per_cu = cus = 0;
     }
-    gesl_reset_f64<<<1, 256, 0, s>>>(flags, (int)N, status);
+    gesl_reset_f64<<<(unsigned)((2 * n + 255) / 256), 256, 0, s>>>(work, 2 * n, status);
     if (N <= (int64_t)per_cu * cus / 2) {
-        gesl_persist_f64<<<(unsigned)N, 64, 0, s>>>(A, lda, (int)N, x, work, work + n, flags, status,
+        gesl_persist_f64<<<(unsigned)N, 64, 0, s>>>(A, lda, (int)N, x, work, work + n, status,
                                                     kGesl64SpinLimit);
         return hipGetLastError();
     }

@@ -55,3 +55,14 @@ def test_nan_of_every_pattern_ends(ctx, n):
         st = ctx._L.hpl_gesl(ctx._c, f.ctypes.data, x.ctypes.data, n, n, None)
         assert st == 0, (hex(bits), st)
         assert np.all(np.isnan(x)), hex(bits)
+
+
+@pytest.mark.parametrize("n", [64, 1024])
+def test_nan_of_every_pattern_ends_f64(ctx, n):
+    print(f"f64 gesl of NaN n={n}", flush=True)
+    a, _ = O.generate_ref_f64(n, seed=n)
+    f = O.gefa_nopvt_f64(a)
+    for bits in (0xFFFFFFFFFFFFFFFF, 0x7FFFFFFFFFFFFFFF, 0xFFF7FFFFFFFFFFFF):
+        x = np.full(n, bits, np.uint64).view(np.float64)
+        ctx.gesl_f64(f, x)
+        assert np.all(np.isnan(x)), hex(bits)
