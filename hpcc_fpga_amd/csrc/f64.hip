@@ -23,6 +23,7 @@
 #include "kernels.hpp"
 
 #include <algorithm>
+#include <cstdlib>
 #include <type_traits>
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
@@ -493,14 +494,18 @@ __global__ __launch_bounds__(256) void gesl_gemv_f64(const double* __restrict__ 
 // above.  A solved block is published by agent-scope stores; an entry not yet
 // there holds kEmpty64, a NaN pattern that no published value has (a small
 // kernel fills it in before), so the values are their own flags.  Waits are
-// bounded and a wave that gives up raises status bit 2 and leaves.  The tile of a contribution (and the wave's own diagonal block, the
-// same access) is loaded into the registers that the tile before it leaves,
-// so only the arithmetic follows a wait.
+// bounded and a wave that gives up raises status bit 2 and leaves; the host
+// then solves launch after launch.  The tile of a contribution (and the wave's
+// own diagonal block, the same access) is loaded into the registers that the
+// tile before it leaves, so only the arithmetic follows a wait.
 // Bound: the chain of 2 n / 64 block solves, each a value's trip, 64 steps of
 // contribution and 64 of the solve.  0.91 ms at n = 8192, 2.92 launch after
 // launch, 4 n / 64 of them (n = 1024 0.31 -> 0.11, 32768 12.5 -> 4.3); with
 // drained stores, flags and then the values 1.00, 0.124 and 4.7.
-constexpr long kGesl64SpinLimit = 1L << 22;
+// Polls before a wave gives up, about a second: whoever waits that long shares
+// the device with launches that keep its partners from starting, and solving
+// launch after launch takes milliseconds.
+constexpr long kGesl64SpinLimit = 1L << 20;
 
 constexpr unsigned long long kEmpty64 = ~0ull;
 
@@ -702,13 +707,14 @@ const int* gesl_f64_status(const double* work, int64_t n) {
 }
 
 hipError_t launch_gesl_f64(const double* A, int64_t lda, int64_t n, double* x, double* work,
-                           hipStream_t s) {
+                           hipStream_t s, bool per_block) {
     if (n % FB) return hipErrorInvalidValue;
     int* status = reinterpret_cast<int*>(work + 2 * n);
     const int64_t N = n / FB;
     // Every wave has to be resident at once: at most half of what the device
-    // holds, so that other work on it leaves room (n up to 65536); beyond, or
-    // where the device does not say, launch after launch.
+    // holds, so that other work on it leaves room (n up to 65536), and at most
+    // HPL_GESL_GROUPS; beyond, where the device does not say, or where the
+    // caller asks for it (per_block), launch after launch.
     int per_cu = 0, dev = 0, cus = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
             &per_cu, reinterpret_cast<const void*>(gesl_persist_f64), 64, 0) != hipSuccess ||
@@ -718,9 +724,11 @@ hipError_t launch_gesl_f64(const double* A, int64_t lda, int64_t n, double* x, d
         per_cu = cus = 0;
     }
     gesl_reset_f64<<<(unsigned)((2 * n + 255) / 256), 256, 0, s>>>(work, 2 * n, status);
-    if (N <= (int64_t)per_cu * cus / 2) {
+    int64_t most = per_block ? 0 : (int64_t)per_cu * cus / 2;
+    if (const char* e = getenv("HPL_GESL_GROUPS")) most = std::min<int64_t>(most, atoll(e));
+    if (N <= most) {
         gesl_persist_f64<<<(unsigned)N, 64, 0, s>>>(A, lda, (int)N, x, work, work + n, status,
-                                                    kGesl64SpinLimit);
+                                                    gesl_spin_limit(kGesl64SpinLimit));
         return hipGetLastError();
     }
     for (int64_t k0 = 0; k0 < n; k0 += FB) {

@@ -756,18 +756,19 @@ hipError_t gesl_persist(const float* A, int64_t lda, int64_t n, int B, const flo
                                     s>>>(ws.pf, ws.pb, words, ws.status);
     }
     const unsigned grid = (unsigned)G;
+    const long spins = gesl_spin_limit(kGeslSpinLimit);
     switch (B) {
         case 32:
-            gesl_persist_kernel<32><<<grid, NT, 0, s>>>(A, lda, n, binv, x, ws, kGeslSpinLimit);
+            gesl_persist_kernel<32><<<grid, NT, 0, s>>>(A, lda, n, binv, x, ws, spins);
             break;
         case 64:
-            gesl_persist_kernel<64><<<grid, NT, 0, s>>>(A, lda, n, binv, x, ws, kGeslSpinLimit);
+            gesl_persist_kernel<64><<<grid, NT, 0, s>>>(A, lda, n, binv, x, ws, spins);
             break;
         case 128:
-            gesl_persist_kernel<128><<<grid, NT, 0, s>>>(A, lda, n, binv, x, ws, kGeslSpinLimit);
+            gesl_persist_kernel<128><<<grid, NT, 0, s>>>(A, lda, n, binv, x, ws, spins);
             break;
         default:
-            gesl_persist_kernel<256><<<grid, NT, 0, s>>>(A, lda, n, binv, x, ws, kGeslSpinLimit);
+            gesl_persist_kernel<256><<<grid, NT, 0, s>>>(A, lda, n, binv, x, ws, spins);
             break;
     }
     return hipGetLastError();
@@ -809,6 +810,11 @@ hipError_t launch_gesl(const float* A, int64_t lda, int64_t n, int B, const floa
 }
 
 int64_t gesl_persist_groups(int64_t n, int B) { return persist_groups(n, B); }
+
+long gesl_spin_limit(long most) {
+    const char* e = getenv("HPL_GESL_SPIN");
+    return e ? std::min(most, std::max(0L, atol(e))) : most;
+}
 
 size_t gesl_ws_bytes(int64_t n) {
     // forward and backward shares (B per slice of S: at most kMaxT n floats

@@ -111,6 +111,10 @@ size_t gesl_ws_bytes(int64_t n);
 // floats of pf and of pb that a launch uses: B per slice of at most 64 entries
 inline int64_t gesl_ws_words(int64_t n, int B) { return n / (B < 64 ? B : 64) * B; }
 GeslWs gesl_ws_carve(void* base, int64_t n);  // base: gesl_ws_bytes(n), 16-byte aligned
+// polls after which a wait of a single-launch substitution gives up: `most`, or
+// HPL_GESL_SPIN if that is less (0: at the first miss, which a test of what
+// follows then asks for)
+long gesl_spin_limit(long most);
 // workgroups of the single launch for order n at block B; 0: it does not
 // apply (block above 256, or too many slices per workgroup)
 int64_t gesl_persist_groups(int64_t n, int B);
@@ -184,11 +188,13 @@ hipError_t launch_update_f64(double* C, int64_t ldc, const double* Lt, int64_t l
                              const double* Lt2, const double* T2, int M2, int N2, int K,
                              hipStream_t s);
 // work: gesl_f64_work(n) doubles; *gesl_f64_status(work, n) is non-zero
-// afterwards where a bounded wait of the single launch gave up
+// afterwards where a bounded wait of the single launch gave up (x is then
+// partly overwritten; per_block solves without one, launch after launch, to the
+// same bits)
 int64_t gesl_f64_work(int64_t n);
 const int* gesl_f64_status(const double* work, int64_t n);
 hipError_t launch_gesl_f64(const double* A, int64_t lda, int64_t n, double* x, double* work,
-                           hipStream_t s);
+                           hipStream_t s, bool per_block = false);
 int64_t residual_f64_work(int64_t n);
 hipError_t launch_residual_f64(const double* A, int64_t lda, int64_t n, const double* x,
                                const double* b, double* work, double* out4, hipStream_t s);
