@@ -672,13 +672,12 @@ const GeslWs* gesl_workspace(hpl_ctx* c, GeslWs* ws) {
     return ws;
 }
 
-hpl_status gesl_check(hpl_ctx* c, const GeslWs* ws) {
+hpl_status gesl_gave_up(hpl_ctx* c, const GeslWs* ws, bool* again) {
+    *again = false;
     if (!ws) return HPL_SUCCESS;
     int h = 0;
     HIPCHK(c, c->stage.to_host(c->s0, &h, ws->status, sizeof(int)));
-    if (h & 2)
-        return fail(c, HPL_ERR_HIP,
-                    "substitution: a bounded wait gave up (workgroups not co-resident)");
+    *again = (h & 2) != 0;
     return HPL_SUCCESS;
 }
 
@@ -687,7 +686,8 @@ IrPlan plan_ir(uint64_t n, int nrhs) {
     p.work = (size_t)residual_multi_work((int64_t)n, nrhs) * sizeof(double);
     p.r = (size_t)n * nrhs * sizeof(double);
     p.xs = (size_t)n * nrhs * sizeof(float);
-    p.out = 4 * (size_t)nrhs * sizeof(double);
+    // the norms, behind one column's the status of a single-launch substitution
+    p.out = std::max<size_t>(4 * (size_t)nrhs, 5) * sizeof(double);
     return p;
 }
 
@@ -716,28 +716,21 @@ hpl_status init_pipeline_streams(hpl_ctx* c) {
     return HPL_SUCCESS;
 }
 
-hpl_status ir_solve(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_iter, double tol,
-                    hpl_ir_result* res) {
-    if (nrhs < 1 || nrhs > 16) return fail(c, HPL_ERR_INVALID_ARG, "nrhs %d not in [1,16]", nrhs);
+namespace {
+
+// One refinement from x0 = F^-1 b on, its substitutions by the single launch
+// where ws is given (one column, the status behind the norms in dIrOut); *again:
+// one of them gave up, the answer is void.
+hpl_status refine(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_iter, double tol,
+                  hpl_ir_result* res, const GeslWs* ws, bool* again) {
+    *again = false;
     const int64_t n = (int64_t)c->n;
-    const IrPlan p = plan_ir(c->n, nrhs);
-    hpl_status st = ensure(c, c->dWork, c->capWork, p.work);
-    if (st) return st;
-    st = ensure(c, c->dIrR, c->capIrR, p.r);
-    if (st) return st;
-    st = ensure(c, c->dIrXs, c->capIrXs, p.xs);
-    if (st) return st;
-    st = ensure(c, c->dIrOut, c->capIrOut, p.out);
-    if (st) return st;
-    st = ensure_block_inverses(c);
-    if (st) return st;
-    GeslWs wsbuf;
-    const GeslWs* ws = nrhs == 1 ? gesl_workspace(c, &wsbuf) : nullptr;
     const int B = (int)c->B;
     const int64_t inv_stride = 3 * (B / 32) * 1024;
     // the substitution of several columns: between two residuals, whose
     // partial sums (at least n (nrhs + 1) doubles) it overwrites
     float* scratch = reinterpret_cast<float*>(c->dWork);
+    const size_t out_bytes = 4 * nrhs * sizeof(double) + (ws ? sizeof(int) : 0);
     double sc_in[16], sc_out[16], h[64];
     int iters[16];
     for (int j = 0; j < nrhs; ++j) {
@@ -753,7 +746,15 @@ hpl_status ir_solve(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_
     for (int it = 0;; ++it) {
         HIPCHK(c, launch_residual_multi(c->dA0, (int64_t)c->lda, n, dX, n, dB, n, nrhs, c->dWork,
                                         c->dIrR, n, c->dIrOut, c->s0));
-        HIPCHK(c, c->stage.to_host(c->s0, h, c->dIrOut, 4 * nrhs * sizeof(double)));
+        HIPCHK(c, c->stage.to_host(c->s0, h, c->dIrOut, out_bytes));
+        if (ws) {
+            int status;
+            std::memcpy(&status, h + 4, sizeof status);
+            if (status & 2) {
+                *again = true;
+                return HPL_SUCCESS;
+            }
+        }
         bool any = false;
         for (int j = 0; j < nrhs; ++j) {
             const double* hj = h + 4 * j;
@@ -784,8 +785,32 @@ hpl_status ir_solve(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_
                                     scratch));
         HIPCHK(c, launch_axpy_multi(dX, n, c->dIrXs, n, n, nrhs, sc_out, 0, c->s0));
     }
-    st = gesl_check(c, ws);
+    return HPL_SUCCESS;
+}
+
+}  // namespace
+
+hpl_status ir_solve(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_iter, double tol,
+                    hpl_ir_result* res) {
+    if (nrhs < 1 || nrhs > 16) return fail(c, HPL_ERR_INVALID_ARG, "nrhs %d not in [1,16]", nrhs);
+    const IrPlan p = plan_ir(c->n, nrhs);
+    hpl_status st = ensure(c, c->dWork, c->capWork, p.work);
     if (st) return st;
+    st = ensure(c, c->dIrR, c->capIrR, p.r);
+    if (st) return st;
+    st = ensure(c, c->dIrXs, c->capIrXs, p.xs);
+    if (st) return st;
+    st = ensure(c, c->dIrOut, c->capIrOut, p.out);
+    if (st) return st;
+    st = ensure_block_inverses(c);
+    if (st) return st;
+    GeslWs wsbuf;
+    const GeslWs* ws = nrhs == 1 ? gesl_workspace(c, &wsbuf) : nullptr;
+    if (ws) wsbuf.status = reinterpret_cast<int*>(c->dIrOut + 4);
+    for (bool again = true; again; ws = nullptr) {
+        st = refine(c, nrhs, dB, dX, max_iter, tol, res, ws, &again);
+        if (st) return st;
+    }
     for (int j = 0; j < nrhs; ++j)
         if (!res[j].converged)
             return fail(c, HPL_ERR_NOT_CONVERGED,
@@ -1017,21 +1042,24 @@ hpl_status hpl_gesl_dev(hpl_ctx* c, hpl_timing* t) {
     HIPCHK(c, hipEventRecord(c->e0, c->s0));
     hpl_status st = hplx::ensure_block_inverses(c);
     if (st) return st;
-    if (c->pivoted)
-        HIPCHK(c, launch_gather_f32(c->dx, c->db, c->dPerm, (int64_t)c->n, c->s0));
-    else
-        HIPCHK(c, hipMemcpyAsync(c->dx, c->db, c->n * sizeof(float), hipMemcpyDeviceToDevice,
-                                 c->s0));
     GeslWs wsbuf;
     const GeslWs* ws = hplx::gesl_workspace(c, &wsbuf);
-    HIPCHK(c, launch_gesl(c->dA, (int64_t)c->lda, (int64_t)c->n, (int)c->B, c->dInv,
-                          3 * (c->B / 32) * 1024, c->dx, c->s0, c->binv_ready ? c->dBInv : nullptr,
-                          ws));
-    HIPCHK(c, hipEventRecord(c->e1, c->s0));
-    st = hplx::gesl_check(c, ws);  // waits for the stream where there is a status
-    if (!ws) HIPCHK(c, hipStreamSynchronize(c->s0));
+    for (bool again = true; again; ws = nullptr) {
+        if (c->pivoted)
+            HIPCHK(c, launch_gather_f32(c->dx, c->db, c->dPerm, (int64_t)c->n, c->s0));
+        else
+            HIPCHK(c, hipMemcpyAsync(c->dx, c->db, c->n * sizeof(float), hipMemcpyDeviceToDevice,
+                                     c->s0));
+        HIPCHK(c, launch_gesl(c->dA, (int64_t)c->lda, (int64_t)c->n, (int)c->B, c->dInv,
+                              3 * (c->B / 32) * 1024, c->dx, c->s0,
+                              c->binv_ready ? c->dBInv : nullptr, ws));
+        HIPCHK(c, hipEventRecord(c->e1, c->s0));
+        st = hplx::gesl_gave_up(c, ws, &again);  // waits for the stream where there is a status
+        if (st) return st;
+        if (!ws) HIPCHK(c, hipStreamSynchronize(c->s0));
+    }
     if (t) t->gesl_s = elapsed_s(c);
-    return st;
+    return HPL_SUCCESS;
 }
 
 hpl_status hpl_download(hpl_ctx* c, float* a, uint64_t lda, float* x, hpl_timing* t) {
@@ -1163,21 +1191,26 @@ hpl_status hpl_solve_ir(hpl_ctx* c, uint32_t block, hpl_prec prec, int max_iter,
 namespace {
 
 // z = F^-1 v for an FP64 vector v (FP32 substitution with the resident
-// factor, result promoted); xs is the FP32 scratch of length n.
-hpl_status precond_apply(hpl_ctx* c, const double* v, double* z) {
+// factor, result promoted); xs is the FP32 scratch of length n.  *single: by the
+// single launch where there is one, until it gives up once.
+hpl_status precond_apply(hpl_ctx* c, const double* v, double* z, bool* single) {
     const int64_t n = (int64_t)c->n;
     const int B = (int)c->B;
     const double one = 1.0;
     hpl_status st = hplx::ensure_block_inverses(c);
     if (st) return st;
-    HIPCHK(c, launch_d2f_multi(v, n, c->dIrXs, n, n, 1, &one, c->s0,
-                               c->pivoted ? c->dPerm : nullptr));
-    GeslWs wsbuf;
-    const GeslWs* ws = hplx::gesl_workspace(c, &wsbuf);
-    HIPCHK(c, launch_gesl_multi(c->dA, (int64_t)c->lda, n, B, c->dInv, 3 * (B / 32) * 1024,
-                                c->dIrXs, n, 1, c->s0, c->binv_ready ? c->dBInv : nullptr, ws));
-    st = hplx::gesl_check(c, ws);
-    if (st) return st;
+    for (bool again = true; again;) {
+        HIPCHK(c, launch_d2f_multi(v, n, c->dIrXs, n, n, 1, &one, c->s0,
+                                   c->pivoted ? c->dPerm : nullptr));
+        GeslWs wsbuf;
+        const GeslWs* ws = *single ? hplx::gesl_workspace(c, &wsbuf) : nullptr;
+        HIPCHK(c, launch_gesl_multi(c->dA, (int64_t)c->lda, n, B, c->dInv, 3 * (B / 32) * 1024,
+                                    c->dIrXs, n, 1, c->s0, c->binv_ready ? c->dBInv : nullptr,
+                                    ws));
+        st = hplx::gesl_gave_up(c, ws, &again);
+        if (st) return st;
+        if (again) *single = false;
+    }
     HIPCHK(c, launch_axpy_multi(z, n, c->dIrXs, n, n, 1, &one, 1, c->s0));
     return HPL_SUCCESS;
 }
@@ -1252,8 +1285,9 @@ hpl_status hpl_solve_gmres(hpl_ctx* c, uint32_t block, hpl_prec prec, int restar
     double* W = c->dGmW;
     double* dh = c->dGmC;  // coefficients: [0, m+1) pass 1 / solution, [m+1, 2m+2) pass 2
     double* work = c->dGmWork;
+    bool single = true;
     // x0 = F^-1 b
-    st = precond_apply(c, c->db64, c->dX64);
+    st = precond_apply(c, c->db64, c->dX64, &single);
     if (st) return st;
     std::vector<double> H((size_t)(m + 1) * m), cs(m), sn(m), g(m + 1), h1(m + 1), h2(m + 1),
         y(m), coef(2 * m + 2);
@@ -1267,7 +1301,7 @@ hpl_status hpl_solve_gmres(hpl_ctx* c, uint32_t block, hpl_prec prec, int restar
         berr = hres[0] / (hres[1] * hres[2] + hres[3]);
         if (berr <= tol || outer >= max_iter || !(hres[0] > 0.0) || !(hres[0] < HUGE_VAL)) break;
         // GMRES on F^-1 M d = F^-1 r, d0 = 0: V0 = z / beta
-        st = precond_apply(c, c->dIrR, W);
+        st = precond_apply(c, c->dIrR, W, &single);
         if (st) return st;
         HIPCHK(c, launch_multi_dot(W, n, 1, W, n, dh, work, c->s0));
         double beta2 = 0.0;
@@ -1283,7 +1317,7 @@ hpl_status hpl_solve_gmres(hpl_ctx* c, uint32_t block, hpl_prec prec, int restar
             // W = F^-1 M V_i
             HIPCHK(c, launch_matvec_f64(c->dA0, (int64_t)c->lda, n, V + (int64_t)i * n, W, work,
                                         c->s0));
-            st = precond_apply(c, W, W);
+            st = precond_apply(c, W, W, &single);
             if (st) return st;
             // classical Gram-Schmidt, twice: h = V^T W, W -= V h
             HIPCHK(c, launch_multi_dot(V, n, i + 1, W, n, dh, work, c->s0));

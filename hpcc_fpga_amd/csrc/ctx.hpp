@@ -249,9 +249,11 @@ hpl_status ensure_block_inverses(hpl_ctx* c);
 // Workspace of the single-launch substitution of one right-hand side with the
 // resident factor (in *ws), or null where the per-step launches solve instead
 // (external mode, no full inverses, or a block the single launch does not
-// take).  gesl_check reads its status after the solve (synchronises s0).
+// take).  gesl_gave_up reads its status after the solve (synchronises s0): *again
+// where a bounded wait gave up, as other launches kept its workgroups from being
+// resident together; the caller solves again without the workspace.
 const GeslWs* gesl_workspace(hpl_ctx* c, GeslWs* ws);
-hpl_status gesl_check(hpl_ctx* c, const GeslWs* ws);
+hpl_status gesl_gave_up(hpl_ctx* c, const GeslWs* ws, bool* again);
 
 // Device buffer of at least `bytes` (grown with hipMalloc in the context's own
 // mode, an error in external mode).

@@ -496,8 +496,8 @@ hipError_t gesl_sweeps_mrhs(const float* A, int64_t lda, int64_t n, int B, const
 // to arrive before it.  The workgroups of the next block, which the chain
 // waits for, read the shares until all are there; the others watch one word of
 // each share first, which keeps the traffic of a thousand waiting waves down.
-// Waits are bounded: past the limit the call fails with status bit 2 and every
-// workgroup leaves.  The factor tile of a contribution and the inverse rows of
+// Waits are bounded: past the limit status bit 2 is raised and every workgroup
+// leaves (a context's calls then solve again by the per-step launches).  The factor tile of a contribution and the inverse rows of
 // a share do not depend on the awaited values, so they are loaded before the
 // wait and only the round trip and the arithmetic stay on the critical path.
 // (With drained stores, a flag and then the values, three round trips a block:

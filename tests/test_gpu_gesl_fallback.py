@@ -38,3 +38,35 @@ def test_fp64(monkeypatch, env, n):
             x = b.copy()
             c.gesl_f64(F, x)
             assert np.array_equal(x.view(np.uint64), ref.view(np.uint64))
+
+
+@pytest.mark.parametrize("n,B,pivot", [(2048, 256, False), (1152, 128, False), (1088, 64, False),
+                                       (544, 32, False), (576, 64, True), (2048, 256, True)])
+def test_fp32(monkeypatch, n, B, pivot):
+    """Giving up ends in the launches per block: the bits of a call that starts there
+    (one workgroup cannot own more than 16 slices of 64, or 32, entries)."""
+    g = np.random.default_rng(n + B)
+    a = (g.random((n, n)) - 0.5).astype(np.float32)
+    if not pivot:
+        a[np.arange(n), np.arange(n)] += n
+    b = g.uniform(-1, 1, n)
+    out = {}
+    for name, env in (("groups", {"HPL_GESL_GROUPS": "1"}), ("spin", {"HPL_GESL_SPIN": "0"})):
+        print(f"fp32 gesl {env} n={n} B={B} pivot={pivot}", flush=True)
+        _env(monkeypatch, env)
+        with Context(0) as c:
+            c.keep_original(True)
+            c.set_pivoting(pivot)
+            c.upload(a)
+            c.upload_rhs64(b)
+            c.gefa_dev(B)
+            c.gesl_dev()
+            x = c.download(matrix=False)[1]
+            c.solve_ir(B, "fp32", tol=1e-15)
+            r = c.download_solution64()
+            c.solve_gmres(B, "fp32", tol=1e-15)
+            out[name] = x, r, c.download_solution64(), c.solve_rhs64(b)[0]
+    for p, q in zip(out["groups"], out["spin"]):
+        assert np.all(np.isfinite(p)) and np.array_equal(p, q)
+    ref = np.linalg.solve(a.T.astype(np.float64), b)
+    assert np.max(np.abs(out["spin"][1] - ref)) <= 1e-9 * np.max(np.abs(ref))
