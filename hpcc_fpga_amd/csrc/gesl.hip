@@ -497,7 +497,8 @@ hipError_t gesl_sweeps_mrhs(const float* A, int64_t lda, int64_t n, int B, const
 // waits for, read the shares until all are there; the others watch one word of
 // each share first, which keeps the traffic of a thousand waiting waves down.
 // Waits are bounded: past the limit status bit 2 is raised and every workgroup
-// leaves (a context's calls then solve again by the per-step launches).  The factor tile of a contribution and the inverse rows of
+// leaves with NaN in its slices of x (a context's calls then solve again by the
+// per-step launches).  The factor tile of a contribution and the inverse rows of
 // a share do not depend on the awaited values, so they are loaded before the
 // wait and only the round trip and the arithmetic stay on the critical path.
 // (With drained stores, a flag and then the values, three round trips a block:
@@ -554,6 +555,8 @@ __global__ __launch_bounds__(NT) void gesl_persist_kernel(const float* __restric
     for (int k = 0; k < own; ++k)
         for (int c = t; c < S; c += NT) {
             zown[k * S + c] = x[(int64_t)(g + k * G) * S + c];
+            // what stays where a wait gives up, for callers that cannot read the status
+            x[(int64_t)(g + k * G) * S + c] = __uint_as_float(0x7fc00000u);
             if (kCarry) zlo[k * S + c] = 0.0f;
         }
 

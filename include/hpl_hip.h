@@ -382,6 +382,9 @@ hpl_status hpl_kernel_bytes(hpl_ctx* ctx, double* bytes);
  * device pointer to n floats (16-byte aligned) holding b on entry and x on
  * return.  stream is the hipStream_t to enqueue on (NULL: the null stream);
  * the call only enqueues work, so synchronise that stream before reading x.
+ * The solve is one launch of up to half the workgroups that the device holds;
+ * where other launches keep part of them from starting for seconds, their
+ * waits give up and x comes out with NaN in it.
  * The block is hpl_gesl's (the largest power of two <= 256 dividing n; n must
  * be a multiple of 32) and the result equals hpl_gesl's bit for bit.  The
  * diagonal-block inverses and the solve's state, about n * (416 + 8 * block)

@@ -70,3 +70,28 @@ def test_fp32(monkeypatch, n, B, pivot):
         assert np.all(np.isfinite(p)) and np.array_equal(p, q)
     ref = np.linalg.solve(a.T.astype(np.float64), b)
     assert np.max(np.abs(out["spin"][1] - ref)) <= 1e-9 * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("n", [544, 1088, 2048])
+def test_noalloc_shows_that_it_gave_up(monkeypatch, n):
+    """hpl_gesl_noalloc only enqueues work and cannot solve again: NaN in x instead."""
+    import torch
+
+    print(f"noalloc n={n}", flush=True)
+    a, b, _, _ = O.generate_ref(n, seed=n)
+    f = O.gefa_nopvt(a)
+    F = torch.from_numpy(f).cuda()
+    with Context(0) as c:
+        ref = b.copy()
+        _env(monkeypatch, {})
+        c._check(c._L.hpl_gesl(c._c, f.ctypes.data, ref.ctypes.data, n, n, None))
+        for env in ({"HPL_GESL_SPIN": "0"}, {}):
+            _env(monkeypatch, env)
+            x = torch.from_numpy(b).cuda()
+            assert c._L.hpl_gesl_noalloc(F.data_ptr(), n, n, x.data_ptr(), None) == 0
+            torch.cuda.synchronize()
+            x = x.cpu().numpy()
+            if env:
+                assert np.any(np.isnan(x))
+            else:
+                assert np.array_equal(x, ref)
