@@ -482,26 +482,31 @@ __global__ __launch_bounds__(PNT) void panel_pivot_kernel(
             const int rl = r0 + 8 * (lane & 7);
             const float lv = rl >= rs1 ? lcol[rl] : 0.0f;
             for (int jb = c + 2; jb < B; jb += 64) {
-                const int j = jb + lane;
-                if (j >= B) continue;
+                // lanes past the last column read it too and store nothing: every
+                // lane stays active, as v_readlane wants of those it reads
+                const bool in = jb + lane < B;
+                const int j = in ? jb + lane : B - 1;
                 const float uj = urow[j];
                 float* q = tile + r0 * LDT + j;
+                float v[8];
                 if (r0 >= rs1) {
-                    float v[8];
 #pragma unroll
                     for (int i = 0; i < 8; ++i) v[i] = q[8 * i * LDT];
 #pragma unroll
                     for (int i = 0; i < 8; ++i) v[i] = v[i] + bcast_lane(lv, i) * uj;
+                    if (in)
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) q[8 * i * LDT] = v[i];
+                        for (int i = 0; i < 8; ++i) q[8 * i * LDT] = v[i];
                 } else {
                     // part of the rows lie above: only those from rs1 on
-                    float v[8];
 #pragma unroll
                     for (int i = 0; i < 8; ++i) v[i] = r0 + 8 * i >= rs1 ? q[8 * i * LDT] : 0.0f;
 #pragma unroll
-                    for (int i = 0; i < 8; ++i)
-                        if (r0 + 8 * i >= rs1) q[8 * i * LDT] = v[i] + bcast_lane(lv, i) * uj;
+                    for (int i = 0; i < 8; ++i) v[i] = v[i] + bcast_lane(lv, i) * uj;
+                    if (in)
+#pragma unroll
+                        for (int i = 0; i < 8; ++i)
+                            if (r0 + 8 * i >= rs1) q[8 * i * LDT] = v[i];
                 }
             }
         }
