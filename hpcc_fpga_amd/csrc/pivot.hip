@@ -63,6 +63,7 @@
 #include "kernels.hpp"
 
 #include <algorithm>
+#include <cstdlib>
 
 namespace {
 
@@ -680,9 +681,12 @@ namespace {
 // 128-column panel alone, us, with 64 / 128 / 256 rows: m = 2048 377 / 440 /
 // 572, 6144 396 / 443 / 556, 12288 426 / 461 / 556, 16384 461 / 462 / 561; with
 // 32 rows 6144 takes 457 (twice the slots to poll).
+// HPL_PANEL_ROWS (64, 128 or 256) asks for one of them at any m.
 int panel_rows_sh(int64_t m, int B) {
     const int most = B >= 256 ? 7 : 8;
-    return std::min(most, m <= 64 * 128 ? 6 : m <= 128 * 128 ? 7 : 8);
+    int sh = m <= 64 * 128 ? 6 : m <= 128 * 128 ? 7 : 8;
+    if (const char* e = getenv("HPL_PANEL_ROWS")) sh = atoi(e) >= 256 ? 8 : atoi(e) >= 128 ? 7 : 6;
+    return std::min(most, sh);
 }
 }  // namespace
 
