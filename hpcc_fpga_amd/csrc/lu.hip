@@ -55,51 +55,53 @@ __device__ __forceinline__ float bcast(float v, int lane) {
 
 // d[i] += m[i], i < N, in the lanes that the mask M has in each half of the wave:
 // one change of the exec mask instead of a select per value (every lane of the
-// wave is active here)
+// wave is active here).  The compiler does not look into the text: d is written
+// before all of m is read (+&), and a DPP move may follow at once, which needs two
+// wait states after the last sum -- the move to exec is one, s_nop 0 the other.
 template <unsigned M, int N>
 __device__ __forceinline__ void add_in(float* d, const float* m) {
     static_assert(N >= 1 && N <= 8, "up to eight values");
     if constexpr (N == 1)
         asm("s_mov_b32 exec_lo, %2\n\ts_mov_b32 exec_hi, %2\n\t"
             "v_add_f32 %0, %0, %1\n\t"
-            "s_mov_b64 exec, -1"
-            : "+v"(d[0])
+            "s_mov_b64 exec, -1\n\ts_nop 0"
+            : "+&v"(d[0])
             : "v"(m[0]), "i"(M));
     else if constexpr (N == 2)
         asm("s_mov_b32 exec_lo, %4\n\ts_mov_b32 exec_hi, %4\n\t"
             "v_add_f32 %0, %0, %2\n\tv_add_f32 %1, %1, %3\n\t"
-            "s_mov_b64 exec, -1"
-            : "+v"(d[0]), "+v"(d[1])
+            "s_mov_b64 exec, -1\n\ts_nop 0"
+            : "+&v"(d[0]), "+&v"(d[1])
             : "v"(m[0]), "v"(m[1]), "i"(M));
     else if constexpr (N == 3)
         asm("s_mov_b32 exec_lo, %6\n\ts_mov_b32 exec_hi, %6\n\t"
             "v_add_f32 %0, %0, %3\n\tv_add_f32 %1, %1, %4\n\t"
             "v_add_f32 %2, %2, %5\n\t"
-            "s_mov_b64 exec, -1"
-            : "+v"(d[0]), "+v"(d[1]), "+v"(d[2])
+            "s_mov_b64 exec, -1\n\ts_nop 0"
+            : "+&v"(d[0]), "+&v"(d[1]), "+&v"(d[2])
             : "v"(m[0]), "v"(m[1]), "v"(m[2]), "i"(M));
     else if constexpr (N == 4)
         asm("s_mov_b32 exec_lo, %8\n\ts_mov_b32 exec_hi, %8\n\t"
             "v_add_f32 %0, %0, %4\n\tv_add_f32 %1, %1, %5\n\t"
             "v_add_f32 %2, %2, %6\n\tv_add_f32 %3, %3, %7\n\t"
-            "s_mov_b64 exec, -1"
-            : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3])
+            "s_mov_b64 exec, -1\n\ts_nop 0"
+            : "+&v"(d[0]), "+&v"(d[1]), "+&v"(d[2]), "+&v"(d[3])
             : "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "i"(M));
     else if constexpr (N == 5)
         asm("s_mov_b32 exec_lo, %10\n\ts_mov_b32 exec_hi, %10\n\t"
             "v_add_f32 %0, %0, %5\n\tv_add_f32 %1, %1, %6\n\t"
             "v_add_f32 %2, %2, %7\n\tv_add_f32 %3, %3, %8\n\t"
             "v_add_f32 %4, %4, %9\n\t"
-            "s_mov_b64 exec, -1"
-            : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]), "+v"(d[4])
+            "s_mov_b64 exec, -1\n\ts_nop 0"
+            : "+&v"(d[0]), "+&v"(d[1]), "+&v"(d[2]), "+&v"(d[3]), "+&v"(d[4])
             : "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "v"(m[4]), "i"(M));
     else if constexpr (N == 6)
         asm("s_mov_b32 exec_lo, %12\n\ts_mov_b32 exec_hi, %12\n\t"
             "v_add_f32 %0, %0, %6\n\tv_add_f32 %1, %1, %7\n\t"
             "v_add_f32 %2, %2, %8\n\tv_add_f32 %3, %3, %9\n\t"
             "v_add_f32 %4, %4, %10\n\tv_add_f32 %5, %5, %11\n\t"
-            "s_mov_b64 exec, -1"
-            : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]), "+v"(d[4]), "+v"(d[5])
+            "s_mov_b64 exec, -1\n\ts_nop 0"
+            : "+&v"(d[0]), "+&v"(d[1]), "+&v"(d[2]), "+&v"(d[3]), "+&v"(d[4]), "+&v"(d[5])
             : "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "v"(m[4]), "v"(m[5]), "i"(M));
     else if constexpr (N == 7)
         asm("s_mov_b32 exec_lo, %14\n\ts_mov_b32 exec_hi, %14\n\t"
@@ -107,8 +109,8 @@ __device__ __forceinline__ void add_in(float* d, const float* m) {
             "v_add_f32 %2, %2, %9\n\tv_add_f32 %3, %3, %10\n\t"
             "v_add_f32 %4, %4, %11\n\tv_add_f32 %5, %5, %12\n\t"
             "v_add_f32 %6, %6, %13\n\t"
-            "s_mov_b64 exec, -1"
-            : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]), "+v"(d[4]), "+v"(d[5]), "+v"(d[6])
+            "s_mov_b64 exec, -1\n\ts_nop 0"
+            : "+&v"(d[0]), "+&v"(d[1]), "+&v"(d[2]), "+&v"(d[3]), "+&v"(d[4]), "+&v"(d[5]), "+&v"(d[6])
             : "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "v"(m[4]), "v"(m[5]), "v"(m[6]), "i"(M));
     else if constexpr (N == 8)
         asm("s_mov_b32 exec_lo, %16\n\ts_mov_b32 exec_hi, %16\n\t"
@@ -116,9 +118,9 @@ __device__ __forceinline__ void add_in(float* d, const float* m) {
             "v_add_f32 %2, %2, %10\n\tv_add_f32 %3, %3, %11\n\t"
             "v_add_f32 %4, %4, %12\n\tv_add_f32 %5, %5, %13\n\t"
             "v_add_f32 %6, %6, %14\n\tv_add_f32 %7, %7, %15\n\t"
-            "s_mov_b64 exec, -1"
-            : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]), "+v"(d[4]), "+v"(d[5]), "+v"(d[6]),
-              "+v"(d[7])
+            "s_mov_b64 exec, -1\n\ts_nop 0"
+            : "+&v"(d[0]), "+&v"(d[1]), "+&v"(d[2]), "+&v"(d[3]), "+&v"(d[4]), "+&v"(d[5]), "+&v"(d[6]),
+              "+&v"(d[7])
             : "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "v"(m[4]), "v"(m[5]), "v"(m[6]),
               "v"(m[7]), "i"(M));
 }

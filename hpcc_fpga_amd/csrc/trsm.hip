@@ -53,13 +53,14 @@ namespace {
 //
 // pf, pb, status: the substitution's shares, cleared for a launch that follows.
 // ----------------------------------------------------------------------------
-// d[k] += m[k] s in the lanes that the mask M has in each half of the wave
+// d[k] += m[k] s in the lanes that the mask M has in each half of the wave (every
+// lane of the wave is active here; early clobbers and s_nop as in lu.hip's add_in)
 template <unsigned M>
 __device__ __forceinline__ void fma_in(float (&d)[4], const float (&m)[4], float s) {
     asm("s_mov_b32 exec_lo, %9\n\ts_mov_b32 exec_hi, %9\n\t"
         "v_fmac_f32 %0, %4, %8\n\tv_fmac_f32 %1, %5, %8\n\t"
-        "v_fmac_f32 %2, %6, %8\n\tv_fmac_f32 %3, %7, %8\n\ts_mov_b64 exec, -1"
-        : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3])
+        "v_fmac_f32 %2, %6, %8\n\tv_fmac_f32 %3, %7, %8\n\ts_mov_b64 exec, -1\n\ts_nop 0"
+        : "+&v"(d[0]), "+&v"(d[1]), "+&v"(d[2]), "+&v"(d[3])
         : "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "v"(s), "i"(M));
 }
 
@@ -117,7 +118,8 @@ __global__ __launch_bounds__(128) void prep_kernel(const float* __restrict__ A, 
     const int q = top ? blk : blk - NQ;
     load_sub(q * 32, q * 32);
     __syncthreads();
-    const int r = t & 15, g = (t >> 4) & 3, w = t >> 6;
+    // (w for the whole wave, so that its branches are scalar ones)
+    const int r = t & 15, g = (t >> 4) & 3, w = __builtin_amdgcn_readfirstlane(t >> 6);
     // coefficients S[j][r]: top D[r][j], left D[j][r]
     auto coeff = [&](float (&s)[16], int j0, int r0) {
         if (top) {
