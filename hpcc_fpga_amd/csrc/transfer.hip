@@ -5,6 +5,21 @@
 
 namespace hplx {
 
+namespace {
+
+// Memory that the runtime made or has registered (pinned, managed, device): its
+// copies need no staging.
+bool runtime_knows(const void* p) {
+    hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return at.type != hipMemoryTypeUnregistered;
+}
+
+}  // namespace
+
 hipError_t HostStage::make() {
     if (mem_) return hipSuccess;
     hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&mem_), kBufs * kBytes,
@@ -42,6 +57,9 @@ hipError_t HostStage::to_device(hipStream_t s, void* dev, size_t dev_pitch, cons
     // bytes from a row's start to the next one's (or to its own end)
     const size_t span = rows > 1 ? dev_pitch : width;
     if (width > span) return hipErrorInvalidValue;
+    if (runtime_knows(host))
+        return hipMemcpy2DAsync(dev, dev_pitch, host, host_pitch, width, rows,
+                                hipMemcpyHostToDevice, s);
     hipError_t e = make();
     if (e != hipSuccess) return e;
     if (span > kBytes) {  // row by row, each in pieces
@@ -73,6 +91,7 @@ hipError_t HostStage::to_device(hipStream_t s, void* dev, size_t dev_pitch, cons
 }
 
 hipError_t HostStage::to_device(hipStream_t s, void* dev, const void* host, size_t bytes) {
+    if (runtime_knows(host)) return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
     const size_t whole = bytes / kBytes, done = whole * kBytes;
     hipError_t e = to_device(s, dev, kBytes, host, kBytes, kBytes, whole);
     if (e != hipSuccess || done == bytes) return e;
@@ -81,6 +100,10 @@ hipError_t HostStage::to_device(hipStream_t s, void* dev, const void* host, size
 }
 
 hipError_t HostStage::to_host(hipStream_t s, void* host, const void* dev, size_t bytes) {
+    if (runtime_knows(host)) {
+        hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);
+        return e == hipSuccess ? hipStreamSynchronize(s) : e;
+    }
     const size_t whole = bytes / kBytes, done = whole * kBytes;
     hipError_t e = to_host(s, host, kBytes, dev, kBytes, kBytes, whole);
     if (e != hipSuccess || done == bytes) return e;
@@ -93,6 +116,11 @@ hipError_t HostStage::to_host(hipStream_t s, void* host, size_t host_pitch, cons
     if (!width || !rows) return hipSuccess;
     const size_t span = rows > 1 ? dev_pitch : width;
     if (width > span) return hipErrorInvalidValue;
+    if (runtime_knows(host)) {
+        hipError_t e = hipMemcpy2DAsync(host, host_pitch, dev, dev_pitch, width, rows,
+                                        hipMemcpyDeviceToHost, s);
+        return e == hipSuccess ? hipStreamSynchronize(s) : e;
+    }
     hipError_t e = make();
     if (e != hipSuccess) return e;
     if (span > kBytes) {

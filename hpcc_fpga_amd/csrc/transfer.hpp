@@ -12,20 +12,23 @@ namespace hplx {
 // and used by one thread at a time.  Made on first use, given back by free().
 //
 // The runtime moves a pitched copy from ordinary host memory row by row, each
-// row pinned and queued by itself (about 10 us a row where the buffer has not
-// been seen before: 27 ms for the three transfers of a 1024 x 1024 solve, 1.3
-// ms through these buffers), and its copies were seen to overtake or be
-// overtaken by kernels of the same stream under a profiler.  Here rows are
+// row pinned and queued by itself (about 10 us a row: 27 ms for the three
+// transfers of a 1024 x 1024 solve, 1.3 ms through these buffers).  Here rows are
 // packed at the device's pitch by the host while the previous piece is on its
-// way, so the device sees plain copies from pinned memory.
+// way, so the device sees plain copies from pinned memory.  Buffers that the
+// runtime knows -- the caller's own pinned, managed or device memory -- are copied
+// from or to directly: a copy through the host's caches halves their rate (n =
+// 4096 up 1.2 ms direct and 2.2 staged, down 1.2 and 2.9; 16384 19 and 36, 19 and
+// 45).
 class HostStage {
    public:
     ~HostStage() { free(); }
     // `rows` rows of `width` bytes, `pitch` apart on each side.  to_device: the
-    // device rows' bytes between width and pitch become zero where the pitch
-    // fits a buffer (the last row's excepted; else they stay); the host buffer
-    // may be reused on return, the copies run on `s`.  to_host: returns when the rows are in place, after everything
-    // enqueued on `s` before.
+    // copies run on `s`; an ordinary host buffer may be reused on return (of such a
+    // one the device rows' bytes between width and pitch become zero where the
+    // pitch fits a staging buffer, the last row's excepted), one that the runtime
+    // knows once `s` has got there.  to_host: returns when the rows are in place,
+    // after everything enqueued on `s` before.
     hipError_t to_device(hipStream_t s, void* dev, size_t dev_pitch, const void* host,
                          size_t host_pitch, size_t width, size_t rows);
     hipError_t to_host(hipStream_t s, void* host, size_t host_pitch, const void* dev,
