@@ -20,18 +20,18 @@ bool runtime_knows(const void* p) {
 
 }  // namespace
 
-hipError_t HostStage::make() {
-    if (mem_) return hipSuccess;
-    hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&mem_), kBufs * kBytes,
+hipError_t HostStage::Ring::make() {
+    if (mem) return hipSuccess;
+    hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&mem), kBufs * bytes,
                                  hipHostMallocDefault);
     if (e != hipSuccess) {
-        mem_ = nullptr;
+        mem = nullptr;
         return e;
     }
-    for (hipEvent_t& ev : ev_) {
-        e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    for (hipEvent_t& v : ev) {
+        e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
         if (e != hipSuccess) {
-            ev = nullptr;
+            v = nullptr;
             free();
             return e;
         }
@@ -39,16 +39,21 @@ hipError_t HostStage::make() {
     return hipSuccess;
 }
 
-void HostStage::free() {
-    for (hipEvent_t& ev : ev_) {
-        if (ev) {
-            (void)hipEventSynchronize(ev);  // its last copy
-            (void)hipEventDestroy(ev);
+void HostStage::Ring::free() {
+    for (hipEvent_t& v : ev) {
+        if (v) {
+            (void)hipEventSynchronize(v);  // its last copy
+            (void)hipEventDestroy(v);
         }
-        ev = nullptr;
+        v = nullptr;
     }
-    if (mem_) (void)hipHostFree(mem_);
-    mem_ = nullptr;
+    if (mem) (void)hipHostFree(mem);
+    mem = nullptr;
+}
+
+hipError_t HostStage::make() {
+    const hipError_t e = small_.make();
+    return e == hipSuccess ? large_.make() : e;
 }
 
 hipError_t HostStage::to_device(hipStream_t s, void* dev, size_t dev_pitch, const void* host,
@@ -60,22 +65,23 @@ hipError_t HostStage::to_device(hipStream_t s, void* dev, size_t dev_pitch, cons
     if (runtime_knows(host))
         return hipMemcpy2DAsync(dev, dev_pitch, host, host_pitch, width, rows,
                                 hipMemcpyHostToDevice, s);
-    hipError_t e = make();
+    Ring& R = ring((rows - 1) * span + width);
+    hipError_t e = R.make();
     if (e != hipSuccess) return e;
-    if (span > kBytes) {  // row by row, each in pieces
+    if (span > kLarge) {  // row by row, each in pieces
         for (size_t r = 0; r < rows && e == hipSuccess; ++r)
             e = to_device(s, static_cast<char*>(dev) + r * dev_pitch,
                           static_cast<const char*>(host) + r * host_pitch, width);
         return e;
     }
-    const size_t per = std::max<size_t>(1, kBytes / span);
+    const size_t per = std::max<size_t>(1, R.bytes / span);
     for (size_t r = 0; r < rows; r += per) {
         const size_t nr = std::min(per, rows - r);
-        const int b = next_;
-        next_ = (next_ + 1) % kBufs;
-        e = hipEventSynchronize(ev_[b]);  // the buffer's previous copy
+        const int b = R.next;
+        R.next = (R.next + 1) % kBufs;
+        e = hipEventSynchronize(R.ev[b]);  // the buffer's previous copy
         if (e != hipSuccess) return e;
-        char* buf = mem_ + b * kBytes;
+        char* buf = R.mem + b * R.bytes;
         for (size_t i = 0; i < nr; ++i) {
             std::memcpy(buf + i * span, static_cast<const char*>(host) + (r + i) * host_pitch,
                         width);
@@ -84,7 +90,7 @@ hipError_t HostStage::to_device(hipStream_t s, void* dev, size_t dev_pitch, cons
         const size_t bytes = r + nr < rows ? nr * span : (nr - 1) * span + width;
         e = hipMemcpyAsync(static_cast<char*>(dev) + r * span, buf, bytes, hipMemcpyHostToDevice,
                            s);
-        if (e == hipSuccess) e = hipEventRecord(ev_[b], s);
+        if (e == hipSuccess) e = hipEventRecord(R.ev[b], s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -92,8 +98,8 @@ hipError_t HostStage::to_device(hipStream_t s, void* dev, size_t dev_pitch, cons
 
 hipError_t HostStage::to_device(hipStream_t s, void* dev, const void* host, size_t bytes) {
     if (runtime_knows(host)) return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
-    const size_t whole = bytes / kBytes, done = whole * kBytes;
-    hipError_t e = to_device(s, dev, kBytes, host, kBytes, kBytes, whole);
+    const size_t whole = bytes / kLarge, done = whole * kLarge;
+    hipError_t e = to_device(s, dev, kLarge, host, kLarge, kLarge, whole);
     if (e != hipSuccess || done == bytes) return e;
     return to_device(s, static_cast<char*>(dev) + done, bytes - done,
                      static_cast<const char*>(host) + done, bytes - done, bytes - done, 1);
@@ -104,8 +110,8 @@ hipError_t HostStage::to_host(hipStream_t s, void* host, const void* dev, size_t
         hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e;
     }
-    const size_t whole = bytes / kBytes, done = whole * kBytes;
-    hipError_t e = to_host(s, host, kBytes, dev, kBytes, kBytes, whole);
+    const size_t whole = bytes / kLarge, done = whole * kLarge;
+    hipError_t e = to_host(s, host, kLarge, dev, kLarge, kLarge, whole);
     if (e != hipSuccess || done == bytes) return e;
     return to_host(s, static_cast<char*>(host) + done, bytes - done,
                    static_cast<const char*>(dev) + done, bytes - done, bytes - done, 1);
@@ -121,17 +127,18 @@ hipError_t HostStage::to_host(hipStream_t s, void* host, size_t host_pitch, cons
                                         hipMemcpyDeviceToHost, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e;
     }
-    hipError_t e = make();
+    Ring& R = ring((rows - 1) * span + width);
+    hipError_t e = R.make();
     if (e != hipSuccess) return e;
-    if (span > kBytes) {
+    if (span > kLarge) {
         for (size_t r = 0; r < rows && e == hipSuccess; ++r)
             e = to_host(s, static_cast<char*>(host) + r * host_pitch,
                         static_cast<const char*>(dev) + r * dev_pitch, width);
         return e;
     }
-    const size_t per = std::max<size_t>(1, kBytes / span);
+    const size_t per = std::max<size_t>(1, R.bytes / span);
     const size_t pieces = (rows + per - 1) / per;
-    const int first = next_;
+    const int first = R.next;
     // up to kBufs pieces on their way while the oldest is unpacked
     for (size_t p = 0, q = 0; q < pieces; ++q) {
         for (; p < pieces && p < q + kBufs; ++p) {
@@ -139,23 +146,23 @@ hipError_t HostStage::to_host(hipStream_t s, void* host, size_t host_pitch, cons
             const size_t bytes = p + 1 < pieces ? nr * span : (nr - 1) * span + width;
             const int b = (int)((first + p) % kBufs);
             if (p < (size_t)kBufs) {  // what an earlier call left in the buffer
-                e = hipEventSynchronize(ev_[b]);
+                e = hipEventSynchronize(R.ev[b]);
                 if (e != hipSuccess) return e;
             }
-            e = hipMemcpyAsync(mem_ + b * kBytes, static_cast<const char*>(dev) + p * per * span,
+            e = hipMemcpyAsync(R.mem + b * R.bytes, static_cast<const char*>(dev) + p * per * span,
                                bytes, hipMemcpyDeviceToHost, s);
-            if (e == hipSuccess) e = hipEventRecord(ev_[b], s);
+            if (e == hipSuccess) e = hipEventRecord(R.ev[b], s);
             if (e != hipSuccess) return e;
         }
         const int b = (int)((first + q) % kBufs);
-        e = hipEventSynchronize(ev_[b]);
+        e = hipEventSynchronize(R.ev[b]);
         if (e != hipSuccess) return e;
         const size_t nr = std::min(per, rows - q * per);
         for (size_t i = 0; i < nr; ++i)
             std::memcpy(static_cast<char*>(host) + (q * per + i) * host_pitch,
-                        mem_ + b * kBytes + i * span, width);
+                        R.mem + b * R.bytes + i * span, width);
     }
-    next_ = (int)((first + pieces) % kBufs);
+    R.next = (int)((first + pieces) % kBufs);
     return hipSuccess;
 }
 

@@ -36,17 +36,31 @@ class HostStage {
     // contiguous bytes
     hipError_t to_device(hipStream_t s, void* dev, const void* host, size_t bytes);
     hipError_t to_host(hipStream_t s, void* host, const void* dev, size_t bytes);
+    // all buffers at once, for who cannot fail later; free() gives them back
     hipError_t make();
-    void free();
+    void free() {
+        small_.free();
+        large_.free();
+    }
 
    private:
     static constexpr int kBufs = 4;
-    // 1 MiB: packed in 30 us, on its way for 20 us; shorter pieces pay the
-    // launch of a copy, longer ones the wait for the first and last piece
-    static constexpr size_t kBytes = 1u << 20;
-    char* mem_ = nullptr;
-    hipEvent_t ev_[kBufs] = {};
-    int next_ = 0;
+    // Up to 64 KiB (status words, norms, vectors of small orders) through small
+    // buffers, so that only a context that moves more holds the 4 MiB of the
+    // large ones.  Those are 1 MiB each: packed in 30 us, on its way for 20 us;
+    // shorter pieces pay the launch of a copy, longer ones the wait for the first
+    // and last piece.
+    static constexpr size_t kSmall = 64u << 10, kLarge = 1u << 20;
+    struct Ring {
+        size_t bytes;  // of one buffer
+        char* mem = nullptr;
+        hipEvent_t ev[kBufs] = {};
+        int next = 0;
+        hipError_t make();
+        void free();
+    };
+    Ring& ring(size_t bytes) { return bytes <= kSmall ? small_ : large_; }
+    Ring small_{kSmall}, large_{kLarge};
 };
 
 }  // namespace hplx

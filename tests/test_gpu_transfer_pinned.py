@@ -64,3 +64,21 @@ def test_pinned_right_hand_sides():
         c._check(c._L.hpl_solve_rhs64(c._c, nrhs, b.ctypes.data, n + 3, x.ctypes.data, n + 7, 50,
                                       1e-14 * n, res))
     assert np.array_equal(x[:, :n].T, ref)
+
+
+@pytest.mark.parametrize("n", [1, 124, 128, 132, 8192, 8196])
+def test_around_the_small_buffers(n):
+    """Transfers of up to 64 KiB take small staging buffers, longer ones large ones:
+    matrices and vectors on either side, in turn."""
+    print(f"small transfers n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    a = rng.random((n, n), np.float32)
+    with Context(0) as c:
+        for rep in range(5):  # more calls than buffers
+            b = rng.random(n)
+            c.upload(a, b.astype(np.float32))
+            c.upload_rhs64(b)
+            f, b64, _ = c.download_vectors()
+            assert np.array_equal(b64, b) and np.array_equal(f, b.astype(np.float32))
+            if n < 8192 or rep == 0:
+                assert np.array_equal(c.download(matrix=True, solution=False)[0], a)
