@@ -16,6 +16,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <numeric>
 #include <string>
 #include <vector>
@@ -28,8 +29,9 @@ namespace {
 
 constexpr int kMaxBatchOrder = 1024;  // LDS holds the two strips of the largest system
 constexpr int kBuckets = 4;
-constexpr int kSingleGets = 4;              // solutions fetched one by one
-constexpr size_t kMaxFetch = 256u << 20;
+constexpr int64_t kAheadBytes = 4 << 20;  // solutions copied ahead of hpl_batch_get
+constexpr int64_t kAllBytes = 32 << 20;   // where all of them are copied
+constexpr int64_t kCopyBytes = 1 << 19;   // what a copy moves in the time it takes to start
 
 struct Bucket {
     int hi = 0;         // largest padded order in the bucket
@@ -78,13 +80,25 @@ struct hpl_batch {
     double graph_tol = -1.0;
     int cus = 256;
     std::string err;
-    // hpl_batch_get: after a few solutions fetched one by one since the last
-    // solve, all of them and the results are copied at once into pinned memory
-    // (at most kMaxFetch bytes) and further calls read them there
     hplx::HostStage stage;
-    char* hAll = nullptr;  // v_total doubles, then nsys results
-    int gets = 0;          // calls since dx64 and dRes were last written
-    bool fetched = false;
+    // hpl_batch_get's copies ahead: the solutions, then the results, of the
+    // systems [ahead_lo, ahead_hi) in pinned memory, dropped whenever dx64 and
+    // dRes are written
+    std::mutex get_mu;
+    char* ahead = nullptr;
+    size_t cap_ahead = 0;
+    const double* ahead_x = nullptr;
+    const BatchResult* ahead_r = nullptr;
+    int ahead_lo = 0, ahead_hi = 0;
+    int last_get = -2;  // the system of the last call
+    int window = 1;     // systems copied by the last call that copied
+    int copies = 0;     // such calls since then
+    void drop_ahead() {
+        std::lock_guard<std::mutex> lk(get_mu);
+        ahead_lo = ahead_hi = copies = 0;
+        last_get = -2;
+        window = 1;
+    }
 };
 
 namespace {
@@ -289,7 +303,7 @@ void hpl_batch_destroy(hpl_batch* b) {
     if (!b) return;
     if (b->s0) (void)hipStreamSynchronize(b->s0);
     drop_graph(b);
-    if (b->hAll) (void)hipHostFree(b->hAll);
+    if (b->ahead) (void)hipHostFree(b->ahead);
     for (void* p : {(void*)b->dSys, (void*)b->dOrder, (void*)b->dCounters, (void*)b->dA,
                     (void*)b->dA0, (void*)b->db64, (void*)b->dx64, (void*)b->drs, (void*)b->dxs,
                     (void*)b->dRes, (void*)b->dBad})
@@ -356,8 +370,7 @@ hpl_status hpl_batch_autotune(hpl_batch* b, hpl_prec prec, int max_iter, double 
         return bfail(b, HPL_ERR_UNSUPPORTED, "batched solves run FP16 or FP32 trailing updates");
     const bool f16 = prec == HPL_PREC_FP16;
     drop_graph(b);
-    b->fetched = false;
-    b->gets = 0;
+    b->drop_ahead();
     const int cands[3] = {128, 256, 512};
     for (int i = 0; i < kBuckets; ++i) {
         Bucket& k = b->buckets[i];
@@ -464,8 +477,7 @@ hpl_status hpl_batch_solve(hpl_batch* b, hpl_prec prec, int max_iter, double tol
         b->graph_iter = max_iter;
         b->graph_tol = tol_per_n;
     }
-    b->fetched = false;
-    b->gets = 0;
+    b->drop_ahead();
     BCHK(b, hipEventRecord(b->t0, b->s0));
     BCHK(b, hipGraphLaunch(b->exec, b->s0));
     BCHK(b, hipEventRecord(b->t1, b->s0));
@@ -496,36 +508,84 @@ hpl_status hpl_batch_solve(hpl_batch* b, hpl_prec prec, int max_iter, double tol
     return HPL_SUCCESS;
 }
 
+}  // extern "C"
+
+namespace {
+
+// The solutions and results of systems lo .. hi - 1 into b->ahead; none of them
+// where there is no pinned memory for them.
+hpl_status copy_ahead(hpl_batch* b, int lo, int hi) {
+    const int64_t v0 = b->sys[lo].v_off, v1 = hi < b->nsys ? b->sys[hi].v_off : b->v_total;
+    const size_t xb = (size_t)(v1 - v0) * sizeof(double), rb = (hi - lo) * sizeof(BatchResult);
+    if (xb + rb > b->cap_ahead) {
+        if (b->ahead) (void)hipHostFree(b->ahead);
+        // room for the further, longer ones too
+        const size_t most = (size_t)b->v_total * sizeof(double) + b->nsys * sizeof(BatchResult);
+        const size_t cap = std::max(xb + rb, std::min<size_t>(most, 2 * kAheadBytes));
+        b->cap_ahead = 0;
+        if (hipHostMalloc(reinterpret_cast<void**>(&b->ahead), cap, hipHostMallocDefault) !=
+            hipSuccess) {
+            (void)hipGetLastError();
+            b->ahead = nullptr;
+            return HPL_SUCCESS;
+        }
+        b->cap_ahead = cap;
+    }
+    BCHK(b, hipMemcpyAsync(b->ahead, b->dx64 + v0, xb, hipMemcpyDeviceToHost, b->s0));
+    BCHK(b, hipMemcpyAsync(b->ahead + xb, b->dRes + lo, rb, hipMemcpyDeviceToHost, b->s0));
+    BCHK(b, hipStreamSynchronize(b->s0));
+    b->ahead_x = reinterpret_cast<const double*>(b->ahead);
+    b->ahead_r = reinterpret_cast<const BatchResult*>(b->ahead + xb);
+    b->ahead_lo = lo;
+    b->ahead_hi = hi;
+    return HPL_SUCCESS;
+}
+
+}  // namespace
+
+extern "C" {
+
+// A copy takes 25 us whatever its size, so systems read in ascending order are
+// copied ahead, twice as many each time up to kAheadBytes (4096 solutions took
+// 118 ms one by one, 2 ms so; one or two read here and there pay for no others).
+// In another order all of them are copied, up to kAllBytes, once the single copies
+// have taken the time of that.
 hpl_status hpl_batch_get(hpl_batch* b, int s, double* x, int* iterations, double* berr) {
     if (!b || s < 0 || s >= b->nsys) return HPL_ERR_INVALID_ARG;
     const BatchSystem& sy = b->sys[s];
     BatchResult r;
-    // A copy of one solution costs 25 us whatever its size, one of everything
-    // about 0.2 ms per 10 MB: 4096 solutions took 118 ms one by one, 2 ms so.
-    const size_t xb = (size_t)b->v_total * sizeof(double), rb = b->nsys * sizeof(BatchResult);
-    if (!b->fetched && ++b->gets > kSingleGets && xb + rb <= kMaxFetch) {
-        if (!b->hAll &&
-            hipHostMalloc(reinterpret_cast<void**>(&b->hAll), xb + rb, hipHostMallocDefault) !=
-                hipSuccess) {
-            (void)hipGetLastError();
-            b->hAll = nullptr;
+    std::lock_guard<std::mutex> lk(b->get_mu);
+    if (s < b->ahead_lo || s >= b->ahead_hi) {
+        const bool next = s == b->last_get + 1;
+        b->window = next ? std::min(2 * b->window, b->nsys) : 1;
+        int lo = s, hi = s + 1;
+        const int64_t all = b->v_total * (int64_t)sizeof(double);
+        if (!next && b->copies * kCopyBytes > all && all <= kAllBytes) {
+            lo = 0;
+            hi = b->nsys;
+        } else {
+            while (hi < b->nsys && hi - s < b->window &&
+                   (b->sys[hi].v_off + b->sys[hi].npad - sy.v_off) * (int64_t)sizeof(double) <=
+                       kAheadBytes)
+                ++hi;
         }
-        if (b->hAll) {
-            BCHK(b, hipMemcpyAsync(b->hAll, b->dx64, xb, hipMemcpyDeviceToHost, b->s0));
-            BCHK(b, hipMemcpyAsync(b->hAll + xb, b->dRes, rb, hipMemcpyDeviceToHost, b->s0));
-            BCHK(b, hipStreamSynchronize(b->s0));
-            b->fetched = true;
+        ++b->copies;
+        b->ahead_lo = b->ahead_hi = 0;
+        if (hi - lo > 1) {
+            hpl_status st = copy_ahead(b, lo, hi);
+            if (st) return st;
         }
     }
-    if (b->fetched) {
+    if (s >= b->ahead_lo && s < b->ahead_hi) {
         if (x)
-            std::memcpy(x, reinterpret_cast<const double*>(b->hAll) + sy.v_off,
+            std::memcpy(x, b->ahead_x + (sy.v_off - b->sys[b->ahead_lo].v_off),
                         sy.n * sizeof(double));
-        std::memcpy(&r, b->hAll + xb + s * sizeof r, sizeof r);
+        r = b->ahead_r[s - b->ahead_lo];
     } else {
         if (x) BCHK(b, b->stage.to_host(b->s0, x, b->dx64 + sy.v_off, sy.n * sizeof(double)));
         BCHK(b, b->stage.to_host(b->s0, &r, b->dRes + s, sizeof r));
     }
+    b->last_get = s;
     if (iterations) *iterations = r.iterations;
     if (berr) *berr = r.backward_error;
     return HPL_SUCCESS;
