@@ -10,6 +10,7 @@ import os
 
 import numpy as np
 import pytest
+import torch  # before the library: one HIP runtime for both
 
 from hpcc_fpga_amd import Context
 from oracle import oracle as O
@@ -75,8 +76,6 @@ def test_fp32(monkeypatch, n, B, pivot):
 @pytest.mark.parametrize("n", [544, 1088, 2048])
 def test_noalloc_shows_that_it_gave_up(monkeypatch, n):
     """hpl_gesl_noalloc only enqueues work and cannot solve again: NaN in x instead."""
-    import torch
-
     print(f"noalloc n={n}", flush=True)
     a, b, _, _ = O.generate_ref(n, seed=n)
     f = O.gefa_nopvt(a)

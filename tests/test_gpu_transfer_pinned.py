@@ -5,6 +5,7 @@ buffers in the same context, and where the caller reuses a buffer after the call
 """
 import numpy as np
 import pytest
+import torch  # before the library: one HIP runtime for both
 
 from hpcc_fpga_amd import Context
 
@@ -12,8 +13,6 @@ pytestmark = pytest.mark.gpu
 
 
 def _pinned(shape, dtype):
-    import torch
-
     t = torch.empty(shape, dtype={np.float32: torch.float32, np.float64: torch.float64}[dtype],
                     pin_memory=True)
     return t.numpy()
