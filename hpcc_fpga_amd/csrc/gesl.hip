@@ -582,14 +582,23 @@ __global__ __launch_bounds__(NT) void gesl_persist_kernel(const float* __restric
         *reinterpret_cast<f32x4*>(&red[rg * S + 4 * cg]) = a;
         __syncthreads();
         if (t < S) {
-            float sum = 0.0f;
-#pragma unroll 8
-            for (int r = 0; r < RG; ++r) sum += red[r * S + t];
             if (kCarry) {
-                const float z = out[t], y = fmaf(sign, sum, zlo[k * S + t]), w = z + y;
+                // (pairwise: a chain of these sums would round more than the sums
+                // over whole blocks did)
+                float v[RG];
+#pragma unroll
+                for (int r = 0; r < RG; ++r) v[r] = red[r * S + t];
+#pragma unroll
+                for (int h = RG / 2; h > 0; h /= 2)
+#pragma unroll
+                    for (int r = 0; r < h; ++r) v[r] += v[r + h];
+                const float z = out[t], y = fmaf(sign, v[0], zlo[k * S + t]), w = z + y;
                 zlo[k * S + t] = fabsf(z) >= fabsf(y) ? y - (w - z) : z - (w - y);
                 out[t] = w;
             } else {
+                float sum = 0.0f;
+#pragma unroll 8
+                for (int r = 0; r < RG; ++r) sum += red[r * S + t];
                 out[t] = out[t] + sign * sum;
             }
         }
