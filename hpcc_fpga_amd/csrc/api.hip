@@ -728,8 +728,8 @@ hpl_status refine(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_it
     const int B = (int)c->B;
     const int64_t inv_stride = 3 * (B / 32) * 1024;
     // the substitution of several columns: between two residuals, whose
-    // partial sums (at least n (nrhs + 1) doubles) it overwrites
-    float* scratch = reinterpret_cast<float*>(c->dWork);
+    // partial sums (at least n (nrhs + 1) doubles, 2 n (nrhs + 1) floats) it overwrites
+    float* scratch = nrhs > 1 || c->pivoted ? reinterpret_cast<float*>(c->dWork) : nullptr;
     const size_t out_bytes = 4 * nrhs * sizeof(double) + (ws ? sizeof(int) : 0);
     double sc_in[16], sc_out[16], h[64];
     int iters[16];
@@ -1042,6 +1042,15 @@ hpl_status hpl_gesl_dev(hpl_ctx* c, hpl_timing* t) {
     HIPCHK(c, hipEventRecord(c->e0, c->s0));
     hpl_status st = hplx::ensure_block_inverses(c);
     if (st) return st;
+    // two columns for a pivoted factor's launches per block (the single launch's
+    // workspace is larger)
+    float* scratch = nullptr;
+    if (c->pivoted) {
+        if (ensure(c, c->dGeslWs, c->capGeslWs, gesl_ws_bytes((int64_t)c->n)) == HPL_SUCCESS)
+            scratch = static_cast<float*>(c->dGeslWs);
+        else
+            c->err.clear();
+    }
     GeslWs wsbuf;
     const GeslWs* ws = hplx::gesl_workspace(c, &wsbuf);
     for (bool again = true; again; ws = nullptr) {
@@ -1052,7 +1061,7 @@ hpl_status hpl_gesl_dev(hpl_ctx* c, hpl_timing* t) {
                                      c->s0));
         HIPCHK(c, launch_gesl(c->dA, (int64_t)c->lda, (int64_t)c->n, (int)c->B, c->dInv,
                               3 * (c->B / 32) * 1024, c->dx, c->s0,
-                              c->binv_ready ? c->dBInv : nullptr, ws));
+                              c->binv_ready ? c->dBInv : nullptr, ws, scratch));
         HIPCHK(c, hipEventRecord(c->e1, c->s0));
         st = hplx::gesl_gave_up(c, ws, &again);  // waits for the stream where there is a status
         if (st) return st;
@@ -1205,8 +1214,8 @@ hpl_status precond_apply(hpl_ctx* c, const double* v, double* z, bool* single) {
         GeslWs wsbuf;
         const GeslWs* ws = *single ? hplx::gesl_workspace(c, &wsbuf) : nullptr;
         HIPCHK(c, launch_gesl_multi(c->dA, (int64_t)c->lda, n, B, c->dInv, 3 * (B / 32) * 1024,
-                                    c->dIrXs, n, 1, c->s0, c->binv_ready ? c->dBInv : nullptr,
-                                    ws));
+                                    c->dIrXs, n, 1, c->s0, c->binv_ready ? c->dBInv : nullptr, ws,
+                                    c->pivoted ? reinterpret_cast<float*>(c->dWork) : nullptr));
         st = hplx::gesl_gave_up(c, ws, &again);
         if (st) return st;
         if (again) *single = false;

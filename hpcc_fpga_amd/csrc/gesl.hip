@@ -394,13 +394,19 @@ __device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// out[r][e] := (ASSIGN ? 0 : out[r][e]) + SIGN sum_{p < B} W[p * ldw + e] v[r][p]
+// What becomes of a product: stored, added to the sum that is there, or added with
+// that sum's rounding errors carried along in a second array (lo; from zero on where
+// `first`), as gesl_persist_kernel does for its sums over blocks of 32.
+enum class Out { Store, Add, Carry };
+
+// out[r][e] := (Store ? 0 : out[r][e]) + SIGN sum_{p < B} W[p * ldw + e] v[r][p]
 // for the 32 entries e of workgroup blockIdx.x, r < nr <= 16
-template <int SIGN, bool ASSIGN>
+template <int SIGN, Out OUT>
 __global__ __launch_bounds__(NT) void gesl_mrhs_kernel(const float* __restrict__ W, int64_t ldw,
                                                        int B, const float* __restrict__ v,
                                                        float* __restrict__ out, int64_t ldx,
-                                                       int nr) {
+                                                       int nr, float* __restrict__ lo,
+                                                       bool first) {
     __shared__ float red[4][16][33];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int c = lane & 15, kk = lane >> 4;
@@ -446,31 +452,54 @@ __global__ __launch_bounds__(NT) void gesl_mrhs_kernel(const float* __restrict__
         const int e = t & 31;
         float sum = red[0][r][e];
         for (int g = 1; g < waves; ++g) sum += red[g][r][e];
-        float* o = out + (int64_t)r * ldx + e0 + e;
-        *o = ASSIGN ? SIGN * sum : *o + SIGN * sum;
+        const int64_t i = (int64_t)r * ldx + e0 + e;
+        if constexpr (OUT == Out::Store) {
+            out[i] = SIGN * sum;
+        } else if constexpr (OUT == Out::Add) {
+            out[i] = out[i] + SIGN * sum;
+        } else {
+            const float z = out[i], y = SIGN * sum + (first ? 0.0f : lo[i]), w = z + y;
+            lo[i] = fabsf(z) >= fabsf(y) ? y - (w - z) : z - (w - y);
+            out[i] = w;
+        }
     }
 }
 
+// Y: nr columns, with blocks of 32 another nr for the carried errors behind them
 hipError_t gesl_sweeps_mrhs(const float* A, int64_t lda, int64_t n, int B, const float* binv,
                             float* X, float* Y, int64_t ldx, int nr, hipStream_t s) {
     const int N = (int)(n / B);
     const int64_t BB = (int64_t)B * B;
     const unsigned gb = (unsigned)(B / 32);
-    gesl_mrhs_kernel<1, true><<<gb, NT, 0, s>>>(binv, B, B, X, Y, ldx, nr);
+    float* lo = B == 32 ? Y + (int64_t)nr * ldx : nullptr;
+    auto solve = [&](auto sign, const float* W, const float* v, float* out) {
+        gesl_mrhs_kernel<sign.value, Out::Store><<<gb, NT, 0, s>>>(W, B, B, v, out, ldx, nr,
+                                                                   nullptr, false);
+    };
+    // entries e0 .. e0 + len - 1 of `out` by the solved block at q0
+    auto update = [&](auto sign, int64_t q0, int64_t e0, int64_t len, const float* v, float* out,
+                      bool first) {
+        const unsigned grid = (unsigned)(len / 32);
+        if (lo)
+            gesl_mrhs_kernel<sign.value, Out::Carry><<<grid, NT, 0, s>>>(
+                A + q0 * lda + e0, lda, B, v, out + e0, ldx, nr, lo + e0, first);
+        else
+            gesl_mrhs_kernel<sign.value, Out::Add><<<grid, NT, 0, s>>>(
+                A + q0 * lda + e0, lda, B, v, out + e0, ldx, nr, nullptr, false);
+    };
+    constexpr std::integral_constant<int, 1> fwd;
+    constexpr std::integral_constant<int, -1> bwd;
+    // (the first update of a sweep reaches all entries that any later one does)
+    solve(fwd, binv, X, Y);
     for (int q = 0; q + 1 < N; ++q) {
         const int64_t q0 = (int64_t)q * B, e0 = q0 + B;
-        gesl_mrhs_kernel<1, false><<<(unsigned)((n - e0) / 32), NT, 0, s>>>(
-            A + q0 * lda + e0, lda, B, Y + q0, X + e0, ldx, nr);
-        gesl_mrhs_kernel<1, true><<<gb, NT, 0, s>>>(binv + (int64_t)(q + 1) * 2 * BB, B, B, X + e0,
-                                                    Y + e0, ldx, nr);
+        update(fwd, q0, e0, n - e0, Y + q0, X, q == 0);
+        solve(fwd, binv + (int64_t)(q + 1) * 2 * BB, X + e0, Y + e0);
     }
     for (int q = N - 1; q >= 0; --q) {
         const int64_t q0 = (int64_t)q * B;
-        gesl_mrhs_kernel<-1, true><<<gb, NT, 0, s>>>(binv + (int64_t)q * 2 * BB + BB, B, B, Y + q0,
-                                                     X + q0, ldx, nr);
-        if (q)
-            gesl_mrhs_kernel<-1, false><<<(unsigned)(q0 / 32), NT, 0, s>>>(A + q0 * lda, lda, B,
-                                                                           X + q0, Y, ldx, nr);
+        solve(bwd, binv + (int64_t)q * 2 * BB + BB, Y + q0, X + q0);
+        if (q) update(bwd, q0, 0, q0, X + q0, Y, q == N - 1);
     }
     return hipGetLastError();
 }
@@ -800,6 +829,8 @@ hipError_t launch_gesl_multi(const float* A, int64_t lda, int64_t n, int B, cons
         const int64_t G = nr == 1 && binv && ws && (lda & 3) == 0 ? persist_groups(n, B) : 0;
         if (G > 0)
             e = gesl_persist(A, lda, n, B, binv, Xr, *ws, G, s);
+        else if (nr == 1 && binv && B == 32 && scratch)
+            e = gesl_sweeps_mrhs(A, lda, n, B, binv, Xr, scratch, ldx, 1, s);
         else if (nr == 1 && binv && B <= 256)
             e = gesl_sweeps_split(A, lda, n, B, binv, Xr, s);
         else if (nr == 1)
@@ -817,8 +848,8 @@ hipError_t launch_gesl_multi(const float* A, int64_t lda, int64_t n, int B, cons
 
 hipError_t launch_gesl(const float* A, int64_t lda, int64_t n, int B, const float* inv,
                        int64_t inv_stride, float* x, hipStream_t s, const float* binv,
-                       const GeslWs* ws) {
-    return launch_gesl_multi(A, lda, n, B, inv, inv_stride, x, n, 1, s, binv, ws);
+                       const GeslWs* ws, float* scratch) {
+    return launch_gesl_multi(A, lda, n, B, inv, inv_stride, x, n, 1, s, binv, ws, scratch);
 }
 
 int64_t gesl_persist_groups(int64_t n, int B) { return persist_groups(n, B); }

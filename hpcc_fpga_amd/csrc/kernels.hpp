@@ -124,10 +124,13 @@ int64_t gesl_persist_groups(int64_t n, int B);
 // persistent launch; otherwise two launches per block step.
 hipError_t launch_gesl(const float* A, int64_t lda, int64_t n, int B, const float* inv,
                        int64_t inv_stride, float* x, hipStream_t s, const float* binv = nullptr,
-                       const GeslWs* ws = nullptr);
+                       const GeslWs* ws = nullptr, float* scratch = nullptr);
 // nrhs right-hand sides, column r at X + r * ldx (ldx a multiple of 4, >= n);
 // blocks up to 256 for more than 4 right-hand sides.  Several right-hand
-// sides with binv need scratch: nrhs columns of the same leading dimension.
+// sides with binv need scratch: nrhs columns of the same leading dimension, twice
+// as many with blocks of 32.  One right-hand side with binv, blocks of 32 and
+// scratch (two columns) is solved by those launches too where the single one does
+// not apply: they carry the sums' rounding errors along, as that does.
 hipError_t launch_gesl_multi(const float* A, int64_t lda, int64_t n, int B, const float* inv,
                              int64_t inv_stride, float* X, int64_t ldx, int nrhs, hipStream_t s,
                              const float* binv = nullptr, const GeslWs* ws = nullptr,

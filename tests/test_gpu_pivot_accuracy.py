@@ -3,8 +3,8 @@
 A pivoted factor is substituted in blocks of 32, so a sum over the order has n / 32
 terms where whole panel blocks had n / B; the substitutions carry the sums' rounding
 errors along.  The bounds are the mean backward errors that the substitution by whole
-blocks reached (16 columns; 24 matrices of order 1024 with block 128; the mean's
-standard error was 0.25e-8).
+blocks reached (16 columns; 10 matrices of order 8192 with block 64, 24 of order 1024
+with block 128; the means' standard errors were 0.7e-8 and 0.25e-8).
 """
 import numpy as np
 import pytest
@@ -32,5 +32,11 @@ def _backward_errors(monkeypatch, env, n, B, seeds, together):
     return np.mean(out)
 
 
-def test_one_column(monkeypatch):
-    assert _backward_errors(monkeypatch, {}, 1024, 128, range(8), False) <= 1.87e-7
+def test_several_columns(monkeypatch):
+    assert _backward_errors(monkeypatch, {}, 8192, 64, range(3), True) <= 4.97e-7
+
+
+# one column; and by the launches that follow where the single launch gives up
+@pytest.mark.parametrize("env", [{}, {"HPL_GESL_GROUPS": "1"}])
+def test_one_column(monkeypatch, env):
+    assert _backward_errors(monkeypatch, env, 1024, 128, range(8), False) <= 1.87e-7
