@@ -645,12 +645,16 @@ hpl_status alloc_factor_workspace(hpl_ctx* c, uint32_t B) { return alloc_factor_
 hpl_status ensure_block_inverses(hpl_ctx* c) {
     if (c->binv_ready) return HPL_SUCCESS;
     const uint32_t B = c->B;
-    if (B > 256) return HPL_SUCCESS;  // sequential diagonal solves
-    const hplx::WsPlan w = plan_factor_ws(c->n, B, c->prec, 1);
-    hpl_status st = ensure(c, c->dBInv, c->capBInv, w.binv);
-    if (st && c->pivoted) {
-        c->err.clear();  // no room: the per-step launches solve
+    // above 256, and in a pivoted factor's panel blocks, sequential diagonal solves
+    if (B > 256 || (c->pivoted && B != 32)) return HPL_SUCCESS;
+    hpl_status st = HPL_ERR_OUT_OF_MEMORY;
+    if (c->block_inverses)
+        st = ensure(c, c->dBInv, c->capBInv, plan_factor_ws(c->n, B, c->prec, 1).binv);
+    else if (!c->pivoted)
         return HPL_SUCCESS;
+    if (st && c->pivoted) {
+        c->err.clear();  // no room: launches per panel block, by its 32 x 32 inverses
+        return prep_solve_blocks(c, c->pivot_block);
     }
     if (st) return st;
     HIPCHK(c, launch_block_inverse(c->dA, (int64_t)c->lda, (int64_t)c->n, (int)B, c->dInv,
@@ -857,6 +861,7 @@ hpl_status hpl_create(int device, hpl_ctx** out) {
     if (const char* e = getenv("HPL_BULK_SLICES")) c->bulk_slices = std::max(0, atoi(e));
     if (const char* e = getenv("HPL_STRIP_SOLVE")) 
         c->strip_inverse = !strcmp(e, "inverse") ? 1 : !strcmp(e, "recurrence") ? 0 : -1;
+    if (const char* e = getenv("HPL_GESL_INVERSES")) c->block_inverses = atoi(e) != 0;
     if (const char* e = getenv("HPL_CHAIN_CUS")) c->chain_cus = std::max(0, atoi(e));
     if (hipDeviceGetAttribute(&c->num_cu, hipDeviceAttributeMultiprocessorCount, device) !=
         hipSuccess)
@@ -1011,7 +1016,7 @@ hpl_status hpl_gefa_dev(hpl_ctx* c, uint32_t block, hpl_prec prec, hpl_timing* t
     c->binv_ready = false;
     // the pipelined schedule also fills the substitution's diagonal-block
     // inverses (off its critical path), so the first solve need not
-    c->binv_in_gefa = c->lt_linear && block <= 256;
+    c->binv_in_gefa = c->lt_linear && block <= 256 && c->block_inverses;
     if (c->binv_in_gefa) {
         const hplx::WsPlan w = hplx::plan_factor_ws(c->n, block, c->prec, 1);
         if (ensure(c, c->dBInv, c->capBInv, w.binv) != HPL_SUCCESS) {
@@ -1029,6 +1034,7 @@ hpl_status hpl_gefa_dev(hpl_ctx* c, uint32_t block, hpl_prec prec, hpl_timing* t
     if (t) t->gefa_s = elapsed_s(c);
     if (st) return st;
     c->B = c->pivoting ? 32 : block;  // a pivoted factor is substituted in blocks of 32
+    c->pivot_block = block;
     c->factored = true;
     c->pivoted = c->pivoting;
     c->binv_ready = c->binv_in_gefa;
@@ -1204,10 +1210,10 @@ namespace {
 // single launch where there is one, until it gives up once.
 hpl_status precond_apply(hpl_ctx* c, const double* v, double* z, bool* single) {
     const int64_t n = (int64_t)c->n;
-    const int B = (int)c->B;
     const double one = 1.0;
     hpl_status st = hplx::ensure_block_inverses(c);
     if (st) return st;
+    const int B = (int)c->B;
     for (bool again = true; again;) {
         HIPCHK(c, launch_d2f_multi(v, n, c->dIrXs, n, n, 1, &one, c->s0,
                                    c->pivoted ? c->dPerm : nullptr));

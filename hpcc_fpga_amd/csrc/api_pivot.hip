@@ -105,8 +105,10 @@ namespace hplx {
 // refined at n = 4096: 13.7 -> 5.0 ms).  Residual of an unrefined solution,
 // means over 8 to 16 matrices: n = 1024 8.1e-7 -> 7.9e-7, 2048 1.13e-6 ->
 // 1.17e-6, 4096 1.67e-6 -> 1.57e-6, 6144 2.05e-6 -> 2.03e-6.
-hpl_status prep_solve_blocks(hpl_ctx* c) {
-    PCHK(c, launch_prep_all(c->dA, (int64_t)c->lda, 32, (int)(c->n / 32), c->dInv, 3 * 1024, c->s0));
+hpl_status prep_solve_blocks(hpl_ctx* c, uint32_t B) {
+    PCHK(c, launch_prep_all(c->dA, (int64_t)c->lda, (int)B, (int)(c->n / B), c->dInv,
+                            3 * (B / 32) * 1024, c->s0));
+    c->B = B;
     return HPL_SUCCESS;
 }
 
@@ -186,7 +188,7 @@ hpl_status gefa_pivot(hpl_ctx* c, uint32_t B) {
     if (rest_pending) PCHK(c, hipStreamWaitEvent(s, c->evP, 0));
     PCHK(c, launch_transpose_square(c->dA, lda, n, s));
     // the substitution's 32 x 32 inverses, from the final factor
-    if (hpl_status ps = prep_solve_blocks(c)) return ps;
+    if (hpl_status ps = prep_solve_blocks(c, 32)) return ps;
     return HPL_SUCCESS;
 }
 
@@ -287,9 +289,9 @@ hpl_status hpl_gesl_pvt(hpl_ctx* c, const float* lu, float* b, const int32_t* ip
     PCHK(c, c->stage.to_device(c->s0, c->dPiv, ipvt, n * sizeof(int32_t)));
     PCHK(c, c->stage.to_device(c->s0, c->dPerm, perm.data(), n * sizeof(int32_t)));
     PCHK(c, c->stage.to_device(c->s0, c->dDiagU, u.data(), n * sizeof(float)));
-    st = hplx::prep_solve_blocks(c);
+    st = hplx::prep_solve_blocks(c, 32);
     if (st) return st;
-    c->B = 32;
+    c->pivot_block = B;
     c->factored = true;
     c->pivoted = true;
     c->binv_ready = false;

@@ -109,6 +109,10 @@ struct hpl_ctx {
     size_t capBInv = 0;
     void* dGeslWs = nullptr;    // workspace of the single-launch substitution
     size_t capGeslWs = 0;
+    // whether the substitution applies whole inverses (HPL_GESL_INVERSES=0: the
+    // sequential diagonal solves, as where there is no room for dBInv)
+    bool block_inverses = true;
+    uint32_t pivot_block = 0;   // the panel block of the pivoted factor
     bool binv_ready = false;    // dBInv holds the inverses of the current factor
     bool binv_in_gefa = false;  // the running factorisation fills dBInv
     // BF16 factorisation: the current steps' diagonal-block inverses for
@@ -263,8 +267,9 @@ hpl_status alloc_factor_workspace(hpl_ctx* c, uint32_t B);
 // Partial-pivoting factorisation of the resident matrix (FP32, B <= 256) on
 // stream s0, leaving the factor, dPiv, dPerm, dDiagU and the GESL inverses.
 hpl_status gefa_pivot(hpl_ctx* c, uint32_t B);
-// the 32 x 32 inverses that a pivoted factor's substitution applies, into dInv
-hpl_status prep_solve_blocks(hpl_ctx* c);
+// the 32 x 32 inverses that a pivoted factor's substitution applies, into dInv, for
+// blocks of B (c->B from then on)
+hpl_status prep_solve_blocks(hpl_ctx* c, uint32_t B);
 // Rewrite a downloaded pivoted factor (host, row-major, lda) into gefa_ref's
 // layout: u_kk on the diagonal, each column's multipliers in the row order of
 // its own step.

@@ -94,3 +94,39 @@ def test_noalloc_shows_that_it_gave_up(monkeypatch, n):
                 assert np.any(np.isnan(x))
             else:
                 assert np.array_equal(x, ref)
+
+
+@pytest.mark.parametrize("n,B,prec,pivot", [(96, 32, "fp32", False), (320, 64, "fp32", False),
+                                            (512, 128, "bf16", False), (1024, 256, "fp32", False),
+                                            (96, 32, "fp32", True), (768, 256, "fp32", True)])
+@pytest.mark.parametrize("nrhs", [1, 3, 16])
+def test_without_whole_inverses(monkeypatch, n, B, prec, pivot, nrhs):
+    """What is left where the inverses find no room: a launch per block that solves the
+    diagonal system by its 32 x 32 inverses, for each width of right-hand sides."""
+    print(f"no inverses n={n} B={B} {prec} pivot={pivot} nrhs={nrhs}", flush=True)
+    _env(monkeypatch, {"HPL_GESL_INVERSES": "0"})
+    g = np.random.default_rng(n + nrhs)
+    a = (g.random((n, n)) - 0.5).astype(np.float32)
+    if not pivot:
+        a[np.arange(n), np.arange(n)] += n
+    b = g.uniform(-1, 1, (n, nrhs))
+    with Context(0) as c:
+        c.keep_original(True)
+        c.set_pivoting(pivot)
+        c.upload(a, b[:, 0].astype(np.float32))
+        c.gefa_dev(B, prec)
+        c.gesl_dev()
+        x0 = c.download(matrix=False)[1]
+        x, res = c.solve_rhs64(b)
+        c.upload_rhs64(b[:, 0])
+        c.solve_gmres(B, prec)  # (raises where it does not converge)
+        y = c.download_solution64()
+    M = a.astype(np.float64).T
+    r = np.abs(b - M @ x).max(axis=0)
+    scale = np.abs(M).sum(axis=1).max() * np.abs(x).max(axis=0) + np.abs(b).max(axis=0)
+    assert all(q["converged"] for q in res) and np.all(r <= 1e-14 * n * scale)
+    assert np.abs(b[:, 0] - M @ y).max() <= 1e-14 * n * scale[0]
+    # unrefined: the FP32 backward error grows like sqrt(n); BF16's own update error apart
+    if prec == "fp32":
+        r0 = np.abs(b[:, 0] - M @ x0).max()
+        assert r0 <= 64 * np.sqrt(n) * 2.0 ** -24 * (scale[0] + np.abs(b).max())
