@@ -127,6 +127,7 @@ class HipExecutor : public hplserve::Executor {
             S.c->device = cfg_.device;
             S.c->external = true;
             S.c->lookahead = false;
+            S.c->strip_inverse = 0;  // (a slot has no buffers for the strips' inverses)
             S.c->depth_fp32 = S.c->depth_lp = 1;
             slots_.push_back(S);
             if (hplx::init_streams(S.c) != HPL_SUCCESS)
