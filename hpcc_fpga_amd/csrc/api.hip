@@ -117,6 +117,17 @@ hpl_status alloc_system(hpl_ctx* c, uint64_t n) {
 
 size_t lp_elem_bytes(int prec) { return prec == HPL_PREC_FP8 ? 1 : 2; }
 
+// Whether a BF16 factorisation solves its strips by the diagonal blocks'
+// inverses: their product reads the strips once and has no chain, but needs
+// the full inverses on the critical path before it.  Up to order 16384 the
+// recurrence (mostly trsm_split_kernel's) is the faster: GEFA n = 1024 B = 128
+// 0.40 ms by inverses, 0.34 by the recurrence, 4096 B = 256 1.99 and 1.59, 8192
+// 4.54 and 3.93, 16384 13.83 and 13.69, then 24576 25.4 and 25.6, 32768 44.7
+// and 45.2.
+bool strips_by_inverse(const hpl_ctx* c) {
+    return c->strip_inverse < 0 ? c->n > 16384 : c->strip_inverse > 0;
+}
+
 hpl_status alloc_factor_ws(hpl_ctx* c, uint32_t B) {
     const hplx::WsPlan w = hplx::plan_factor_ws(c->n, B, c->prec, c->depth, c->lt_linear);
     hpl_status st = ensure(c, c->dLt, c->capLt, w.lt);
@@ -125,7 +136,7 @@ hpl_status alloc_factor_ws(hpl_ctx* c, uint32_t B) {
     if (st) return st;
     st = ensure(c, c->dInv, c->capInv, w.inv);
     if (st) return st;
-    st = ensure(c, c->dTinv, c->capTinv, c->strip_inverse != 0 ? w.tinv : 0);
+    st = ensure(c, c->dTinv, c->capTinv, strips_by_inverse(c) ? w.tinv : 0);
     if (st) return st;
     st = ensure(c, c->dLpT, c->capLpT, w.lp);
     if (st) return st;
@@ -253,17 +264,6 @@ hpl_status factor_diag(hpl_ctx* c, hipStream_t st, int64_t off, uint32_t B, floa
     HIPCHK(c, launch_gemm_update_f32(c->dA + (off + h) * lda + off + h, lda, DT + h, ldt,
                                      c->dA + off * lda + off + h, lda, h, h, h, st));
     return factor_diag(c, st, off + h, h, DT + h * ldt + h, ldt, inv + (h / 32) * 1024, inv_ts);
-}
-
-// Whether a BF16 factorisation solves its strips by the diagonal blocks'
-// inverses: their product reads the strips once and has no chain, but needs
-// the full inverses on the critical path before it.  Up to order 16384 the
-// recurrence (mostly trsm_split_kernel's) is the faster: GEFA n = 1024 B = 128
-// 0.40 ms by inverses, 0.34 by the recurrence, 4096 B = 256 1.99 and 1.59, 8192
-// 4.54 and 3.93, 16384 13.83 and 13.69, then 24576 25.4 and 25.6, 32768 44.7
-// and 45.2.
-bool strips_by_inverse(const hpl_ctx* c) {
-    return c->strip_inverse < 0 ? c->n > 16384 : c->strip_inverse > 0;
 }
 
 // Step k's buffer of diagonal-block inverses for the strip solves of the

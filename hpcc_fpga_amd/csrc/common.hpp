@@ -19,6 +19,11 @@ __device__ __forceinline__ f32x16 mfma32(float a, float b, f32x16 c) {
 __device__ __forceinline__ int acc_row(int r, int lane) {
     return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
 }
+// v_mfma_f32_16x16x4_f32: D(16x16) += A(16x4) * B(4x16).  Lane l holds
+// A[l%16][l/16] and B[l/16][l%16]; accumulator register r D[4*(l/16) + r][l%16].
+__device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
 
 // Ordering of LDS traffic between lanes of one wavefront (no hardware barrier
 // needed when only one wave touches the region).

@@ -24,7 +24,6 @@
 
 #include <algorithm>
 #include <cstdlib>
-#include <type_traits>
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
@@ -114,14 +113,6 @@ __device__ __forceinline__ double from_half64(double v) {
     const auto a = __builtin_amdgcn_permlane32_swap(l, l, false, false);
     const auto b = __builtin_amdgcn_permlane32_swap(g, g, false, false);
     return __longlong_as_double((long long)(((uint64_t)b[H] << 32) | a[H]));
-}
-
-template <int J, int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (J < N) {
-        f(std::integral_constant<int, J>{});
-        static_for<J + 1, N>(f);
-    }
 }
 
 template <bool TOP>

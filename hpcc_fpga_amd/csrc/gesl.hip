@@ -390,10 +390,6 @@ hipError_t gesl_sweeps_split(const float* A, int64_t lda, int64_t n, int B, cons
 // products on vector instructions took 156 us a step, 10 ms for the two
 // solves of a refinement; solve_rhs64 as a whole 12.17 -> 1.57 ms.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
 // What becomes of a product: stored, added to the sum that is there, or added with
 // that sum's rounding errors carried along in a second array (lo; from zero on where
 // `first`), as gesl_persist_kernel does for its sums over blocks of 32.

@@ -503,10 +503,6 @@ __global__ __launch_bounds__(64) void trsm_reg_kernel(float* __restrict__ A, int
 // GEFA: n = 1024 B = 128 0.378 -> 0.324 ms, 2048 0.853 -> 0.738, 4096 B = 256
 // 2.51 -> 1.94, B = 64 2.15 -> 2.00; FP8 n = 6144 B = 128 3.3 -> 2.95, B = 256
 // 3.69 -> 2.86.
-__device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
 template <int B>
 constexpr int kSplitWaves = B / 32 < 4 ? B / 32 : 4;  // per half
 
