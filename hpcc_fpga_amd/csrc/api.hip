@@ -668,6 +668,9 @@ const GeslWs* gesl_workspace(hpl_ctx* c, GeslWs* ws) {
     // once, and their single launches could not all be co-resident
     if (c->external || !c->binv_ready || gesl_persist_groups((int64_t)c->n, (int)c->B) <= 0)
         return nullptr;
+    // a pivoted factor of one block waits for nothing: two plain launches (22 us
+    // with the copy of b and the call, 29 as a single one and its status)
+    if (c->pivoted && c->n == c->B) return nullptr;
     if (ensure(c, c->dGeslWs, c->capGeslWs, gesl_ws_bytes((int64_t)c->n)) != HPL_SUCCESS) {
         c->err.clear();
         return nullptr;  // no room: the per-step launches solve
@@ -690,8 +693,9 @@ IrPlan plan_ir(uint64_t n, int nrhs) {
     p.work = (size_t)residual_multi_work((int64_t)n, nrhs) * sizeof(double);
     p.r = (size_t)n * nrhs * sizeof(double);
     p.xs = (size_t)n * nrhs * sizeof(float);
-    // the norms, behind one column's the status of a single-launch substitution
-    p.out = std::max<size_t>(4 * (size_t)nrhs, 5) * sizeof(double);
+    // the norms, behind those of a few columns the single launches' status words
+    p.out = 4 * (size_t)nrhs * sizeof(double);
+    if (nrhs <= kGeslSingleColumns) p.out += kGeslSingleColumns * sizeof(int);
     return p;
 }
 
@@ -723,8 +727,8 @@ hpl_status init_pipeline_streams(hpl_ctx* c) {
 namespace {
 
 // One refinement from x0 = F^-1 b on, its substitutions by the single launch
-// where ws is given (one column, the status behind the norms in dIrOut); *again:
-// one of them gave up, the answer is void.
+// where ws is given (its status words behind the norms in dIrOut); *again: one of
+// them gave up, the answer is void.
 hpl_status refine(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_iter, double tol,
                   hpl_ir_result* res, const GeslWs* ws, bool* again) {
     *again = false;
@@ -733,8 +737,8 @@ hpl_status refine(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_it
     const int64_t inv_stride = 3 * (B / 32) * 1024;
     // the substitution of several columns: between two residuals, whose
     // partial sums (at least n (nrhs + 1) doubles, 2 n (nrhs + 1) floats) it overwrites
-    float* scratch = nrhs > 1 || c->pivoted ? reinterpret_cast<float*>(c->dWork) : nullptr;
-    const size_t out_bytes = 4 * nrhs * sizeof(double) + (ws ? sizeof(int) : 0);
+    float* scratch = reinterpret_cast<float*>(c->dWork);
+    const size_t out_bytes = 4 * nrhs * sizeof(double) + (ws ? nrhs * sizeof(int) : 0);
     double sc_in[16], sc_out[16], h[64];
     int iters[16];
     for (int j = 0; j < nrhs; ++j) {
@@ -745,19 +749,18 @@ hpl_status refine(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_it
     const int* perm = c->pivoted ? c->dPerm : nullptr;
     HIPCHK(c, launch_d2f_multi(dB, n, c->dIrXs, n, n, nrhs, sc_in, c->s0, perm));
     HIPCHK(c, launch_gesl_multi(c->dA, (int64_t)c->lda, n, B, c->dInv, inv_stride, c->dIrXs, n,
-                                nrhs, c->s0, c->binv_ready ? c->dBInv : nullptr, ws, scratch));
+                                nrhs, c->s0, c->binv_ready ? c->dBInv : nullptr, ws, scratch,
+                                c->pivoted));
     HIPCHK(c, launch_axpy_multi(dX, n, c->dIrXs, n, n, nrhs, sc_out, 1, c->s0));
     for (int it = 0;; ++it) {
         HIPCHK(c, launch_residual_multi(c->dA0, (int64_t)c->lda, n, dX, n, dB, n, nrhs, c->dWork,
                                         c->dIrR, n, c->dIrOut, c->s0));
         HIPCHK(c, c->stage.to_host(c->s0, h, c->dIrOut, out_bytes));
         if (ws) {
-            int status;
-            std::memcpy(&status, h + 4, sizeof status);
-            if (status & 2) {
-                *again = true;
-                return HPL_SUCCESS;
-            }
+            int status[kGeslSingleColumns];
+            std::memcpy(status, h + 4 * nrhs, nrhs * sizeof(int));
+            for (int j = 0; j < nrhs; ++j) *again = *again || (status[j] & 2);
+            if (*again) return HPL_SUCCESS;
         }
         bool any = false;
         for (int j = 0; j < nrhs; ++j) {
@@ -786,7 +789,7 @@ hpl_status refine(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_it
         HIPCHK(c, launch_d2f_multi(c->dIrR, n, c->dIrXs, n, n, nrhs, sc_in, c->s0, perm));
         HIPCHK(c, launch_gesl_multi(c->dA, (int64_t)c->lda, n, B, c->dInv, inv_stride, c->dIrXs,
                                     n, nrhs, c->s0, c->binv_ready ? c->dBInv : nullptr, ws,
-                                    scratch));
+                                    scratch, c->pivoted));
         HIPCHK(c, launch_axpy_multi(dX, n, c->dIrXs, n, n, nrhs, sc_out, 0, c->s0));
     }
     return HPL_SUCCESS;
@@ -809,8 +812,9 @@ hpl_status ir_solve(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_
     st = ensure_block_inverses(c);
     if (st) return st;
     GeslWs wsbuf;
-    const GeslWs* ws = nrhs == 1 ? gesl_workspace(c, &wsbuf) : nullptr;
-    if (ws) wsbuf.status = reinterpret_cast<int*>(c->dIrOut + 4);
+    const bool single = nrhs == 1 || (c->pivoted && nrhs <= kGeslSingleColumns);
+    const GeslWs* ws = single ? gesl_workspace(c, &wsbuf) : nullptr;
+    if (ws) wsbuf.status = reinterpret_cast<int*>(c->dIrOut + 4 * nrhs);
     for (bool again = true; again; ws = nullptr) {
         st = refine(c, nrhs, dB, dX, max_iter, tol, res, ws, &again);
         if (st) return st;
@@ -1067,7 +1071,8 @@ hpl_status hpl_gesl_dev(hpl_ctx* c, hpl_timing* t) {
                                      c->s0));
         HIPCHK(c, launch_gesl(c->dA, (int64_t)c->lda, (int64_t)c->n, (int)c->B, c->dInv,
                               3 * (c->B / 32) * 1024, c->dx, c->s0,
-                              c->binv_ready ? c->dBInv : nullptr, ws, scratch));
+                              c->binv_ready ? c->dBInv : nullptr, ws, scratch,
+                              c->pivoted));
         HIPCHK(c, hipEventRecord(c->e1, c->s0));
         st = hplx::gesl_gave_up(c, ws, &again);  // waits for the stream where there is a status
         if (st) return st;
@@ -1221,7 +1226,7 @@ hpl_status precond_apply(hpl_ctx* c, const double* v, double* z, bool* single) {
         const GeslWs* ws = *single ? hplx::gesl_workspace(c, &wsbuf) : nullptr;
         HIPCHK(c, launch_gesl_multi(c->dA, (int64_t)c->lda, n, B, c->dInv, 3 * (B / 32) * 1024,
                                     c->dIrXs, n, 1, c->s0, c->binv_ready ? c->dBInv : nullptr, ws,
-                                    c->pivoted ? reinterpret_cast<float*>(c->dWork) : nullptr));
+                                    reinterpret_cast<float*>(c->dWork), c->pivoted));
         st = hplx::gesl_gave_up(c, ws, &again);
         if (st) return st;
         if (again) *single = false;

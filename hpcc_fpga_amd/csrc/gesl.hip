@@ -461,13 +461,13 @@ __global__ __launch_bounds__(NT) void gesl_mrhs_kernel(const float* __restrict__
     }
 }
 
-// Y: nr columns, with blocks of 32 another nr for the carried errors behind them
+// Y: nr columns, with carry another nr for the carried errors behind them
 hipError_t gesl_sweeps_mrhs(const float* A, int64_t lda, int64_t n, int B, const float* binv,
-                            float* X, float* Y, int64_t ldx, int nr, hipStream_t s) {
+                            float* X, float* Y, int64_t ldx, int nr, bool carry, hipStream_t s) {
     const int N = (int)(n / B);
     const int64_t BB = (int64_t)B * B;
     const unsigned gb = (unsigned)(B / 32);
-    float* lo = B == 32 ? Y + (int64_t)nr * ldx : nullptr;
+    float* lo = carry ? Y + (int64_t)nr * ldx : nullptr;
     auto solve = [&](auto sign, const float* W, const float* v, float* out) {
         gesl_mrhs_kernel<sign.value, Out::Store><<<gb, NT, 0, s>>>(W, B, B, v, out, ldx, nr,
                                                                    nullptr, false);
@@ -815,24 +815,30 @@ hipError_t gesl_persist(const float* A, int64_t lda, int64_t n, int B, const flo
 
 hipError_t launch_gesl_multi(const float* A, int64_t lda, int64_t n, int B, const float* inv,
                              int64_t inv_stride, float* X, int64_t ldx, int nrhs, hipStream_t s,
-                             const float* binv, const GeslWs* ws, float* scratch) {
-    if (B > 512 || B < 32 || B % 32 || n % B || nrhs < 1 || (nrhs > 1 && (ldx < n || ldx % 4 || (binv && !scratch))))
+                             const float* binv, const GeslWs* ws, float* scratch, bool carry) {
+    if (B > 512 || B < 32 || B % 32 || n % B || nrhs < 1 ||
+        (nrhs > 1 && (ldx < n || ldx % 4 || (binv && !scratch))))
         return hipErrorInvalidValue;
     for (int r0 = 0; r0 < nrhs; r0 += 16) {
         const int nr = std::min(16, nrhs - r0);
         float* Xr = X + (int64_t)r0 * ldx;
-        hipError_t e;
-        const int64_t G = nr == 1 && binv && ws && (lda & 3) == 0 ? persist_groups(n, B) : 0;
-        if (G > 0)
-            e = gesl_persist(A, lda, n, B, binv, Xr, *ws, G, s);
-        else if (nr == 1 && binv && B == 32 && scratch)
-            e = gesl_sweeps_mrhs(A, lda, n, B, binv, Xr, scratch, ldx, 1, s);
+        hipError_t e = hipSuccess;
+        const bool single = nr == 1 || (carry && nr <= kGeslSingleColumns);
+        const int64_t G = single && binv && ws && (lda & 3) == 0 ? persist_groups(n, B) : 0;
+        if (G > 0) {
+            for (int r = 0; r < nr && e == hipSuccess; ++r) {
+                GeslWs w = *ws;
+                w.status += r;
+                e = gesl_persist(A, lda, n, B, binv, Xr + r * ldx, w, G, s);
+            }
+        } else if (nr == 1 && binv && carry && scratch)
+            e = gesl_sweeps_mrhs(A, lda, n, B, binv, Xr, scratch, ldx, 1, true, s);
         else if (nr == 1 && binv && B <= 256)
             e = gesl_sweeps_split(A, lda, n, B, binv, Xr, s);
         else if (nr == 1)
             e = gesl_sweeps<1>(A, lda, n, B, inv, inv_stride, Xr, ldx, 1, s);
         else if (binv && B <= 256)
-            e = gesl_sweeps_mrhs(A, lda, n, B, binv, Xr, scratch, ldx, nr, s);
+            e = gesl_sweeps_mrhs(A, lda, n, B, binv, Xr, scratch, ldx, nr, carry, s);
         else if (nr <= 4)
             e = gesl_sweeps<4>(A, lda, n, B, inv, inv_stride, Xr, ldx, nr, s);
         else
@@ -844,8 +850,8 @@ hipError_t launch_gesl_multi(const float* A, int64_t lda, int64_t n, int B, cons
 
 hipError_t launch_gesl(const float* A, int64_t lda, int64_t n, int B, const float* inv,
                        int64_t inv_stride, float* x, hipStream_t s, const float* binv,
-                       const GeslWs* ws, float* scratch) {
-    return launch_gesl_multi(A, lda, n, B, inv, inv_stride, x, n, 1, s, binv, ws, scratch);
+                       const GeslWs* ws, float* scratch, bool carry) {
+    return launch_gesl_multi(A, lda, n, B, inv, inv_stride, x, n, 1, s, binv, ws, scratch, carry);
 }
 
 int64_t gesl_persist_groups(int64_t n, int B) { return persist_groups(n, B); }

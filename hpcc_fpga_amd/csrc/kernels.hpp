@@ -122,19 +122,24 @@ int64_t gesl_persist_groups(int64_t n, int B);
 // or null for the sequential diagonal solve with the 32 x 32 inverses.  With
 // binv, one right-hand side and a workspace, the substitution is a single
 // persistent launch; otherwise two launches per block step.
+// carry (blocks of 32): sums over blocks carry their rounding errors along, which
+// the launches for several right-hand sides do in twice the scratch; they then
+// take one right-hand side too, where the single launch does not apply.
 hipError_t launch_gesl(const float* A, int64_t lda, int64_t n, int B, const float* inv,
                        int64_t inv_stride, float* x, hipStream_t s, const float* binv = nullptr,
-                       const GeslWs* ws = nullptr, float* scratch = nullptr);
+                       const GeslWs* ws = nullptr, float* scratch = nullptr, bool carry = false);
 // nrhs right-hand sides, column r at X + r * ldx (ldx a multiple of 4, >= n);
-// blocks up to 256 for more than 4 right-hand sides.  Several right-hand
-// sides with binv need scratch: nrhs columns of the same leading dimension, twice
-// as many with blocks of 32.  One right-hand side with binv, blocks of 32 and
-// scratch (two columns) is solved by those launches too where the single one does
-// not apply: they carry the sums' rounding errors along, as that does.
+// blocks up to 256 for more than 4 right-hand sides.  Several right-hand sides
+// with binv need scratch: nrhs columns of the same leading dimension.  With carry
+// and a workspace, up to kGeslSingleColumns go one by one by the single launch,
+// which leaves column r's status at ws->status[r]: in blocks of 32 the launches
+// per block step take 0.4 ms a solve at n = 1024 and 3.5 at 9216, whatever the
+// count, a single launch 0.1 and 0.83.
+constexpr int kGeslSingleColumns = 4;
 hipError_t launch_gesl_multi(const float* A, int64_t lda, int64_t n, int B, const float* inv,
                              int64_t inv_stride, float* X, int64_t ldx, int nrhs, hipStream_t s,
                              const float* binv = nullptr, const GeslWs* ws = nullptr,
-                             float* scratch = nullptr);
+                             float* scratch = nullptr, bool carry = false);
 
 // partial pivoting (pivot.hip); X is the transposed matrix X[i][j] = M(i, j)
 hipError_t launch_transpose_square(float* A, int64_t ld, int64_t n, hipStream_t s);

@@ -66,7 +66,8 @@ def test_fp32(monkeypatch, n, B, pivot):
             c.solve_ir(B, "fp32", tol=1e-15)
             r = c.download_solution64()
             c.solve_gmres(B, "fp32", tol=1e-15)
-            out[name] = x, r, c.download_solution64(), c.solve_rhs64(b)[0]
+            out[name] = (x, r, c.download_solution64(), c.solve_rhs64(b)[0],
+                         c.solve_rhs64(np.stack([b, -2.0 * b[::-1], b ** 2], axis=1))[0])
     for p, q in zip(out["groups"], out["spin"]):
         assert np.all(np.isfinite(p)) and np.array_equal(p, q)
     ref = np.linalg.solve(a.T.astype(np.float64), b)
