@@ -8,7 +8,8 @@ namespace hplx {
 namespace {
 
 // Memory that the runtime made or has registered (pinned, managed, device): its
-// copies need no staging.
+// copies need no staging.  Asking costs 3 us, more than a host copy of a small
+// buffer, so it is for longer transfers.
 bool runtime_knows(const void* p) {
     hipPointerAttribute_t at{};
     if (hipPointerGetAttributes(&at, p) != hipSuccess) {
@@ -62,10 +63,11 @@ hipError_t HostStage::to_device(hipStream_t s, void* dev, size_t dev_pitch, cons
     // bytes from a row's start to the next one's (or to its own end)
     const size_t span = rows > 1 ? dev_pitch : width;
     if (width > span) return hipErrorInvalidValue;
-    if (runtime_knows(host))
+    const size_t total = (rows - 1) * span + width;
+    if (total > kSmall && runtime_knows(host))
         return hipMemcpy2DAsync(dev, dev_pitch, host, host_pitch, width, rows,
                                 hipMemcpyHostToDevice, s);
-    Ring& R = ring((rows - 1) * span + width);
+    Ring& R = ring(total);
     hipError_t e = R.make();
     if (e != hipSuccess) return e;
     if (span > kLarge) {  // row by row, each in pieces
@@ -97,7 +99,8 @@ hipError_t HostStage::to_device(hipStream_t s, void* dev, size_t dev_pitch, cons
 }
 
 hipError_t HostStage::to_device(hipStream_t s, void* dev, const void* host, size_t bytes) {
-    if (runtime_knows(host)) return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
+    if (bytes > kSmall && runtime_knows(host))
+        return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
     const size_t whole = bytes / kLarge, done = whole * kLarge;
     hipError_t e = to_device(s, dev, kLarge, host, kLarge, kLarge, whole);
     if (e != hipSuccess || done == bytes) return e;
@@ -106,7 +109,7 @@ hipError_t HostStage::to_device(hipStream_t s, void* dev, const void* host, size
 }
 
 hipError_t HostStage::to_host(hipStream_t s, void* host, const void* dev, size_t bytes) {
-    if (runtime_knows(host)) {
+    if (bytes > kSmall && runtime_knows(host)) {
         hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e;
     }
@@ -122,12 +125,13 @@ hipError_t HostStage::to_host(hipStream_t s, void* host, size_t host_pitch, cons
     if (!width || !rows) return hipSuccess;
     const size_t span = rows > 1 ? dev_pitch : width;
     if (width > span) return hipErrorInvalidValue;
-    if (runtime_knows(host)) {
+    const size_t total = (rows - 1) * span + width;
+    if (total > kSmall && runtime_knows(host)) {
         hipError_t e = hipMemcpy2DAsync(host, host_pitch, dev, dev_pitch, width, rows,
                                         hipMemcpyDeviceToHost, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e;
     }
-    Ring& R = ring((rows - 1) * span + width);
+    Ring& R = ring(total);
     hipError_t e = R.make();
     if (e != hipSuccess) return e;
     if (span > kLarge) {

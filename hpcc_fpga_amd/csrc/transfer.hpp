@@ -15,11 +15,11 @@ namespace hplx {
 // row pinned and queued by itself (about 10 us a row: 27 ms for the three
 // transfers of a 1024 x 1024 solve, 1.3 ms through these buffers).  Here rows are
 // packed at the device's pitch by the host while the previous piece is on its
-// way, so the device sees plain copies from pinned memory.  Buffers that the
-// runtime knows -- the caller's own pinned, managed or device memory -- are copied
-// from or to directly: a copy through the host's caches halves their rate (n =
-// 4096 up 1.2 ms direct and 2.2 staged, down 1.2 and 2.9; 16384 19 and 36, 19 and
-// 45).
+// way, so the device sees plain copies from pinned memory.  Longer transfers of
+// buffers that the runtime knows -- the caller's own pinned, managed or device
+// memory -- are copied from or to directly: a copy through the host's caches halves
+// their rate (n = 4096 up 1.2 ms direct and 2.2 staged, down 1.2 and 2.9; 16384 19
+// and 36, 19 and 45).
 class HostStage {
    public:
     ~HostStage() { free(); }
