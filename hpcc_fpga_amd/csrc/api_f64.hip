@@ -304,17 +304,21 @@ hpl_status hpl_gesl_dev_f64(hpl_ctx* c, hpl_timing* t) {
     FCHK(c, hipSetDevice(c->device));
     FCHK(c, hipEventRecord(c->e0, c->s0));
     const int64_t n = (int64_t)c->n64;
-    // where the single launch gave up (its waves were not resident together,
-    // as other launches held the device), again from b launch after launch
-    for (const bool per_block : {false, true}) {
+    // One block waits for nothing.  Where the single launch gave up (its waves were
+    // not resident together, as other launches held the device), again from b launch
+    // after launch.
+    for (bool again = true, per_block = n == f64_block(); again; per_block = true) {
         FCHK(c, hipMemcpyAsync(c->dX64s, c->dB64s, c->n64 * sizeof(double),
                                hipMemcpyDeviceToDevice, c->s0));
         FCHK(c, launch_gesl_f64(c->dA64, (int64_t)c->lda64, n, c->dX64s, c->dWork64, c->s0,
                                 per_block));
         FCHK(c, hipEventRecord(c->e1, c->s0));
         int h = 0;
-        FCHK(c, c->stage.to_host(c->s0, &h, gesl_f64_status(c->dWork64, n), sizeof h));
-        if (!h) break;
+        if (per_block)
+            FCHK(c, hipStreamSynchronize(c->s0));
+        else
+            FCHK(c, c->stage.to_host(c->s0, &h, gesl_f64_status(c->dWork64, n), sizeof h));
+        again = h != 0;
     }
     if (t) t->gesl_s = seconds(c->e0, c->e1);
     return HPL_SUCCESS;

@@ -706,21 +706,24 @@ hipError_t launch_gesl_f64(const double* A, int64_t lda, int64_t n, double* x, d
     // holds, so that other work on it leaves room (n up to 65536), and at most
     // HPL_GESL_GROUPS; beyond, where the device does not say, or where the
     // caller asks for it (per_block), launch after launch.
-    int per_cu = 0, dev = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void*>(gesl_persist_f64), 64, 0) != hipSuccess ||
-        hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-        (void)hipGetLastError();
-        per_cu = cus = 0;
-    }
-    gesl_reset_f64<<<(unsigned)((2 * n + 255) / 256), 256, 0, s>>>(work, 2 * n, status);
-    int64_t most = per_block ? 0 : (int64_t)per_cu * cus / 2;
-    if (const char* e = getenv("HPL_GESL_GROUPS")) most = std::min<int64_t>(most, atoll(e));
-    if (N <= most) {
-        gesl_persist_f64<<<(unsigned)N, 64, 0, s>>>(A, lda, (int)N, x, work, work + n, status,
-                                                    gesl_spin_limit(kGesl64SpinLimit));
-        return hipGetLastError();
+    if (!per_block) {
+        int per_cu = 0, dev = 0, cus = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per_cu, reinterpret_cast<const void*>(gesl_persist_f64), 64, 0) != hipSuccess ||
+            hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
+                hipSuccess) {
+            (void)hipGetLastError();
+            per_cu = cus = 0;
+        }
+        gesl_reset_f64<<<(unsigned)((2 * n + 255) / 256), 256, 0, s>>>(work, 2 * n, status);
+        int64_t most = (int64_t)per_cu * cus / 2;
+        if (const char* e = getenv("HPL_GESL_GROUPS")) most = std::min<int64_t>(most, atoll(e));
+        if (N <= most) {
+            gesl_persist_f64<<<(unsigned)N, 64, 0, s>>>(A, lda, (int)N, x, work, work + n, status,
+                                                        gesl_spin_limit(kGesl64SpinLimit));
+            return hipGetLastError();
+        }
     }
     for (int64_t k0 = 0; k0 < n; k0 += FB) {
         gesl_diag_fwd_f64<<<1, 64, 0, s>>>(A, lda, k0, x);

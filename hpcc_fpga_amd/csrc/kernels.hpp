@@ -198,7 +198,7 @@ hipError_t launch_update_f64(double* C, int64_t ldc, const double* Lt, int64_t l
 // work: gesl_f64_work(n) doubles; *gesl_f64_status(work, n) is non-zero
 // afterwards where a bounded wait of the single launch gave up (x is then
 // partly overwritten; per_block solves without one, launch after launch, to the
-// same bits)
+// same bits, and leaves the status alone)
 int64_t gesl_f64_work(int64_t n);
 const int* gesl_f64_status(const double* work, int64_t n);
 hipError_t launch_gesl_f64(const double* A, int64_t lda, int64_t n, double* x, double* work,
