@@ -390,20 +390,11 @@ hipError_t gesl_sweeps_split(const float* A, int64_t lda, int64_t n, int B, cons
 // products on vector instructions took 156 us a step, 10 ms for the two
 // solves of a refinement; solve_rhs64 as a whole 12.17 -> 1.57 ms.
 // ---------------------------------------------------------------------------
-// What becomes of a product: stored, added to the sum that is there, or added with
-// that sum's rounding errors carried along in a second array (lo; from zero on where
-// `first`), as gesl_persist_kernel does for its sums over blocks of 32.
-enum class Out { Store, Add, Carry };
-
-// out[r][e] := (Store ? 0 : out[r][e]) + SIGN sum_{p < B} W[p * ldw + e] v[r][p]
-// for the 32 entries e of workgroup blockIdx.x, r < nr <= 16
-template <int SIGN, Out OUT>
-__global__ __launch_bounds__(NT) void gesl_mrhs_kernel(const float* __restrict__ W, int64_t ldw,
-                                                       int B, const float* __restrict__ v,
-                                                       float* __restrict__ out, int64_t ldx,
-                                                       int nr, float* __restrict__ lo,
-                                                       bool first) {
-    __shared__ float red[4][16][33];
+// red[g][r][e] := sum over wave g's rows p of W[p * ldw + e0 + e] v[r][p], for the 32
+// entries e0 .. of workgroup blockIdx.x and r < nr <= 16; returns the waves
+__device__ __forceinline__ int mrhs_product(const float* __restrict__ W, int64_t ldw, int B,
+                                            const float* __restrict__ v, int64_t ldx, int nr,
+                                            float (&red)[4][16][33]) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int c = lane & 15, kk = lane >> 4;
     const int waves = min(4, B / 16), rows = B / waves;  // 16, 32 or 64 rows per wave
@@ -444,20 +435,45 @@ __global__ __launch_bounds__(NT) void gesl_mrhs_kernel(const float* __restrict__
         }
     }
     __syncthreads();
+    return waves;
+}
+
+// out[r][e] := (ASSIGN ? 0 : out[r][e]) + SIGN sum_{p < B} W[p * ldw + e] v[r][p]
+template <int SIGN, bool ASSIGN>
+__global__ __launch_bounds__(NT) void gesl_mrhs_kernel(const float* __restrict__ W, int64_t ldw,
+                                                       int B, const float* __restrict__ v,
+                                                       float* __restrict__ out, int64_t ldx,
+                                                       int nr) {
+    __shared__ float red[4][16][33];
+    const int waves = mrhs_product(W, ldw, B, v, ldx, nr, red);
+    const int t = threadIdx.x, e = t & 31;
     for (int r = t >> 5; r < nr; r += NT / 32) {
-        const int e = t & 31;
         float sum = red[0][r][e];
         for (int g = 1; g < waves; ++g) sum += red[g][r][e];
-        const int64_t i = (int64_t)r * ldx + e0 + e;
-        if constexpr (OUT == Out::Store) {
-            out[i] = SIGN * sum;
-        } else if constexpr (OUT == Out::Add) {
-            out[i] = out[i] + SIGN * sum;
-        } else {
-            const float z = out[i], y = SIGN * sum + (first ? 0.0f : lo[i]), w = z + y;
-            lo[i] = fabsf(z) >= fabsf(y) ? y - (w - z) : z - (w - y);
-            out[i] = w;
-        }
+        float* o = out + (int64_t)r * ldx + (int64_t)blockIdx.x * 32 + e;
+        *o = ASSIGN ? SIGN * sum : *o + SIGN * sum;
+    }
+}
+
+// The same addition with the sum's rounding errors carried along in lo (from zero on
+// where `first`), as gesl_persist_kernel does for its sums over blocks of 32.
+template <int SIGN>
+__global__ __launch_bounds__(NT) void gesl_mrhs_carry_kernel(const float* __restrict__ W,
+                                                             int64_t ldw, int B,
+                                                             const float* __restrict__ v,
+                                                             float* __restrict__ out,
+                                                             float* __restrict__ lo, int64_t ldx,
+                                                             int nr, bool first) {
+    __shared__ float red[4][16][33];
+    const int waves = mrhs_product(W, ldw, B, v, ldx, nr, red);
+    const int t = threadIdx.x, e = t & 31;
+    for (int r = t >> 5; r < nr; r += NT / 32) {
+        float sum = red[0][r][e];
+        for (int g = 1; g < waves; ++g) sum += red[g][r][e];
+        const int64_t i = (int64_t)r * ldx + (int64_t)blockIdx.x * 32 + e;
+        const float z = out[i], y = SIGN * sum + (first ? 0.0f : lo[i]), w = z + y;
+        lo[i] = fabsf(z) >= fabsf(y) ? y - (w - z) : z - (w - y);
+        out[i] = w;
     }
 }
 
@@ -469,19 +485,18 @@ hipError_t gesl_sweeps_mrhs(const float* A, int64_t lda, int64_t n, int B, const
     const unsigned gb = (unsigned)(B / 32);
     float* lo = carry ? Y + (int64_t)nr * ldx : nullptr;
     auto solve = [&](auto sign, const float* W, const float* v, float* out) {
-        gesl_mrhs_kernel<sign.value, Out::Store><<<gb, NT, 0, s>>>(W, B, B, v, out, ldx, nr,
-                                                                   nullptr, false);
+        gesl_mrhs_kernel<sign.value, true><<<gb, NT, 0, s>>>(W, B, B, v, out, ldx, nr);
     };
     // entries e0 .. e0 + len - 1 of `out` by the solved block at q0
     auto update = [&](auto sign, int64_t q0, int64_t e0, int64_t len, const float* v, float* out,
                       bool first) {
         const unsigned grid = (unsigned)(len / 32);
         if (lo)
-            gesl_mrhs_kernel<sign.value, Out::Carry><<<grid, NT, 0, s>>>(
-                A + q0 * lda + e0, lda, B, v, out + e0, ldx, nr, lo + e0, first);
+            gesl_mrhs_carry_kernel<sign.value><<<grid, NT, 0, s>>>(
+                A + q0 * lda + e0, lda, B, v, out + e0, lo + e0, ldx, nr, first);
         else
-            gesl_mrhs_kernel<sign.value, Out::Add><<<grid, NT, 0, s>>>(
-                A + q0 * lda + e0, lda, B, v, out + e0, ldx, nr, nullptr, false);
+            gesl_mrhs_kernel<sign.value, false><<<grid, NT, 0, s>>>(A + q0 * lda + e0, lda, B, v,
+                                                                    out + e0, ldx, nr);
     };
     constexpr std::integral_constant<int, 1> fwd;
     constexpr std::integral_constant<int, -1> bwd;
