@@ -519,7 +519,7 @@ hpl_status copy_ahead(hpl_batch* b, int lo, int hi) {
     const size_t xb = (size_t)(v1 - v0) * sizeof(double), rb = (hi - lo) * sizeof(BatchResult);
     if (xb + rb > b->cap_ahead) {
         if (b->ahead) (void)hipHostFree(b->ahead);
-        // room for the further, longer ones too
+        // room for the longest piece to come (one allocation, about a millisecond)
         const size_t most = (size_t)b->v_total * sizeof(double) + b->nsys * sizeof(BatchResult);
         const size_t cap = std::max(xb + rb, std::min<size_t>(most, 2 * kAheadBytes));
         b->cap_ahead = 0;
@@ -571,7 +571,8 @@ hpl_status hpl_batch_get(hpl_batch* b, int s, double* x, int* iterations, double
         }
         ++b->copies;
         b->ahead_lo = b->ahead_hi = 0;
-        if (hi - lo > 1) {
+        // (one alone too once there is the memory: two copies and one wait)
+        if (hi - lo > 1 || b->cap_ahead >= (size_t)sy.npad * sizeof(double) + sizeof r) {
             hpl_status st = copy_ahead(b, lo, hi);
             if (st) return st;
         }
