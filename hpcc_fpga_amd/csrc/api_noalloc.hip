@@ -76,7 +76,8 @@ extern "C" hpl_status hpl_gesl_noalloc(const float* lu, uint64_t n, uint64_t lda
     float* binv = base + inv_floats;  // inv_floats is a multiple of 1024: 4 KiB aligned
     // binv_floats = 2 n B, a multiple of 64: the workspace stays 256-byte aligned
     GeslWs ws = gesl_ws_carve(binv + binv_floats, (int64_t)n);
-    ws.cleared = true;  // by the first launch
+    ws.cleared = true;     // by the first launch
+    ws.spins = 1L << 22;   // giving up leaves NaN
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (launch_prep_all(lu, (int64_t)lda, (int)B, (int)N, inv, inv_stride, s, &ws) !=
             hipSuccess ||

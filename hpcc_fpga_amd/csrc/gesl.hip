@@ -548,7 +548,6 @@ hipError_t gesl_sweeps_mrhs(const float* A, int64_t lda, int64_t n, int B, const
 // ---------------------------------------------------------------------------
 constexpr int kMaxOwn = 16;            // slices per workgroup (LDS capacity)
 constexpr int kMaxT = 4;               // shares per block (B / S, B <= 256)
-constexpr long kGeslSpinLimit = 1L << 22;
 
 __device__ __forceinline__ void pub_f(float* p, float v) {
     const unsigned u = __float_as_uint(v);
@@ -808,7 +807,7 @@ hipError_t gesl_persist(const float* A, int64_t lda, int64_t n, int B, const flo
                                     s>>>(ws.pf, ws.pb, words, ws.status);
     }
     const unsigned grid = (unsigned)G;
-    const long spins = gesl_spin_limit(kGeslSpinLimit);
+    const long spins = gesl_spin_limit(ws.spins);
     switch (B) {
         case 32:
             gesl_persist_kernel<32><<<grid, NT, 0, s>>>(A, lda, n, binv, x, ws, spins);

@@ -106,6 +106,8 @@ struct GeslWs {
     float* pb;  // backward partial solutions, B per slice
     int* status;
     bool cleared = false;
+    // polls before a wait gives up, about a second; more where nothing follows
+    long spins = 1L << 20;
 };
 size_t gesl_ws_bytes(int64_t n);
 // floats of pf and of pb that a launch uses: B per slice of at most 64 entries
