@@ -645,16 +645,12 @@ hpl_status alloc_factor_workspace(hpl_ctx* c, uint32_t B) { return alloc_factor_
 hpl_status ensure_block_inverses(hpl_ctx* c) {
     if (c->binv_ready) return HPL_SUCCESS;
     const uint32_t B = c->B;
-    // above 256, and in a pivoted factor's panel blocks, sequential diagonal solves
-    if (B > 256 || (c->pivoted && B != 32)) return HPL_SUCCESS;
-    hpl_status st = HPL_ERR_OUT_OF_MEMORY;
-    if (c->block_inverses)
-        st = ensure(c, c->dBInv, c->capBInv, plan_factor_ws(c->n, B, c->prec, 1).binv);
-    else if (!c->pivoted)
-        return HPL_SUCCESS;
+    if (B > 256 || !c->block_inverses) return HPL_SUCCESS;  // sequential diagonal solves
+    const hplx::WsPlan w = plan_factor_ws(c->n, B, c->prec, 1);
+    hpl_status st = ensure(c, c->dBInv, c->capBInv, w.binv);
     if (st && c->pivoted) {
-        c->err.clear();  // no room: launches per panel block, by its 32 x 32 inverses
-        return prep_solve_blocks(c, c->pivot_block);
+        c->err.clear();  // no room: launches per panel block, by the 32 x 32 inverses
+        return HPL_SUCCESS;
     }
     if (st) return st;
     HIPCHK(c, launch_block_inverse(c->dA, (int64_t)c->lda, (int64_t)c->n, (int)B, c->dInv,
@@ -668,9 +664,6 @@ const GeslWs* gesl_workspace(hpl_ctx* c, GeslWs* ws) {
     // once, and their single launches could not all be co-resident
     if (c->external || !c->binv_ready || gesl_persist_groups((int64_t)c->n, (int)c->B) <= 0)
         return nullptr;
-    // a pivoted factor of one block waits for nothing: two plain launches (22 us
-    // with the copy of b and the call, 29 as a single one and its status)
-    if (c->pivoted && c->n == c->B) return nullptr;
     if (ensure(c, c->dGeslWs, c->capGeslWs, gesl_ws_bytes((int64_t)c->n)) != HPL_SUCCESS) {
         c->err.clear();
         return nullptr;  // no room: the per-step launches solve
@@ -695,7 +688,7 @@ IrPlan plan_ir(uint64_t n, int nrhs) {
     p.xs = (size_t)n * nrhs * sizeof(float);
     // the norms, behind those of a few columns the single launches' status words
     p.out = 4 * (size_t)nrhs * sizeof(double);
-    if (nrhs <= kGeslSingleColumns) p.out += kGeslSingleColumns * sizeof(int);
+    if (nrhs <= kGeslSingleColumns) p.out += 2 * sizeof(double);
     return p;
 }
 
@@ -724,6 +717,21 @@ hpl_status init_pipeline_streams(hpl_ctx* c) {
     return HPL_SUCCESS;
 }
 
+bool few_panels(const hpl_ctx* c) {
+    return c->pivoted && c->n <= 256 && c->n <= 2 * (uint64_t)c->pivot_block;
+}
+
+hipError_t substitute(hpl_ctx* c, float* X, int nrhs, const GeslWs* ws, float* scratch,
+                      bool panels) {
+    const int64_t n = (int64_t)c->n;
+    if (c->pivoted && (panels || !c->binv_ready))
+        return launch_gesl_panels(c->dA, (int64_t)c->lda, n, (int)c->pivot_block, c->dInv, X, n,
+                                  nrhs, c->s0);
+    return launch_gesl_multi(c->dA, (int64_t)c->lda, n, (int)c->B, c->dInv,
+                             3 * (c->B / 32) * 1024, X, n, nrhs, c->s0,
+                             c->binv_ready ? c->dBInv : nullptr, ws, scratch, c->pivoted);
+}
+
 namespace {
 
 // One refinement from x0 = F^-1 b on, its substitutions by the single launch
@@ -733,8 +741,6 @@ hpl_status refine(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_it
                   hpl_ir_result* res, const GeslWs* ws, bool* again) {
     *again = false;
     const int64_t n = (int64_t)c->n;
-    const int B = (int)c->B;
-    const int64_t inv_stride = 3 * (B / 32) * 1024;
     // the substitution of several columns: between two residuals, whose
     // partial sums (at least n (nrhs + 1) doubles, 2 n (nrhs + 1) floats) it overwrites
     float* scratch = reinterpret_cast<float*>(c->dWork);
@@ -748,9 +754,7 @@ hpl_status refine(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_it
     // x0 = F^-1 b in FP32, promoted (a pivoted factor solves for P b)
     const int* perm = c->pivoted ? c->dPerm : nullptr;
     HIPCHK(c, launch_d2f_multi(dB, n, c->dIrXs, n, n, nrhs, sc_in, c->s0, perm));
-    HIPCHK(c, launch_gesl_multi(c->dA, (int64_t)c->lda, n, B, c->dInv, inv_stride, c->dIrXs, n,
-                                nrhs, c->s0, c->binv_ready ? c->dBInv : nullptr, ws, scratch,
-                                c->pivoted));
+    HIPCHK(c, substitute(c, c->dIrXs, nrhs, ws, scratch, false));
     HIPCHK(c, launch_axpy_multi(dX, n, c->dIrXs, n, n, nrhs, sc_out, 1, c->s0));
     for (int it = 0;; ++it) {
         HIPCHK(c, launch_residual_multi(c->dA0, (int64_t)c->lda, n, dX, n, dB, n, nrhs, c->dWork,
@@ -787,9 +791,7 @@ hpl_status refine(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_it
         // correction: F d = r / ||r|| in FP32, x += ||r|| d in FP64 (inactive
         // columns get scale 0 and stay unchanged)
         HIPCHK(c, launch_d2f_multi(c->dIrR, n, c->dIrXs, n, n, nrhs, sc_in, c->s0, perm));
-        HIPCHK(c, launch_gesl_multi(c->dA, (int64_t)c->lda, n, B, c->dInv, inv_stride, c->dIrXs,
-                                    n, nrhs, c->s0, c->binv_ready ? c->dBInv : nullptr, ws,
-                                    scratch, c->pivoted));
+        HIPCHK(c, substitute(c, c->dIrXs, nrhs, ws, scratch, false));
         HIPCHK(c, launch_axpy_multi(dX, n, c->dIrXs, n, n, nrhs, sc_out, 0, c->s0));
     }
     return HPL_SUCCESS;
@@ -812,7 +814,7 @@ hpl_status ir_solve(hpl_ctx* c, int nrhs, const double* dB, double* dX, int max_
     st = ensure_block_inverses(c);
     if (st) return st;
     GeslWs wsbuf;
-    const bool single = nrhs == 1 || (c->pivoted && nrhs <= kGeslSingleColumns);
+    const bool single = nrhs <= gesl_single_columns((int64_t)c->n, c->pivoted);
     const GeslWs* ws = single ? gesl_workspace(c, &wsbuf) : nullptr;
     if (ws) wsbuf.status = reinterpret_cast<int*>(c->dIrOut + 4 * nrhs);
     for (bool again = true; again; ws = nullptr) {
@@ -1050,29 +1052,27 @@ hpl_status hpl_gesl_dev(hpl_ctx* c, hpl_timing* t) {
     if (!c->factored) return fail(c, HPL_ERR_STATE, "hpl_gesl_dev before a successful GEFA");
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, hipEventRecord(c->e0, c->s0));
-    hpl_status st = hplx::ensure_block_inverses(c);
+    const bool panels = hplx::few_panels(c);
+    hpl_status st = panels ? HPL_SUCCESS : hplx::ensure_block_inverses(c);
     if (st) return st;
     // two columns for a pivoted factor's launches per block (the single launch's
     // workspace is larger)
     float* scratch = nullptr;
-    if (c->pivoted) {
+    if (c->pivoted && !panels) {
         if (ensure(c, c->dGeslWs, c->capGeslWs, gesl_ws_bytes((int64_t)c->n)) == HPL_SUCCESS)
             scratch = static_cast<float*>(c->dGeslWs);
         else
             c->err.clear();
     }
     GeslWs wsbuf;
-    const GeslWs* ws = hplx::gesl_workspace(c, &wsbuf);
+    const GeslWs* ws = panels ? nullptr : hplx::gesl_workspace(c, &wsbuf);
     for (bool again = true; again; ws = nullptr) {
         if (c->pivoted)
             HIPCHK(c, launch_gather_f32(c->dx, c->db, c->dPerm, (int64_t)c->n, c->s0));
         else
             HIPCHK(c, hipMemcpyAsync(c->dx, c->db, c->n * sizeof(float), hipMemcpyDeviceToDevice,
                                      c->s0));
-        HIPCHK(c, launch_gesl(c->dA, (int64_t)c->lda, (int64_t)c->n, (int)c->B, c->dInv,
-                              3 * (c->B / 32) * 1024, c->dx, c->s0,
-                              c->binv_ready ? c->dBInv : nullptr, ws, scratch,
-                              c->pivoted));
+        HIPCHK(c, hplx::substitute(c, c->dx, 1, ws, scratch, panels));
         HIPCHK(c, hipEventRecord(c->e1, c->s0));
         st = hplx::gesl_gave_up(c, ws, &again);  // waits for the stream where there is a status
         if (st) return st;
@@ -1216,17 +1216,15 @@ namespace {
 hpl_status precond_apply(hpl_ctx* c, const double* v, double* z, bool* single) {
     const int64_t n = (int64_t)c->n;
     const double one = 1.0;
-    hpl_status st = hplx::ensure_block_inverses(c);
+    const bool panels = hplx::few_panels(c);
+    hpl_status st = panels ? HPL_SUCCESS : hplx::ensure_block_inverses(c);
     if (st) return st;
-    const int B = (int)c->B;
     for (bool again = true; again;) {
         HIPCHK(c, launch_d2f_multi(v, n, c->dIrXs, n, n, 1, &one, c->s0,
                                    c->pivoted ? c->dPerm : nullptr));
         GeslWs wsbuf;
-        const GeslWs* ws = *single ? hplx::gesl_workspace(c, &wsbuf) : nullptr;
-        HIPCHK(c, launch_gesl_multi(c->dA, (int64_t)c->lda, n, B, c->dInv, 3 * (B / 32) * 1024,
-                                    c->dIrXs, n, 1, c->s0, c->binv_ready ? c->dBInv : nullptr, ws,
-                                    reinterpret_cast<float*>(c->dWork), c->pivoted));
+        const GeslWs* ws = *single && !panels ? hplx::gesl_workspace(c, &wsbuf) : nullptr;
+        HIPCHK(c, hplx::substitute(c, c->dIrXs, 1, ws, reinterpret_cast<float*>(c->dWork), panels));
         st = hplx::gesl_gave_up(c, ws, &again);
         if (st) return st;
         if (again) *single = false;

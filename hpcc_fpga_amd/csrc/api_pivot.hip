@@ -100,15 +100,15 @@ namespace hplx {
 // applying a whole B x B inverse loses up to a digit there (B = 256, uniform
 // matrices: 1.8e-3 against 4e-4 with 32 x 32).  So c->B is 32 for it and the
 // substitutions that apply whole inverses take the 32 x 32 ones: one launch for
-// a right-hand side (n = 6144: 1.4 ms as 96 launches, now 0.49; n = 16384
-// B = 256 5.1 -> 1.6; n = 64 0.019 -> 0.014), the MFMA sweeps for several (16
-// refined at n = 4096: 13.7 -> 5.0 ms).  Residual of an unrefined solution,
-// means over 8 to 16 matrices: n = 1024 8.1e-7 -> 7.9e-7, 2048 1.13e-6 ->
-// 1.17e-6, 4096 1.67e-6 -> 1.57e-6, 6144 2.05e-6 -> 2.03e-6.
-hpl_status prep_solve_blocks(hpl_ctx* c, uint32_t B) {
-    PCHK(c, launch_prep_all(c->dA, (int64_t)c->lda, (int)B, (int)(c->n / B), c->dInv,
-                            3 * (B / 32) * 1024, c->s0));
-    c->B = B;
+// a right-hand side (n = 6144 B = 128: 1.13 ms as 96 launches, now 0.45; n = 16384
+// B = 256 5.0 -> 1.5), the MFMA sweeps for more than three (16 refined at n = 4096
+// B = 256: 19.9 -> 5.0 ms); a launch per panel block, without whole inverses, is
+// left for small orders (few_panels) and where the inverses find no room.
+// Backward error of an unrefined solution, means over 16 columns of 12 to 24
+// matrices, by panel blocks and in blocks of 32: n = 1024 B = 128 1.87e-7 and
+// 1.58e-7, 2048 B = 256 2.78e-7 and 2.11e-7, 6144 B = 128 4.23e-7 and 3.27e-7.
+hpl_status prep_solve_blocks(hpl_ctx* c) {
+    PCHK(c, launch_prep_all(c->dA, (int64_t)c->lda, 32, (int)(c->n / 32), c->dInv, 3 * 1024, c->s0));
     return HPL_SUCCESS;
 }
 
@@ -188,7 +188,7 @@ hpl_status gefa_pivot(hpl_ctx* c, uint32_t B) {
     if (rest_pending) PCHK(c, hipStreamWaitEvent(s, c->evP, 0));
     PCHK(c, launch_transpose_square(c->dA, lda, n, s));
     // the substitution's 32 x 32 inverses, from the final factor
-    if (hpl_status ps = prep_solve_blocks(c, 32)) return ps;
+    if (hpl_status ps = prep_solve_blocks(c)) return ps;
     return HPL_SUCCESS;
 }
 
@@ -289,8 +289,9 @@ hpl_status hpl_gesl_pvt(hpl_ctx* c, const float* lu, float* b, const int32_t* ip
     PCHK(c, c->stage.to_device(c->s0, c->dPiv, ipvt, n * sizeof(int32_t)));
     PCHK(c, c->stage.to_device(c->s0, c->dPerm, perm.data(), n * sizeof(int32_t)));
     PCHK(c, c->stage.to_device(c->s0, c->dDiagU, u.data(), n * sizeof(float)));
-    st = hplx::prep_solve_blocks(c, 32);
+    st = hplx::prep_solve_blocks(c);
     if (st) return st;
+    c->B = 32;
     c->pivot_block = B;
     c->factored = true;
     c->pivoted = true;

@@ -258,6 +258,15 @@ hpl_status ensure_block_inverses(hpl_ctx* c);
 // resident together; the caller solves again without the workspace.
 const GeslWs* gesl_workspace(hpl_ctx* c, GeslWs* ws);
 hpl_status gesl_gave_up(hpl_ctx* c, const GeslWs* ws, bool* again);
+// X := F^-1 X for nrhs columns (leading dimension n) on s0; panels: a pivoted
+// factor by a launch per panel block (also where its inverses found no room).
+hipError_t substitute(hpl_ctx* c, float* X, int nrhs, const GeslWs* ws, float* scratch,
+                      bool panels);
+// Whether that is the faster for one column and a call that waits for it: up to
+// two panel blocks and order 256, four launches and no status to fetch (n = 64
+// with block 64 24 us, 32 as a single launch; 128 with block 64 34 and 36, 256
+// with 256 41 and 45, 512 with 256 75 and 65).
+bool few_panels(const hpl_ctx* c);
 
 // Device buffer of at least `bytes` (grown with hipMalloc in the context's own
 // mode, an error in external mode).
@@ -267,9 +276,8 @@ hpl_status alloc_factor_workspace(hpl_ctx* c, uint32_t B);
 // Partial-pivoting factorisation of the resident matrix (FP32, B <= 256) on
 // stream s0, leaving the factor, dPiv, dPerm, dDiagU and the GESL inverses.
 hpl_status gefa_pivot(hpl_ctx* c, uint32_t B);
-// the 32 x 32 inverses that a pivoted factor's substitution applies, into dInv, for
-// blocks of B (c->B from then on)
-hpl_status prep_solve_blocks(hpl_ctx* c, uint32_t B);
+// the 32 x 32 inverses that a pivoted factor's substitution applies, into dInv
+hpl_status prep_solve_blocks(hpl_ctx* c);
 // Rewrite a downloaded pivoted factor (host, row-major, lda) into gefa_ref's
 // layout: u_kk on the diagonal, each column's multipliers in the row order of
 // its own step.

@@ -112,12 +112,20 @@ __device__ __forceinline__ void block_gemv(const float* __restrict__ A, int64_t 
     }
 }
 
+// Where a block's 32 x 32 inverses lie: those of one type `type` floats after the
+// type before, those of one sub-block `sub` after the one before.  By panels
+// (launch_prep for blocks of B): type = B * 32, sub = 1024; prepared for blocks
+// of 32: type = 1024, sub = 3072.
+struct InvAt {
+    int type, sub;
+};
+
 // Solve the B x B diagonal system starting at Qoff for nr right-hand sides,
 // forward (unit lower) or backward (upper), in place in X.
 template <int NR, bool FWD>
 __device__ void diag_solve(const float* __restrict__ A, int64_t lda, int64_t Qoff, int B,
-                           const float* __restrict__ invT, float* __restrict__ X, int64_t ldx,
-                           int nr, float* ybuf, float* part, float* zbuf) {
+                           const float* __restrict__ invT, int sub, float* __restrict__ X,
+                           int64_t ldx, int nr, float* ybuf, float* part, float* zbuf) {
     constexpr int MAXB = gesl_cfg<NR>::MAXB;
     const int t = threadIdx.x;
     const int NQ = B / 32;
@@ -161,7 +169,7 @@ __device__ void diag_solve(const float* __restrict__ A, int64_t lda, int64_t Qof
             const int r = idx >> 5, ii = idx & 31;
             // y_s = X z with X^T stored: X[ii][j] = invT[j][ii]
             float y = 0.0f;
-            const float* Xs = invT + s * 1024;
+            const float* Xs = invT + (int64_t)s * sub;
 #pragma unroll 8
             for (int j = 0; j < 32; ++j) y = fmaf(Xs[j * 32 + ii], zbuf[r * 32 + j], y);
             ybuf[r * MAXB + 32 * s + ii] = y;
@@ -188,12 +196,11 @@ template <int NR>
 __global__ __launch_bounds__(NT) void gesl_fwd_kernel(const float* __restrict__ A, int64_t lda,
                                                       int64_t n, int B, int q,
                                                       const float* __restrict__ inv,
-                                                      int64_t inv_stride,
+                                                      int64_t inv_stride, InvAt at,
                                                       float* __restrict__ X, int64_t ldx, int nr) {
     constexpr int MAXB = gesl_cfg<NR>::MAXB, CH = gesl_cfg<NR>::CH;
     __shared__ gesl_smem<NR> sm;
     const int t = threadIdx.x;
-    const int NQ = B / 32;
     const int64_t qoff = (int64_t)q * B;
     if (q >= 0) {
         for (int idx = t; idx < nr * B; idx += NT) {
@@ -213,8 +220,8 @@ __global__ __launch_bounds__(NT) void gesl_fwd_kernel(const float* __restrict__ 
             }
             __syncthreads();
         }
-        diag_solve<NR, true>(A, lda, Q, B, inv + (int64_t)(q + 1) * inv_stride + NQ * 1024, X, ldx,
-                             nr, sm.ybuf, sm.part, sm.zbuf);
+        diag_solve<NR, true>(A, lda, Q, B, inv + (int64_t)(q + 1) * inv_stride + at.type, at.sub,
+                             X, ldx, nr, sm.ybuf, sm.part, sm.zbuf);
         return;
     }
     // entries [(q+2)B, n) in chunks of CH
@@ -227,12 +234,11 @@ template <int NR>
 __global__ __launch_bounds__(NT) void gesl_bwd_kernel(const float* __restrict__ A, int64_t lda,
                                                       int B, int q, int N,
                                                       const float* __restrict__ inv,
-                                                      int64_t inv_stride,
+                                                      int64_t inv_stride, InvAt at,
                                                       float* __restrict__ X, int64_t ldx, int nr) {
     constexpr int MAXB = gesl_cfg<NR>::MAXB, CH = gesl_cfg<NR>::CH;
     __shared__ gesl_smem<NR> sm;
     const int t = threadIdx.x;
-    const int NQ = B / 32;
     const int64_t qoff = (int64_t)q * B;
     if (q < N) {
         for (int idx = t; idx < nr * B; idx += NT) {
@@ -251,8 +257,8 @@ __global__ __launch_bounds__(NT) void gesl_bwd_kernel(const float* __restrict__ 
             }
             __syncthreads();
         }
-        diag_solve<NR, false>(A, lda, Q, B, inv + (int64_t)(q - 1) * inv_stride + 2 * NQ * 1024, X,
-                              ldx, nr, sm.ybuf, sm.part, sm.zbuf);
+        diag_solve<NR, false>(A, lda, Q, B, inv + (int64_t)(q - 1) * inv_stride + 2 * at.type,
+                              at.sub, X, ldx, nr, sm.ybuf, sm.part, sm.zbuf);
         return;
     }
     // entries [0, (q-1)B)
@@ -263,19 +269,20 @@ __global__ __launch_bounds__(NT) void gesl_bwd_kernel(const float* __restrict__ 
 
 template <int NR>
 hipError_t gesl_sweeps(const float* A, int64_t lda, int64_t n, int B, const float* inv,
-                       int64_t inv_stride, float* X, int64_t ldx, int nr, hipStream_t s) {
+                       int64_t inv_stride, InvAt at, float* X, int64_t ldx, int nr,
+                       hipStream_t s) {
     constexpr int CH = gesl_cfg<NR>::CH;
     if (B > gesl_cfg<NR>::MAXB) return hipErrorInvalidValue;
     const int N = (int)(n / B);
     for (int q = -1; q <= N - 2; ++q) {
         const int64_t rest = n - (int64_t)(q + 2) * B;
         const int grid = 1 + (q >= 0 ? (int)((rest + CH - 1) / CH) : 0);
-        gesl_fwd_kernel<NR><<<grid, NT, 0, s>>>(A, lda, n, B, q, inv, inv_stride, X, ldx, nr);
+        gesl_fwd_kernel<NR><<<grid, NT, 0, s>>>(A, lda, n, B, q, inv, inv_stride, at, X, ldx, nr);
     }
     for (int q = N; q >= 1; --q) {
         const int64_t rest = (int64_t)(q - 1) * B;
         const int grid = 1 + (q < N ? (int)((rest + CH - 1) / CH) : 0);
-        gesl_bwd_kernel<NR><<<grid, NT, 0, s>>>(A, lda, B, q, N, inv, inv_stride, X, ldx, nr);
+        gesl_bwd_kernel<NR><<<grid, NT, 0, s>>>(A, lda, B, q, N, inv, inv_stride, at, X, ldx, nr);
     }
     return hipGetLastError();
 }
@@ -825,7 +832,24 @@ hipError_t gesl_persist(const float* A, int64_t lda, int64_t n, int B, const flo
     return hipGetLastError();
 }
 
+// nr <= 16 right-hand sides by a launch per block step
+hipError_t gesl_steps(const float* A, int64_t lda, int64_t n, int B, const float* inv,
+                      int64_t inv_stride, InvAt at, float* X, int64_t ldx, int nr,
+                      hipStream_t s) {
+    return nr == 1   ? gesl_sweeps<1>(A, lda, n, B, inv, inv_stride, at, X, ldx, 1, s)
+           : nr <= 4 ? gesl_sweeps<4>(A, lda, n, B, inv, inv_stride, at, X, ldx, nr, s)
+                     : gesl_sweeps<16>(A, lda, n, B, inv, inv_stride, at, X, ldx, nr, s);
+}
+
 }  // namespace
+
+hipError_t launch_gesl_panels(const float* A, int64_t lda, int64_t n, int B, const float* inv,
+                              float* X, int64_t ldx, int nrhs, hipStream_t s) {
+    if (B > 256 || B < 32 || B % 32 || n % B || nrhs < 1 || nrhs > 16 ||
+        (nrhs > 1 && (ldx < n || ldx % 4)))
+        return hipErrorInvalidValue;
+    return gesl_steps(A, lda, n, B, inv, B / 32 * 3072, InvAt{1024, 3072}, X, ldx, nrhs, s);
+}
 
 hipError_t launch_gesl_multi(const float* A, int64_t lda, int64_t n, int B, const float* inv,
                              int64_t inv_stride, float* X, int64_t ldx, int nrhs, hipStream_t s,
@@ -837,8 +861,9 @@ hipError_t launch_gesl_multi(const float* A, int64_t lda, int64_t n, int B, cons
         const int nr = std::min(16, nrhs - r0);
         float* Xr = X + (int64_t)r0 * ldx;
         hipError_t e = hipSuccess;
-        const bool single = nr == 1 || (carry && nr <= kGeslSingleColumns);
-        const int64_t G = single && binv && ws && (lda & 3) == 0 ? persist_groups(n, B) : 0;
+        const int64_t G = nr <= gesl_single_columns(n, carry) && binv && ws && (lda & 3) == 0
+                              ? persist_groups(n, B)
+                              : 0;
         if (G > 0) {
             for (int r = 0; r < nr && e == hipSuccess; ++r) {
                 GeslWs w = *ws;
@@ -849,14 +874,10 @@ hipError_t launch_gesl_multi(const float* A, int64_t lda, int64_t n, int B, cons
             e = gesl_sweeps_mrhs(A, lda, n, B, binv, Xr, scratch, ldx, 1, true, s);
         else if (nr == 1 && binv && B <= 256)
             e = gesl_sweeps_split(A, lda, n, B, binv, Xr, s);
-        else if (nr == 1)
-            e = gesl_sweeps<1>(A, lda, n, B, inv, inv_stride, Xr, ldx, 1, s);
-        else if (binv && B <= 256)
+        else if (nr > 1 && binv && B <= 256)
             e = gesl_sweeps_mrhs(A, lda, n, B, binv, Xr, scratch, ldx, nr, carry, s);
-        else if (nr <= 4)
-            e = gesl_sweeps<4>(A, lda, n, B, inv, inv_stride, Xr, ldx, nr, s);
         else
-            e = gesl_sweeps<16>(A, lda, n, B, inv, inv_stride, Xr, ldx, nr, s);
+            e = gesl_steps(A, lda, n, B, inv, inv_stride, InvAt{B * 32, 1024}, Xr, ldx, nr, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -864,8 +885,8 @@ hipError_t launch_gesl_multi(const float* A, int64_t lda, int64_t n, int B, cons
 
 hipError_t launch_gesl(const float* A, int64_t lda, int64_t n, int B, const float* inv,
                        int64_t inv_stride, float* x, hipStream_t s, const float* binv,
-                       const GeslWs* ws, float* scratch, bool carry) {
-    return launch_gesl_multi(A, lda, n, B, inv, inv_stride, x, n, 1, s, binv, ws, scratch, carry);
+                       const GeslWs* ws) {
+    return launch_gesl_multi(A, lda, n, B, inv, inv_stride, x, n, 1, s, binv, ws);
 }
 
 int64_t gesl_persist_groups(int64_t n, int B) { return persist_groups(n, B); }

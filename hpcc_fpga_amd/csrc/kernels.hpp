@@ -124,24 +124,33 @@ int64_t gesl_persist_groups(int64_t n, int B);
 // or null for the sequential diagonal solve with the 32 x 32 inverses.  With
 // binv, one right-hand side and a workspace, the substitution is a single
 // persistent launch; otherwise two launches per block step.
-// carry (blocks of 32): sums over blocks carry their rounding errors along, which
-// the launches for several right-hand sides do in twice the scratch; they then
-// take one right-hand side too, where the single launch does not apply.
 hipError_t launch_gesl(const float* A, int64_t lda, int64_t n, int B, const float* inv,
                        int64_t inv_stride, float* x, hipStream_t s, const float* binv = nullptr,
-                       const GeslWs* ws = nullptr, float* scratch = nullptr, bool carry = false);
+                       const GeslWs* ws = nullptr);
 // nrhs right-hand sides, column r at X + r * ldx (ldx a multiple of 4, >= n);
 // blocks up to 256 for more than 4 right-hand sides.  Several right-hand sides
-// with binv need scratch: nrhs columns of the same leading dimension.  With carry
-// and a workspace, up to kGeslSingleColumns go one by one by the single launch,
-// which leaves column r's status at ws->status[r]: in blocks of 32 the launches
-// per block step take 0.4 ms a solve at n = 1024 and 3.5 at 9216, whatever the
-// count, a single launch 0.1 and 0.83.
-constexpr int kGeslSingleColumns = 4;
+// with binv need scratch: nrhs columns of the same leading dimension.
+// carry (blocks of 32): sums over blocks carry their rounding errors along, which
+// the launches for several right-hand sides do in twice the scratch; they then
+// take one right-hand side too, where the single launch does not apply.  With
+// carry and a workspace, up to gesl_single_columns go one by one by the single
+// launch, which leaves column r's status at ws->status[r]: in blocks of 32 the
+// launches per block step take 0.4 ms a solve at n = 1024 and 3.5 at 9216,
+// whatever the count, a single launch 0.1 and 0.83; at n = 64 two columns take
+// as long either way.
+constexpr int kGeslSingleColumns = 3;
+inline int gesl_single_columns(int64_t n, bool carry) {
+    return carry && n >= 128 ? kGeslSingleColumns : 1;
+}
 hipError_t launch_gesl_multi(const float* A, int64_t lda, int64_t n, int B, const float* inv,
                              int64_t inv_stride, float* X, int64_t ldx, int nrhs, hipStream_t s,
                              const float* binv = nullptr, const GeslWs* ws = nullptr,
                              float* scratch = nullptr, bool carry = false);
+
+// nrhs <= 16 right-hand sides by a launch per block of B <= 256 and its 32 x 32
+// inverses, as launch_prep_all writes those of blocks of 32
+hipError_t launch_gesl_panels(const float* A, int64_t lda, int64_t n, int B, const float* inv,
+                              float* X, int64_t ldx, int nrhs, hipStream_t s);
 
 // partial pivoting (pivot.hip); X is the transposed matrix X[i][j] = M(i, j)
 hipError_t launch_transpose_square(float* A, int64_t ld, int64_t n, hipStream_t s);

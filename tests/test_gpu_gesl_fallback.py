@@ -131,3 +131,29 @@ def test_without_whole_inverses(monkeypatch, n, B, prec, pivot, nrhs):
     if prec == "fp32":
         r0 = np.abs(b[:, 0] - M @ x0).max()
         assert r0 <= 64 * np.sqrt(n) * 2.0 ** -24 * (scale[0] + np.abs(b).max())
+
+
+@pytest.mark.parametrize("n,B", [(32, 32), (64, 32), (64, 64), (128, 64), (256, 128), (256, 256)])
+def test_few_panels(monkeypatch, n, B):
+    """Small pivoted factors are solved by a launch per panel block: no further off than
+    gesl_ref in FP32, whether or not there is room for whole inverses."""
+    print(f"few panels n={n} B={B}", flush=True)
+    g = np.random.default_rng(n + B)
+    a = (g.random((n, n)) - 0.5).astype(np.float32)
+    b = g.uniform(-1, 1, n).astype(np.float32)
+    x = []
+    for env in ({}, {"HPL_GESL_INVERSES": "0"}):
+        _env(monkeypatch, env)
+        with Context(0) as c:
+            c.set_pivoting(True)
+            c.upload(a, b)
+            c.gefa_dev(B)
+            c.gesl_dev()
+            x.append(c.download(matrix=False)[1])
+            f, _ = c.download(matrix=True, solution=False)
+            ipvt = c.pivots()
+    assert np.array_equal(x[0], x[1])
+    ref = np.linalg.solve(a.T.astype(np.float64), b.astype(np.float64))
+    seq = O.gesl_pvt(f, b.copy(), ipvt)
+    err = np.max(np.abs(x[0] - ref))
+    assert err <= 8 * max(np.max(np.abs(seq - ref)), 2.0 ** -24 * np.max(np.abs(ref)))
