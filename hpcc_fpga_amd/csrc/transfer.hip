@@ -52,11 +52,6 @@ void HostStage::Ring::free() {
     mem = nullptr;
 }
 
-hipError_t HostStage::make() {
-    const hipError_t e = small_.make();
-    return e == hipSuccess ? large_.make() : e;
-}
-
 hipError_t HostStage::to_device(hipStream_t s, void* dev, size_t dev_pitch, const void* host,
                                 size_t host_pitch, size_t width, size_t rows) {
     if (!width || !rows) return hipSuccess;

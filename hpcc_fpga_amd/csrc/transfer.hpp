@@ -36,8 +36,9 @@ class HostStage {
     // contiguous bytes
     hipError_t to_device(hipStream_t s, void* dev, const void* host, size_t bytes);
     hipError_t to_host(hipStream_t s, void* host, const void* dev, size_t bytes);
-    // all buffers at once, for who cannot fail later; free() gives them back
-    hipError_t make();
+    // the large buffers, which serve every size, for who cannot fail later (both
+    // sets cost a server of four slots 1.1 ms more); free() gives them back
+    hipError_t make() { return large_.make(); }
     void free() {
         small_.free();
         large_.free();
@@ -46,10 +47,10 @@ class HostStage {
    private:
     static constexpr int kBufs = 4;
     // Up to 64 KiB (status words, norms, vectors of small orders) through small
-    // buffers, so that only a context that moves more holds the 4 MiB of the
-    // large ones.  Those are 1 MiB each: packed in 30 us, on its way for 20 us;
-    // shorter pieces pay the launch of a copy, longer ones the wait for the first
-    // and last piece.
+    // buffers while there are no large ones, so that only a context that moves more
+    // holds their 4 MiB.  Those are 1 MiB each: packed in 30 us, on its way for 20
+    // us; shorter pieces pay the launch of a copy, longer ones the wait for the
+    // first and last piece.
     static constexpr size_t kSmall = 64u << 10, kLarge = 1u << 20;
     struct Ring {
         size_t bytes;  // of one buffer
@@ -59,7 +60,7 @@ class HostStage {
         hipError_t make();
         void free();
     };
-    Ring& ring(size_t bytes) { return bytes <= kSmall ? small_ : large_; }
+    Ring& ring(size_t bytes) { return bytes <= kSmall && !large_.mem ? small_ : large_; }
     Ring small_{kSmall}, large_{kLarge};
 };
 
