@@ -550,8 +550,8 @@ hipError_t gesl_sweeps_mrhs(const float* A, int64_t lda, int64_t n, int B, const
 // wait and only the round trip and the arithmetic stay on the critical path.
 // (With drained stores, a flag and then the values, three round trips a block:
 // n = 1024 B = 64 71 us, now 57; 2048 B = 128 81, 64; 7488 B = 64 435, 369; in
-// blocks of 32 n = 6144 680, 491; n = 32768 B = 256 1417, 1262, 65536 4.67 ms,
-// 4.12.)
+// blocks of 32 n = 6144 680, 491, and 446 with the pairwise sums of its shares;
+// n = 32768 B = 256 1417, 1262, 65536 4.67 ms, 4.12.)
 // ---------------------------------------------------------------------------
 constexpr int kMaxOwn = 16;            // slices per workgroup (LDS capacity)
 constexpr int kMaxT = 4;               // shares per block (B / S, B <= 256)

@@ -270,7 +270,8 @@ hpl_status hpl_batch_autotune(hpl_batch* batch, hpl_prec prec, int max_iter, dou
 hpl_status hpl_batch_set_blocked(hpl_batch* batch, int blocked);
 hpl_status hpl_batch_solve(hpl_batch* batch, hpl_prec prec, int max_iter, double tol_per_n,
                            hpl_batch_stats* stats);
-/* Refined solution (n doubles), corrections and backward error of system s. */
+/* Refined solution (n doubles), corrections and backward error of system s.
+ * Several threads may fetch from one batch at a time while none solves it. */
 hpl_status hpl_batch_get(hpl_batch* batch, int s, double* x, int* iterations, double* berr);
 /* The padded matrix (npad x npad, npad = n rounded up to 32) and right-hand
  * side (npad doubles) of system s as stored on the device. */
